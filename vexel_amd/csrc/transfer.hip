@@ -5,139 +5,10 @@
 // copies (and takes the page faults of) each on the calling thread: 32 MiB take 3.4 ms where the bus needs 0.6 ms.
 // Here the pieces go through a ring of pinned memory one behind the other, and a few threads of the backend copy
 // those that have arrived while later ones are on their way. Small uploads go through pinned memory without waiting.
-#include <string.h>
-
-#include <algorithm>
-#include <atomic>
-#include <condition_variable>
-#include <mutex>
-#include <thread>
-#include <vector>
-
 #include "common.h"
+#include "transfer_ring.h"
 
 namespace vx {
-
-struct Mover {
-    static constexpr int SLOTS = 16, MAX_WORKERS = 6;
-    static constexpr size_t SLOT = (size_t)1 << 20;
-    struct Piece {
-        char *dst;
-        const char *src;
-        size_t bytes;
-    };
-    struct Job {
-        std::vector<Piece> pieces;
-        std::vector<std::atomic<char>> copied;
-        std::atomic<int> next{0}, arrived{0};
-        std::atomic<bool> failed{false};
-        explicit Job(std::vector<Piece> p) : pieces(std::move(p)), copied(pieces.size()) {
-            for (auto &c : copied) c.store(0);
-        }
-    };
-    char *ring = nullptr;
-    hipEvent_t events[SLOTS] = {};
-    std::vector<std::thread> workers;
-    std::mutex call, mu;  // one transfer at a time; the fields below
-    std::condition_variable wake, left;
-    Job *job = nullptr;
-    uint64_t turn = 0;
-    int inside = 0;
-    bool stop = false;
-
-    ~Mover() {
-        {
-            std::lock_guard<std::mutex> g(mu);
-            stop = true;
-        }
-        wake.notify_all();
-        for (auto &t : workers) t.join();
-        for (hipEvent_t e : events)
-            if (e) (void)hipEventDestroy(e);
-        if (ring) (void)hipHostFree(ring);
-    }
-    bool start() {
-        if (hipHostMalloc((void **)&ring, SLOTS * SLOT, hipHostMallocDefault) != hipSuccess) {
-            ring = nullptr;
-            return false;
-        }
-        for (hipEvent_t &e : events)
-            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                e = nullptr;
-                return false;
-            }
-        const int n = std::min<int>(MAX_WORKERS, std::max(1u, std::thread::hardware_concurrency()) - 1);
-        try {
-            for (int i = 0; i < n; i++) workers.emplace_back([this] { work(); });
-        } catch (...) {  // (fewer threads, or none: the caller copies as well)
-        }
-        return true;
-    }
-    // Takes pieces as they arrive until none is left.
-    void run(Job &j) {
-        const int n = (int)j.pieces.size();
-        for (;;) {
-            const int i = j.next.fetch_add(1);
-            if (i >= n) return;
-            while (j.arrived.load(std::memory_order_acquire) <= i) {
-                if (j.failed.load()) return;
-                std::this_thread::yield();
-            }
-            memcpy(j.pieces[i].dst, ring + (size_t)(i % SLOTS) * SLOT, j.pieces[i].bytes);
-            j.copied[i].store(1, std::memory_order_release);
-        }
-    }
-    void work() {
-        uint64_t seen = 0;
-        std::unique_lock<std::mutex> l(mu);
-        for (;;) {
-            wake.wait(l, [&] { return stop || (job && turn != seen); });
-            if (stop) return;
-            seen = turn;
-            Job *j = job;
-            inside++;
-            l.unlock();
-            run(*j);
-            l.lock();
-            if (--inside == 0) left.notify_all();
-        }
-    }
-    // Everything before on the stream is done when this returns.
-    hipError_t move(hipStream_t stream, Job &j) {
-        const int n = (int)j.pieces.size();
-        hipError_t err = hipSuccess;
-        int sent = 0;
-        for (int got = 0; got < n && err == hipSuccess; got++) {
-            while (sent < n && err == hipSuccess) {
-                if (sent >= SLOTS) {  // the slot's last piece has to be out of it
-                    while (sent == got && !j.copied[sent - SLOTS].load(std::memory_order_acquire)) std::this_thread::yield();
-                    if (!j.copied[sent - SLOTS].load(std::memory_order_acquire)) break;
-                }
-                const Piece &p = j.pieces[sent];
-                err = hipMemcpyAsync(ring + (size_t)(sent % SLOTS) * SLOT, p.src, p.bytes, hipMemcpyDeviceToHost, stream);
-                if (err == hipSuccess) err = hipEventRecord(events[sent % SLOTS], stream);
-                sent++;
-            }
-            if (err == hipSuccess) err = hipEventSynchronize(events[got % SLOTS]);
-            if (err != hipSuccess) break;
-            j.arrived.store(got + 1, std::memory_order_release);
-            if (got == 0) {  // (the threads sleep through the work that the first piece waits for)
-                {
-                    std::lock_guard<std::mutex> g(mu);
-                    job = &j;
-                    turn++;
-                }
-                wake.notify_all();
-            }
-        }
-        if (err != hipSuccess) j.failed.store(true);
-        else run(j);
-        std::unique_lock<std::mutex> l(mu);
-        job = nullptr;
-        left.wait(l, [&] { return inside == 0; });
-        return err;
-    }
-};
 
 void mover_destroy(Mover *m) { delete m; }
 
@@ -179,7 +50,7 @@ static int download(vx_backend *be, int n, void *const *dst, const void *const *
         std::lock_guard<std::mutex> g(be->stage_mu);
         if (!be->mover) {
             be->mover = new Mover();
-            if (!be->mover->start()) {
+            if (!be->mover->start(std::min<int>(Mover::MAX_WORKERS, std::max(1u, std::thread::hardware_concurrency()) - 1))) {
                 delete be->mover;
                 be->mover = nullptr;
                 (void)hipGetLastError();
