@@ -172,6 +172,83 @@ def test_matmul_packed_with_scales_at_their_limits(be, fmt, m, kind):
     be.reset_pool()
 
 
+def _balanced_k_quant(rng, fmt, n, k):
+    """Weights as quantizing zero-mean ones gives them: codes bell-shaped about the middle, minima that take the middle off."""
+    sb = (n, k // 256)
+    b = rng.integers(0, 256, sb + (nx.BLOCK_BYTES[fmt],), dtype=np.uint8)
+    d = (0.0005 * (1 + rng.random(sb + (1,)))).astype(np.float16)
+    if fmt == nx.FMT_Q6_K:
+        b[..., 208:210] = d.view(np.uint8)
+        q = np.clip(np.rint(32 + 9 * rng.standard_normal(sb + (2, 4, 32))), 0, 63).astype(np.uint8)
+        b[..., 0:128] = ((q[..., 0:2, :] & 15) | (q[..., 2:4, :] & 15) << 4).reshape(sb + (128,))
+        h = q >> 4
+        b[..., 128:192] = (h[..., 0, :] | h[..., 1, :] << 2 | h[..., 2, :] << 4 | h[..., 3, :] << 6).reshape(sb + (64,))
+        b[..., 192:208] = (rng.integers(64, 128, sb + (16,)) * rng.choice([-1, 1], sb + (16,))).astype(np.int8).view(np.uint8)
+        return b.reshape(n, -1)
+    wide = fmt == nx.FMT_Q5_K
+    b[..., 0:2], b[..., 2:4] = d.view(np.uint8), (d * np.float16(15.5 if wide else 7.5)).view(np.uint8)
+    s = rng.integers(32, 64, sb + (8,)).astype(np.uint8)
+    b[..., 4:8] = b[..., 8:12] = (s[..., :4] & 63) | (s[..., 4:] >> 4) << 6
+    b[..., 12:16] = (s[..., 4:] & 15) | (s[..., 4:] & 15) << 4
+    z = rng.standard_normal(sb + (8, 32))
+    q = np.clip(np.rint(15.5 + 7 * z if wide else 7.5 + 3.5 * z), 0, 31 if wide else 15).astype(np.uint8)
+    b[..., 16 + 32 * wide:] = ((q[..., 0::2, :] & 15) | (q[..., 1::2, :] & 15) << 4).reshape(sb + (128,))
+    if wide:
+        b[..., 16:48] = np.bitwise_or.reduce((q >> 4) << np.arange(8, dtype=np.uint8)[:, None], axis=-2)
+    return b.reshape(n, -1)
+
+
+def _exact_k_quant(fmt, w, n, k):
+    """The weights in float64 (gguf.Dequantize rounds d * sc * q - dmin * m to float32)."""
+    sb = (n, k // 256)
+    b = w.reshape(sb + (-1,))
+    half = lambda x: np.ascontiguousarray(x).view(np.float16).astype(np.float64)
+    if fmt == nx.FMT_Q6_K:
+        q = np.empty(sb + (2, 4, 32))
+        lo, hi = b[..., 0:128].reshape(sb + (2, 2, 32)), b[..., 128:192].reshape(sb + (2, 1, 32))
+        q[..., 0:2, :], q[..., 2:4, :] = lo & 15, lo >> 4
+        q += (((hi >> np.array([0, 2, 4, 6], dtype=np.uint8)[:, None]) & 3) << 4) - 32.0
+        sc = np.ascontiguousarray(b[..., 192:208]).view(np.int8).astype(np.float64)
+        return (half(b[..., 208:210])[..., None] * sc[..., None] * q.reshape(sb + (16, 16))).reshape(n, k)
+    wide = fmt == nx.FMT_Q5_K
+    s = b[..., 4:16].astype(np.int64)
+    sc = np.concatenate([s[..., 0:4] & 63, (s[..., 8:12] & 15) | (s[..., 0:4] >> 6) << 4], -1)
+    mn = np.concatenate([s[..., 4:8] & 63, (s[..., 8:12] >> 4) | (s[..., 4:8] >> 6) << 4], -1)
+    qs = b[..., 16 + 32 * wide:].reshape(sb + (4, 32))
+    q = np.stack([qs & 15, qs >> 4], axis=-2).reshape(sb + (8, 32)).astype(np.float64)
+    if wide:
+        q += ((b[..., None, 16:48] >> np.arange(8, dtype=np.uint8)[:, None]) & 1) * 16.0
+    return (half(b[..., 0:2])[..., None] * sc[..., None] * q - half(b[..., 2:4])[..., None] * mn[..., None]).reshape(n, k)
+
+
+# Relative error (2-norm) of the products against float64, in 1e-7, for one row, for 2 .. 64 rows and for more: what kernels leave that
+# put d * sc on every block's own sum and take the minima off block by block, the largest measured on these matrices (2.87, 2.58 and 2.60;
+# 5.27, 2.56 and 2.67; 5.20, 1.05 and 1.25), and 1 to 5 % for the seed. With the scales in the operands no precision is given away.
+ROUNDING = {nx.FMT_Q4_K: (2.9, 2.7, 2.73), nx.FMT_Q5_K: (5.4, 2.7, 2.8), nx.FMT_Q6_K: (5.3, 1.1, 1.3)}
+
+
+# both ends of the streaming kernel and of its four-tile form; 65 and more rows in few and in many slices of K
+@pytest.mark.parametrize("n,k", [(2048, 2048), (512, 4096)])
+@pytest.mark.parametrize("m", [2, 32, 33, 64, 65, 200])
+@pytest.mark.parametrize("fmt", [nx.FMT_Q4_K, nx.FMT_Q5_K, nx.FMT_Q6_K])
+def test_scales_in_the_operands_round_no_more_than_scales_on_the_sums(be, fmt, m, n, k):
+    rng = np.random.default_rng(1000 * fmt + m + k)
+    w = _balanced_k_quant(rng, fmt, n, k)
+    deq = _exact_k_quant(fmt, w, n, k)
+    a = rng.standard_normal((max(m, 24 // m * m), k)).astype(np.float32)  # (24 rows at least: the error of one scatters)
+    dw, _ = _packed(be, w, n, k, fmt)
+    got = np.empty((len(a), n), dtype=np.float32)
+    for r in range(0, len(a), m):
+        da, dout = be.upload(a[r:r + m]), be.alloc(m * n * 4)
+        be.matmul_quant(fmt, da, dw, dout, None, m, n, k)
+        got[r:r + m] = be.download(dout, (m, n), np.float32)
+    want = a.astype(np.float64) @ deq.T
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    be.free(dw)
+    be.reset_pool()
+    assert err <= ROUNDING[fmt][0 if m == 1 else 1 if m <= 64 else 2] * 1e-7, err
+
+
 @pytest.mark.parametrize("fmt", FMTS)
 def test_matmul_packed_many_rows_independent_of_batch(be, fmt):
     """A row has the same bits in any batch with the same number of 64-row groups (the K slicing depends on that
