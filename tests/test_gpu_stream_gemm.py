@@ -229,7 +229,7 @@ ROUNDING = {nx.FMT_Q4_K: (2.9, 2.7, 2.73), nx.FMT_Q5_K: (5.4, 2.7, 2.8), nx.FMT_
 
 # both ends of the streaming kernel and of its four-tile form; 65 and more rows in few and in many slices of K
 @pytest.mark.parametrize("n,k", [(2048, 2048), (512, 4096)])
-@pytest.mark.parametrize("m", [2, 32, 33, 64, 65, 200])
+@pytest.mark.parametrize("m", [1, 2, 32, 33, 64, 65, 200])
 @pytest.mark.parametrize("fmt", [nx.FMT_Q4_K, nx.FMT_Q5_K, nx.FMT_Q6_K])
 def test_scales_in_the_operands_round_no_more_than_scales_on_the_sums(be, fmt, m, n, k):
     rng = np.random.default_rng(1000 * fmt + m + k)

@@ -789,15 +789,22 @@ __device__ __forceinline__ void mv3_dots(const uint32_t (&lo)[4], const uint32_t
     tb = b[0] + (b[1] << 8) + (b[2] << 16);
 }
 // The scales and minima of sub-blocks 2 g and 2 g + 1 (getScaleMinK4, dequant.go:400-409) from the head of a super-block, and
-// d (sc0 ta + sc1 tb) - dmin (mn0 s0 + mn1 s1).
+// d (sc0 ta + sc1 tb) - dmin (mn0 s0 + mn1 s1). The sums enter less CENTER times the activation's, exact integers, and the minima
+// less what that leaves out: the two parts, which otherwise are twice the result's size and cancel, round at its size
+// (16384 x 2048 of Q4_K, relative error against float64: 2.9e-7 for the parts as they stand, 2.6e-7 so, 2.8e-7 in the first form;
+// 22016 x 4096 14.0 -> 14.5 us, 4096 x 4096 the same).
+template <int CENTER>
 __device__ __forceinline__ float mv3_k_value(mv_u32x4 h, int g, int ta, int tb, const uint32_t (&x)[MV2_XSTRIDE]) {
     const int sh = 16 * (g & 1);
     const uint32_t w0 = h[1] >> sh, w1 = h[2] >> sh, w2 = h[3] >> sh;
     const uint32_t sc = g < 2 ? w0 & 0x3F3Fu : (w2 & 0x0F0Fu) | ((w0 >> 2) & 0x3030u);
     const uint32_t mn = g < 2 ? w1 & 0x3F3Fu : ((w2 >> 4) & 0x0F0Fu) | ((w1 >> 2) & 0x3030u);
-    const float fs = fmaf((float)(sc & 0xFF), (float)ta, (float)(sc >> 8 & 0xFF) * (float)tb);
-    const float fm = fmaf((float)(mn & 0xFF), (float)(int)x[24], (float)(mn >> 8 & 0xFF) * (float)(int)x[25]);
-    return fmaf(h2f((uint16_t)(h[0] & 0xFFFF)), fs, -(h2f((uint16_t)(h[0] >> 16)) * fm)) * __uint_as_float(x[26]);
+    const float d = h2f((uint16_t)(h[0] & 0xFFFF)), dm = h2f((uint16_t)(h[0] >> 16));
+    const float d0 = d * (float)(sc & 0xFF), d1 = d * (float)(sc >> 8 & 0xFF);  // (exact, as are dm's products)
+    const float c0 = fmaf((float)CENTER, d0, -(dm * (float)(mn & 0xFF))), c1 = fmaf((float)CENTER, d1, -(dm * (float)(mn >> 8 & 0xFF)));
+    const int s0 = (int)x[24], s1 = (int)x[25];
+    const float a = fmaf(d0, (float)(ta - CENTER * s0), c0 * (float)s0), b = fmaf(d1, (float)(tb - CENTER * s1), c1 * (float)s1);
+    return (a + b) * __uint_as_float(x[26]);
 }
 struct K3_Q4_0 {
     static constexpr int BYTES = 18, SHARES = 1, BITS = 23, APART = 16;
@@ -855,7 +862,7 @@ struct K3_Q4_K {  // share: low and high nibbles of qs[32 g + 16 h .. + 15], g =
         for (int i = 0; i < 4; i++) lo[i] = w.c[i] & 0x0F0F0F0Fu, hi[i] = (w.c[i] >> 4) & 0x0F0F0F0Fu;
         int ta, tb;
         mv3_dots(lo, hi, x, ta, tb);
-        return mv3_k_value(w.h, share >> 1, ta, tb, x);
+        return mv3_k_value<8>(w.h, share >> 1, ta, tb, x);
     }
 };
 struct K3_Q5_K {  // as Q4_K; bit 2 g (2 g + 1) of qh[16 h + i] is the fifth bit of a low (high) nibble
@@ -878,7 +885,7 @@ struct K3_Q5_K {  // as Q4_K; bit 2 g (2 g + 1) of qh[16 h + i] is the fifth bit
         }
         int ta, tb;
         mv3_dots(lo, hi, x, ta, tb);
-        return mv3_k_value(w.h, g, ta, tb, x);
+        return mv3_k_value<16>(w.h, g, ta, tb, x);
     }
 };
 struct K3_Q6_K {  // share (n, a, h): low and high nibbles of ql[64 n + 32 a + 16 h ..], bits 2 a and 4 + 2 a of qh[32 n + 16 h ..]
@@ -1238,7 +1245,7 @@ int launch_fmt(vx_backend *be, int fmt, MvArgs &a) {
         VX_CHECK_LAUNCH();
         return VX_OK;
     }
-    // (K-quants: faster at every size measured, 2048 x 2048 to 32000 x 4096: Q4_K 22016 x 4096 20.1 -> 14.1 us, 4096 x 11008
+    // (K-quants: faster at every size measured, 2048 x 2048 to 32000 x 4096: Q4_K 22016 x 4096 20.1 -> 14.5 us, 4096 x 11008
     // 16.0 -> 10.4, 2048 x 5632 8.2 -> 4.8; Q6_K 24.4 -> 22.3, 18.8 -> 14.2, 9.7 -> 5.6; Q5_K 23.2 -> 16.9, 18.0 -> 11.5)
     if ((fmt == VX_Q4_K && launch_third_form<K3_Q4_K>(be, a)) || (fmt == VX_Q5_K && launch_third_form<K3_Q5_K>(be, a)) ||
         (fmt == VX_Q6_K && launch_third_form<K3_Q6_K>(be, a))) {
