@@ -1127,6 +1127,30 @@ def test_paged_multiquery_pairs_of_blocks(be, hq, hk, d, qn, keys):
     be.reset_pool()
 
 
+# the pairs of a row tile in four, two and one shares; the token in the second block of the first and of the last pair
+@pytest.mark.parametrize("hq,hk,d,qn", [(8, 2, 128, 64), (4, 4, 64, 64), (64, 4, 64, 256), (64, 8, 128, 512)])
+@pytest.mark.parametrize("pair", [0, -1])
+def test_paged_multiquery_value_that_is_not_finite(be, hq, hk, d, qn, pair):
+    """A later row's value that overflowed f16 stays out of the row tiles that end before its block."""
+    rng = np.random.default_rng(qn + pair)
+    bs, nb = 16, qn // 16
+    bt = rng.permutation(nb).astype(np.int32)
+    pool = _make_pool(rng, True, nb, bs, hk, d).reshape(nb, 2, bs, hk, d)
+    block = 2 * (pair % (nb // 2)) + 1
+    q = rng.standard_normal((qn, hq, d)).astype(np.float32)
+    kvl = np.arange(1, qn + 1, dtype=np.int32)
+    dq, dbt, dk, out = be.upload(q), be.upload(bt), be.upload(kvl), []
+    for value in (None, np.inf):
+        if value is not None:
+            pool[bt[block], 1, 4] = np.float16(value).view(np.uint16)
+        do = be.alloc(q.nbytes)
+        be.sdpa_paged_decode_multiquery(dq, be.upload(pool.reshape(-1)), dbt, do, dk, nb, bs, hq, hk, d, np.float32(1 / math.sqrt(d)), qn, pool_is_f16=True)
+        out.append(be.download(do, q.shape, np.float32))
+    assert np.isfinite(out[0]).all()
+    assert np.array_equal(out[0][:16 * block], out[1][:16 * block]) and not np.isfinite(out[1][16 * block + 4:]).any()
+    be.reset_pool()
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])

@@ -879,6 +879,7 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
     }
     constexpr int PT = 2 * HOT_BS;  // tokens of a pair of blocks
     const int n_pairs = idle ? 0 : (len_max + PT - 1) / PT;
+    const int len_top = __builtin_amdgcn_readfirstlane(len_max);
     const int tok_row = 4 * (c16 & 3) + (c16 >> 2);  // this lane's K row of a block as A operand
     constexpr int KP = D + 8;                        // halves per staged row (rows 4 banks apart)
     // [share][buffer][K, V][row of the pair]; behind the loop the shares' outputs lie there
@@ -907,9 +908,12 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                 for (int b = 0; b < 2; b++) sc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk[b], ql[t][s], sc[t][b], 0, 0, 0);
             }
         }
+        // A second block that none of the wave's rows sees has weights of 0 only, but a value there may be infinite: the first block's
+        // values once more then.
+        const _Float16 *const vs2 = vs + ((2 * pi + 1) * HOT_BS < len_top ? HOT_BS * KP : 0);
         halfv vv[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) vv[i] = *(const halfv *)&vs[((i >> 2) * HOT_BS + 4 * (i & 3) + g4) * KP + c16 * NT];
+        for (int i = 0; i < 8; i++) vv[i] = *(const halfv *)&(i < 4 ? vs : vs2)[(4 * (i & 3) + g4) * KP + c16 * NT];
 #pragma unroll
         for (int t = 0; t < QT; t++) {
             float sv[8], gm = -INFINITY;
