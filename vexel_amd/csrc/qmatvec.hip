@@ -23,6 +23,7 @@
 //     exchange, the four waves through LDS, in a fixed order.
 #include "common.h"
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 using namespace vx;
@@ -1085,13 +1086,17 @@ bool launch_third_form(vx_backend *be, MvArgs &a) {
                          (a.rope.head_dim & (a.rope.head_dim - 1)) != 0 || ((uintptr_t)a.rope.q_out & 7) != 0))
         return false;
     a.row_bytes = (size_t)(a.K / (32 * F::SHARES)) * F::BYTES;
-    static int attr = 0;
-    if (attr == 0) {
-        (void)hipFuncSetAttribute((const void *)qmatvec3_kernel<F>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-        attr = 1;
+    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_kernel<F>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    (void)attr;
+    // workgroups a compute unit holds, asked for once per length of the row (backends may call from several threads)
+    constexpr int LONGEST = 120 * 1024 / (MV2_XSTRIDE * 4);
+    static std::atomic<int> resident[LONGEST + 1];
+    std::atomic<int> &known = resident[a.K / 32];
+    int per_cu = known.load(std::memory_order_relaxed);
+    if (per_cu == 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, qmatvec3_kernel<F>, MV_THREADS, lds) != hipSuccess || per_cu < 1) per_cu = 1;
+        known.store(per_cu, std::memory_order_relaxed);
     }
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, qmatvec3_kernel<F>, MV_THREADS, lds) != hipSuccess || per_cu < 1) per_cu = 1;
     const int n_passes = a.pair > 0 ? a.pair : ceil_div(a.N, 2);
     // as many workgroups as fit at once, or fewer when that makes every wave's number of passes equal
     const int wgs = ceil_div(n_passes, MV_WAVES), trips = ceil_div(wgs, per_cu * device_cus(be));
