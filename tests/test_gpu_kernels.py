@@ -603,8 +603,13 @@ def test_single_row_qkv_finishes_its_rows(be, fqk, fv):
     for name, out in (("wq", dq), ("wk", dk), ("wv", dv)):
         be.matmul_quant(fm[name], dnorm, dW[name], out, None, 1, dims[name][0], hidden)
     be.rope_store_paged(dq, dk, dv, dpos, dslots, dpool, True, 1, hq, hk, d, bs, theta)
+    dpeak = be.upload(np.eye(1, 16, 7, dtype=np.float32))
     be.rope_table_prepare(dpos, 1, d, theta)
+    # The launches that leave the rows to a kernel behind them take the position from its buffer, the others the table: another
+    # position there now (by a kernel, not by a copy, which would end the table) tells them apart.
+    be.argmax_rows(dpeak, 1, 16, dpos)
     be.decode_attn_qkv(dx, dn1, eps, False, qw["wq"], qw["wk"], qw["wv"], 1, dpos, dslots, dpool2, True, hq, hk, d, bs, theta, dq2)
+    assert be.download(dpos, (1,), np.int32)[0] == 7
     q_ref, q = be.download(dq, (hidden,), np.float32), be.download(dq2, (hidden,), np.float32)
     assert np.all(np.abs(q - q_ref) <= 2e-5 * np.abs(q_ref).max() + 1e-6)
     ref, got = (nx.f16_to_f32_array(be.download(p, pool.shape, pool.dtype)) for p in (dpool, dpool2))
