@@ -604,15 +604,24 @@ template <typename T, int MT, int NT, int WAVES, int KIND>
 void launch_few_as(vx_backend *be, const LinArgs &p, int slices) {
     linear_few_kernel<T, MT, NT, WAVES, KIND, false><<<dim3((p.n >> 4) / NT, slices, p.o.groups), 64 * WAVES, 0, be->stream>>>(p);
 }
-// The kernel that holds its activations: more than 16 rows (16 rows: 13312 x 2048 15.7 us against 13.7, but 32000 x 2048 24.5 against
-// 27.5 and gate|up of 11264 x 2048 12.9 against 13.7), more than 1024 inputs to a slice (32 rows: 2048 x 4096 in eight slices
+int compute_units(vx_backend *be) {
+    static const int cus = [&] {
+        int n = 0;
+        return (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, be->device) == hipSuccess && n > 0) ? n : 256;
+    }();
+    return cus;
+}
+
+// The kernel that holds its activations: more than 16 rows (at 16 the maps it would serve are not told apart by their size: 13312 x 2048
+// is slower with it, 15.7 us against 13.7, 32000 x 2048 and gate|up of 11264 x 2048 are faster, 24.5 against 27.5 and 12.9
+// against 13.7; it is not built for them), more than 1024 inputs to a slice (32 rows: 2048 x 4096 in eight slices
 // 6.5 us against 7.0, 8192 x 128 3.7 against 4.5) and no more to a wave than its registers hold. 32 and 64 rows: 13312 x 2048
 // 22.7 -> 15.7 and 37 -> 20 us, gate|up 17.5 -> 15.5 and 24 -> 20, 32000 x 2048 34 -> 29 and 73 -> 35.
 template <int MT, int KIND>
 bool launch_hold(vx_backend *be, const LinArgs &p, int slices) {
     const int per_wave = ceil_div(ceil_div(p.k >> 5, slices), 8), units = (p.n >> 4) / (KIND == VX_LIN_SWIGLU ? 2 : 1);
     if (per_wave <= 4 || per_wave > (MT == 4 ? 8 : 16)) return false;
-    const dim3 grid(std::max(1, std::min(units, 256 / (slices * p.o.groups))), slices, p.o.groups);
+    const dim3 grid(std::max(1, std::min(units, compute_units(be) / (slices * p.o.groups))), slices, p.o.groups);
     if (per_wave <= 8)
         linear_hold_kernel<MT, 8, KIND><<<grid, 512, 0, be->stream>>>(p);
     else if constexpr (MT < 4)
@@ -645,14 +654,14 @@ void launch_many(vx_backend *be, const LinArgs &p, int slices) {
 }
 
 // The tile whose launch is the shortest: the first workgroup of every compute unit takes `first`, each further one `more`, in
-// microseconds per 2048 inputs as measured over 65 .. 4096 rows of 2048 .. 13312 outputs (2048 x 11264 x 2048: 128 x 256 89 us,
+// tenths of a microsecond per 2048 inputs as measured over 65 .. 4096 rows of 2048 .. 13312 outputs (2048 x 11264 x 2048: 128 x 256 89 us,
 // 128 x 128 116, 64 x 128 161; 2048 x 2048 x 5632: 79, 61, 83; 128 x 11264 x 2048: 34, 25, 21 and 21 for 64 x 64).
-void many_tile(int n, int rows, int slices, bool wide, int *bm, int *bn) {
+void many_tile(int n, int rows, int slices, bool wide, int cus, int *bm, int *bn) {
     const struct { int bm, bn, first, more; } tiles[] = {{128, 256, 330, 270}, {128, 128, 245, 190}, {64, 128, 200, 120}, {64, 64, 156, 80}};
     int64_t best = INT64_MAX;
     for (const auto &t : tiles) {
         if (t.bn == 256 && !wide) continue;
-        const int64_t wgs = (int64_t)ceil_div(rows, t.bm) * ceil_div(n, t.bn) * slices, cost = t.first + t.more * ((wgs + 255) / 256 - 1);
+        const int64_t wgs = (int64_t)ceil_div(rows, t.bm) * ceil_div(n, t.bn) * slices, cost = t.first + t.more * ((wgs + cus - 1) / cus - 1);
         if (cost < best) best = cost, *bm = t.bm, *bn = t.bn;
     }
 }
@@ -689,7 +698,7 @@ int launch(vx_backend *be, const LinArgs &p, int slices) {
         // (a map that writes a transcendental of each product and has few inputs is bound by that: its workgroups overlap better
         // in two rounds than in one, 2048 x 8192 x 128 33.7 us against 24.3)
         constexpr bool WIDE = KIND != VX_LIN_SOFTPLUS;
-        many_tile(p.n, p.rows, slices * p.o.groups, WIDE, &bm, &bn);
+        many_tile(p.n, p.rows, slices * p.o.groups, WIDE, compute_units(be), &bm, &bn);
         if constexpr (sizeof(T) == 4) {
             launch_many<T, 64, 64, KIND>(be, p, slices);
         } else if (bn == 64) {
@@ -748,7 +757,7 @@ int launch_experts(vx_backend *be, const LinArgs &p, int step_rows, int max_tile
             // (the wide tile where it surely leaves every compute unit a workgroup: an expert's last tile may be short, so up to
             // `experts` of the tiles are. 8 experts of 8192 x 4096, 2 of them per row, 2048 rows: 427 -> 314 us;
             // 64 of 2816 x 2048, 6 per row: 277 -> 197)
-            if ((int64_t)(max_tiles - p.experts) * ceil_div(n, 256) >= 256)
+            if ((int64_t)(max_tiles - p.experts) * ceil_div(n, 256) >= compute_units(be))
                 launch_many_experts<T, 128, 256, KIND>(be, p, step_rows, max_tiles);
             else
                 launch_many_experts<T, 128, 128, KIND>(be, p, step_rows, max_tiles);
