@@ -117,7 +117,7 @@ def test_linear_held_activations(be, kind, rows, n, k):
 def test_linear_wide_tiles(be, kind, n, rows, k):
     """Products large enough for tiles of 128 rows x 256 outputs (a last tile of six and two rows short of a tile and 96 and
     32 outputs; one to three steps of the inputs): the first 65 rows are bit for bit those of a step of 65 rows, whose tiles
-    are 64 x 64, and the plain map is the product."""
+    are narrower, and the plain map is the product."""
     rng = np.random.default_rng(n + k + kind)
     w = lz.bf16_round(rng.standard_normal((n, k)) / 8)
     p, n_pad, k_pad = packed(be, w)
@@ -145,6 +145,76 @@ def test_linear_wide_tiles(be, kind, n, rows, k):
         p, _, _ = packed(be, w)
     for x, y in zip(*res):
         assert np.isfinite(x).all() and np.any(x != 0) and np.array_equal(x, y)
+
+
+FORMS = ["rotary", "silu", "forget", "softplus", "relu2", "groups", "a_rows", "softcap", "mult"]
+
+
+# (rows, the rows of the older kernel's step): activations held, two and four tiles of 16 rows, 5 and 8 steps to a wave; the tile of 128
+# x 256 (softplus: the widest that kind has), with a short last tile, against narrower ones
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("n,k,rows,few", [(2080, 1088, 20, 16), (96, 1984, 33, 16), (2080, 1984, 64, 16), (8544, 192, 1030, 65)])
+def test_linear_kinds_by_held_activations_and_wide_tiles(be, form, n, k, rows, few):
+    """Every kind of result and every way to take the activations by the kernels of many outputs: the product in float64, and the
+    first rows bit for bit those of a step that the older kernels take."""
+    rng = np.random.default_rng(n + k + rows)
+    sg = lambda x: 1.0 / (1.0 + np.exp(-x))
+    groups = 2 if form == "groups" else 1
+    w, a = lz.bf16_round(rng.standard_normal((groups * n, k)) / np.sqrt(k) * 2), grid(rng.standard_normal((rows, groups * k)), BF16)
+    y = np.concatenate([a[:, g * k:(g + 1) * k].astype(np.float64) @ w[g * n:(g + 1) * n].T.astype(np.float64) for g in range(groups)], 1)
+    split, f32 = n // 64 * 32, form in ("softplus", "groups", "softcap")
+    bias, keep = rng.standard_normal(n).astype(np.float32), rng.choice([0.0, 0.02, 0.5, 1.0], n).astype(np.float32)
+    ang, order = rng.uniform(-3, 3, (rows, 5)), rng.permutation(rows).astype(np.int32)
+    cols, rest, want = groups * n, None, y
+    if form in ("rotary", "silu", "forget"):
+        cols, rest, want = split, y[:, split:], y[:, :split].copy()
+        if form == "rotary":
+            h = want.reshape(rows, -1, 32)
+            u, v, c, s = h[..., 8:18:2].copy(), h[..., 9:18:2].copy(), np.cos(ang)[:, None], np.sin(ang)[:, None]
+            h[..., 8:18:2], h[..., 9:18:2] = u * c - v * s, v * c + u * s
+        else:
+            silu = split if form == "silu" else 16
+            want[:, :silu] *= sg(want[:, :silu])
+            if form == "forget":
+                rest = keep[:n - split] * sg(-(rest + bias[:n - split]))
+    elif form == "softplus":
+        want = lz.softplus(y + bias)
+    elif form == "relu2":
+        want = np.maximum(y + bias, 0) ** 2
+    elif form == "softcap":
+        want = 1.5 * np.tanh(y / 1.5)
+    elif form == "mult":
+        want = 0.37 * y
+    res = []
+    for r in (rows, few):
+        p, n_pad, k_pad = packed(be, w)
+        assert (n_pad, k_pad) == (groups * n, k)
+        out, out2 = blank(be, (r, cols), F32 if f32 else BF16), blank(be, (r, n - split), F32)
+        kw = dict(kind={"rotary": 5, "silu": 7, "forget": 8, "softplus": 4, "relu2": 9}.get(form, 0), out=out, ldo=cols, cols=cols, out_f32=int(f32))
+        if rest is not None:
+            kw.update(split=split, out2=out2, ldo2=n - split, silu_cols=16, bias=be.upload(bias), keep=be.upload(keep), rot_stride=32, rot_first=8, rot_pairs=5,
+                      rot_tab=be.upload(np.stack([np.cos(ang), np.sin(ang)], -1).astype(np.float32)[:r]))
+        elif form in ("softplus", "relu2"):
+            kw.update(bias=be.upload(bias))
+        elif form == "groups":
+            kw.update(groups=2, a_group=k, out_group=n, cols=n)
+        elif form == "softcap":
+            kw.update(softcap=1.5)
+        elif form == "mult":
+            kw.update(mult=0.37)
+        rows_of = np.arange(rows)
+        if form == "a_rows":
+            kw.update(a_rows=be.upload(order[:r]))
+            rows_of = order
+        be.linear(BF16, up(be, a, BF16), groups * k, p, n, k, r, lin_out(**kw))
+        got, got2 = down(be, out, (r, cols), F32 if f32 else BF16), down(be, out2, (r, n - split), F32)
+        # (32-bit results: the tolerance of a float32 sum of that many products)
+        close(got, want[rows_of[:r]], F32 if f32 else BF16, form)
+        if rest is not None:
+            close(got2, rest[:r], F32, form)
+        res.append((got[:few], got2[:few] if rest is not None else got[:few]))
+        be.reset_pool()
+    assert all(np.array_equal(x, y) for x, y in zip(*res))
 
 
 @pytest.mark.parametrize("act", ACTS)
