@@ -252,8 +252,8 @@ typedef struct vx_qweight {
  * bits; Q5_K: one byte per code and the scales as for Q4_K, 9.5 bits), kept by the backend under the matrix' address until
  * vx_qweight_unpack, vx_free of the matrix, a library write into its bytes or vx_backend_destroy. While it exists,
  * every quantized matmul entry point and fused decode block that is given the matrix (by the same data pointer, alone
- * or as part of a Q|K|V or gate|up group) with 2 .. 64 activation rows (Q4_K, Q5_K: 2 .. 32) streams the packed copy, and with more than 64 rows reads
- * it tile by tile; other row counts read the GGUF rows, which stay where they are. vx_dequantize_packed: gguf.Dequantize of the packed copy
+ * or as part of a Q|K|V or gate|up group) with 2 .. 64 activation rows streams the packed copy, and with more than 64 rows reads
+ * it tile by tile; a single row reads the GGUF rows, which stay where they are. vx_dequantize_packed: gguf.Dequantize of the packed copy
  * (pkg/gguf/dequant.go:16-145, 272-470), bit for bit what vx_dequantize gives for the rows. */
 int vx_qweight_pack(vx_backend *be, const vx_qweight *w);
 int vx_qweight_unpack(vx_backend *be, const vx_qweight *w);

@@ -58,8 +58,9 @@ __global__ void __launch_bounds__(kThreads) rmsnorm_kernel(const float *x, const
     const float *xr = x + (size_t)blockIdx.x * cols;
     float *orow = out + (size_t)blockIdx.x * cols;
     float ss = 0.f;
-    // Up to 4096 columns the row and the weights are asked for at once and kept: a single row is bound by trips to memory
-    // (4096 columns 11.7 us in two loops over them, 4.6 now; the same sums).
+    // Up to 16 columns a thread the row and the weights are asked for at once and kept: a single row is bound by trips to memory
+    // (4096 columns 11.7 us in two loops over them, 4.6 now; the same sums). Wider rows take the loops; whether more registers
+    // or threads would serve them is not measured.
     constexpr int U = 16;
     if (cols <= U * kThreads) {
         float v[U], wv[U];
