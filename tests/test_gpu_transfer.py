@@ -77,3 +77,15 @@ def test_staged_uploads(be):
     be.call("vx_to_device_staged", d, big.ctypes.data, big.size)
     assert np.array_equal(be.download(d, (big.size,), np.uint8), big)
     be.free(d)
+
+
+# sources at addresses that 16-byte, 4-byte and single-byte loads serve; both sides of a piece of 64 KB
+@pytest.mark.parametrize("at", [16, 4, 1])
+@pytest.mark.parametrize("size", [576 * KB - 1, 576 * KB, 576 * KB + 17])
+def test_download_from_any_address(be, at, size):
+    src = np.random.default_rng(size + at).integers(0, 256, size + 32, dtype=np.uint8)
+    d = be.upload(src, permanent=True)
+    out = np.zeros(size + 1, dtype=np.uint8)
+    be.to_host(out[:-1], d + at)
+    assert np.array_equal(out[:-1], src[at:at + size]) and out[-1] == 0
+    be.free(d)

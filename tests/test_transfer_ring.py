@@ -71,3 +71,69 @@ def test_every_piece_arrives(ring, helpers):
     sizes = [1, 15, 16, 17, 32, 40, 41, 200]
     r = subprocess.run([ring, str(helpers)] + [str(n) for n in sizes], capture_output=True, text=True, timeout=30)
     assert r.returncode == 0 and r.stdout.split("\n")[:-1] == ["%d ok" % n for n in sizes], (r.returncode, r.stdout)
+
+
+# A sender that keeps a launch back until the stream is asked, as a kernel may be late; "lost" leaves the last launch out.
+SENDER = HARNESS[:HARNESS.index("int main")] + r"""
+#include <atomic>
+#include <thread>
+struct Late : vx::Mover::Sender {
+    std::deque<std::thread> running;
+    bool lose = false;
+    int sends = 0;
+    hipError_t send(hipStream_t, const vx::Mover &m, const vx::Mover::Job &j, int from, int to) override {
+        if (to - from < 1 || to - from > vx::Mover::SENT_MOST) return 5;
+        sends++;
+        if (lose && to == (int)j.pieces.size()) return 0;
+        if (!running.empty()) running.back().join(), running.pop_back();  // (one launch behind the other)
+        running.emplace_back([&m, &j, from, to] {
+            for (int i = from; i < to; i++) {
+                std::this_thread::yield();
+                if (i >= vx::Mover::SENT_SLOTS && !j.copied[i - vx::Mover::SENT_SLOTS].load()) abort();  // the slot is still in use
+                memcpy(m.ring + (size_t)(i % vx::Mover::SENT_SLOTS) * vx::Mover::SENT_SLOT, j.pieces[i].src, j.pieces[i].bytes);
+                __atomic_store_n(m.marks + (size_t)(i % vx::Mover::SENT_SLOTS) * vx::Mover::MARK_STEP, vx::Mover::mark_of(j, i), __ATOMIC_RELEASE);
+            }
+        });
+        return 0;
+    }
+    void wait() { while (!running.empty()) running.back().join(), running.pop_back(); }
+    hipError_t ask(hipStream_t, bool *over) override { *over = lose; return 0; }
+    hipError_t lost() override { return 9; }
+};
+int main(int argc, char **argv) {
+    const int helpers = atoi(argv[1]);
+    vx::Mover m;
+    m.marks = (uint64_t *)calloc(vx::Mover::SENT_SLOTS * vx::Mover::MARK_STEP, 8);
+    Late *late = new Late;
+    m.sender = late;
+    if (!m.start(helpers) || (int)m.workers.size() != helpers) return 2;
+    const size_t piece = 4099;
+    for (int i = 2; i < argc; i++) {
+        const int n = abs(atoi(argv[i]));
+        late->lose = atoi(argv[i]) < 0;
+        std::string from(n * piece, 0), to(n * piece, 0);
+        for (size_t k = 0; k < from.size(); k++) from[k] = (char)(k * 2654435761u >> 13);
+        std::vector<vx::Mover::Piece> pieces;
+        for (int k = 0; k < n; k++) pieces.push_back({&to[k * piece], &from[k * piece], piece});
+        vx::Mover::Job job(std::move(pieces));
+        const int rc = m.move(0, job);
+        late->wait();
+        if (late->lose ? rc != 9 : rc != 0 || from != to) return 3;
+        printf("%d ok\n", atoi(argv[i]));
+        fflush(stdout);
+    }
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("helpers", [0, 1, 6])
+def test_every_sent_piece_arrives(tmp_path, helpers):
+    """Both sides of a launch (64 pieces), of the ring (256 slots) and of several turns of it; a stream that ends without its
+    last launch is an error and not a wait without an end, and what comes after it is whole again."""
+    src, exe = tmp_path / "sent.cpp", tmp_path / "sent"
+    src.write_text(SENDER)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "vexel_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    sizes = [1, 63, 64, 65, 255, 256, 257, -3, 320, 321, -300, 1000]
+    r = subprocess.run([str(exe), str(helpers)] + [str(n) for n in sizes], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.split("\n")[:-1] == ["%d ok" % n for n in sizes], (r.returncode, r.stdout)

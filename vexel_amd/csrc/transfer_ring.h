@@ -1,5 +1,5 @@
 // The ring of pinned memory that large downloads go through, and the threads behind it (transfer.hip). Nothing here but the
-// HIP calls of one copy at a time, declared by whoever includes it.
+// HIP calls of one copy at a time, declared by whoever includes it; a kernel that sends many pieces at once comes from outside.
 #pragma once
 #include <string.h>
 
@@ -15,6 +15,9 @@ namespace vx {
 struct Mover {
     static constexpr int SLOTS = 16, MAX_WORKERS = 6;
     static constexpr size_t SLOT = (size_t)1 << 20;
+    // With a sender the same ring has more and smaller slots, and a mark behind each that says which piece is in it.
+    static constexpr int SENT_SLOTS = 256, SENT_MOST = 64, MARK_STEP = 8;  // (marks on cache lines of their own)
+    static constexpr size_t SENT_SLOT = SLOTS * SLOT / SENT_SLOTS;
     struct Piece {
         char *dst;
         const char *src;
@@ -23,13 +26,27 @@ struct Mover {
     struct Job {
         std::vector<Piece> pieces;
         std::vector<std::atomic<char>> copied;
-        std::atomic<int> next{0}, arrived{0};
+        std::atomic<int> next{0}, arrived{0}, done{0};
         std::atomic<bool> failed{false};
+        uint64_t mark = 0;      // of the pieces of the ring's first turn, with a sender
+        bool by_sender = true;  // where there is one
         explicit Job(std::vector<Piece> p) : pieces(std::move(p)), copied(pieces.size()) {
             for (auto &c : copied) c.store(0);
         }
     };
+    // Puts pieces into the ring by a kernel: one launch for up to SENT_MOST of them instead of a copy and an event each.
+    struct Sender {
+        virtual ~Sender() {}
+        // Enqueues pieces from .. to - 1: each to its slot, then its mark behind it.
+        virtual hipError_t send(hipStream_t stream, const Mover &m, const Job &j, int from, int to) = 0;
+        // hipSuccess while the stream has work left, *over once it has none
+        virtual hipError_t ask(hipStream_t stream, bool *over) = 0;
+        virtual hipError_t lost() = 0;  // the error for pieces that will not come
+    };
     char *ring = nullptr;
+    uint64_t *marks = nullptr;  // [SENT_SLOTS * MARK_STEP], pinned
+    Sender *sender = nullptr;
+    uint64_t last_mark = 0;  // (no mark is ever used again)
     hipEvent_t events[SLOTS] = {};
     std::vector<std::thread> workers;
     std::mutex call, mu;  // one transfer at a time; the fields below
@@ -49,10 +66,12 @@ struct Mover {
         for (hipEvent_t e : events)
             if (e) (void)hipEventDestroy(e);
         if (ring) (void)hipHostFree(ring);
+        if (marks) (void)hipHostFree(marks);
+        delete sender;
     }
     // helpers: threads beside the caller, who copies as well; fewer, or none, where the system gives no more
     bool start(int helpers) {
-        if (hipHostMalloc((void **)&ring, SLOTS * SLOT, hipHostMallocDefault) != hipSuccess) {
+        if (!ring && hipHostMalloc((void **)&ring, SLOTS * SLOT, hipHostMallocDefault) != hipSuccess) {
             ring = nullptr;
             return false;
         }
@@ -67,14 +86,22 @@ struct Mover {
         }
         return true;
     }
+    bool sends(const Job &j) const { return sender && j.by_sender; }
+    const char *slot_of(const Job &j, int i) const { return sends(j) ? ring + (size_t)(i % SENT_SLOTS) * SENT_SLOT : ring + (size_t)(i % SLOTS) * SLOT; }
+    static uint64_t mark_of(const Job &j, int i) { return j.mark + (uint64_t)(i / SENT_SLOTS); }
+    bool here(const Job &j, int i) const {
+        if (sends(j)) return __atomic_load_n(marks + (size_t)(i % SENT_SLOTS) * MARK_STEP, __ATOMIC_ACQUIRE) == mark_of(j, i);
+        return i < j.arrived.load(std::memory_order_acquire);
+    }
     void copy(Job &j, int i) {
-        memcpy(j.pieces[i].dst, ring + (size_t)(i % SLOTS) * SLOT, j.pieces[i].bytes);
+        memcpy(j.pieces[i].dst, slot_of(j, i), j.pieces[i].bytes);
         j.copied[i].store(1, std::memory_order_release);
+        j.done.fetch_add(1, std::memory_order_release);
     }
     // Copies the next piece if it has arrived.
     bool take_arrived(Job &j) {
         int i = j.next.load();
-        while (i < j.arrived.load(std::memory_order_acquire))
+        while (i < (int)j.pieces.size() && here(j, i))
             if (j.next.compare_exchange_weak(i, i + 1)) {
                 copy(j, i);
                 return true;
@@ -87,12 +114,62 @@ struct Mover {
         for (;;) {
             const int i = j.next.fetch_add(1);
             if (i >= n) return;
-            while (j.arrived.load(std::memory_order_acquire) <= i) {
+            while (!here(j, i)) {
                 if (j.failed.load()) return;
                 std::this_thread::yield();
             }
             copy(j, i);
         }
+    }
+    void wake_workers(Job &j) {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            job = &j;
+            turn++;
+        }
+        wake.notify_all();
+    }
+    // The threads are out of the job when this returns.
+    void finish() {
+        std::unique_lock<std::mutex> l(mu);
+        job = nullptr;
+        left.wait(l, [&] { return inside == 0; });
+    }
+    // move() with a sender: the caller enqueues up to SENT_MOST pieces whenever their slots are free, and copies what has arrived
+    // in between. It never waits for a piece without asking now and then whether the stream still works.
+    hipError_t move_sent(hipStream_t stream, Job &j) {
+        const int n = (int)j.pieces.size();
+        hipError_t err = hipSuccess;
+        j.mark = last_mark + 1;
+        last_mark += (uint64_t)((n - 1) / SENT_SLOTS) + 1;
+        int sent = 0, out = 0;  // pieces enqueued; pieces before `out` are out of their slots
+        bool awake = false;
+        for (uint32_t polls = 1; j.done.load(std::memory_order_acquire) < n && err == hipSuccess; polls++) {
+            while (out < sent && j.copied[out].load(std::memory_order_acquire)) out++;
+            if (sent < n) {
+                const int to = std::min(n, sent + SENT_MOST);
+                if (to - SENT_SLOTS <= out) {
+                    err = sender->send(stream, *this, j, sent, to);
+                    sent = to;
+                    continue;
+                }
+            }
+            if (!awake && here(j, 0)) {  // (the threads sleep through the work that the first piece waits for)
+                awake = true;
+                wake_workers(j);
+            }
+            if (take_arrived(j)) continue;
+            std::this_thread::yield();
+            if (polls % 8192 == 0) {  // a stream that has ended without the pieces will not bring them
+                bool over = false;
+                err = sender->ask(stream, &over);
+                for (int i = out; i < sent && over && err == hipSuccess; i++)
+                    if (!here(j, i) && !j.copied[i].load(std::memory_order_acquire)) err = sender->lost();
+            }
+        }
+        if (err != hipSuccess) j.failed.store(true);
+        finish();
+        return err;
     }
     void work() {
         uint64_t seen = 0;
@@ -111,6 +188,7 @@ struct Mover {
     }
     // Everything before on the stream is done when this returns.
     hipError_t move(hipStream_t stream, Job &j) {
+        if (sends(j)) return move_sent(stream, j);
         const int n = (int)j.pieces.size();
         hipError_t err = hipSuccess;
         int sent = 0;
@@ -129,20 +207,11 @@ struct Mover {
             if (err == hipSuccess) err = hipEventSynchronize(events[got % SLOTS]);
             if (err != hipSuccess) break;
             j.arrived.store(got + 1, std::memory_order_release);
-            if (got == 0) {  // (the threads sleep through the work that the first piece waits for)
-                {
-                    std::lock_guard<std::mutex> g(mu);
-                    job = &j;
-                    turn++;
-                }
-                wake.notify_all();
-            }
+            if (got == 0) wake_workers(j);  // (the threads sleep through the work that the first piece waits for)
         }
         if (err != hipSuccess) j.failed.store(true);
         else run(j);
-        std::unique_lock<std::mutex> l(mu);
-        job = nullptr;
-        left.wait(l, [&] { return inside == 0; });
+        finish();
         return err;
     }
 };
