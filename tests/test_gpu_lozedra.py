@@ -526,6 +526,13 @@ def test_attention_many_rows(be, heads, start, lens):
     run_attention(be, BF16, Batch(be, [start, 40, 0], [lens, 1, 3], seed=4), heads, heads // 4, 16, 16, seed=1)
 
 
+@pytest.mark.parametrize("lens", [(64,), (68,), (128,), (132,), (30, 98), (256,), (400,), (512,), (300, 212), (516,)])
+def test_attention_long_tiles_beside_short_ones(be, lens):
+    """Both sides of the numbers of tiles (256 and 512 workgroups) between which the second half of them goes from short to long, for
+    one, two and four waves to the same queries; one and two sequences."""
+    run_attention(be, BF16, Batch(be, [7] * len(lens), list(lens), seed=6), 64, 16, 16, 16, seed=2)
+
+
 @pytest.mark.parametrize("act", ACTS)
 @pytest.mark.parametrize("length,back", [(1, 0), (17, 16), (33, 32), (130, 129), (257, 256), (700, 699), (700, 444), (700, 129), (700, 1)])
 def test_attention_far_key(be, act, length, back):

@@ -23,7 +23,7 @@ struct AttnArgs {
     int vec_q, vec_o;  // vector access to q / gate and out
     int lut_lds;
     // prefill
-    int tile_rows, tiles, min_rows;
+    int tile_rows, tiles, min_rows, first_round;
     // decode
     const int32_t *items;
     int piece, pieces;
@@ -94,6 +94,15 @@ template <int KD, int VD, int MAPS, bool NT> struct Keys {
     }
     __device__ __forceinline__ void load_k(int b0, int b1) {
         const bf16 *base = pool + (size_t)(k_sel ? b1 : b0) * blk;
+        if (kp == 32 * KD) {  // (no lane has to be left out)
+#pragma unroll
+            for (int kk = 0; kk < KD; kk++)
+#pragma unroll
+                for (int m = 0; m < MAPS; m++)
+#pragma unroll
+                    for (int t = 0; t < 2; t++) k[m][t][kk] = ld8<NT>(base + m * BS * kp + ko[t] + kk * 32 + kd);
+            return;
+        }
 #pragma unroll
         for (int kk = 0; kk < KD; kk++) {
             const int d = kk * 32 + kd;
@@ -150,12 +159,16 @@ template <int KD, int VD, int QT> struct Queries {
             for (int j = 0; j < 8; j++) s[j] = fmaf((j < 4 ? st0[j & 3] : st1[j & 3]), factor, far[t]);
         } else {
             const int last = a.p.bias_len - 1, n0 = pos[t] - key;
+            float b[8];
+            if (a.lut_lds) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int n = min(max(n0 - j, 0), last) + lut[t];
-                const float b = a.lut_lds ? s_lut[n] : a.p.bias[n] * kLog2e;
-                s[j] = fmaf((j < 4 ? st0[j & 3] : st1[j & 3]), factor, b);
+                for (int j = 0; j < 8; j++) b[j] = s_lut[min(max(n0 - j, 0), last) + lut[t]];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++) b[j] = a.p.bias[min(max(n0 - j, 0), last) + lut[t]] * kLog2e;
             }
+#pragma unroll
+            for (int j = 0; j < 8; j++) s[j] = fmaf((j < 4 ? st0[j & 3] : st1[j & 3]), factor, b[j]);
         }
         if (!whole) {
 #pragma unroll
