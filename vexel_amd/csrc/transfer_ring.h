@@ -2,6 +2,7 @@
 // HIP calls of one copy at a time, declared by whoever includes it; a kernel that sends many pieces at once comes from outside.
 #pragma once
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
@@ -121,6 +122,17 @@ struct Mover {
             copy(j, i);
         }
     }
+    // Has the pages of a piece's destination made, whatever is in them. A caller's memory is often fresh, and threads that copy into the
+    // same few megabytes of it wait for each other's page faults; false where the system does not know how.
+    static bool make_pages(const Piece &p) {
+#ifdef MADV_POPULATE_WRITE
+        const uintptr_t page = 4096, a = (uintptr_t)p.dst / page * page, b = ((uintptr_t)p.dst + p.bytes + page - 1) / page * page;
+        return madvise((void *)a, b - a, MADV_POPULATE_WRITE) == 0;
+#else
+        (void)p;
+        return false;
+#endif
+    }
     void wake_workers(Job &j) {
         {
             std::lock_guard<std::mutex> g(mu);
@@ -136,13 +148,13 @@ struct Mover {
         left.wait(l, [&] { return inside == 0; });
     }
     // move() with a sender: the caller enqueues up to SENT_MOST pieces whenever their slots are free, and copies what has arrived
-    // in between. It never waits for a piece without asking now and then whether the stream still works.
+    // in between; while nothing has, it makes the destination's pages. It never waits for a piece without asking now and then whether the stream still works.
     hipError_t move_sent(hipStream_t stream, Job &j) {
         const int n = (int)j.pieces.size();
         hipError_t err = hipSuccess;
         j.mark = last_mark + 1;
         last_mark += (uint64_t)((n - 1) / SENT_SLOTS) + 1;
-        int sent = 0, out = 0;  // pieces enqueued; pieces before `out` are out of their slots
+        int sent = 0, out = 0, made = 0;  // pieces enqueued; pieces before `out` are out of their slots; pieces whose pages are made
         bool awake = false;
         for (uint32_t polls = 1; j.done.load(std::memory_order_acquire) < n && err == hipSuccess; polls++) {
             while (out < sent && j.copied[out].load(std::memory_order_acquire)) out++;
@@ -159,7 +171,9 @@ struct Mover {
                 wake_workers(j);
             }
             if (take_arrived(j)) continue;
-            std::this_thread::yield();
+            made = std::max(made, j.next.load());
+            if (made < n) made = make_pages(j.pieces[made]) ? made + 1 : n;
+            else std::this_thread::yield();
             if (polls % 8192 == 0) {  // a stream that has ended without the pieces will not bring them
                 bool over = false;
                 err = sender->ask(stream, &over);
