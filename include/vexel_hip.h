@@ -70,6 +70,8 @@ int vx_to_host_many(vx_backend *be, int n, void *const *dst_host, const void *co
 /* vx_to_device that does not wait for the copy: src_host may be changed at once, and later calls on this backend see the
  * bytes; whoever reads dst by other means waits (vx_sync). More than 64 KiB: vx_to_device. */
 int vx_to_device_staged(vx_backend *be, void *dst, const void *src_host, size_t bytes);
+/* The same of n ranges that do not overlap, in few launches; a null dst or zero bytes is left out. */
+int vx_to_device_staged_many(vx_backend *be, int n, void *const *dst, const void *const *src_host, const size_t *bytes);
 /* Backend.Sync */
 int vx_sync(vx_backend *be);
 /* BufferCopier.CopyBuffer / CopyBufferBatched (backend.go:38-43): device to device. */

@@ -89,3 +89,27 @@ def test_download_from_any_address(be, at, size):
     be.to_host(out[:-1], d + at)
     assert np.array_equal(out[:-1], src[at:at + size]) and out[-1] == 0
     be.free(d)
+
+
+# more ranges than a launch holds; sizes at the edges of 4 and 16 bytes, none and more than the staging takes; any alignment; more
+# than the staging memory in all
+@pytest.mark.parametrize("sizes", [[4, 0, 4], [4] * 3, [1, 3, 4, 15, 16, 17, 64, 1000] * 20, [64 * KB, 64 * KB + 1, 12, 64 * KB - 3] * 4, [40 * KB] * 30])
+@pytest.mark.parametrize("shift", [0, 4, 1])
+def test_staged_uploads_of_several_ranges(be, sizes, shift):
+    rng = np.random.default_rng(len(sizes) + shift)
+    src = [rng.integers(0, 256, max(1, s), dtype=np.uint8)[:s] for s in sizes]
+    at = np.cumsum([0] + [(s + 31) // 16 * 16 for s in sizes])
+    total = int(at[-1]) + 32
+    want = rng.integers(0, 256, total, dtype=np.uint8)
+    d = be.upload(want, permanent=True)
+    n = len(sizes)
+    for _ in range(2):
+        dst = (C.c_void_p * (n + 1))(*([d + int(a) + shift for a in at[:-1]] + [None]))
+        frm = (C.c_void_p * (n + 1))(*([s.ctypes.data for s in src] + [want.ctypes.data]))
+        num = (C.c_size_t * (n + 1))(*(sizes + [9]))
+        be.call("vx_to_device_staged_many", n + 1, dst, frm, num)
+        for s, a in zip(src, at):
+            want[a + shift:a + shift + s.size] = s
+            s[:] = 255 - s                                 # the bytes are taken when the call returns
+        assert np.array_equal(be.download(d, (total,), np.uint8), want)
+    be.free(d)

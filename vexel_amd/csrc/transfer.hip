@@ -18,6 +18,20 @@ namespace vx {
 void mover_destroy(Mover *m) { delete m; }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// n bytes by the threads of a workgroup, in pieces of what both addresses are aligned to
+__device__ __forceinline__ void copy_bytes(char *dst, const char *src, uint32_t n, int tid, int threads) {
+    const uintptr_t at = (uintptr_t)dst | (uintptr_t)src;
+    uint32_t done = 0;
+    if ((at & 15) == 0) {
+        for (uint32_t k = tid; k < n / 16; k += threads) ((u32x4 *)dst)[k] = ((const u32x4 *)src)[k];
+        done = n / 16 * 16;
+    } else if ((at & 3) == 0) {
+        for (uint32_t k = tid; k < n / 4; k += threads) ((uint32_t *)dst)[k] = ((const uint32_t *)src)[k];
+        done = n / 4 * 4;
+    }
+    for (uint32_t k = done + tid; k < n; k += threads) dst[k] = src[k];
+}
+
 struct SendArgs {
     const char *src[Mover::SENT_MOST];
     uint32_t bytes[Mover::SENT_MOST];
@@ -37,31 +51,34 @@ __global__ void __launch_bounds__(SEND_THREADS) send_kernel(const SendArgs a) {
         const char *src = a.src[p];
         char *dst = a.ring + (size_t)slot * Mover::SENT_SLOT;
         const uint32_t n = a.bytes[p];
-        uint32_t done = 0;
-        if (((uintptr_t)src & 15) == 0) {
+        if (n == Mover::SENT_SLOT && ((uintptr_t)src & 15) == 0) {
             const u32x4 *s4 = (const u32x4 *)src;
-            u32x4 *d4 = (u32x4 *)dst;
-            if (n == Mover::SENT_SLOT) {
-                u32x4 v[SEND_VECS];
+            u32x4 v[SEND_VECS];
 #pragma unroll
-                for (int k = 0; k < SEND_VECS; k++) v[k] = s4[tid + k * SEND_THREADS];
+            for (int k = 0; k < SEND_VECS; k++) v[k] = s4[tid + k * SEND_THREADS];
 #pragma unroll
-                for (int k = 0; k < SEND_VECS; k++) d4[tid + k * SEND_THREADS] = v[k];
-            } else {
-                for (uint32_t k = tid; k < n / 16; k += SEND_THREADS) d4[k] = s4[k];
-            }
-            done = n / 16 * 16;
-        } else if (((uintptr_t)src & 3) == 0) {
-            for (uint32_t k = tid; k < n / 4; k += SEND_THREADS) ((uint32_t *)dst)[k] = ((const uint32_t *)src)[k];
-            done = n / 4 * 4;
+            for (int k = 0; k < SEND_VECS; k++) ((u32x4 *)dst)[tid + k * SEND_THREADS] = v[k];
+        } else {
+            copy_bytes(dst, src, n, tid, SEND_THREADS);
         }
-        for (uint32_t k = done + tid; k < n; k += SEND_THREADS) dst[k] = src[k];
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");  // (system scope: each thread's bytes are there before any thread is past the barrier)
         __syncthreads();
         if (tid == 0)
             __hip_atomic_store(a.marks + (size_t)slot * Mover::MARK_STEP, a.mark + (uint64_t)(i / Mover::SENT_SLOTS), __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+
+// Small uploads that lie in pinned memory one behind the other, a workgroup each.
+constexpr int SCATTER_MOST = 64;
+struct ScatterArgs {
+    const char *from;
+    char *dst[SCATTER_MOST];
+    uint32_t at[SCATTER_MOST], bytes[SCATTER_MOST];
+};
+__global__ void __launch_bounds__(SEND_THREADS) scatter_kernel(const ScatterArgs a) {
+    const int i = blockIdx.x;
+    copy_bytes(a.dst[i], a.from + a.at[i], a.bytes[i], threadIdx.x, SEND_THREADS);
 }
 
 namespace {
@@ -227,6 +244,61 @@ int vx_to_device_staged(vx_backend *be, void *dst, const void *src_host, size_t 
     memcpy(at, src_host, bytes);
     VX_CHECK_HIP(hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, be->stream));
     return VX_OK;
+}
+
+// What bounds a step's small uploads is the host: each copy of the runtime's is 6 us of it, 66 of them (the tables of 32 sequences
+// that have all come to a new block) 400 us before the step's first kernel. One launch brings 64.
+int vx_to_device_staged_many(vx_backend *be, int n, void *const *dst, const void *const *src_host, const size_t *bytes) {
+    int rc = enter(be);
+    if (rc) return rc;
+    if (n == 0) return VX_OK;
+    VX_REQUIRE(n > 0 && dst && src_host && bytes, "vx_to_device_staged: bad arguments");
+    VX_REQUIRE(!be->capturing, "vx_to_device_staged during graph capture");
+    int small = 0;
+    for (int i = 0; i < n; i++) {
+        VX_REQUIRE(!dst[i] || bytes[i] == 0 || src_host[i] != nullptr, "vx_to_device_staged: null source");
+        small += dst[i] && bytes[i] > 0 && bytes[i] <= UP_MOST;
+    }
+    if (small <= 2) {
+        for (int i = 0; i < n; i++)
+            if (rc = vx_to_device_staged(be, dst[i], src_host[i], bytes[i]); rc) return rc;
+        return VX_OK;
+    }
+    ScatterArgs a;
+    int m = 0;
+    size_t used = 0;  // of the staging memory, by the launch in the making
+    std::unique_lock<std::mutex> g(be->stage_mu);
+    auto launch = [&]() -> int {
+        if (m == 0) return VX_OK;
+        scatter_kernel<<<m, SEND_THREADS, 0, be->stream>>>(a);
+        be->stage_used += used;
+        m = 0, used = 0;
+        VX_CHECK_LAUNCH();
+        return VX_OK;
+    };
+    for (int i = 0; i < n; i++) {
+        if (!dst[i] || bytes[i] == 0) continue;
+        if (bytes[i] > UP_MOST || !readable(be, dst[i], bytes[i])) {
+            if (rc = launch(); rc) return rc;
+            g.unlock();
+            if (rc = vx_to_device_staged(be, dst[i], src_host[i], bytes[i]); rc) return rc;
+            g.lock();
+            continue;
+        }
+        const size_t room = (bytes[i] + 63) / 64 * 64;
+        if (m == SCATTER_MOST || be->stage_used + used + room > UP_BYTES)
+            if (rc = launch(); rc) return rc;
+        if (be->stage_used + room > UP_BYTES) {
+            VX_CHECK_HIP(hipStreamSynchronize(be->stream));
+            be->stage_used = 0;
+        }
+        if (m == 0) a.from = (const char *)be->host_stage + UP_AT + be->stage_used;
+        items_written(be, dst[i], bytes[i]);
+        memcpy((char *)be->host_stage + UP_AT + be->stage_used + used, src_host[i], bytes[i]);
+        a.dst[m] = (char *)dst[i], a.at[m] = (uint32_t)used, a.bytes[m] = (uint32_t)bytes[i];
+        m++, used += room;
+    }
+    return launch();
 }
 
 }  // extern "C"

@@ -263,6 +263,15 @@ SeqState *find_seq(vh_model *m, int64_t id);
 int create_seq_locked(vh_model *m, int64_t id);
 int sync_pool_to_device(vh_model *m);
 
+// Small uploads that go together (vx_to_device_staged_many). The sources are read by send().
+struct Uploads {
+    std::vector<void *> dst;
+    std::vector<const void *> src;
+    std::vector<size_t> bytes;
+    void add(void *d, const void *s, size_t n) { dst.push_back(d), src.push_back(s), bytes.push_back(n); }
+    int send(vx_backend *be) const { return vx_to_device_staged_many(be, (int)dst.size(), dst.data(), src.data(), bytes.data()); }
+};
+
 // A model whose mixer program is complete in m->mix (weights included): caches, states, activations.
 int mix_finish(vh_model *m);
 // Embedding of b.rows tokens -> layer runs -> final norm and head of n_want rows (want: device row numbers, NULL = the

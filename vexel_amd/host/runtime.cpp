@@ -67,23 +67,26 @@ int create_seq_locked(vh_model *m, int64_t id) {  // gpu_block_pool.go:126-135 (
 int sync_pool_to_device(vh_model *m) {
     BlockPool &p = m->pool;
     const int mb = m->cfg.max_blocks_per_seq;
+    Uploads up;
+    std::vector<int32_t> counts(p.seqs.size() + 1);
+    size_t n = 0;
     for (auto &kv : p.seqs) {
-        SeqState &s = kv.second;
+        const SeqState &s = kv.second;
         if (!s.dirty) continue;
         if ((int)s.table.size() > mb)
             return fail("sequence %lld needs %zu blocks, the table holds %d", (long long)kv.first, s.table.size(), mb);
-        if (!s.table.empty())
-            VXC(vx_to_device_staged(m->be, m->d_tables + (size_t)s.slot * mb, s.table.data(), s.table.size() * 4));
-        int32_t nb = (int32_t)s.table.size();
-        VXC(vx_to_device_staged(m->be, m->d_num_blocks + s.slot, &nb, 4));
-        s.dirty = false;
+        up.add(m->d_tables + (size_t)s.slot * mb, s.table.data(), s.table.size() * 4);
+        counts[n] = (int32_t)s.table.size();
+        up.add(m->d_num_blocks + s.slot, &counts[n++], 4);
     }
     if (p.free_dirty) {
-        if (!p.free_list.empty()) VXC(vx_to_device_staged(m->be, m->d_free, p.free_list.data(), p.free_list.size() * 4));
-        int32_t fc = (int32_t)p.free_list.size();
-        VXC(vx_to_device_staged(m->be, m->d_free_count, &fc, 4));
-        p.free_dirty = false;
+        up.add(m->d_free, p.free_list.data(), p.free_list.size() * 4);
+        counts[n] = (int32_t)p.free_list.size();
+        up.add(m->d_free_count, &counts[n], 4);
     }
+    VXC(up.send(m->be));
+    for (auto &kv : p.seqs) kv.second.dirty = false;
+    p.free_dirty = false;
     return VH_OK;
 }
 
@@ -959,10 +962,12 @@ int vh_sample_last_logits(vh_model *m, int rows, const float *temperature, const
     float *d_u = (float *)vx_alloc(be, (size_t)rows * 4);
     int32_t *d_k = (int32_t *)vx_alloc(be, (size_t)rows * 4), *d_out = (int32_t *)vx_alloc(be, (size_t)rows * 4);
     if (!d_t || !d_p || !d_u || !d_k || !d_out) return fail("sampling buffers: %s", vx_last_error());
-    VXC(vx_to_device_staged(be, d_t, temperature, (size_t)rows * 4));
-    VXC(vx_to_device_staged(be, d_k, top_k, (size_t)rows * 4));
-    VXC(vx_to_device_staged(be, d_p, top_p, (size_t)rows * 4));
-    VXC(vx_to_device_staged(be, d_u, uniform, (size_t)rows * 4));
+    Uploads how;
+    how.add(d_t, temperature, (size_t)rows * 4);
+    how.add(d_k, top_k, (size_t)rows * 4);
+    how.add(d_p, top_p, (size_t)rows * 4);
+    how.add(d_u, uniform, (size_t)rows * 4);
+    VXC(how.send(be));
     if (m->arch.final_softcap > 0.f)  // scheduler.go:772-773: the logits a request is sampled from are capped first
         for (int r = 0; r < rows; r++)
             if (temperature[r] > 0.f)
@@ -1017,11 +1022,13 @@ int vh_prefill(vh_model *m, const int32_t *tokens, int n, int64_t seq_id, int st
     float *logits = fa((size_t)out_rows * c.vocab);
     if (!d_tok || !d_page || !d_offs || !d_kvl || !d_bt || !x || !norm || !q || !k || !v || !attn || !gate || !up || !logits)
         return fail("prefill buffers: %s", vx_last_error());
-    VXC(vx_to_device_staged(be, d_tok, tokens, (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_page, page.data(), (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_offs, offs.data(), (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_kvl, kvl.data(), (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_bt, table.data(), table.size() * 4));
+    Uploads arrays;
+    arrays.add(d_tok, tokens, (size_t)n * 4);
+    arrays.add(d_page, page.data(), (size_t)n * 4);
+    arrays.add(d_offs, offs.data(), (size_t)n * 4);
+    arrays.add(d_kvl, kvl.data(), (size_t)n * 4);
+    arrays.add(d_bt, table.data(), table.size() * 4);
+    VXC(arrays.send(be));
     VXC(vx_embedding(be, d_tok, n, m->embedding, x, c.vocab, c.hidden));               // decode.go:1005-1010
     VHC(g_scale_embedding(m, x, n));                                                   // decode.go:1030
     const float scale = (float)(1.0 / sqrt((double)c.head_dim));
@@ -1311,14 +1318,16 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
     float *logits = fa((size_t)n * c.vocab);
     if (!d_tok || !d_pos || !d_slot || !d_am || !d_mask || !x || !norm || !q || !k || !v || !attn || !gate || !up || !logits)
         return fail("verification buffers: %s", vx_last_error());
-    VXC(vx_to_device_staged(be, d_tok, tok.data(), (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_pos, pos.data(), (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_slot, slot_map.data(), (size_t)n * 4));
-    VXC(vx_to_device_staged(be, d_mask, mask.data(), mask.size()));
+    Uploads arrays;
+    arrays.add(d_tok, tok.data(), (size_t)n * 4);
+    arrays.add(d_pos, pos.data(), (size_t)n * 4);
+    arrays.add(d_slot, slot_map.data(), (size_t)n * 4);
+    arrays.add(d_mask, mask.data(), mask.size());
+    std::vector<int32_t> ent_rows, ent_lens, info, moff;
     int32_t *d_ent_rows = nullptr, *d_ent_lens = nullptr, *d_info = nullptr, *d_moff = nullptr;
     int entries = 0, max_start = 0;
     if (rg) {
-        std::vector<int32_t> ent_rows, ent_lens, info((size_t)n * 4), moff(n);
+        info.resize((size_t)n * 4), moff.resize(n);
         for (int i = 0; i < n_seqs; i++) {
             const SeqRows &s = sr[i];
             max_start = std::max(max_start, s.start);
@@ -1335,11 +1344,12 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
         entries = (int)ent_rows.size();
         d_ent_rows = ia(entries), d_ent_lens = ia(entries), d_info = ia((size_t)n * 4), d_moff = ia(n);
         if (!d_ent_rows || !d_ent_lens || !d_info || !d_moff) return fail("verification buffers: %s", vx_last_error());
-        VXC(vx_to_device_staged(be, d_ent_rows, ent_rows.data(), (size_t)entries * 4));
-        VXC(vx_to_device_staged(be, d_ent_lens, ent_lens.data(), (size_t)entries * 4));
-        VXC(vx_to_device_staged(be, d_info, info.data(), (size_t)n * 16));
-        VXC(vx_to_device_staged(be, d_moff, moff.data(), (size_t)n * 4));
+        arrays.add(d_ent_rows, ent_rows.data(), (size_t)entries * 4);
+        arrays.add(d_ent_lens, ent_lens.data(), (size_t)entries * 4);
+        arrays.add(d_info, info.data(), (size_t)n * 16);
+        arrays.add(d_moff, moff.data(), (size_t)n * 4);
     }
+    VXC(arrays.send(be));
     VXC(vx_embedding(be, d_tok, n, m->embedding, x, c.vocab, c.hidden));
     VHC(g_scale_embedding(m, x, n));
     const float scale = (float)(1.0 / sqrt((double)c.head_dim));
@@ -1462,9 +1472,11 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
         const int chains = (int)chain_off.size() - 1;
         int32_t *d_co = ia(chain_off.size()), *d_src = ia(move_src.size()), *d_dst = ia(move_dst.size());
         if (!d_co || !d_src || !d_dst) return fail("verification buffers: %s", vx_last_error());
-        VXC(vx_to_device_staged(be, d_co, chain_off.data(), chain_off.size() * 4));
-        VXC(vx_to_device_staged(be, d_src, move_src.data(), move_src.size() * 4));
-        VXC(vx_to_device_staged(be, d_dst, move_dst.data(), move_dst.size() * 4));
+        Uploads moves;
+        moves.add(d_co, chain_off.data(), chain_off.size() * 4);
+        moves.add(d_src, move_src.data(), move_src.size() * 4);
+        moves.add(d_dst, move_dst.data(), move_dst.size() * 4);
+        VXC(moves.send(be));
         for (int l = 0; l < c.num_layers; l++)
             VXC(vx_paged_kv_move(be, m->kv[l], c.kv_fp16, d_co, d_src, d_dst, chains, c.num_kv_heads, c.head_dim,
                                  c.block_size));

@@ -30,6 +30,7 @@ SIGNATURES = {
     "vx_to_host": (_i, [_vp, _vp, _vp, _sz]),
     "vx_to_host_many": (_i, [_vp, _i, _vp, _vp, _vp]),
     "vx_to_device_staged": (_i, [_vp, _vp, _vp, _sz]),
+    "vx_to_device_staged_many": (_i, [_vp, _i, _vp, _vp, _vp]),
     "vx_sync": (_i, [_vp]),
     "vx_copy_buffer": (_i, [_vp, _vp, _sz, _vp, _sz, _sz]),
     "vx_begin_batch": (_i, [_vp]),
