@@ -1156,6 +1156,18 @@ def test_paged_multiquery_value_that_is_not_finite(be, hq, hk, d, qn, pair):
     be.reset_pool()
 
 
+# steps of 64 keys: one key more and less, a block and a pair and a block into the next step; the last block of a step not finite
+@pytest.mark.parametrize("keys", [63, 64, 65, 80, 97, 128, 129, 193])
+@pytest.mark.parametrize("hq,hk,d,qn", [(8, 2, 128, 17), (4, 4, 64, 16), (32, 8, 128, 512), (16, 16, 128, 300), (64, 4, 64, 512), (64, 8, 128, 512)])
+def test_paged_multiquery_steps_of_64_keys(be, hq, hk, d, qn, keys):
+    test_paged_multiquery_pairs_of_blocks(be, hq, hk, d, qn, keys)
+
+
+@pytest.mark.parametrize("hq,hk,d,qn", [(8, 2, 128, 64), (64, 4, 64, 256), (32, 8, 128, 512), (64, 8, 128, 512)])
+def test_paged_multiquery_value_that_is_not_finite_late_in_a_step(be, hq, hk, d, qn):
+    test_paged_multiquery_value_that_is_not_finite(be, hq, hk, d, qn, 1)
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])

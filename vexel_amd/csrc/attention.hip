@@ -790,6 +790,18 @@ __global__ void __launch_bounds__(256, 3) paged_decode_gqa_kernel(
     finish_split<D, G, RG>(s_m, s_l, s_acc, partial, seq, kvh, split, kv_len, num_q_heads, num_kv_heads, max_splits, mg, tps);
 }
 
+// The operand of 32 rows by 16 columns from rows in LDS: a lane's address is that of four columns of a row (lane c of 16: row c / 4 of
+// its four, columns 4 (c & 3) ..); it gets column c of the 16, the four rows at `a` and then the four at `b`.
+__device__ __forceinline__ half8 read_columns(const _Float16 *a, const _Float16 *b) {
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4v *Lds;
+    const short4v x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)a), y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((Lds)b);
+    half8 r;
+    __builtin_memcpy(&r, &x, 8);
+    __builtin_memcpy((char *)&r + 8, &y, 8);
+    return r;
+}
+
 // Many query rows of one sequence over its paged F16 context, each row with its own number of visible keys (the
 // later chunks of a prompt, linear verification): paged_decode_gqa_kernel's two matrix-core products and operand
 // layouts, with QT tiles of 16 consecutive query rows of one head per wave instead of 16 (row, head) queries of one
@@ -798,25 +810,29 @@ __global__ void __launch_bounds__(256, 3) paged_decode_gqa_kernel(
 // shares of the pairs of blocks (pair b belongs to share b % KS). The NSUB waves of a share bring each pair into LDS
 // together, whole rows per load instruction, and read their operands from there, so the K/V rows pass through the
 // memory system once per workgroup; the shares' (m, l, O) meet in LDS at the end and share 0 writes the rows.
-// A step is a pair of blocks: the values' product then fills a 16 x 16 x 32 instruction (with one block it took a 16 x 16 x 16
-// one, the same time for half the work) and maximum, rescaling and barrier come once per 32 keys. What is left is bound by
-// the vector instructions of the softmax and the operands' halves beside the matrix cores. 512 rows over 4096 keys, 32 / 8
-// heads of 128: 136 -> 102 us.
-// grid = (ceil(G * row tiles / NSUB), num_kv_heads); block = 64 * NSUB * KS.
+// A step is two pairs of blocks where LDS holds them (one with four shares of 128 columns): the values' product fills a 16 x 16 x 32
+// instruction, maximum, rescaling and barrier come once per 64 keys, and one pair's weights go beside the other's product. The
+// values' operands are read from LDS by columns (read_columns), not put together from rows by 32 permutes a pair. A KV head's workgroups
+// are a grid's neighbours eight apart, so with eight KV heads they run on one die and find its rows in that die's L2.
+// What is left is waiting: the matrix pipes are busy a third of the time, vector and matrix instructions could issue in half
+// of it; two waves a SIMD go through the same chain (scores, softmax, weights, values) at the same time. 512 rows over 4096 keys, 32 / 8
+// heads of 128: 104 -> 88 us (rescaling by need 99, steps of 64 keys and the dies 88; operands by columns alone changed nothing
+// but the registers). 32 rows a wave: 98.
+// grid = (num_kv_heads, ceil(G * row tiles / NSUB)); block = 64 * NSUB * KS.
+constexpr float MQ_LAZY = 5.f;  // a row's reference follows its largest score once that is 2^5 above it: 2^10 p stays below 2^15
 template <int D, int QT, int KS, int NSUB = 4>
 __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *__restrict__ q, const _Float16 *__restrict__ pool,
                                                          const int32_t *__restrict__ table, const int32_t *__restrict__ kv_lens,
                                                          float *__restrict__ out, int query_len, int max_keys, int num_q_heads,
                                                          int num_kv_heads, float scale) {
     constexpr int NS = D / 32, NT = D / 16;
-    typedef _Float16 halfv __attribute__((ext_vector_type(NT)));
-    const int kvh = blockIdx.y, G = num_q_heads / num_kv_heads;
+    const int kvh = blockIdx.x, G = num_q_heads / num_kv_heads;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = wave % NSUB, ksub = wave / NSUB;  // which of the workgroup's NSUB (head, row group) pairs, which share of the blocks
     const int row_groups = (query_len + 16 * QT - 1) / (16 * QT);
-    const bool idle = blockIdx.x * NSUB + sub >= G * row_groups;  // (a wave without work walks no block; it still meets the others)
-    const int combo = min((int)blockIdx.x * NSUB + sub, G * row_groups - 1);
+    const bool idle = blockIdx.y * NSUB + sub >= G * row_groups;  // (a wave without work walks no block; it still meets the others)
+    const int combo = min((int)blockIdx.y * NSUB + sub, G * row_groups - 1);
     const int head = kvh * G + combo % G, r0 = (combo / G) * 16 * QT;
     const int c16 = lane & 15, g4 = lane >> 4;
     const size_t hs = (size_t)num_kv_heads * D, part = (size_t)HOT_BS * hs, qs = (size_t)num_q_heads * D;
@@ -881,50 +897,57 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
     const int n_pairs = idle ? 0 : (len_max + PT - 1) / PT;
     const int len_top = __builtin_amdgcn_readfirstlane(len_max);
     const int tok_row = 4 * (c16 & 3) + (c16 >> 2);  // this lane's K row of a block as A operand
-    constexpr int KP = D + 8;                        // halves per staged row (rows 4 banks apart)
+    constexpr int KP = D + 8, VP = D + 16;           // halves per staged row of K (rows 4 banks apart) and of V (8 banks)
     // [share][buffer][K, V][row of the pair]; behind the loop the shares' outputs lie there
-    constexpr int STAGE = PT * KP, SO_FLOATS = (KS - 1) * NSUB * QT * 4 * NT * 64;
-    constexpr int SMEM = KS * 4 * STAGE * 2 > SO_FLOATS * 4 ? KS * 4 * STAGE * 2 : SO_FLOATS * 4;
+    // pairs to a buffer: two where LDS holds them, so that the waves meet half as often and one pair's scores can go beside the other's
+    // weights
+    constexpr int PAIRS = KS * 2 * 2 * PT * (KP + VP) * 2 <= 150 * 1024 ? 2 : 1;
+    constexpr int STAGE = PAIRS * PT * (KP + VP), V_AT = PAIRS * PT * KP, SO_FLOATS = (KS - 1) * NSUB * QT * 4 * NT * 64;
+    constexpr int SMEM = KS * 2 * STAGE * 2 > SO_FLOATS * 4 ? KS * 2 * STAGE * 2 : SO_FLOATS * 4;
     __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
     _Float16 *const stg = (_Float16 *)smem;
-    // One pair of blocks against the wave's query tiles: scores of both blocks side by side, one maximum and one rescaling for the
-    // pair, and the values' product over 32 tokens in one instruction (lane group g: tokens 4 i + g of either block).
-    auto compute = [&](int pi, const _Float16 *ks, const _Float16 *vs) __attribute__((always_inline)) {
-        const int tok0 = pi * PT + g4;                   // score 4 b + i of a tile: token tok0 + 16 b + 4 i
-        const bool open = (pi + 1) * PT <= len_min;      // every row of the wave sees the whole pair
-        float4v sc[QT][2];
+    // A buffer's blocks against the wave's query tiles: all scores, one maximum and one rescaling, and the values' product over 32 tokens
+    // in one instruction (lane group g: tokens 4 i + g of either block of a pair).
+    constexpr int NB = 2 * PAIRS;
+    auto compute = [&](int gi, const _Float16 *ks, const _Float16 *vs) __attribute__((always_inline)) {
+        const int tok0 = gi * NB * HOT_BS + g4;                   // score 4 b + i of a tile: token tok0 + 16 b + 4 i
+        const bool open = (gi + 1) * NB * HOT_BS <= len_min;      // every row of the wave sees them all
+        float4v sc[QT][NB];
 #pragma unroll
-        for (int t = 0; t < QT; t++) sc[t][0] = sc[t][1] = (float4v){0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < QT; t++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) sc[t][b] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            half8 kk[2];
+            half8 kk[NB];
 #pragma unroll
-            for (int b = 0; b < 2; b++) kk[b] = *(const half8 *)&ks[(b * HOT_BS + tok_row) * KP + g4 * (D / 4) + 8 * s];
+            for (int b = 0; b < NB; b++) kk[b] = *(const half8 *)&ks[(b * HOT_BS + tok_row) * KP + g4 * (D / 4) + 8 * s];
 #pragma unroll
             for (int t = 0; t < QT; t++) {
 #pragma unroll
-                for (int b = 0; b < 2; b++) sc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk[b], qh[t][s], sc[t][b], 0, 0, 0);
+                for (int b = 0; b < NB; b++) sc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk[b], qh[t][s], sc[t][b], 0, 0, 0);
 #pragma unroll
-                for (int b = 0; b < 2; b++) sc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk[b], ql[t][s], sc[t][b], 0, 0, 0);
+                for (int b = 0; b < NB; b++) sc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kk[b], ql[t][s], sc[t][b], 0, 0, 0);
             }
         }
-        // A second block that none of the wave's rows sees has weights of 0 only, but a value there may be infinite: the first block's
+        // A block that none of the wave's rows sees has weights of 0 only, but a value there may be infinite: the first block's
         // values once more then.
-        const _Float16 *const vs2 = vs + ((2 * pi + 1) * HOT_BS < len_top ? HOT_BS * KP : 0);
-        halfv vv[8];
+        const _Float16 *v_row[NB];
 #pragma unroll
-        for (int i = 0; i < 8; i++) vv[i] = *(const halfv *)&(i < 4 ? vs : vs2)[(4 * (i & 3) + g4) * KP + c16 * NT];
+        for (int b = 0; b < NB; b++)
+            v_row[b] = vs + (4 * (c16 >> 2) + g4) * VP + (c16 & 3) * 4 + ((gi * NB + b) * HOT_BS < len_top ? b * HOT_BS * VP : 0);
 #pragma unroll
         for (int t = 0; t < QT; t++) {
-            float sv[8], gm = -INFINITY;
+            float gm = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                sv[i] = (open || tok0 + 16 * (i >> 2) + 4 * (i & 3) < lim[t]) ? sc[t][i >> 2][i & 3] * q_inv[t] : -INFINITY;
-                gm = fmaxf(gm, sv[i]);
-            }
-            gm = fmaxf(gm, __shfl_xor(gm, 16, 64));
-            gm = fmaxf(gm, __shfl_xor(gm, 32, 64));
-            if (__builtin_amdgcn_ballot_w64(gm > m_run[t]) != 0) {
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (!open && tok0 + 16 * b + 4 * i >= lim[t]) sc[t][b][i] = -INFINITY;
+                    gm = fmaxf(gm, sc[t][b][i]);
+                }
+            gm = max_of_quarters(gm) * q_inv[t] - 10.f;  // (q_inv: a power of two)
+            if (__builtin_amdgcn_ballot_w64(gm > m_run[t] + MQ_LAZY) != 0) {
                 const float m_new = fmaxf(m_run[t], gm);
                 const float alpha = exp2f(m_run[t] - m_new);  // (m_new is finite in every lane that gets here with gm > m_run; 1 elsewhere)
                 const float a_own = gm > m_run[t] ? alpha : 1.f;
@@ -938,21 +961,24 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                 }
             }
             const float m_use = m_run[t] == -INFINITY ? 0.f : m_run[t];  // (a row that has seen no key yet: every weight 0)
-            half8 ph, pl;
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                // (2^10 p; below 2^-126 it is 0, which is 2^-136 of the row's largest weight)
-                const float pw = __builtin_amdgcn_exp2f(sv[i] - m_use + 10.f);
-                l_run[t] += pw;
-                const HalfPair hl = split_hl(pw);
-                ph[i] = hl.h;
-                pl[i] = hl.l;
-            }
+            for (int p = 0; p < PAIRS; p++) {
+                half8 ph, pl;
 #pragma unroll
-            for (int e = 0; e < NT; e++) {
-                const half8 vb = {vv[0][e], vv[1][e], vv[2][e], vv[3][e], vv[4][e], vv[5][e], vv[6][e], vv[7][e]};
-                o[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb, o[t][e], 0, 0, 0);
-                o[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb, o[t][e], 0, 0, 0);
+                for (int i = 0; i < 8; i++) {
+                    // (2^10 p and up to 2^5 of that; below 2^-126 it is 0, which is 2^-136 of the row's largest weight)
+                    const float pw = __builtin_amdgcn_exp2f(fmaf(sc[t][2 * p + (i >> 2)][i & 3], q_inv[t], -m_use));
+                    l_run[t] += pw;
+                    const HalfPair hl = split_hl(pw);
+                    ph[i] = hl.h;
+                    pl[i] = hl.l;
+                }
+#pragma unroll
+                for (int e = 0; e < NT; e++) {
+                    const half8 vb = read_columns(v_row[2 * p] + 16 * e, v_row[2 * p + 1] + 16 * e);
+                    o[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb, o[t][e], 0, 0, 0);
+                    o[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb, o[t][e], 0, 0, 0);
+                }
             }
         }
     };
@@ -961,7 +987,7 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
         // rows per load instruction, once for all of them, and each reads its operands from there: one pass over
         // the K/V rows per workgroup instead of one per wave. Two buffers, one barrier per pair; the loop runs to
         // the longest of the workgroup's row tiles for every wave.
-        constexpr int TG = NSUB * 64, PIECES = PT * D / 8, PPT = (PIECES + TG - 1) / TG;
+        constexpr int TG = NSUB * 64, PIECES = PAIRS * PT * D / 8, PPT = (PIECES + TG - 1) / TG;
         static_assert(PIECES % TG == 0, "every lane moves whole pieces");
         __shared__ int s_wg[2];
         if (tid == 0) s_wg[0] = s_wg[1] = 0;
@@ -975,40 +1001,51 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
         const int last_block = max((wg_len + HOT_BS - 1) / HOT_BS - 1, 0);
         const int tg = sub * 64 + lane;
         half8 kreg[PPT], vreg[PPT];
-        auto issue = [&](int pi) {
-            // (a pair whose second block is beyond the last takes that one twice: its keys are masked, its values cleared)
-            const int b0 = __builtin_amdgcn_readfirstlane(table[2 * pi]), b1 = __builtin_amdgcn_readfirstlane(table[min(2 * pi + 1, last_block)]);
+        // Numbers of a pair's blocks, asked for a pair before the rows. (A pair whose second block is beyond the last takes that one twice:
+        // its keys are masked, its values cleared.)
+        int blk[2 * PAIRS];
+        auto number = [&](int gi) {
+#pragma unroll
+            for (int i = 0; i < 2 * PAIRS; i++) blk[i] = __builtin_amdgcn_readfirstlane(table[min(2 * PAIRS * gi + i, last_block)]);
+        };
+        auto issue = [&]() {
 #pragma unroll
             for (int j = 0; j < PPT; j++) {
                 const int pc = j * TG + tg, row = pc / (D / 8), c8 = pc % (D / 8);
-                const _Float16 *base = pool + (size_t)(row < HOT_BS ? b0 : b1) * 2 * part + (size_t)kvh * D + (size_t)(row & (HOT_BS - 1)) * hs + c8 * 8;
+                int b = blk[0];
+#pragma unroll
+                for (int i = 1; i < 2 * PAIRS; i++) b = row >= i * HOT_BS ? blk[i] : b;
+                const _Float16 *base = pool + (size_t)b * 2 * part + (size_t)kvh * D + (size_t)(row & (HOT_BS - 1)) * hs + c8 * 8;
                 // (plain loads: the workgroups of other row tiles and heads read the same rows, from the die's L2)
                 kreg[j] = *(const half8 *)base;
                 vreg[j] = *(const half8 *)(base + part);
             }
         };
-        auto commit = [&](int pi, _Float16 *to) {
+        auto commit = [&](int gi, _Float16 *to) {
 #pragma unroll
             for (int j = 0; j < PPT; j++) {
                 const int pc = j * TG + tg, row = pc / (D / 8), c8 = pc % (D / 8);
                 half8 v = vreg[j];
-                if (pi * PT + row >= wg_len) v = (half8){0, 0, 0, 0, 0, 0, 0, 0};  // rows past the sequence's end may hold anything
+                if (gi * PAIRS * PT + row >= wg_len) v = (half8){0, 0, 0, 0, 0, 0, 0, 0};  // rows past the sequence's end may hold anything
                 *(half8 *)&to[row * KP + c8 * 8] = kreg[j];
-                *(half8 *)&to[STAGE + row * KP + c8 * 8] = v;
+                *(half8 *)&to[V_AT + row * VP + c8 * 8] = v;
             }
         };
-        const int iters = (wg_pairs + KS - 1) / KS;
-        if (ksub < wg_pairs) issue(ksub);
+        const int wg_groups = (wg_pairs + PAIRS - 1) / PAIRS, iters = (wg_groups + KS - 1) / KS;
+        number(ksub);
+        if (ksub < wg_groups) issue();
+        number(ksub + KS);
         for (int it = 0; it < iters; it++) {
-            const int pi = it * KS + ksub;
-            _Float16 *const at = stg + (size_t)(ksub * 2 + (it & 1)) * 2 * STAGE;
-            if (pi < wg_pairs) commit(pi, at);
-            if (pi + KS < wg_pairs) issue(pi + KS);
+            const int gi = it * KS + ksub;
+            _Float16 *const at = stg + (size_t)(ksub * 2 + (it & 1)) * STAGE;
+            if (gi < wg_groups) commit(gi, at);
+            if (gi + KS < wg_groups) issue();
+            number(gi + 2 * KS);
             __syncthreads();
-            if (pi < n_pairs) compute(pi, at, at + STAGE);  // (beyond: none of this wave's rows sees a key of the pair)
+            if (gi * PAIRS < n_pairs) compute(gi, at, at + V_AT);  // (beyond: none of this wave's rows sees a key of them)
         }
     }
-    // lane (c16, g4) holds O[row 4 g4 + i][columns c16 * NT .. + NT - 1] of every tile; the row's sum of weights is
+    // lane (c16, g4) holds O[row 4 g4 + i][columns 16 e + c16] of every tile; the row's sum of weights is
     // spread over the four lanes (row, 0..3). With KS > 1 the waves that took the other shares of the blocks hand
     // their (m, l, O) over through LDS - every value in the slot of the lane that holds the same element - and the
     // wave with share 0 adds them in share order.
@@ -1061,8 +1098,7 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
             }
             const float inv = L > 0.f ? 1.f / L : 0.f;
             if (qi >= query_len) continue;
-            float *op = out + (size_t)qi * qs + (size_t)head * D + c16 * NT;
-            float y[NT];
+            float *op = out + (size_t)qi * qs + (size_t)head * D + c16;
 #pragma unroll
             for (int e = 0; e < NT; e++) {
                 float acc = o[t][e][i] * w[0];
@@ -1070,10 +1106,8 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
 #pragma unroll
                     for (int k2 = 1; k2 < KS; k2++) acc += s_o[k2 - 1][sub][t][e * 4 + i][lane] * w[k2];
                 }
-                y[e] = acc * inv;
+                op[16 * e] = acc * inv;
             }
-#pragma unroll
-            for (int e = 0; e < NT; e += 4) *(float4 *)(op + e) = make_float4(y[e], y[e + 1], y[e + 2], y[e + 3]);
         }
     }
 }
@@ -1924,7 +1958,7 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
         const int max_keys = num_blocks * block_size;
 #define VX_MQ(DD, KK, NS)                                                                                                 \
     if (head_dim == DD && share == KK)                                                                                    \
-        paged_mq_kernel<DD, QT, KK, NS><<<dim3(ceil_div(combos, NS), num_kv_heads), 64 * NS * KK, 0, be->stream>>>(         \
+        paged_mq_kernel<DD, QT, KK, NS><<<dim3(num_kv_heads, ceil_div(combos, NS)), 64 * NS * KK, 0, be->stream>>>(         \
             q, pool, block_table, kv_lens, out, query_len, max_keys, num_q_heads, num_kv_heads, scale);
         // (heads of 128 with four shares: two pairs a workgroup, so that a wave keeps 256 registers)
         VX_MQ(128, 1, 4) VX_MQ(128, 2, 4) VX_MQ(128, 4, 2) VX_MQ(64, 1, 4) VX_MQ(64, 2, 4) VX_MQ(64, 4, 4)

@@ -61,19 +61,6 @@ template <bool NT> __device__ __forceinline__ bf16x8 ld8(const bf16 *p) {
     return NT ? __builtin_nontemporal_load((const bf16x8 *)p) : *(const bf16x8 *)p;
 }
 
-// The largest of the four lanes with the same lane % 16. (The copies are opaque: of two equal operands the compiler takes both results for
-// equal as well.)
-__device__ __forceinline__ float max_of_quarters(float v) {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    unsigned a = __builtin_bit_cast(unsigned, v), b = a;
-    asm("" : "+v"(b));
-    u32x2 p = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a, b, false, false));  // lanes 16 apart
-    a = b = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)p[0]), __builtin_bit_cast(float, (unsigned)p[1])));
-    asm("" : "+v"(b));
-    p = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a, b, false, false));        // lanes 32 apart
-    return fmaxf(__builtin_bit_cast(float, (unsigned)p[0]), __builtin_bit_cast(float, (unsigned)p[1]));
-}
-
 // The keys of one group of 32 for a wave: K (of every map) as two 16 x (32 KD) operands, V^T as VD 16 x 32 operands.
 template <int KD, int VD, int MAPS, bool NT> struct Keys {
     bf16x8 k[MAPS][2][KD];

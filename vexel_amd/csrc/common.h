@@ -212,4 +212,17 @@ int run_matvec_fused(vx_backend *be, int fmt, const void *const *ws, const int *
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// The largest of the four lanes with the same lane % 16. (The copies are opaque: of two equal operands the compiler takes both results for
+// equal as well.)
+__device__ __forceinline__ float max_of_quarters(float v) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    unsigned a = __builtin_bit_cast(unsigned, v), b = a;
+    asm("" : "+v"(b));
+    u32x2 p = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a, b, false, false));  // lanes 16 apart
+    a = b = __builtin_bit_cast(unsigned, fmaxf(__builtin_bit_cast(float, (unsigned)p[0]), __builtin_bit_cast(float, (unsigned)p[1])));
+    asm("" : "+v"(b));
+    p = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a, b, false, false));        // lanes 32 apart
+    return fmaxf(__builtin_bit_cast(float, (unsigned)p[0]), __builtin_bit_cast(float, (unsigned)p[1]));
+}
+
 }  // namespace vx
