@@ -863,6 +863,35 @@ def test_sdpa_and_prefill(be):
         be.reset_pool()
 
 
+# around a share (32 keys) and a step (64) of the tiled kernel; growing: the largest score of a row is among its last keys, so that
+# the shares' maxima are far apart and both are rescaled
+@pytest.mark.parametrize("s", [1, 31, 32, 33, 63, 64, 65, 96, 97, 160, 257])
+@pytest.mark.parametrize("hq,hk,d,growing", [(4, 1, 128, False), (2, 2, 64, True), (2, 1, 128, True)])
+def test_sdpa_prefill_shares_of_a_step(be, s, hq, hk, d, growing):
+    rng = np.random.default_rng(s + d)
+    q = rng.standard_normal((s, hq, d)).astype(np.float32)
+    k = rng.standard_normal((s, hk, d)).astype(np.float32)
+    if growing:
+        q = np.abs(q)
+        k = np.abs(k) * (np.arange(s, dtype=np.float32)[:, None, None] / 32 - 1)
+    v = rng.standard_normal((s, hk, d)).astype(np.float32)
+    sc = np.float32(1 / math.sqrt(d))
+    dq, dk, dv = be.upload(q), be.upload(k), be.upload(v)
+    do = be.alloc(q.nbytes)
+    be.sdpa_prefill(dq, dk, dv, do, s, hq, hk, d, sc)
+    q64, k64, v64 = q.astype(np.float64), np.repeat(k.astype(np.float64), hq // hk, 1), np.repeat(v.astype(np.float64), hq // hk, 1)
+    z = np.einsum("ihd,jhd->hij", q64, k64) * float(sc)
+    z = np.where(np.tril(np.ones((s, s), bool)), z, -np.inf)
+    size = np.einsum("ihd,jhd->hij", np.abs(q64), np.abs(k64)) * float(sc)
+    w = np.exp(z - z.max(-1, keepdims=True))
+    want = np.einsum("hij,jhd->ihd", w / w.sum(-1, keepdims=True), v64)
+    # a score is off by 2^-21 of the sum of its products' sizes at most (the halves keep 22 bits, the sums 24); a weight by as much
+    # of itself, twice with its row's sum
+    tol = 2.0 ** -20 * (1 + np.where(np.isfinite(z), size, 0).max()) * np.abs(v64).max()
+    assert np.abs(be.download(do, q.shape, np.float32) - want).max() <= tol
+    be.reset_pool()
+
+
 def _make_pool(rng, f16, nblocks, bs, hk, d):
     elems = nblocks * 2 * bs * hk * d
     vals = rng.standard_normal(elems).astype(np.float32)

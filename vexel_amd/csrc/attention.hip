@@ -1258,15 +1258,20 @@ __global__ void __launch_bounds__(64) tree_merge_kernel(const float *__restrict_
 
 // --------------------------------------------------------------------------------------------
 // Dense causal prefill (Backend.SDPAPrefill, backend.go:389; math of backend/cpu/cpu.go:568-632 per query):
-// FlashAttention-2 style. grid = (query tiles of 64, Hq); block = 256 = 4 waves of 16 queries.
-// Per 32-key tile: K goes to LDS as f16 rows, V transposed ([d][key], so that a lane's eight keys of one column are
-// 16 contiguous bytes); S = Q K^T and O += P V run on v_mfma_f32_16x16x32_f16 with every float32 operand split in
+// FlashAttention-2 style. grid = (query tiles of 64, Hq); block = 512 = two shares of a step's 64 keys x 4 waves of 16 queries.
+// Per step K and V go to LDS as f16 rows (the values' operands are read from there by columns, see read_columns); S = Q K^T and
+// O += P V run on v_mfma_f32_16x16x32_f16 with every float32 operand split in
 // two f16 halves (x = hi + lo, about 22 significant bits, float32 accumulation): Q and P always, K and V when they
 // come as float32 (dense prefill; the products hi*hi + hi*lo + lo*hi, the lo*lo term is below float32's last bit),
 // not when they are the f16 rows of the paged pool, which are exact. The softmax is online in the exp2 domain; P
-// crosses from the MFMA output layout to the operand layout through a wave-private LDS tile. LDS row pitches are
-// an odd number of 16-byte slots, so the 16 lanes of an operand read land in 16 different slots.
-constexpr int FA_BQ = 64, FA_BK = 32;
+// crosses from the MFMA output layout to the operand layout through a wave-private LDS tile; the shares' (m, l, O) meet
+// through LDS at the end. LDS row pitches are an odd number of 16-byte slots, so the 16 lanes of an operand read land in 16 different slots.
+// Bound by the chain of a step (rows to LDS, scores, softmax, weights, values) and the splitting of float32 rows beside it, so: two
+// waves a SIMD with half the keys each, products in chains that do not wait for each other, O rescaled only where a maximum has
+// grown, and no value turned by 2-byte stores. 32 heads of 128: 77 rows 11.3 -> 9.8 us, 128 14.0 -> 11.1, 256 24.0 -> 18.4, 512 43.7 -> 32.6
+// (values by columns and rows loaded along their length alone: 10.4, 12.5, 21.2, 38.6); 512 rows over 4000 paged keys in blocks of 32,
+// 8 KV heads: 263 -> 177 us.
+constexpr int FA_BQ = 64, FA_BK = 32, FA_SHARES = 2, FA_THREADS = 256 * FA_SHARES;
 
 template <int N>
 __device__ __forceinline__ float row16_max(float t) {  // max over the 16 lanes of a row; every lane gets it
@@ -1291,20 +1296,23 @@ struct PagedSrc {
 };
 
 template <int D, bool CAP = false, bool PAGED = false>
-__global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restrict__ q, const float *__restrict__ k,
+__global__ void __launch_bounds__(FA_THREADS) prefill_fa2_kernel(const float *__restrict__ q, const float *__restrict__ k,
                                                           const float *__restrict__ v, float *__restrict__ out, int S,
                                                           int num_q_heads, int num_kv_heads, float scale,
                                                           float softcap = 0.f, PagedSrc paged = PagedSrc()) {
-    constexpr int KP = D + 8, VP = FA_BK + 8, PP = FA_BK + 4;  // halves per K row, halves per V^T row, floats per P row
+    constexpr int KP = D + 8, PP = FA_BK + 4;  // halves per K or V row, floats per P row
     constexpr int NLO = PAGED ? 1 : 2;                           // [0]: hi halves, [1]: lo halves (float32 sources only)
-    __shared__ __attribute__((aligned(16))) _Float16 Ks[NLO][FA_BK * KP];
-    __shared__ __attribute__((aligned(16))) _Float16 Vt[NLO][D * VP];
-    __shared__ __attribute__((aligned(16))) float Ps[4][16 * PP];
+    constexpr int STEP = FA_BK * FA_SHARES, HALVES = NLO * STEP * KP;  // keys of a step
+    __shared__ __attribute__((aligned(16))) _Float16 kv_lds[2 * HALVES];
+    __shared__ __attribute__((aligned(16))) float Ps[4 * FA_SHARES][16 * PP];
+    _Float16(*const Ks)[STEP * KP] = (_Float16(*)[STEP * KP])kv_lds, (*const Vs)[STEP * KP] = (_Float16(*)[STEP * KP])(kv_lds + HALVES);
     __shared__ int len_max[5];  // PAGED: the longest key range among each wave's 16 queries, [4]: among all 64
     const int qt = blockIdx.x, h = blockIdx.y, kvh = h / (num_q_heads / num_kv_heads);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, g = lane >> 4;
-    const int q0 = qt * FA_BQ + wave * 16;  // the wave's first query
+    const int wq = wave & 3, share = wave >> 2;
+    const int q0 = qt * FA_BQ + wq * 16;  // the wave's first query
     const size_t qs = (size_t)num_q_heads * D, ks = (size_t)num_kv_heads * D;
     int lim[4];  // keys 0 .. lim[i]-1 are visible to the lane's query row 4g + i
 #pragma unroll
@@ -1316,11 +1324,11 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
         if (tid < 5) len_max[tid] = 0;
         __syncthreads();
         const int m4 = max(max(lim[0], lim[1]), max(lim[2], lim[3]));
-        atomicMax(&len_max[wave], m4);
+        atomicMax(&len_max[wq], m4);
         atomicMax(&len_max[4], m4);
         __syncthreads();
     }
-    const int wave_keys = PAGED ? len_max[wave] : min(q0 + 15, S - 1) + 1;  // keys any of the wave's queries sees
+    const int wave_keys = PAGED ? len_max[wq] : min(q0 + 15, S - 1) + 1;  // keys any of the wave's queries sees
 
     // Q as the A operand: lane (row c16, columns 32s + 8g .. + 7), pre-multiplied by scale*log2(e), hi + lo
     half8 qh[D / 32], ql[D / 32];
@@ -1351,19 +1359,19 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
     }
     const int last_q = min(qt * FA_BQ + FA_BQ - 1, S - 1);
     const int n_keys = PAGED ? len_max[4] : last_q + 1;  // keys 0 .. n_keys-1 are visible to some query of the tile
-    const int n_tiles = (n_keys + FA_BK - 1) / FA_BK;
+    const int n_steps = (n_keys + STEP - 1) / STEP;
     // A tile's rows as they come from memory: requested a tile ahead, so that their way is covered by the
-    // arithmetic of the tile before (a thread's pieces: key idx % 32, columns 8 (idx / 32) .. + 7).
+    // arithmetic of the tile before (a thread's pieces: key idx / (D / 8), columns 8 (idx % (D / 8)) .. + 7).
     constexpr int NIDX = FA_BK * (D / 8) / 256;
-    static_assert(NIDX * 256 == FA_BK * (D / 8), "whole trips of the 256 threads over a tile");
+    static_assert(NIDX * FA_THREADS == STEP * (D / 8), "whole trips of the threads over a step's rows");
     float4 rk[PAGED ? 1 : NIDX][2], rv[PAGED ? 1 : NIDX][2];
     half8 rkh[PAGED ? NIDX : 1], rvh[PAGED ? NIDX : 1];
     auto fetch = [&](int kt) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NIDX; t++) {
-            const int idx = tid + 256 * t;
-            const int key = idx % FA_BK, d8 = (idx / FA_BK) * 8;  // (lanes run over keys: V^T's 2-byte stores fill whole rows)
-            const int ki = kt * FA_BK + key;
+            const int idx = tid + FA_THREADS * t;
+            const int key = idx / (D / 8), d8 = idx % (D / 8) * 8;
+            const int ki = kt * STEP + key;
             if constexpr (PAGED) {
                 const half8 z = {0, 0, 0, 0, 0, 0, 0, 0};
                 rkh[t] = z;
@@ -1388,12 +1396,12 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
             }
         }
     };
-    // what fetch() brought, as f16 halves into the LDS tiles (K rows, V transposed)
+    // what fetch() brought, as f16 halves into the LDS tiles
     auto stash = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < NIDX; t++) {
-            const int idx = tid + 256 * t;
-            const int key = idx % FA_BK, d8 = (idx / FA_BK) * 8;
+            const int idx = tid + FA_THREADS * t;
+            const int key = idx / (D / 8), d8 = idx % (D / 8) * 8;
             half8 kh = {0, 0, 0, 0, 0, 0, 0, 0}, vh = kh, kl = kh, vl = kh;
             if constexpr (PAGED) {
                 kh = rkh[t];
@@ -1410,40 +1418,45 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
                 }
             }
             *(half8 *)(&Ks[0][key * KP + d8]) = kh;
-#pragma unroll
-            for (int e = 0; e < 8; e++) Vt[0][(d8 + e) * VP + key] = vh[e];
+            *(half8 *)(&Vs[0][key * KP + d8]) = vh;
             if (!PAGED) {
                 *(half8 *)(&Ks[NLO - 1][key * KP + d8]) = kl;
-#pragma unroll
-                for (int e = 0; e < 8; e++) Vt[NLO - 1][(d8 + e) * VP + key] = vl[e];
+                *(half8 *)(&Vs[NLO - 1][key * KP + d8]) = vl;
             }
         }
     };
-    if (n_tiles > 0) fetch(0);
-    for (int kt = 0; kt < n_tiles; kt++) {
-        __syncthreads();  // the previous tile's reads are done
+    if (n_steps > 0) fetch(0);
+    for (int kt = 0; kt < n_steps; kt++) {
+        __syncthreads();  // the previous step's reads are done
         stash();
-        if (kt + 1 < n_tiles) fetch(kt + 1);
+        if (kt + 1 < n_steps) fetch(kt + 1);
         __syncthreads();
-        if (kt * FA_BK >= wave_keys) continue;  // every key of the tile is beyond what the wave's queries see
+        const int key0 = kt * STEP + share * FA_BK;
+        if (key0 >= wave_keys) continue;  // every key of the share is beyond what the wave's queries see
         // S = Q K^T for the wave's 16 queries x 32 keys: lane holds S[row 4g+i][key cb*16 + c16]
-        float4v sc[FA_BK / 16];
+        float4v sc[FA_BK / 16], low[FA_BK / 16];  // the large products and the small ones, a chain each
 #pragma unroll
-        for (int cb = 0; cb < FA_BK / 16; cb++) {
-            float4v acc = {0.f, 0.f, 0.f, 0.f};
-            const int ko = (cb * 16 + c16) * KP + 8 * g;  // key cb*16 + c16, columns 32s + 8g .. + 7
+        for (int cb = 0; cb < FA_BK / 16; cb++) sc[cb] = low[cb] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int s = 0; s < D / 32; s++) {
-                const half8 b = *(const half8 *)(&Ks[0][ko + 32 * s]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[s], b, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[s], b, acc, 0, 0, 0);
-                if (!PAGED) {
-                    const half8 bl = *(const half8 *)(&Ks[NLO - 1][ko + 32 * s]);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[s], bl, acc, 0, 0, 0);
-                }
+        for (int s = 0; s < D / 32; s++) {
+            half8 b[FA_BK / 16], bl[PAGED ? 1 : FA_BK / 16];
+#pragma unroll
+            for (int cb = 0; cb < FA_BK / 16; cb++) {
+                const int ko = (share * FA_BK + cb * 16 + c16) * KP + 8 * g + 32 * s;  // key cb*16 + c16, columns 32s + 8g .. + 7
+                b[cb] = *(const half8 *)(&Ks[0][ko]);
+                if constexpr (!PAGED) bl[cb] = *(const half8 *)(&Ks[NLO - 1][ko]);
             }
-            sc[cb] = acc;
+#pragma unroll
+            for (int cb = 0; cb < FA_BK / 16; cb++) sc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[s], b[cb], sc[cb], 0, 0, 0);
+#pragma unroll
+            for (int cb = 0; cb < FA_BK / 16; cb++) low[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ql[s], b[cb], low[cb], 0, 0, 0);
+            if constexpr (!PAGED) {
+#pragma unroll
+                for (int cb = 0; cb < FA_BK / 16; cb++) low[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(qh[s], bl[cb], low[cb], 0, 0, 0);
+            }
         }
+#pragma unroll
+        for (int cb = 0; cb < FA_BK / 16; cb++) sc[cb] += low[cb];
         if (CAP) {
             const float cap2 = softcap * kLog2e, inv_cap2 = 1.f / cap2;
 #pragma unroll
@@ -1458,7 +1471,7 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
             float mx = -INFINITY;
 #pragma unroll
             for (int cb = 0; cb < FA_BK / 16; cb++) {
-                const int ki = kt * FA_BK + cb * 16 + c16;
+                const int ki = key0 + cb * 16 + c16;
                 if (ki >= lim[i]) sc[cb][i] = -INFINITY;
                 mx = fmaxf(mx, sc[cb][i]);
             }
@@ -1481,10 +1494,12 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
             l_run[i] = l_run[i] * alpha[i] + rs;
             m_run[i] = m_new;
         }
+        if (__builtin_amdgcn_ballot_w64(alpha[0] != 1.f || alpha[1] != 1.f || alpha[2] != 1.f || alpha[3] != 1.f) != 0) {
 #pragma unroll
-        for (int db = 0; db < D / 16; db++)
+            for (int db = 0; db < D / 16; db++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) o[db][i] *= alpha[i];
+                for (int i = 0; i < 4; i++) o[db][i] *= alpha[i];
+        }
         // P: MFMA output layout -> operand layout through the wave's LDS tile
         float *pt = &Ps[wave][0];
 #pragma unroll
@@ -1504,18 +1519,55 @@ __global__ void __launch_bounds__(256) prefill_fa2_kernel(const float *__restric
                 pl[e] = t.l;
             }
         }
-        // O += P V: lane holds O[row 4g+i][d = db*16 + c16]; B operand: column d, keys 8g .. 8g + 7 of V^T
+        // O += P V: lane holds O[row 4g+i][d = db*16 + c16]; B operand: column d, keys 8g .. 8g + 7, read from V's rows by columns
+        constexpr int AT = 4;  // column tiles at a time: their products are chains of their own
 #pragma unroll
-        for (int db = 0; db < D / 16; db++) {
-            const int vo = (db * 16 + c16) * VP + 8 * g;
-            const half8 vb = *(const half8 *)(&Vt[0][vo]);
-            o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb, o[db], 0, 0, 0);
-            o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb, o[db], 0, 0, 0);
-            if (!PAGED) {
-                const half8 vl = *(const half8 *)(&Vt[NLO - 1][vo]);
-                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vl, o[db], 0, 0, 0);
+        for (int d0 = 0; d0 < D / 16; d0 += AT) {
+            half8 vb[AT], vl[PAGED ? 1 : AT];
+#pragma unroll
+            for (int j = 0; j < AT; j++) {
+                const int vo = (share * FA_BK + 8 * g + (c16 >> 2)) * KP + (d0 + j) * 16 + 4 * (c16 & 3);
+                vb[j] = read_columns(&Vs[0][vo], &Vs[0][vo + 4 * KP]);
+                if constexpr (!PAGED) vl[j] = read_columns(&Vs[NLO - 1][vo], &Vs[NLO - 1][vo + 4 * KP]);
+            }
+#pragma unroll
+            for (int j = 0; j < AT; j++) o[d0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vb[j], o[d0 + j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < AT; j++) o[d0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pl, vb[j], o[d0 + j], 0, 0, 0);
+            if constexpr (!PAGED) {
+#pragma unroll
+                for (int j = 0; j < AT; j++) o[d0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ph, vl[j], o[d0 + j], 0, 0, 0);
             }
         }
+    }
+    // The second share's sums join the first's through LDS: its output where the rows were, (m, l) where the weights were.
+    static_assert(FA_SHARES == 2 && 4 * (D / 16) * 64 * sizeof(float4v) <= sizeof kv_lds && 4 * 2 * 64 * sizeof(float4v) <= sizeof Ps, "two shares' sums in LDS");
+    float4v *const so = (float4v *)kv_lds + wq * (D / 16) * 64 + lane, *const sm = (float4v *)&Ps[0][0] + wq * 2 * 64 + lane;
+    __syncthreads();
+    if (share == 1) {
+#pragma unroll
+        for (int db = 0; db < D / 16; db++) so[db * 64] = o[db];
+        sm[0] = (float4v){m_run[0], m_run[1], m_run[2], m_run[3]};
+        sm[64] = (float4v){l_run[0], l_run[1], l_run[2], l_run[3]};
+    }
+    __syncthreads();
+    if (share == 1) return;
+    float f0[4], f1[4];
+    {
+        const float4v m1 = sm[0], l1 = sm[64];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float m = fmaxf(m_run[i], m1[i]);
+            f0[i] = m_run[i] == -INFINITY ? 0.f : exp2f(m_run[i] - m);
+            f1[i] = m1[i] == -INFINITY ? 0.f : exp2f(m1[i] - m);
+            l_run[i] = l_run[i] * f0[i] + l1[i] * f1[i];
+        }
+    }
+#pragma unroll
+    for (int db = 0; db < D / 16; db++) {
+        const float4v o1 = so[db * 64];
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[db][i] = o[db][i] * f0[i] + o1[i] * f1[i];
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -1779,13 +1831,13 @@ static int sdpa_prefill_dense(vx_backend *be, const float *q, const float *k, co
         const dim3 grid(ceil_div(seq_len, FA_BQ), num_q_heads);
         if (softcap > 0.f) {
             if (head_dim == 128)
-                prefill_fa2_kernel<128, true><<<grid, 256, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale, softcap);
+                prefill_fa2_kernel<128, true><<<grid, FA_THREADS, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale, softcap);
             else
-                prefill_fa2_kernel<64, true><<<grid, 256, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale, softcap);
+                prefill_fa2_kernel<64, true><<<grid, FA_THREADS, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale, softcap);
         } else if (head_dim == 128)
-            prefill_fa2_kernel<128><<<grid, 256, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale);
+            prefill_fa2_kernel<128><<<grid, FA_THREADS, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale);
         else
-            prefill_fa2_kernel<64><<<grid, 256, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale);
+            prefill_fa2_kernel<64><<<grid, FA_THREADS, 0, be->stream>>>(q, k, v, out, seq_len, num_q_heads, num_kv_heads, scale);
         VX_CHECK_LAUNCH();
         return VX_OK;
     }
@@ -1970,10 +2022,10 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
         PagedSrc src = {(const _Float16 *)kv_pool, block_table, kv_lens, block_size};
         dim3 grid(ceil_div(query_len, FA_BQ), num_q_heads);
         if (head_dim == 128)
-            prefill_fa2_kernel<128, false, true><<<grid, 256, 0, be->stream>>>(q, nullptr, nullptr, out, query_len, num_q_heads,
+            prefill_fa2_kernel<128, false, true><<<grid, FA_THREADS, 0, be->stream>>>(q, nullptr, nullptr, out, query_len, num_q_heads,
                                                                                num_kv_heads, scale, 0.f, src);
         else
-            prefill_fa2_kernel<64, false, true><<<grid, 256, 0, be->stream>>>(q, nullptr, nullptr, out, query_len, num_q_heads,
+            prefill_fa2_kernel<64, false, true><<<grid, FA_THREADS, 0, be->stream>>>(q, nullptr, nullptr, out, query_len, num_q_heads,
                                                                               num_kv_heads, scale, 0.f, src);
         VX_CHECK_LAUNCH();
         return VX_OK;
