@@ -513,6 +513,39 @@ def test_fused_decode_blocks_equal_the_unfused_sequence(be, fmt, rows, hidden, f
     be.reset_pool()
 
 
+# past 32 rows (no epilogue), past a table of 64 rows, the largest table and one row more (no table); dense: K and V rows beside the pool
+@pytest.mark.parametrize("dense", [False, True])
+@pytest.mark.parametrize("rows", [2, 33, 65, 512, 1024, 1025])
+def test_angle_table_of_many_rows(be, rows, dense):
+    rng = np.random.default_rng(rows)
+    hidden, hq, hk, d, bs, eps, theta, fmt = 512, 4, 2, 128, 16, 1e-5, 10000.0, nx.FMT_Q8_0
+    kvd, nblocks = hk * d, (rows + 15) // 16
+    dims = dict(wq=(hidden, hidden), wk=(kvd, hidden), wv=(kvd, hidden))
+    qw = {n: be.qweight(fmt, be.upload(qz.random_quant(fmt, rng, *dims[n])), *dims[n]) for n in dims}
+    dx, dn = be.upload(rng.standard_normal((rows, hidden)).astype(np.float32)), be.upload(np.ones(hidden, dtype=np.float32))
+    dpos = be.upload(rng.integers(0, 5000, rows).astype(np.int32))
+    dslots = be.upload(rng.permutation(nblocks * bs)[:rows].astype(np.int32))
+    pool = np.zeros(nblocks * 2 * bs * kvd, dtype=np.float16)
+    outs = []
+    for table in (False, True):
+        dpool, dq, dk, dv = be.upload(pool), be.alloc(rows * hidden * 4), be.alloc(rows * kvd * 4), be.alloc(rows * kvd * 4)
+        if table:
+            be.rope_table_prepare(dpos, rows, d, theta)
+        if dense:
+            be.prefill_attn_qkv(dx, dn, eps, False, qw["wq"], qw["wk"], qw["wv"], None, None, None, rows, dpos, dslots, dpool, True,
+                                hq, hk, d, bs, theta, d, False, dq, dk, dv)
+        else:
+            be.decode_attn_qkv(dx, dn, eps, False, qw["wq"], qw["wk"], qw["wv"], rows, dpos, dslots, dpool, True, hq, hk, d, bs, theta, dq)
+        outs.append([be.download(dq, (rows, hidden), np.float32), be.download(dpool, pool.shape, pool.dtype)] +
+                    ([be.download(dk, (rows, kvd), np.float32), be.download(dv, (rows, kvd), np.float32)] if dense else []))
+    for a, b in zip(*outs):
+        if rows > 32 or dense:
+            assert np.array_equal(a, b)
+        else:  # (a launch that finishes its own rows may add the products in another order: neighbours in the pool's 11 bits)
+            assert np.abs(a.astype(np.float32) - b).max() <= 2.0 ** -10 * np.abs(a).max()
+    be.reset_pool()
+
+
 @pytest.mark.parametrize("rows", [1, 5, 32, 40])
 @pytest.mark.parametrize("fqk,fv", [(nx.FMT_Q4_K, nx.FMT_Q6_K), (nx.FMT_Q4_0, nx.FMT_Q8_0)])
 def test_decode_attn_qkv_with_v_in_another_format(be, rows, fqk, fv):

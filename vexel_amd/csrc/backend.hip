@@ -200,6 +200,7 @@ void vx_reset_pool(vx_backend *be) {
     for (auto &c : be->chunks) c.used = 0;
     be->cur_chunk = 0;
     be->items.valid = false;  // a kv_lens array taken from the pool is about to be reused
+    be->rope_tab_pos = nullptr;  // (and a positions array)
 }
 
 int vx_to_device(vx_backend *be, void *dst, const void *src_host, size_t bytes) {

@@ -47,7 +47,7 @@ struct PoolChunk {
 }  // namespace vx
 
 // chunk-parallel prepares: up to 512 rows x 64 chunks of 256 columns; two [64][512] float arrays of per-chunk sums of squares
-#define VX_ROPE_TAB_ROWS 64
+#define VX_ROPE_TAB_ROWS 1024
 #define VX_ATTN_CNT 16384
 // ints from one counter to the next: arrivals at counters that share a line wait for one another (one sequence of 2048 tokens,
 // 32 heads of 128: 14.8 us with counters side by side, 11.5 with one per 256 bytes)
