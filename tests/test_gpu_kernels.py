@@ -546,6 +546,33 @@ def test_angle_table_of_many_rows(be, rows, dense):
     be.reset_pool()
 
 
+def test_angle_table_of_a_graph_is_not_taken_for_another(be):
+    rng = np.random.default_rng(12)
+    rows, hidden, hq, hk, d, bs, eps, theta, fmt = 40, 512, 4, 2, 128, 16, 1e-5, 10000.0, nx.FMT_Q8_0
+    kvd, nblocks = hk * d, 3
+    dims = dict(wq=(hidden, hidden), wk=(kvd, hidden), wv=(kvd, hidden))
+    qw = {n: be.qweight(fmt, be.upload(qz.random_quant(fmt, rng, *dims[n])), *dims[n]) for n in dims}
+    dx, dn = be.upload(rng.standard_normal((rows, hidden)).astype(np.float32)), be.upload(np.ones(hidden, dtype=np.float32))
+    dpos, dother = (be.upload(rng.integers(0, 5000, rows).astype(np.int32)) for _ in range(2))
+    dslots, dpool = be.upload(np.arange(rows, dtype=np.int32)), be.upload(np.zeros(nblocks * 2 * bs * kvd, dtype=np.float16))
+    dq = be.alloc(rows * hidden * 4)
+
+    def project():
+        be.decode_attn_qkv(dx, dn, eps, False, qw["wq"], qw["wk"], qw["wv"], rows, dpos, dslots, dpool, True, hq, hk, d, bs, theta, dq)
+        return be.download(dq, (rows, hidden), np.float32)
+
+    want = project()
+    be.graph_begin_capture()
+    be.rope_table_prepare(dother, rows, d, theta)
+    graph = be.graph_end_capture()
+    for _ in range(3):
+        be.rope_table_prepare(dpos, rows, d, theta)
+        be.graph_launch(graph)   # (fills the table for the other positions)
+        assert np.array_equal(project(), want)
+    be.graph_destroy(graph)
+    be.reset_pool()
+
+
 @pytest.mark.parametrize("rows", [1, 5, 32, 40])
 @pytest.mark.parametrize("fqk,fv", [(nx.FMT_Q4_K, nx.FMT_Q6_K), (nx.FMT_Q4_0, nx.FMT_Q8_0)])
 def test_decode_attn_qkv_with_v_in_another_format(be, rows, fqk, fv):

@@ -255,6 +255,7 @@ int vx_graph_end_capture(vx_backend *be, vx_graph **out) {
     be->capturing = false;
     hipGraph_t graph = nullptr;
     VX_CHECK_HIP(hipStreamEndCapture(be->stream, &graph));
+    be->rope_tab_pos = nullptr;  // (a table recorded in the graph has not been filled; each replay fills it anew)
     VX_REQUIRE(out != nullptr, "out is null");
     vx_graph *g = new vx_graph();
     g->graph = graph;
@@ -274,6 +275,7 @@ int vx_graph_launch(vx_backend *be, vx_graph *g) {
     if (rc) return rc;
     VX_REQUIRE(g && g->exec, "null graph");
     VX_CHECK_HIP(hipGraphLaunch(g->exec, be->stream));
+    be->rope_tab_pos = nullptr;  // (the graph may have filled the table for positions of its own)
     return VX_OK;
 }
 
