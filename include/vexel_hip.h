@@ -277,7 +277,7 @@ int vx_decode_attn_qkv_supported(const vx_qweight *wq, const vx_qweight *wk, con
  * (one launch per layer less), with the same arithmetic; a call whose projection leaves K slices' sums (more rows, the
  * formats with a min term, V in another format) reads its cos / sin from the table in the RoPE + store launch that
  * follows. The table falls when the library writes to a caller's
- * buffer (vx_pack_batch, vx_decode_advance, vx_to_device, vx_copy_buffer), with vx_reset_pool and with graphs (vx_graph_end_capture, vx_graph_launch); a caller that changes the positions by
+ * buffer (vx_pack_batch, vx_decode_advance, vx_to_device, vx_copy_buffer), with vx_reset_pool and with graphs (vx_graph_begin_capture, vx_graph_end_capture, vx_graph_launch); a caller that changes the positions by
  * other means must call this again (or not at all: without a table nothing changes). No counterpart in the reference,
  * which recomputes the angles in every layer (backend/cpu/cpu.go:226-303). */
 int vx_rope_table_prepare(vx_backend *be, const int32_t *positions, int rows, int head_dim, float theta);

@@ -570,6 +570,17 @@ def test_angle_table_of_a_graph_is_not_taken_for_another(be):
         be.graph_launch(graph)   # (fills the table for the other positions)
         assert np.array_equal(project(), want)
     be.graph_destroy(graph)
+    # and a call recorded while a table of its positions stands does not read what stands there at the time of a replay
+    be.rope_table_prepare(dpos, rows, d, theta)
+    be.graph_begin_capture()
+    be.decode_attn_qkv(dx, dn, eps, False, qw["wq"], qw["wk"], qw["wv"], rows, dpos, dslots, dpool, True, hq, hk, d, bs, theta, dq)
+    graph = be.graph_end_capture()
+    for _ in range(3):
+        be.to_device(dq, np.zeros((rows, hidden), dtype=np.float32))
+        be.rope_table_prepare(dother, rows, d, theta)
+        be.graph_launch(graph)
+        assert np.array_equal(be.download(dq, (rows, hidden), np.float32), want)
+    be.graph_destroy(graph)
     be.reset_pool()
 
 

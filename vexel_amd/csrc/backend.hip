@@ -245,6 +245,7 @@ int vx_graph_begin_capture(vx_backend *be) {
     VX_CHECK_HIP(hipStreamSynchronize(be->stream));
     VX_CHECK_HIP(hipStreamBeginCapture(be->stream, hipStreamCaptureModeThreadLocal));
     be->capturing = true;
+    be->rope_tab_pos = nullptr;  // (a table filled before is another one by the time of a replay)
     return VX_OK;
 }
 
@@ -253,9 +254,9 @@ int vx_graph_end_capture(vx_backend *be, vx_graph **out) {
     if (rc) return rc;
     VX_REQUIRE(be->capturing, "no capture active");
     be->capturing = false;
+    be->rope_tab_pos = nullptr;  // (a table recorded in the graph has not been filled; each replay fills it anew)
     hipGraph_t graph = nullptr;
     VX_CHECK_HIP(hipStreamEndCapture(be->stream, &graph));
-    be->rope_tab_pos = nullptr;  // (a table recorded in the graph has not been filled; each replay fills it anew)
     VX_REQUIRE(out != nullptr, "out is null");
     vx_graph *g = new vx_graph();
     g->graph = graph;
