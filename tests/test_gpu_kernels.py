@@ -1268,6 +1268,62 @@ def test_paged_multiquery_value_that_is_not_finite_late_in_a_step(be, hq, hk, d,
     test_paged_multiquery_value_that_is_not_finite(be, hq, hk, d, qn, 1)
 
 
+# the blocks of a row tile in four, two and one shares, both widths
+MQ_SHARES = [(8, 2, 128, 64), (4, 4, 64, 64), (32, 8, 128, 512), (64, 4, 64, 256), (64, 8, 128, 512), (64, 4, 64, 512)]
+
+
+def _mq_out(be, q, k, v, kvl, hq, hk, d, sc, seed):
+    """Keys and values [keys, hk, d] (float16) in a pool of 16-token blocks in any order, and what each row of q gets."""
+    bs, keys, qn = 16, len(k), len(q)
+    nb = (keys + bs - 1) // bs
+    bt = np.random.default_rng(seed).permutation(nb).astype(np.int32)
+    pool = np.zeros((nb, 2, bs, hk, d), dtype=np.float16)
+    for part, x in enumerate((k, v)):
+        rows = np.zeros((nb * bs, hk, d), dtype=np.float16)
+        rows[:keys] = x
+        pool[bt, part] = rows.reshape(nb, bs, hk, d)
+    do = be.alloc(q.nbytes)
+    be.sdpa_paged_decode_multiquery(be.upload(q), be.upload(pool.reshape(-1)), be.upload(bt), do, be.upload(kvl), nb, bs, hq, hk, d, sc, qn, pool_is_f16=True)
+    out = be.download(do, q.shape, np.float32)
+    be.reset_pool()
+    return out
+
+
+def _softmax_mean64(z, kvl, v, group):
+    """z [rows, hq, keys]: scores in natural units, float64; every row's own number of keys."""
+    z = np.where(np.arange(z.shape[-1])[None, None, :] < kvl[:, None, None], z, -np.inf)
+    w = np.exp(z - z.max(-1, keepdims=True))
+    w /= w.sum(-1, keepdims=True)
+    return np.matmul(w.transpose(1, 0, 2), np.repeat(v.astype(np.float64), group, 1).transpose(1, 0, 2)).transpose(1, 0, 2)
+
+
+# From 2^24 on the neighbours of a score are 2 apart and more, and 5 or 10 below it is no number: the weights still have to fit f16.
+# keys in an order in which a share's maximum rises by one to three such steps at a time; rows of positive and of negative scores
+@pytest.mark.parametrize("e", [22, 24, 25, 26, 27, 28])
+@pytest.mark.parametrize("first", [0, 1])
+@pytest.mark.parametrize("hq,hk,d,qn", MQ_SHARES)
+def test_paged_multiquery_large_scores(be, hq, hk, d, qn, first, e):
+    rng = np.random.default_rng(e + first + qn)
+    keys = 600
+    ulp = 2.0 ** (e - 23)
+    up = first + np.cumsum([0, 3, 1, 2, 3, 1, 1, 2, 3, 3, 1, 2, 3, 1, 2, 1, 3, 3, 2])[np.arange(keys) // 32]
+    k = np.zeros((keys, hk, d), dtype=np.float16)
+    k[:, :, 0], k[:, :, 8] = 272, up[:, None]
+    v = rng.standard_normal((keys, hk, d)).astype(np.float16)
+    q = np.zeros((qn, hq, d), dtype=np.float32)
+    q[:, :, 0], q[:, :, 8] = 2.0 ** (e - 8) * rng.choice([1, -1], (qn, hq)), ulp
+    sc = np.float32(0.6931472)  # (times log2(e) 1 in float32, so that a score in base 2 is 272 q[0] + up q[8] and no rounding)
+    assert sc * np.float32(1.4426950408889634) == 1
+    kvl = rng.integers(1, keys + 1, qn).astype(np.int32)
+    kvl[0] = keys
+    got = _mq_out(be, q, k, v, kvl, hq, hk, d, sc, qn)
+    rows = np.unique(np.r_[0:40, qn // 2, qn - 18:qn].clip(0, qn - 1))
+    z = np.broadcast_to(math.log(2) * ulp * up, (len(rows), hq, keys))
+    want = _softmax_mean64(z, kvl[rows], v, hq // hk)
+    # scores and the references' distances to them are exact; weights of 22 bits, sums of 24 over up to 600 keys, mostly of one sign
+    assert np.abs(got[rows] - want).max() <= 2.0 ** -17 * np.abs(v.astype(np.float64)).max()
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])

@@ -819,7 +819,9 @@ __device__ __forceinline__ half8 read_columns(const _Float16 *a, const _Float16 
 // heads of 128: 104 -> 88 us (rescaling by need 99, steps of 64 keys and the dies 88; operands by columns alone changed nothing
 // but the registers). 32 rows a wave: 98.
 // grid = (num_kv_heads, ceil(G * row tiles / NSUB)); block = 64 * NSUB * KS.
-constexpr float MQ_LAZY = 5.f;  // a row's reference follows its largest score once that is 2^5 above it: 2^10 p stays below 2^15
+// A row's reference lies 10 below its largest score (the weights are 2^10 p) and follows it once that is more than 15 above: a weight
+// fits f16 as long as its exponent, a difference of two floats that are near each other and so exact, stays below 16.
+constexpr float MQ_MOST = 15.f;
 template <int D, int QT, int KS, int NSUB = 4>
 __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *__restrict__ q, const _Float16 *__restrict__ pool,
                                                          const int32_t *__restrict__ table, const int32_t *__restrict__ kv_lens,
@@ -946,11 +948,13 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                     if (!open && tok0 + 16 * b + 4 * i >= lim[t]) sc[t][b][i] = -INFINITY;
                     gm = fmaxf(gm, sc[t][b][i]);
                 }
-            gm = max_of_quarters(gm) * q_inv[t] - 10.f;  // (q_inv: a power of two)
-            if (__builtin_amdgcn_ballot_w64(gm > m_run[t] + MQ_LAZY) != 0) {
-                const float m_new = fmaxf(m_run[t], gm);
-                const float alpha = exp2f(m_run[t] - m_new);  // (m_new is finite in every lane that gets here with gm > m_run; 1 elsewhere)
-                const float a_own = gm > m_run[t] ? alpha : 1.f;
+            const float top = max_of_quarters(gm) * q_inv[t];  // (q_inv: a power of two)
+            if (__builtin_amdgcn_ballot_w64(top - m_run[t] > MQ_MOST) != 0) {
+                // (from 2^27 on the float next to 10 below may be 16 below: the score itself then)
+                const float below = top - 10.f, ref = top - below > MQ_MOST ? top : below;
+                const float m_new = fmaxf(m_run[t], ref);
+                const float alpha = exp2f(m_run[t] - m_new);  // (m_new is finite in every lane that gets here with ref > m_run; 1 elsewhere)
+                const float a_own = ref > m_run[t] ? alpha : 1.f;
                 m_run[t] = m_new;
                 l_run[t] *= a_own;
 #pragma unroll
