@@ -1324,6 +1324,24 @@ def test_paged_multiquery_large_scores(be, hq, hk, d, qn, first, e):
     assert np.abs(got[rows] - want).max() <= 2.0 ** -17 * np.abs(v.astype(np.float64)).max()
 
 
+@pytest.mark.parametrize("hq,hk,d,qn", MQ_SHARES)
+def test_paged_multiquery_scores_beyond_the_range_of_float32(be, hq, hk, d, qn):
+    """Not a number and no zeros, in their rows alone."""
+    keys = 200
+    rng = np.random.default_rng(5)
+    k, v = (rng.standard_normal((keys, hk, d)).astype(np.float16) for _ in range(2))
+    k[:, :, 0] = 32768
+    q = rng.standard_normal((qn, hq, d)).astype(np.float32)
+    q[:, :, 0] = 0
+    kvl = np.full(qn, keys, dtype=np.int32)
+    sc = np.float32(1 / math.sqrt(d))
+    want = _mq_out(be, q, k, v, kvl, hq, hk, d, sc, 1)
+    q[5, :, 0] = 2.0 ** 120
+    got = _mq_out(be, q, k, v, kvl, hq, hk, d, sc, 1)
+    assert np.isnan(got[5]).all() and np.isfinite(want).all()
+    assert np.array_equal(np.delete(got, 5, 0), np.delete(want, 5, 0))
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])

@@ -955,7 +955,7 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                 const float m_new = fmaxf(m_run[t], ref);
                 const float alpha = exp2f(m_run[t] - m_new);  // (m_new is finite in every lane that gets here with ref > m_run; 1 elsewhere)
                 const float a_own = ref > m_run[t] ? alpha : 1.f;
-                m_run[t] = m_new;
+                m_run[t] = m_new == INFINITY ? NAN : m_new;  // (a score beyond float32: fmaf's exact product minus infinity would be a weight of 0)
                 l_run[t] *= a_own;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
