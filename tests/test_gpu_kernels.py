@@ -1342,6 +1342,21 @@ def test_paged_multiquery_scores_beyond_the_range_of_float32(be, hq, hk, d, qn):
     assert np.array_equal(np.delete(got, 5, 0), np.delete(want, 5, 0))
 
 
+@pytest.mark.parametrize("hq,hk,d,qn", MQ_SHARES)
+def test_paged_multiquery_rows_do_not_depend_on_their_neighbours(be, hq, hk, d, qn):
+    """Every second row's scores grow a little, those between them by far more or not at all: same bits."""
+    rng = np.random.default_rng(qn)
+    keys, sc = 600, np.float32(1 / math.sqrt(d))
+    k, v = (rng.standard_normal((keys, hk, d)).astype(np.float16) for _ in range(2))
+    k[:, :, 0] = (1.0 * (np.arange(keys) // 32) / (float(sc) * math.log2(math.e)))[:, None]
+    q = (0.1 * rng.standard_normal((qn, hq, d))).astype(np.float32)
+    out = []
+    for other in (0.0, 8.0):
+        q[0::2, :, 0], q[1::2, :, 0] = 1.0, other
+        out.append(_mq_out(be, q, k, v, np.full(qn, keys, dtype=np.int32), hq, hk, d, sc, 1))
+    assert np.array_equal(out[0][0::2], out[1][0::2])
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])

@@ -949,13 +949,13 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                     gm = fmaxf(gm, sc[t][b][i]);
                 }
             const float top = max_of_quarters(gm) * q_inv[t];  // (q_inv: a power of two)
-            if (__builtin_amdgcn_ballot_w64(top - m_run[t] > MQ_MOST) != 0) {
-                // (from 2^27 on the float next to 10 below may be 16 below: the score itself then)
+            const bool follow = top - m_run[t] > MQ_MOST;  // (each row by its own scores, whatever its neighbours' are)
+            if (__builtin_amdgcn_ballot_w64(follow) != 0) {
+                // (from 2^27 on the float next to 10 below may be 16 below: the score itself then; a score beyond float32 makes the row not a
+                // number, as fmaf's exact product minus infinity would be a weight of 0)
                 const float below = top - 10.f, ref = top - below > MQ_MOST ? top : below;
-                const float m_new = fmaxf(m_run[t], ref);
-                const float alpha = exp2f(m_run[t] - m_new);  // (m_new is finite in every lane that gets here with ref > m_run; 1 elsewhere)
-                const float a_own = ref > m_run[t] ? alpha : 1.f;
-                m_run[t] = m_new == INFINITY ? NAN : m_new;  // (a score beyond float32: fmaf's exact product minus infinity would be a weight of 0)
+                const float a_own = follow ? exp2f(m_run[t] - ref) : 1.f;
+                if (follow) m_run[t] = ref == INFINITY ? NAN : ref;
                 l_run[t] *= a_own;
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
