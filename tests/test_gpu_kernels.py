@@ -1357,6 +1357,36 @@ def test_paged_multiquery_rows_do_not_depend_on_their_neighbours(be, hq, hk, d, 
     assert np.array_equal(out[0][0::2], out[1][0::2])
 
 
+# Height of a key's score (base 2) by its step of 64 keys (32 with four shares). A reference follows a maximum that is 2^5 above it:
+# just under that and every second step over it; far over it at each step; a share of the steps far below the others; a last key above all.
+@pytest.mark.parametrize("heights", ["under", "over", "share", "last"])
+@pytest.mark.parametrize("hq,hk,d,qn", MQ_SHARES)
+def test_paged_multiquery_growing_scores(be, hq, hk, d, qn, heights):
+    rng = np.random.default_rng(qn + d + len(heights))
+    shares = 1 if hq * qn >= 16 * 2048 else (2 if hq * qn >= 16 * 1024 else 4)
+    step, keys = (32, 300) if shares == 4 else (64, 600)
+    at = np.arange(keys) // step
+    t = {"under": 4.6 * at, "over": 7.0 * at, "share": np.where(at % max(shares, 2) == 1, -60.0, 0.0), "last": np.where(np.arange(keys) == keys - 1, 40.0, 0.0)}[heights]
+    sc = np.float32(1 / math.sqrt(d))
+    k = rng.standard_normal((keys, hk, d)).astype(np.float16)
+    k[:, :, 0] = (t / (float(sc) * math.log2(math.e)))[:, None]
+    v = rng.standard_normal((keys, hk, d)).astype(np.float16)
+    q = (0.1 * rng.standard_normal((qn, hq, d))).astype(np.float32)
+    q[:, :, 0] = rng.choice([1.0, 1.0, 0.5, 0.0, -1.0], (qn, hq))  # the rows of a tile rise, stay or fall
+    kvl = rng.integers(keys - step - 3, keys + 1, qn).astype(np.int32)
+    kvl[:4] = keys
+    kvl[4:8] = [1, step, step + 1, 2 * step]
+    got = _mq_out(be, q, k, v, kvl, hq, hk, d, sc, qn)
+    rows = np.unique(np.r_[0:40, qn // 2, qn - 18:qn].clip(0, qn - 1))
+    k64, q64 = np.repeat(k.astype(np.float64), hq // hk, 1).transpose(1, 2, 0), q[rows].astype(np.float64).transpose(1, 0, 2)
+    z, size = (float(sc) * np.matmul(f(q64), f(k64)).transpose(1, 0, 2) for f in (lambda x: x, np.abs))
+    want = _softmax_mean64(z, kvl[rows], v, hq // hk)
+    # a score is off by 2^-21 of the sum of its products' sizes at most (halves of 22 bits, sums of 24), a weight by as much of itself,
+    # twice with its row's sum
+    tol = 2.0 ** -20 * (1 + size.max()) * np.abs(v.astype(np.float64)).max()
+    assert np.abs(got[rows] - want).max() <= tol
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])
