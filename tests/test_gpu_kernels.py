@@ -1387,6 +1387,22 @@ def test_paged_multiquery_growing_scores(be, hq, hk, d, qn, heights):
     assert np.abs(got[rows] - want).max() <= tol
 
 
+def test_paged_multiquery_more_workgroups_than_a_second_dimension_takes(be):
+    """131090 rows of 32 heads over one KV head: 65552 workgroups a KV head. The rows repeat every 1024, so do their results."""
+    hq, hk, d, qn, keys = 32, 1, 64, 131090, 40
+    rng = np.random.default_rng(6)
+    k, v = (rng.standard_normal((keys, hk, d)).astype(np.float16) for _ in range(2))
+    base = rng.standard_normal((1024, hq, d)).astype(np.float32)
+    q = np.resize(base, (qn, hq, d))
+    sc = np.float32(1 / math.sqrt(d))
+    got = _mq_out(be, q, k, v, np.full(qn, keys, dtype=np.int32), hq, hk, d, sc, 1)
+    z = float(sc) * np.matmul(base.astype(np.float64), k[:, 0].astype(np.float64).T)
+    want = _softmax_mean64(z, np.full(1024, keys), v, hq)
+    _close(got[:1024], want, 1e-5, 3e-6, "first rows")
+    for r in range(1024, qn, 1024):
+        assert np.array_equal(got[r:r + 1024], got[:min(1024, qn - r)]), r
+
+
 # one split (the workgroup's own result, nothing to merge), a full round of eight-split groups for the waves that share a chunk
 # (four for 32 heads of 128, two for 8 x 64) and one split more, a second round
 @pytest.mark.parametrize("hq,hk,d", [(32, 4, 64), (32, 32, 128), (32, 8, 128), (8, 8, 64)])

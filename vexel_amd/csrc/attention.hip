@@ -818,7 +818,8 @@ __device__ __forceinline__ half8 read_columns(const _Float16 *a, const _Float16 
 // of it; two waves a SIMD go through the same chain (scores, softmax, weights, values) at the same time. 512 rows over 4096 keys, 32 / 8
 // heads of 128: 104 -> 88 us (rescaling by need 99, steps of 64 keys and the dies 88; operands by columns alone changed nothing
 // but the registers). 32 rows a wave: 98.
-// grid = (num_kv_heads, ceil(G * row tiles / NSUB)); block = 64 * NSUB * KS.
+// grid = num_kv_heads * ceil(G * row tiles / NSUB), the KV heads next to each other (a second dimension would end at 65536: 131072 rows of
+// 32 heads over one); block = 64 * NSUB * KS.
 // A row's reference lies 10 below its largest score (the weights are 2^10 p) and follows it once that is more than 15 above: a weight
 // fits f16 as long as its exponent, a difference of two floats that are near each other and so exact, stays below 16.
 constexpr float MQ_MOST = 15.f;
@@ -828,13 +829,13 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                                                          float *__restrict__ out, int query_len, int max_keys, int num_q_heads,
                                                          int num_kv_heads, float scale) {
     constexpr int NS = D / 32, NT = D / 16;
-    const int kvh = blockIdx.x, G = num_q_heads / num_kv_heads;
+    const int kvh = blockIdx.x % num_kv_heads, nth = blockIdx.x / num_kv_heads, G = num_q_heads / num_kv_heads;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = wave % NSUB, ksub = wave / NSUB;  // which of the workgroup's NSUB (head, row group) pairs, which share of the blocks
     const int row_groups = (query_len + 16 * QT - 1) / (16 * QT);
-    const bool idle = blockIdx.y * NSUB + sub >= G * row_groups;  // (a wave without work walks no block; it still meets the others)
-    const int combo = min((int)blockIdx.y * NSUB + sub, G * row_groups - 1);
+    const bool idle = nth * NSUB + sub >= G * row_groups;  // (a wave without work walks no block; it still meets the others)
+    const int combo = min(nth * NSUB + sub, G * row_groups - 1);
     const int head = kvh * G + combo % G, r0 = (combo / G) * 16 * QT;
     const int c16 = lane & 15, g4 = lane >> 4;
     const size_t hs = (size_t)num_kv_heads * D, part = (size_t)HOT_BS * hs, qs = (size_t)num_q_heads * D;
@@ -2021,7 +2022,7 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
         const int max_keys = num_blocks * block_size;
 #define VX_MQ(DD, KK, NS)                                                                                                 \
     if (head_dim == DD && share == KK)                                                                                    \
-        paged_mq_kernel<DD, QT, KK, NS><<<dim3(num_kv_heads, ceil_div(combos, NS)), 64 * NS * KK, 0, be->stream>>>(         \
+        paged_mq_kernel<DD, QT, KK, NS><<<num_kv_heads * ceil_div(combos, NS), 64 * NS * KK, 0, be->stream>>>(               \
             q, pool, block_table, kv_lens, out, query_len, max_keys, num_q_heads, num_kv_heads, scale);
         // (heads of 128 with four shares: two pairs a workgroup, so that a wave keeps 256 registers)
         VX_MQ(128, 1, 4) VX_MQ(128, 2, 4) VX_MQ(128, 4, 2) VX_MQ(64, 1, 4) VX_MQ(64, 2, 4) VX_MQ(64, 4, 4)
