@@ -73,35 +73,83 @@ def test_every_piece_arrives(ring, helpers):
     assert r.returncode == 0 and r.stdout.split("\n")[:-1] == ["%d ok" % n for n in sizes], (r.returncode, r.stdout)
 
 
-# A sender that keeps a launch back until the stream is asked, as a kernel may be late; "lost" leaves the last launch out.
-SENDER = HARNESS[:HARNESS.index("int main")] + r"""
+# A sender whose launches run one behind the other on a thread, as on a stream. "h": they begin when the stream is asked about, as behind a
+# long step; "s": a helper thread copies its first piece when the stream has been found at its end; "l": the last launch is lost.
+SENDER = HARNESS[:HARNESS.index('#include "transfer_ring.h"')] + r"""
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <mutex>
 #include <thread>
+static std::thread::id caller;
+static std::atomic<bool> slow{false};
+static std::atomic<int> holding{0}, found_over{0};
+static void await(const std::atomic<int> &what) {
+    for (const auto end = std::chrono::steady_clock::now() + std::chrono::seconds(20); what.load() == 0; std::this_thread::yield())
+        if (std::chrono::steady_clock::now() > end) abort();
+}
+static thread_local bool device = false;
+static void copy_slowly(void *d, const void *s, size_t n) {
+    if (slow.load() && !device) {
+        if (std::this_thread::get_id() == caller) await(holding);  // (so that the helpers get pieces)
+        else holding++, await(found_over);
+    }
+    memcpy(d, s, n);
+}
+#define memcpy copy_slowly
+#include "transfer_ring.h"
 struct Late : vx::Mover::Sender {
-    std::deque<std::thread> running;
-    bool lose = false;
-    int sends = 0;
+    struct Launch { const vx::Mover *m; const vx::Mover::Job *j; int from, to; };
+    std::mutex mu;
+    std::condition_variable more;
+    std::deque<Launch> queue;
+    int free_to_run = 0, launched = 0, finished = 0;
+    bool hold = false, lose = false, stop = false;
+    std::thread runs{[this] { run(); }};
+    ~Late() override {
+        { std::lock_guard<std::mutex> g(mu); stop = true; }
+        more.notify_all();
+        runs.join();
+    }
+    void run() {
+        device = true;
+        std::unique_lock<std::mutex> l(mu);
+        for (;;) {
+            more.wait(l, [&] { return stop || (finished < launched && (!hold || finished < free_to_run)); });
+            if (stop) return;
+            const Launch a = queue.front();
+            l.unlock();
+            for (int i = a.from; i < a.to; i++) {
+                std::this_thread::yield();
+                if (i >= vx::Mover::SENT_SLOTS && !a.j->copied[i - vx::Mover::SENT_SLOTS].load()) abort();  // the slot is still in use
+                memcpy(a.m->ring + (size_t)(i % vx::Mover::SENT_SLOTS) * vx::Mover::SENT_SLOT, a.j->pieces[i].src, a.j->pieces[i].bytes);
+                __atomic_store_n(a.m->marks + (size_t)(i % vx::Mover::SENT_SLOTS) * vx::Mover::MARK_STEP, vx::Mover::mark_of(*a.j, i), __ATOMIC_RELEASE);
+            }
+            l.lock();
+            queue.pop_front();
+            finished++;
+        }
+    }
     hipError_t send(hipStream_t, const vx::Mover &m, const vx::Mover::Job &j, int from, int to) override {
         if (to - from < 1 || to - from > vx::Mover::SENT_MOST) return 5;
-        sends++;
         if (lose && to == (int)j.pieces.size()) return 0;
-        if (!running.empty()) running.back().join(), running.pop_back();  // (one launch behind the other)
-        running.emplace_back([&m, &j, from, to] {
-            for (int i = from; i < to; i++) {
-                std::this_thread::yield();
-                if (i >= vx::Mover::SENT_SLOTS && !j.copied[i - vx::Mover::SENT_SLOTS].load()) abort();  // the slot is still in use
-                memcpy(m.ring + (size_t)(i % vx::Mover::SENT_SLOTS) * vx::Mover::SENT_SLOT, j.pieces[i].src, j.pieces[i].bytes);
-                __atomic_store_n(m.marks + (size_t)(i % vx::Mover::SENT_SLOTS) * vx::Mover::MARK_STEP, vx::Mover::mark_of(j, i), __ATOMIC_RELEASE);
-            }
-        });
+        { std::lock_guard<std::mutex> g(mu); queue.push_back({&m, &j, from, to}); launched++; }
+        more.notify_all();
         return 0;
     }
-    void wait() { while (!running.empty()) running.back().join(), running.pop_back(); }
-    hipError_t ask(hipStream_t, bool *over) override { *over = lose; return 0; }
+    hipError_t ask(hipStream_t, bool *over) override {
+        std::lock_guard<std::mutex> g(mu);
+        free_to_run = launched;
+        more.notify_all();
+        *over = finished == launched;
+        if (*over) found_over++;
+        return 0;
+    }
     hipError_t lost() override { return 9; }
 };
 int main(int argc, char **argv) {
     const int helpers = atoi(argv[1]);
+    caller = std::this_thread::get_id();
     vx::Mover m;
     m.marks = (uint64_t *)calloc(vx::Mover::SENT_SLOTS * vx::Mover::MARK_STEP, 8);
     Late *late = new Late;
@@ -109,17 +157,20 @@ int main(int argc, char **argv) {
     if (!m.start(helpers) || (int)m.workers.size() != helpers) return 2;
     const size_t piece = 4099;
     for (int i = 2; i < argc; i++) {
-        const int n = abs(atoi(argv[i]));
-        late->lose = atoi(argv[i]) < 0;
+        const int n = atoi(argv[i] + strcspn(argv[i], "0123456789"));
+        { std::lock_guard<std::mutex> g(late->mu); late->hold = strchr(argv[i], 'h'), late->lose = strchr(argv[i], 'l'); }
+        slow = strchr(argv[i], 's') && helpers > 0;
+        holding = 0, found_over = 0;
         std::string from(n * piece, 0), to(n * piece, 0);
         for (size_t k = 0; k < from.size(); k++) from[k] = (char)(k * 2654435761u >> 13);
         std::vector<vx::Mover::Piece> pieces;
         for (int k = 0; k < n; k++) pieces.push_back({&to[k * piece], &from[k * piece], piece});
         vx::Mover::Job job(std::move(pieces));
         const int rc = m.move(0, job);
-        late->wait();
         if (late->lose ? rc != 9 : rc != 0 || from != to) return 3;
-        printf("%d ok\n", atoi(argv[i]));
+        if (slow && (holding.load() == 0 || found_over.load() == 0)) return 4;
+        if (late->hold && late->free_to_run == 0) return 6;
+        printf("%s ok\n", argv[i]);
         fflush(stdout);
     }
     return 0;
@@ -129,11 +180,12 @@ int main(int argc, char **argv) {
 
 @pytest.mark.parametrize("helpers", [0, 1, 6])
 def test_every_sent_piece_arrives(tmp_path, helpers):
-    """Both sides of a launch (64 pieces), of the ring (256 slots) and of several turns of it; a stream that ends without its
-    last launch is an error and not a wait without an end, and what comes after it is whole again."""
+    """Both sides of a launch (64 pieces), of the ring (256 slots) and of several turns of it; launches that come late; a stream found
+    at its end while pieces that have arrived are still to be copied, which is no loss; a stream that ends without its last launch,
+    which is an error and not a wait without an end, and what comes after it is whole again."""
     src, exe = tmp_path / "sent.cpp", tmp_path / "sent"
     src.write_text(SENDER)
     subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "vexel_amd", "csrc"), str(src), "-o", str(exe)], check=True)
-    sizes = [1, 63, 64, 65, 255, 256, 257, -3, 320, 321, -300, 1000]
-    r = subprocess.run([str(exe), str(helpers)] + [str(n) for n in sizes], capture_output=True, text=True, timeout=60)
-    assert r.returncode == 0 and r.stdout.split("\n")[:-1] == ["%d ok" % n for n in sizes], (r.returncode, r.stdout)
+    jobs = ["1", "63", "64", "65", "255", "256", "257", "l3", "320", "321", "l300", "1000", "h1", "h257", "h600", "s65", "s257", "s320", "s600", "hs400", "l65", "s256"]
+    r = subprocess.run([str(exe), str(helpers)] + jobs, capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.split("\n")[:-1] == [j + " ok" for j in jobs], (r.returncode, r.stdout)

@@ -170,7 +170,7 @@ struct Mover {
                 awake = true;
                 wake_workers(j);
             }
-            if (take_arrived(j)) continue;
+            if (awake && take_arrived(j)) continue;  // (not before: piece 256 may take the slot that says that they can be woken)
             made = std::max(made, j.next.load());
             if (made < n) made = make_pages(j.pieces[made]) ? made + 1 : n;
             else std::this_thread::yield();
@@ -178,7 +178,7 @@ struct Mover {
                 bool over = false;
                 err = sender->ask(stream, &over);
                 for (int i = out; i < sent && over && err == hipSuccess; i++)
-                    if (!here(j, i) && !j.copied[i].load(std::memory_order_acquire)) err = sender->lost();
+                    if (!here(j, i)) err = sender->lost();  // (no slot has been given to a later piece: those wait for `out`)
             }
         }
         if (err != hipSuccess) j.failed.store(true);
