@@ -16,7 +16,7 @@ HARNESS = r"""
 typedef int hipError_t;
 typedef int hipStream_t;
 typedef int *hipEvent_t;
-enum { hipSuccess = 0, hipMemcpyDeviceToHost = 2, hipHostMallocDefault = 0, hipEventDisableTiming = 2 };
+enum { hipSuccess = 0, hipErrorNotReady = 600, hipMemcpyDeviceToHost = 2, hipHostMallocDefault = 0, hipEventDisableTiming = 2 };
 struct Pending { void *dst; const void *src; size_t bytes; hipEvent_t event; };
 static std::deque<Pending> pending;
 static hipError_t hipHostMalloc(void **p, size_t n, unsigned) { *p = malloc(n); return 0; }
@@ -25,6 +25,9 @@ static hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = new in
 static hipError_t hipEventDestroy(hipEvent_t e) { delete e; return 0; }
 static hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, int, hipStream_t) { pending.push_back({d, s, n, nullptr}); return 0; }
 static hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { pending.back().event = e; return 0; }
+static hipError_t last_error = hipSuccess;
+static hipError_t hipGetLastError() { const hipError_t e = last_error; last_error = hipSuccess; return e; }
+static hipError_t hipStreamQuery(hipStream_t);
 #include <string.h>
 static hipError_t hipEventSynchronize(hipEvent_t e) {
     while (!pending.empty()) {
@@ -36,6 +39,7 @@ static hipError_t hipEventSynchronize(hipEvent_t e) {
     return 0;
 }
 #include "transfer_ring.h"
+static hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 int main(int argc, char **argv) {
     const int helpers = atoi(argv[1]);
     vx::Mover m;
@@ -135,25 +139,28 @@ struct Late : vx::Mover::Sender {
         if (lose && to == (int)j.pieces.size()) return 0;
         { std::lock_guard<std::mutex> g(mu); queue.push_back({&m, &j, from, to}); launched++; }
         more.notify_all();
-        return 0;
+        return hipGetLastError();
     }
-    hipError_t ask(hipStream_t, bool *over) override {
+    hipError_t query() {
         std::lock_guard<std::mutex> g(mu);
         free_to_run = launched;
         more.notify_all();
-        *over = finished == launched;
-        if (*over) found_over++;
-        return 0;
+        if (finished == launched) found_over++;
+        return finished == launched ? hipSuccess : hipErrorNotReady;
     }
     hipError_t lost() override { return 9; }
 };
+static Late *late = nullptr;
+static hipError_t hipStreamQuery(hipStream_t) {  // a runtime that keeps "not ready" as the last error
+    const hipError_t e = late->query();
+    return e == hipSuccess ? e : last_error = e;
+}
 int main(int argc, char **argv) {
     const int helpers = atoi(argv[1]);
     caller = std::this_thread::get_id();
     vx::Mover m;
     m.marks = (uint64_t *)calloc(vx::Mover::SENT_SLOTS * vx::Mover::MARK_STEP, 8);
-    Late *late = new Late;
-    m.sender = late;
+    m.sender = late = new Late;
     if (!m.start(helpers) || (int)m.workers.size() != helpers) return 2;
     const size_t piece = 4099;
     for (int i = 2; i < argc; i++) {

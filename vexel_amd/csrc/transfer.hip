@@ -90,11 +90,6 @@ struct KernelSender : Mover::Sender {
         send_kernel<<<std::min(SEND_GROUPS, to - from), SEND_THREADS, 0, stream>>>(a);
         return hipGetLastError();
     }
-    hipError_t ask(hipStream_t stream, bool *over) override {
-        const hipError_t e = hipStreamQuery(stream);
-        *over = e == hipSuccess;
-        return e == hipErrorNotReady ? hipSuccess : e;
-    }
     hipError_t lost() override { return hipErrorUnknown; }
 };
 

@@ -41,7 +41,13 @@ struct Mover {
         // Enqueues pieces from .. to - 1: each to its slot, then its mark behind it.
         virtual hipError_t send(hipStream_t stream, const Mover &m, const Job &j, int from, int to) = 0;
         // hipSuccess while the stream has work left, *over once it has none
-        virtual hipError_t ask(hipStream_t stream, bool *over) = 0;
+        virtual hipError_t ask(hipStream_t stream, bool *over) {
+            const hipError_t e = hipStreamQuery(stream);
+            *over = e == hipSuccess;
+            if (e != hipErrorNotReady) return e;
+            (void)hipGetLastError();  // (what a query leaves there is not the error of the next launch)
+            return hipSuccess;
+        }
         virtual hipError_t lost() = 0;  // the error for pieces that will not come
     };
     char *ring = nullptr;
