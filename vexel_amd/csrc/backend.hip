@@ -84,7 +84,8 @@ int vx_backend_create(int device_id, vx_backend **out) {
     VX_CHECK_HIP(hipEventCreate(&be->ev0));
     VX_CHECK_HIP(hipEventCreate(&be->ev1));
     be->host_stage_bytes = 1 << 20;
-    VX_CHECK_HIP(hipHostMalloc(&be->host_stage, be->host_stage_bytes, hipHostMallocDefault));
+    // (coherent: kernels read staged uploads there, whose bytes the host writes anew between launches)
+    VX_CHECK_HIP(hipHostMalloc(&be->host_stage, be->host_stage_bytes, hipHostMallocCoherent));
     be->misc_ws_bytes = 1 << 20;
     VX_CHECK_HIP(hipMalloc(&be->misc_ws, be->misc_ws_bytes));
     VX_CHECK_HIP(hipMalloc(&be->rope_tab, (size_t)VX_ROPE_TAB_ROWS * VX_ROPE_TAB_PAIRS * 2 * sizeof(float)));
