@@ -10,6 +10,8 @@
 // behind it costs 13 us beside the bytes, so 4.1 MB in eight pieces took 206 us of 73 and 32.8 MB in 32 pieces 1047 of 586. One
 // kernel sends up to 64 pieces of 64 KiB instead, each with a mark in pinned memory behind it that the threads look at:
 // 4.1 MB in 95 us, 32.8 MB in 633, 1 MB in 44 (88 before). More threads than six, none.
+#include <memory>
+
 #include "common.h"
 #include "transfer_ring.h"
 
@@ -158,14 +160,13 @@ static int download(vx_backend *be, int n, void *const *dst, const void *const *
     Mover *mover = nullptr;
     if (!pinned) {
         std::lock_guard<std::mutex> g(be->stage_mu);
-        if (!be->mover) {
-            be->mover = new Mover();
-            use_sender(be->mover);
-            if (!be->mover->start(std::min<int>(Mover::MAX_WORKERS, std::max(1u, std::thread::hardware_concurrency()) - 1))) {
-                delete be->mover;
-                be->mover = nullptr;
+        if (!be->mover) {  // (kept when it is whole, whatever throws before)
+            std::unique_ptr<Mover> made(new Mover());
+            use_sender(made.get());
+            if (made->start(std::min<int>(Mover::MAX_WORKERS, std::max(1u, std::thread::hardware_concurrency()) - 1)))
+                be->mover = made.release();
+            else
                 (void)hipGetLastError();
-            }
         }
         mover = be->mover;
     }
