@@ -421,9 +421,7 @@ void launch_prefill(vx_backend *be, Args a, const vx_ragged *b) {
     const size_t o = KS > 1 ? (size_t)4 / KS * QT * 16 * (VD * 16 + 4) * 4 : 0;
     // Late tiles, the longest, first. Where the workgroups are all resident from the start, two to a compute unit, the second of a
     // unit's two goes the other way, so that a long one meets a short one (2048 rows of 16 / 4 heads x 128: 79 -> 65 us).
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, be->device) != hipSuccess) cus = 0;
-    const int units = cus / a.p.kv_heads;
+    const int units = be->cus / a.p.kv_heads;
     a.first_round = prefill_waves<KD, VD, QT, MAPS>() == 2 && units > 0 && a.tiles > units && a.tiles <= 2 * units ? units : a.tiles;
     if (a.tiles > 0) prefill_kernel<KD, VD, QT, KS, MAPS><<<a.tiles * a.p.kv_heads, 256, lut > o ? lut : o, be->stream>>>(a);
 }

@@ -73,6 +73,7 @@ int vx_backend_create(int device_id, vx_backend **out) {
     }
     vx_backend *be = new vx_backend();
     be->device = device_id;
+    be->cus = prop.multiProcessorCount;
     {
         int rc = attn_noalloc_init(be);
         if (rc) {

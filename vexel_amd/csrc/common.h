@@ -59,6 +59,7 @@ struct PoolChunk {
 
 struct vx_backend {
     int device = 0;
+    int cus = 0;  // compute units
     hipStream_t stream = nullptr;
     bool capturing = false;
     const char *last_matmul = "";  // kernel family of the last quantized matmul launch (vx_last_matmul_kernel)
