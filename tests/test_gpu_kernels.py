@@ -1,6 +1,7 @@
 """GPU parity: every C-ABI compute entry point against the CPU oracle on the same seeded
 inputs. Integer/byte results (dequantised weights, scatter layout, argmax, packing) are
 compared bit-exactly; floating point within the stated tolerances."""
+import ctypes
 import math
 
 import numpy as np
@@ -513,36 +514,49 @@ def test_fused_decode_blocks_equal_the_unfused_sequence(be, fmt, rows, hidden, f
     be.reset_pool()
 
 
+def _overwrite(be, dst, a):
+    """Bytes into device memory by the runtime alone, which the library does not see."""
+    be.sync()
+    assert ctypes.CDLL("libamdhip64.so").hipMemcpy(ctypes.c_void_p(dst), ctypes.c_void_p(a.ctypes.data), ctypes.c_size_t(a.nbytes), 1) == 0
+
+
 # past 32 rows (no epilogue), past a table of 64 rows, the largest table and one row more (no table); dense: K and V rows beside the pool
 @pytest.mark.parametrize("dense", [False, True])
 @pytest.mark.parametrize("rows", [2, 33, 65, 512, 1024, 1025])
 def test_angle_table_of_many_rows(be, rows, dense):
+    """The positions change behind the library's back once the table is prepared: up to 1024 rows the table's are what counts."""
     rng = np.random.default_rng(rows)
     hidden, hq, hk, d, bs, eps, theta, fmt = 512, 4, 2, 128, 16, 1e-5, 10000.0, nx.FMT_Q8_0
     kvd, nblocks = hk * d, (rows + 15) // 16
     dims = dict(wq=(hidden, hidden), wk=(kvd, hidden), wv=(kvd, hidden))
     qw = {n: be.qweight(fmt, be.upload(qz.random_quant(fmt, rng, *dims[n])), *dims[n]) for n in dims}
     dx, dn = be.upload(rng.standard_normal((rows, hidden)).astype(np.float32)), be.upload(np.ones(hidden, dtype=np.float32))
-    dpos = be.upload(rng.integers(0, 5000, rows).astype(np.int32))
+    first, other = (rng.integers(0, 5000, rows).astype(np.int32) for _ in range(2))
     dslots = be.upload(rng.permutation(nblocks * bs)[:rows].astype(np.int32))
     pool = np.zeros(nblocks * 2 * bs * kvd, dtype=np.float16)
-    outs = []
-    for table in (False, True):
+
+    def project(positions, then=None):
+        dpos = be.upload(positions)
         dpool, dq, dk, dv = be.upload(pool), be.alloc(rows * hidden * 4), be.alloc(rows * kvd * 4), be.alloc(rows * kvd * 4)
-        if table:
+        if then is not None:
             be.rope_table_prepare(dpos, rows, d, theta)
+            _overwrite(be, dpos, then)
         if dense:
             be.prefill_attn_qkv(dx, dn, eps, False, qw["wq"], qw["wk"], qw["wv"], None, None, None, rows, dpos, dslots, dpool, True,
                                 hq, hk, d, bs, theta, d, False, dq, dk, dv)
         else:
             be.decode_attn_qkv(dx, dn, eps, False, qw["wq"], qw["wk"], qw["wv"], rows, dpos, dslots, dpool, True, hq, hk, d, bs, theta, dq)
-        outs.append([be.download(dq, (rows, hidden), np.float32), be.download(dpool, pool.shape, pool.dtype)] +
-                    ([be.download(dk, (rows, kvd), np.float32), be.download(dv, (rows, kvd), np.float32)] if dense else []))
-    for a, b in zip(*outs):
+        return ([be.download(dq, (rows, hidden), np.float32), be.download(dpool, pool.shape, pool.dtype)] +
+                ([be.download(dk, (rows, kvd), np.float32), be.download(dv, (rows, kvd), np.float32)] if dense else []))
+
+    got, want = project(first, other), project(first if rows <= 1024 else other)
+    for a, b in zip(want, got):
         if rows > 32 or dense:
             assert np.array_equal(a, b)
-        else:  # (a launch that finishes its own rows may add the products in another order: neighbours in the pool's 11 bits)
-            assert np.abs(a.astype(np.float32) - b).max() <= 2.0 ** -10 * np.abs(a).max()
+        else:  # (a launch that finishes its own rows may add the products in another order: the sums of 16 steps of 32 columns and of up to
+            # five slices and waves, 24 roundings of 2^-24 on either side of four times the largest result; neighbours in the pool's 11 bits)
+            tol = 2.0 ** -16 if a.dtype == np.float32 else 2.0 ** -10
+            assert np.abs(a.astype(np.float32) - b).max() <= tol * np.abs(a).max()
     be.reset_pool()
 
 
