@@ -270,16 +270,18 @@ int vx_dequantize_packed(vx_backend *be, const vx_qweight *w, float *dst);
  * most 32 rows one launch still computes the three (its row groups shared out between the two formats), otherwise V is
  * a launch of its own between the shared prepare and the shared RoPE + store. */
 int vx_decode_attn_qkv_supported(const vx_qweight *wq, const vx_qweight *wk, const vx_qweight *wv, int head_dim);
-/* Optional, once per step (decode, prompt chunk, verification) before the layers' vx_decode_attn_qkv calls: works out cos / sin of every (row,
- * dimension pair) for positions[0 .. rows-1] (up to 1024 rows, heads up to 256) and keeps them in the backend. While the
- * table stands, a vx_decode_attn_qkv call with the same positions pointer, at most 32 rows, an unbiased interleaved
- * whole-head RoPE and weights laid out for a single K slice rotates and stores its rows inside the projection launch
- * (one launch per layer less), with the same arithmetic; a call whose projection leaves K slices' sums (more rows, the
- * formats with a min term, V in another format) reads its cos / sin from the table in the RoPE + store launch that
- * follows. The table falls when the library writes to a caller's
- * buffer (vx_pack_batch, vx_decode_advance, vx_to_device, vx_copy_buffer), with vx_reset_pool and with graphs (vx_graph_begin_capture, vx_graph_end_capture, vx_graph_launch); a caller that changes the positions by
- * other means must call this again (or not at all: without a table nothing changes). No counterpart in the reference,
- * which recomputes the angles in every layer (backend/cpu/cpu.go:226-303). */
+/* Optional, once per step (decode, prompt chunk, verification) after the step's last upload and before the layers'
+ * vx_decode_attn_qkv, vx_decode_attn_qkv_ex or vx_prefill_attn_qkv calls: works out cos / sin of every (row, dimension
+ * pair) for positions[0 .. rows-1] (up to 1024 rows, heads up to 256) and keeps them in the backend. While the table
+ * stands, a vx_decode_attn_qkv call with the same positions pointer, at most 32 rows, an unbiased interleaved whole-head
+ * RoPE and weights laid out for a single K slice rotates and stores its rows inside the projection launch (one launch
+ * per layer less), with the same arithmetic; a call of that RoPE whose projection leaves K slices' sums (more rows, the
+ * formats with a min term, V in another format, vx_prefill_attn_qkv) reads its cos / sin from the table in the RoPE +
+ * store launch that follows. The table falls whenever the library writes to a caller's buffer, whichever it is (vx_pack_batch,
+ * vx_decode_advance, vx_to_device, vx_to_device_staged, vx_to_device_staged_many, vx_copy_buffer, vx_fill_zero) or frees
+ * one (vx_free), with vx_reset_pool and with graphs (vx_graph_begin_capture, vx_graph_end_capture, vx_graph_launch); a
+ * caller that changes the positions by other means must call this again (or not at all: without a table nothing
+ * changes). No counterpart in the reference, which recomputes the angles in every layer (backend/cpu/cpu.go:226-303). */
 int vx_rope_table_prepare(vx_backend *be, const int32_t *positions, int rows, int head_dim, float theta);
 int vx_decode_attn_qkv(vx_backend *be, const float *x, const float *norm_weight, float eps, int x_prepared,
                        const vx_qweight *wq, const vx_qweight *wk, const vx_qweight *wv, int rows,
