@@ -807,13 +807,13 @@ __device__ __forceinline__ half8 read_columns(const _Float16 *a, const _Float16 
 // layouts, with QT tiles of 16 consecutive query rows of one head per wave instead of 16 (row, head) queries of one
 // KV head and the per-row limits as the mask. A workgroup holds NSUB (head of the KV head's group, row tile) pairs
 // next to each other - the same rows for the heads that share the K/V rows, or neighbouring row tiles - times KS
-// shares of the pairs of blocks (pair b belongs to share b % KS). The NSUB waves of a share bring each pair into LDS
+// shares of the steps (step s belongs to share s % KS). The NSUB waves of a share bring each step's blocks into LDS
 // together, whole rows per load instruction, and read their operands from there, so the K/V rows pass through the
 // memory system once per workgroup; the shares' (m, l, O) meet in LDS at the end and share 0 writes the rows.
-// A step is two pairs of blocks where LDS holds them (one with four shares of 128 columns): the values' product fills a 16 x 16 x 32
-// instruction, maximum, rescaling and barrier come once per 64 keys, and one pair's weights go beside the other's product. The
+// A step is two pairs of blocks, with four shares one pair (PAIRS): the values' product fills a 16 x 16 x 32
+// instruction, maximum, rescaling and barrier come once per 64 (32) keys, and one pair's weights go beside the other's product. The
 // values' operands are read from LDS by columns (read_columns), not put together from rows by 32 permutes a pair. A KV head's workgroups
-// are a grid's neighbours eight apart, so with eight KV heads they run on one die and find its rows in that die's L2.
+// lie num_kv_heads apart in the grid: where that is a multiple of the eight dies, they run on one and find its rows in that die's L2.
 // What is left is waiting: the matrix pipes are busy a third of the time, vector and matrix instructions could issue in half
 // of it; two waves a SIMD go through the same chain (scores, softmax, weights, values) at the same time. 512 rows over 4096 keys, 32 / 8
 // heads of 128: 104 -> 88 us (rescaling by need 99, steps of 64 keys and the dies 88; operands by columns alone changed nothing
@@ -901,9 +901,9 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
     const int len_top = __builtin_amdgcn_readfirstlane(len_max);
     const int tok_row = 4 * (c16 & 3) + (c16 >> 2);  // this lane's K row of a block as A operand
     constexpr int KP = D + 8, VP = D + 16;           // halves per staged row of K (rows 4 banks apart) and of V (8 banks)
-    // [share][buffer][K, V][row of the pair]; behind the loop the shares' outputs lie there
-    // pairs to a buffer: two where LDS holds them, so that the waves meet half as often and one pair's scores can go beside the other's
-    // weights
+    // [share][buffer][K, V][row of the step]; behind the loop the shares' outputs lie there
+    // pairs to a buffer: two, so that the waves meet half as often and one pair's scores can go beside the other's weights, where all
+    // shares' buffers stay below 150 KB (two with four shares take 304 KB, of 64 columns 152: one there)
     constexpr int PAIRS = KS * 2 * 2 * PT * (KP + VP) * 2 <= 150 * 1024 ? 2 : 1;
     constexpr int STAGE = PAIRS * PT * (KP + VP), V_AT = PAIRS * PT * KP, SO_FLOATS = (KS - 1) * NSUB * QT * 4 * NT * 64;
     constexpr int SMEM = KS * 2 * STAGE * 2 > SO_FLOATS * 4 ? KS * 2 * STAGE * 2 : SO_FLOATS * 4;
@@ -988,9 +988,9 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
         }
     };
     {
-        // The NSUB waves that share a pair of blocks (same KV head, same share of the pairs) bring it into LDS together, whole
+        // The NSUB waves that share a step's blocks (same KV head, same share of the steps) bring them into LDS together, whole
         // rows per load instruction, once for all of them, and each reads its operands from there: one pass over
-        // the K/V rows per workgroup instead of one per wave. Two buffers, one barrier per pair; the loop runs to
+        // the K/V rows per workgroup instead of one per wave. Two buffers, one barrier per step; the loop runs to
         // the longest of the workgroup's row tiles for every wave.
         constexpr int TG = NSUB * 64, PIECES = PAIRS * PT * D / 8, PPT = (PIECES + TG - 1) / TG;
         static_assert(PIECES % TG == 0, "every lane moves whole pieces");
@@ -1006,8 +1006,8 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
         const int last_block = max((wg_len + HOT_BS - 1) / HOT_BS - 1, 0);
         const int tg = sub * 64 + lane;
         half8 kreg[PPT], vreg[PPT];
-        // Numbers of a pair's blocks, asked for a pair before the rows. (A pair whose second block is beyond the last takes that one twice:
-        // its keys are masked, its values cleared.)
+        // Numbers of a step's blocks, asked for a step of the share before the rows. (Blocks beyond the last are that one again: their keys
+        // are masked, their values cleared. Number 0 is read where no row sees a key, too: a table has a block at least.)
         int blk[2 * PAIRS];
         auto number = [&](int gi) {
 #pragma unroll
@@ -1062,7 +1062,7 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
         l_run[t] += __shfl_xor(l_run[t], 32, 64);
     }
     if constexpr (KS > 1) {
-        __syncthreads();  // (the last pairs have been read)
+        __syncthreads();  // (the last steps have been read)
 #pragma unroll
         for (int t = 0; t < QT; t++) {
             if (g4 == 0) {
@@ -1156,7 +1156,8 @@ __global__ void __launch_bounds__(D) paged_merge_kernel(const float *__restrict_
 // in 16-byte pieces, and the splits' sums, the keys and the values are asked for together (256 rows of 16 trees, 32 heads of 128: 25 -> 15 us).
 // A row sees its own path only, a few of its tree's keys, and a context has a few splits of the eight that a round holds: which they are
 // is the same in all lanes, so the others are passed over instead of being added with a weight of 0, and 64 registers let all of those
-// rows' waves run at once (15.6 -> 13.9 us; 128 rows 10.7 -> 9.4, 64 rows 7.7 -> 6.9; four heads a workgroup: 16.7).
+// rows' waves run at once (15.6 -> 13.9 us; 128 rows 10.7 -> 9.4, 64 rows 7.7 -> 6.9; four heads a workgroup: 16.7). Heads of 128 would
+// take 66 registers and spill four of them for that, 12 bytes a lane.
 template <int D>
 __global__ void __launch_bounds__(64, 8) tree_merge_kernel(const float *__restrict__ partial, const float *__restrict__ q,
                                                        const _Float16 *__restrict__ pool, const int32_t *__restrict__ bt_matrix,
@@ -2024,7 +2025,7 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
     if (head_dim == DD && share == KK)                                                                                    \
         paged_mq_kernel<DD, QT, KK, NS><<<num_kv_heads * ceil_div(combos, NS), 64 * NS * KK, 0, be->stream>>>(               \
             q, pool, block_table, kv_lens, out, query_len, max_keys, num_q_heads, num_kv_heads, scale);
-        // (heads of 128 with four shares: two pairs a workgroup, so that a wave keeps 256 registers)
+        // (heads of 128 with four shares: two (head, row tile) pairs a workgroup, so that a wave keeps 256 registers)
         VX_MQ(128, 1, 4) VX_MQ(128, 2, 4) VX_MQ(128, 4, 2) VX_MQ(64, 1, 4) VX_MQ(64, 2, 4) VX_MQ(64, 4, 4)
 #undef VX_MQ
         VX_CHECK_LAUNCH();

@@ -77,8 +77,8 @@ __device__ __forceinline__ float diff_factor(const Args &a, int lane, O &&diff) 
 // The four waves of a workgroup: 4 / KS groups of QT x 16 queries (of QT / MAPS x 16 (row, head) pairs), KS waves to a group that
 // take turns at the key groups.
 // What bounds it is the time from a load to its use: a wave asks for the next group's keys behind this one's scores and for this one's
-// values ahead of them. So there are two waves a SIMD wherever a wave's queries, output, keys and values (up to 160 registers) leave
-// room for it, block numbers come a group further ahead than keys, and a wave's number is known to be the same in its lanes.
+// values ahead of them. So there are two waves a SIMD wherever a wave's queries, output, keys and values take up to 160 registers (at 160,
+// KD 4, VD 8 and two tiles, six registers are spilled for it), block numbers come a group further ahead than keys, and a wave's number is known to be the same in its lanes.
 // 2048 rows of 16 / 4 heads x 128 with a bias table: 101 -> 65 us (two waves 96, uniform numbers 85, numbers ahead and no branches
 // per element of the bias 79, long tiles beside short ones 65).
 template <int KD, int VD, int QT, int MAPS> constexpr int prefill_waves() { return 4 * (QT * (KD + VD) + MAPS * 2 * KD + VD) <= 160 ? 2 : 1; }
