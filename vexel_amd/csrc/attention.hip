@@ -903,7 +903,7 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
     constexpr int KP = D + 8, VP = D + 16;           // halves per staged row of K (rows 4 banks apart) and of V (8 banks)
     // [share][buffer][K, V][row of the step]; behind the loop the shares' outputs lie there
     // pairs to a buffer: two, so that the waves meet half as often and one pair's scores can go beside the other's weights, where all
-    // shares' buffers stay below 150 KB (two with four shares take 304 KB, of 64 columns 152: one there)
+    // shares' buffers stay below 150 KB (two with four shares take 280 KB, of 64 columns 152: one there)
     constexpr int PAIRS = KS * 2 * 2 * PT * (KP + VP) * 2 <= 150 * 1024 ? 2 : 1;
     constexpr int STAGE = PAIRS * PT * (KP + VP), V_AT = PAIRS * PT * KP, SO_FLOATS = (KS - 1) * NSUB * QT * 4 * NT * 64;
     constexpr int SMEM = KS * 2 * STAGE * 2 > SO_FLOATS * 4 ? KS * 2 * STAGE * 2 : SO_FLOATS * 4;
