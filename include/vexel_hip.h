@@ -67,6 +67,11 @@ int vx_to_device(vx_backend *be, void *dst, const void *src_host, size_t bytes);
 int vx_to_host(vx_backend *be, void *dst_host, const void *src, size_t bytes);
 /* vx_to_host of n ranges with one wait; a null src or zero bytes is left out. */
 int vx_to_host_many(vx_backend *be, int n, void *const *dst_host, const void *const *src, const size_t *bytes);
+/* A hint, ahead of the work whose results a later vx_to_host_many will bring: threads of the backend make the destinations' pages
+ * (large ordinary memory only) while the caller enqueues it. The memory stays valid until vx_to_host_forget has returned, which
+ * stops them; *token is 0, and nothing is to be forgotten, where there is nothing to do or another download is expected. */
+int vx_to_host_expect(vx_backend *be, int n, void *const *dst_host, const size_t *bytes, int *token);
+void vx_to_host_forget(vx_backend *be, int token);
 /* vx_to_device that does not wait for the copy: src_host may be changed at once, and later calls on this backend see the
  * bytes; whoever reads dst by other means waits (vx_sync). More than 64 KiB: vx_to_device. */
 int vx_to_device_staged(vx_backend *be, void *dst, const void *src_host, size_t bytes);

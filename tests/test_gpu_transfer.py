@@ -113,3 +113,22 @@ def test_staged_uploads_of_several_ranges(be, sizes, shift):
             s[:] = 255 - s                                 # the bytes are taken when the call returns
         assert np.array_equal(be.download(d, (total,), np.uint8), want)
     be.free(d)
+
+
+# both sides of the smallest announced size; fresh memory, memory in use, a destination left out
+@pytest.mark.parametrize("size", [2 * MB - 64, 2 * MB + 5, 9 * MB])
+def test_expected_download(be, size):
+    src = np.random.default_rng(size).integers(0, 256, size, dtype=np.uint8)
+    d = be.upload(src, permanent=True)
+    for used in (False, True):
+        out = np.zeros(size, dtype=np.uint8) if used else np.empty(size, dtype=np.uint8)
+        if used:
+            out[:] = 1
+        token = C.c_int(-1)
+        dst, num = (C.c_void_p * 2)(out.ctypes.data, None), (C.c_size_t * 2)(size, 7)
+        be.call("vx_to_host_expect", 2, dst, num, C.byref(token))
+        assert token.value >= 0 and (token.value == 0 or not used) and (token.value == 0 or size >= 2 * MB)
+        be.to_host(out, d)
+        be.lib_call("vx_to_host_forget", be._h, token.value)
+        assert np.array_equal(out, src)
+    be.free(d)

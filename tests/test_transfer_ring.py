@@ -196,3 +196,72 @@ def test_every_sent_piece_arrives(tmp_path, helpers):
     jobs = ["1", "63", "64", "65", "255", "256", "257", "l3", "320", "321", "l300", "1000", "h1", "h257", "h600", "s65", "s257", "s320", "s600", "hs400", "l65", "s256"]
     r = subprocess.run([str(exe), str(helpers)] + jobs, capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.split("\n")[:-1] == [j + " ok" for j in jobs], (r.returncode, r.stdout)
+
+
+# Memory that is announced before its transfer: all its pages come, what is in it stays, nothing touches it once it is forgotten.
+AHEAD = HARNESS[:HARNESS.index("int main(")] + r"""
+#include <chrono>
+static const size_t PAGE = 4096, N = 600 * PAGE + 123;
+static char *fresh() { return (char *)mmap(nullptr, N, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0); }
+static int missing(const char *p) {
+    int n = 0;
+    for (size_t i = 0; i * PAGE < N; i++) {
+        unsigned char c = 0;
+        if (mincore((void *)(p + i * PAGE), PAGE, &c) != 0 || !(c & 1)) n++;
+    }
+    return n;
+}
+static std::vector<vx::Mover::Piece> pieces_of(char *dst, const char *src) {
+    std::vector<vx::Mover::Piece> p;
+    for (size_t at = 0; at < N; at += vx::Mover::SENT_SLOT) p.push_back({dst + at, src ? src + at : nullptr, std::min(vx::Mover::SENT_SLOT, N - at)});
+    return p;
+}
+int main(int argc, char **argv) {
+    const int helpers = atoi(argv[1]);
+    vx::Mover m;
+    if (!m.start(helpers)) return 2;
+    char *a = fresh();
+    a[5 * PAGE + 7] = 42;
+    if (!vx::Mover::pages_missing(a, N)) return 3;
+    const int t = m.expect(pieces_of(a, nullptr));
+    if ((t != 0) != (helpers > 0)) return 4;
+    if (helpers > 0 && m.expect(pieces_of(a, nullptr)) != 0) return 5;  // one at a time
+    m.forget(t + 1);                                                    // (somebody else's)
+    const auto end = std::chrono::steady_clock::now() + std::chrono::seconds(20);
+    while (helpers > 0 && missing(a) > 0)
+        if (std::chrono::steady_clock::now() > end) return 6;
+    std::string from(N, 0);
+    for (size_t k = 0; k < N; k++) from[k] = (char)(k * 2654435761u >> 13);
+    if (helpers > 0 && (a[5 * PAGE + 7] != 42 || a[5 * PAGE + 8] != 0 || vx::Mover::pages_missing(a, N))) return 7;
+    vx::Mover::Job job(pieces_of(a, from.data()));
+    if (m.move(0, job) != 0 || memcmp(a, from.data(), N) != 0) return 8;  // while it is still announced
+    m.forget(t);
+    m.forget(t);
+    munmap(a, N);
+    for (int i = 0; i < 200; i++) {  // forgotten at once, with and without the transfer, and gone afterwards
+        char *b = fresh();
+        const int u = m.expect(pieces_of(b, nullptr));
+        if ((u != 0) != (helpers > 0) || (u != 0 && u == t)) return 9;
+        if (i % 3 == 0) {
+            vx::Mover::Job again(pieces_of(b, from.data()));
+            if (m.move(0, again) != 0 || memcmp(b, from.data(), N) != 0) return 10;
+        }
+        m.forget(u);
+        munmap(b, N);
+    }
+    char *gone = fresh();  // memory that is not there is nobody's fault
+    munmap(gone, N);
+    m.forget(m.expect(pieces_of(gone, nullptr)));
+    puts("ok");
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("helpers", [0, 1, 6])
+def test_pages_of_expected_transfers(tmp_path, helpers):
+    src, exe = tmp_path / "ahead.cpp", tmp_path / "ahead"
+    src.write_text(AHEAD)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "vexel_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe), str(helpers)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout)

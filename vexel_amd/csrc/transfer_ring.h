@@ -62,6 +62,12 @@ struct Mover {
     uint64_t turn = 0;
     int inside = 0;
     bool stop = false;
+    // Destinations of a transfer that is still to come (expect).
+    std::vector<Piece> ahead;
+    std::atomic<int> ahead_next{0};
+    bool making = false;              // a helper is at it
+    std::atomic<int> ahead_token{0};  // which expect() it is, 0: none
+    int tokens = 0;
 
     ~Mover() {
         {
@@ -147,6 +153,45 @@ struct Mover {
         }
         wake.notify_all();
     }
+    // Whether pages of [dst, dst + bytes) are missing, by a few of them: memory that a caller has used before has them all.
+    static bool pages_missing(const char *dst, size_t bytes) {
+        const uintptr_t page = 4096, first = (uintptr_t)dst / page, last = ((uintptr_t)dst + bytes - 1) / page;
+        for (int i = 0; i <= 4; i++) {
+            unsigned char in_core = 1;
+            if (mincore((void *)((first + (last - first) * (uintptr_t)i / 4) * page), page, &in_core) == 0 && !(in_core & 1)) return true;
+        }
+        return false;
+    }
+    // The pages of these pieces' destinations will be written by a transfer that has not begun: a helper has them made from now on. One:
+    // several wait for each other (64 KiB take one thread 6 us, three at once 40).
+    // -> what forget() takes, 0 where nothing was begun (no helpers, or another transfer is expected already)
+    int expect(std::vector<Piece> pieces) {
+        std::lock_guard<std::mutex> g(mu);
+        if (ahead_token.load() != 0 || workers.empty() || pieces.empty()) return 0;
+        ahead = std::move(pieces);
+        ahead_next.store(0);
+        tokens = tokens == 0x7FFFFFFF ? 1 : tokens + 1;
+        ahead_token.store(tokens);
+        wake.notify_one();
+        return tokens;
+    }
+    // No thread touches what was announced under this token when this returns.
+    void forget(int token) {
+        std::unique_lock<std::mutex> l(mu);
+        if (token == 0 || token != ahead_token.load()) return;
+        ahead_next.store((int)ahead.size());
+        left.wait(l, [&] { return !making; });
+        ahead.clear();
+        ahead_token.store(0);
+    }
+    bool pages_wanted() const { return !making && ahead_next.load() < (int)ahead.size(); }
+    void make_ahead() {
+        for (;;) {
+            const int i = ahead_next.fetch_add(1);
+            if (i >= (int)ahead.size()) return;
+            if (!make_pages(ahead[i])) ahead_next.store((int)ahead.size());
+        }
+    }
     // The threads are out of the job when this returns.
     void finish() {
         std::unique_lock<std::mutex> l(mu);
@@ -177,7 +222,7 @@ struct Mover {
                 wake_workers(j);
             }
             if (awake && take_arrived(j)) continue;  // (not before: piece 256 may take the slot that says that they can be woken)
-            made = std::max(made, j.next.load());
+            made = ahead_token.load() != 0 ? n : std::max(made, j.next.load());
             if (made < n) made = make_pages(j.pieces[made]) ? made + 1 : n;
             else std::this_thread::yield();
             if (polls % 8192 == 0) {  // a stream that has ended without the pieces will not bring them
@@ -195,8 +240,17 @@ struct Mover {
         uint64_t seen = 0;
         std::unique_lock<std::mutex> l(mu);
         for (;;) {
-            wake.wait(l, [&] { return stop || (job && turn != seen); });
+            wake.wait(l, [&] { return stop || (job && turn != seen) || pages_wanted(); });
             if (stop) return;
+            if (!(job && turn != seen)) {
+                making = true;
+                l.unlock();
+                make_ahead();
+                l.lock();
+                making = false;
+                left.notify_all();
+                continue;
+            }
             seen = turn;
             Job *j = job;
             inside++;

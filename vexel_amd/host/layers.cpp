@@ -806,6 +806,7 @@ int mix_step(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_t *q_l
     if (!one_each) VHC(plan_expand(m, n_seqs, q_lens, lens, seq_tables, &ex));
     VXC(vx_pack_batch(be, d_slots, d_pos, one_each ? nullptr : d_q, n_seqs, T, m->d_tables, c.max_blocks_per_seq, m->d_num_blocks,
                       m->d_free, m->d_free_count, c.block_size, d_cu, d_tp, d_sm, d_kvl, m->d_status));
+    const Expected expected(be, logits_out, (size_t)n_want * c.vocab * 4);
     const vx_ragged b{T, n_seqs, one_each ? nullptr : q_lens, max_kv, d_cu, d_tp, d_sm, d_slots, d_kvl, m->d_tables, c.max_blocks_per_seq,
                       c.block_size};
     VHC(mix_forward(m, b, d_tok, acts, ex.rows > 0 ? &ex : nullptr, n_want ? d_want : nullptr, n_want, logits));

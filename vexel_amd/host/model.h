@@ -272,6 +272,21 @@ struct Uploads {
     int send(vx_backend *be) const { return vx_to_device_staged_many(be, (int)dst.size(), dst.data(), src.data(), bytes.data()); }
 };
 
+// A destination of the caller's that a step will fill at its end: its pages are made while the step is enqueued (vx_to_host_expect),
+// until this goes out of scope.
+struct Expected {
+    vx_backend *be;
+    int token = 0;
+    Expected(vx_backend *b, void *dst, size_t bytes) : be(b) {
+        if (dst) (void)vx_to_host_expect(be, 1, &dst, &bytes, &token);
+    }
+    ~Expected() {
+        if (token) vx_to_host_forget(be, token);
+    }
+    Expected(const Expected &) = delete;
+    Expected &operator=(const Expected &) = delete;
+};
+
 // A model whose mixer program is complete in m->mix (weights included): caches, states, activations.
 int mix_finish(vh_model *m);
 // Embedding of b.rows tokens -> layer runs -> final norm and head of n_want rows (want: device row numbers, NULL = the

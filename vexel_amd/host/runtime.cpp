@@ -942,6 +942,7 @@ int vh_decode_batched(vh_model *m, const int32_t *tokens, const int64_t *seq_ids
         VXC(vx_to_device_staged(m->be, m->d_slot_map, slot_map.data(), (size_t)batch * 4));
         VXC(vx_to_device_staged(m->be, m->d_kv_lens, kv_lens.data(), (size_t)batch * 4));
     }
+    const Expected expected(m->be, logits_out, (size_t)batch * c.vocab * 4);
     VHC(forward_decode(m, batch, max_kv));
     void *dst[2] = {argmax_out, logits_out};
     const void *src[2] = {argmax_out ? m->d_next : nullptr, logits_out ? m->logits : nullptr};
@@ -1012,6 +1013,7 @@ int vh_prefill(vh_model *m, const int32_t *tokens, int n, int64_t seq_id, int st
     }
     vx_backend *be = m->be;
     vx_reset_pool(be);
+    const Expected expected(be, logits_out, (size_t)(all_logits ? n : 1) * c.vocab * 4);
     const size_t qd = (size_t)c.num_heads * c.head_dim, kvd = (size_t)c.num_kv_heads * c.head_dim;
     auto fa = [&](size_t count) { return (float *)vx_alloc(be, count * 4); };
     auto ia = [&](size_t count) { return (int32_t *)vx_alloc(be, count * 4); };
@@ -1309,6 +1311,7 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
     }
     vx_backend *be = m->be;
     vx_reset_pool(be);
+    const Expected expected(be, logits_out, (size_t)(n_seqs + nodes_total) * c.vocab * 4);
     const int n = total;
     const size_t qd = (size_t)c.num_heads * c.head_dim, kvd = (size_t)c.num_kv_heads * c.head_dim;
     auto fa = [&](size_t count) { return (float *)vx_alloc(be, count * 4); };

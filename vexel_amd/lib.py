@@ -29,6 +29,8 @@ SIGNATURES = {
     "vx_to_device": (_i, [_vp, _vp, _vp, _sz]),
     "vx_to_host": (_i, [_vp, _vp, _vp, _sz]),
     "vx_to_host_many": (_i, [_vp, _i, _vp, _vp, _vp]),
+    "vx_to_host_expect": (_i, [_vp, _i, _vp, _vp, _vp]),
+    "vx_to_host_forget": (None, [_vp, _i]),
     "vx_to_device_staged": (_i, [_vp, _vp, _vp, _sz]),
     "vx_to_device_staged_many": (_i, [_vp, _i, _vp, _vp, _vp]),
     "vx_sync": (_i, [_vp]),
