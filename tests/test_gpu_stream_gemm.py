@@ -100,6 +100,24 @@ def test_matmul_packed_vs_oracle(be, n, k, m, fmt):
     be.reset_pool()
 
 
+# Workgroups of five and six tiles (1285 over 256 compute units): groups of one, two and four tiles between two barriers with an odd one at
+# the end, units asked for past a workgroup's last tile, sums added up a group later
+@pytest.mark.parametrize("m", [16, 32, 64])
+@pytest.mark.parametrize("fmt", FMTS)
+def test_matmul_packed_several_groups_a_workgroup(be, m, fmt):
+    n, k = 16 * 1285, 256
+    rng = np.random.default_rng(m + fmt)
+    w = qz.random_quant(fmt, rng, n, k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    want = nx.matmul_quant(fmt, a, w, m, n, k)
+    dw, _ = _packed(be, w, n, k, fmt)
+    da, dout = be.upload(a), be.alloc(m * n * 4)
+    be.matmul_quant(fmt, da, dw, dout, None, m, n, k)
+    _close(be.download(dout, (m, n), np.float32), want, 2e-5, 2e-6 * np.abs(want).max() + 1e-7, "%d rows" % m)
+    be.free(dw)
+    be.reset_pool()
+
+
 # more than 64 rows: the kernel whose waves own weight tiles and share the activation through LDS
 # (n, k): fewer tiles than a workgroup's waves own; tiles not a multiple of a wave's; many K slices; a long K
 @pytest.mark.parametrize("n,k", [(16, 256), (80, 1024), (1040, 2304), (4112, 512), (208, 11008)])
