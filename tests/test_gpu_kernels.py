@@ -1663,6 +1663,55 @@ def test_rope_store_paged(be, rope_dim, neox, d):
 
 
 # ------------------------------------------------------------------ packing: bit exact
+@pytest.mark.parametrize("batch", [1, 63, 64, 65, 200])
+@pytest.mark.parametrize("q_lens", ["none", "ones", "mixed"])
+def test_pack_batch_by_waves(be, batch, q_lens):
+    """A launch of as many waves as the batch or its new tokens fill: one wave, its last lanes, two waves, several; new blocks at block edges;
+    the work list left behind gives the attention of the grid bit for bit."""
+    rng = np.random.default_rng(batch + len(q_lens))
+    bs, mb, hq, hk, d = 16, 80, 2, 2, 64
+    pos = rng.integers(0, 1200, batch).astype(np.int32)
+    pos[::3] = pos[::3] // bs * bs                       # the new token opens a block
+    pos[-1] = 511
+    ql = rng.integers(1, 40, batch).astype(np.int32) if q_lens == "mixed" else np.ones(batch, np.int32)
+    slots = rng.permutation(batch).astype(np.int32)
+    had = (pos + bs - 1) // bs
+    need = (pos + ql - 1) // bs + 1 - had
+    perm = rng.permutation(int((had + need).sum()) + 5).astype(np.int32)
+    free = perm[:int(need.sum()) + 5]
+    tables, nblk, at = np.zeros((batch, mb), np.int32), np.zeros(batch, np.int32), free.size
+    for i, s in enumerate(slots):
+        tables[s, :had[i]] = perm[at:at + had[i]]
+        nblk[s] = had[i]
+        at += had[i]
+    want, top = tables.copy(), free.size
+    for i, s in enumerate(slots):
+        want[s, had[i]:had[i] + need[i]] = free[top - need[i]:top][::-1]
+        top -= need[i]
+    tokens = [(s, int(p) + j) for s, p, n in zip(slots, pos, ql) for j in range(n)]
+    total = len(tokens)
+    dt, dn, df, dc = be.upload(tables), be.upload(nblk), be.upload(free), be.upload(np.array([free.size], np.int32))
+    ds, dp, dq = be.upload(slots), be.upload(pos), be.upload(ql)
+    cu, tp, sm, kl, st = be.alloc((batch + 1) * 4), be.alloc(total * 4), be.alloc(total * 4), be.alloc(batch * 4), be.alloc(4)
+    be.pack_batch(ds, dp, 0 if q_lens == "none" else dq, batch, total, dt, mb, dn, df, dc, bs, cu, tp, sm, kl, st)
+    assert be.download(st, (1,), np.int32)[0] == 0 and be.download(dc, (1,), np.int32)[0] == top
+    assert np.array_equal(be.download(cu, (batch + 1,), np.int32), np.concatenate([[0], np.cumsum(ql)]))
+    assert np.array_equal(be.download(tp, (total,), np.int32), [p for _, p in tokens])
+    assert np.array_equal(be.download(sm, (total,), np.int32), [want[s, p // bs] * bs + p % bs for s, p in tokens])
+    assert np.array_equal(be.download(kl, (batch,), np.int32), pos + ql)
+    assert np.array_equal(be.download(dt, tables.shape, np.int32), want)
+    assert np.array_equal(be.download(dn, (batch,), np.int32)[slots], had + need)
+    pool = be.upload(_make_pool(rng, True, perm.size, bs, hk, d))
+    q = be.upload(rng.standard_normal((batch, hq, d)).astype(np.float32))
+    o_list, o_grid, kl2 = be.alloc(batch * hq * d * 4), be.alloc(batch * hq * d * 4), be.alloc(batch * 4)
+    sc = np.float32(1 / math.sqrt(d))
+    be.sdpa_paged_decode_ragged(q, pool, True, dt, kl, o_list, batch, mb, bs, hq, hk, d, sc, mb * bs, table_rows=ds)
+    be.copy_buffer(kl, 0, kl2, 0, batch * 4)
+    be.sdpa_paged_decode_ragged(q, pool, True, dt, kl2, o_grid, batch, mb, bs, hq, hk, d, sc, mb * bs, table_rows=ds)
+    assert np.array_equal(be.download(o_list, (batch, hq, d), np.uint32), be.download(o_grid, (batch, hq, d), np.uint32))
+    be.reset_pool()
+
+
 def test_pack_batch_bit_exact(be):
     rng = np.random.default_rng(40)
     bs, max_blocks, nslots, pool_blocks = 16, 20, 12, 150

@@ -8,6 +8,8 @@
 // order and every layer's free list evolves identically, sequence i's new blocks are the
 // entries free[F-1-rank_i-j], rank_i = exclusive prefix sum of the blocks needed by the
 // sequences before it. Two prefix scans (blocks needed, new tokens) give every output.
+#include <algorithm>
+
 #include "common.h"
 
 using namespace vx;
@@ -16,35 +18,39 @@ namespace {
 
 constexpr int PK_THREADS = 1024;
 
-// Exclusive scan over blockDim.x values held one per thread; returns the exclusive prefix and
-// writes the total to *total (same value in every thread). Each wave scans its 64 values by shuffles, the first wave
-// then the 16 waves' sums (sm: at least PK_THREADS / 64 ints).
-__device__ int block_exclusive_scan(int v, int *sm, int *total) {
+// Exclusive scans over four values of each of blockDim.x threads; returns the exclusive prefixes and writes the totals to *total (the
+// same in every thread). Each wave scans its 64 threads' by shuffles, all four values at every step (a shuffle is waited for, and one
+// after the other they are most of a small step's launch), the first wave then the waves' sums (sm: at least PK_THREADS / 64).
+__device__ int4 block_exclusive_scan4(const int4 v, int4 *sm, int4 *total) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int NWAVES = PK_THREADS / 64;
-    int incl = v;
+    const int n_waves = blockDim.x >> 6;
+    const auto inclusive = [&](int4 x, int most) {
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int t = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += t;
+        for (int off = 1; off < 64; off <<= 1) {
+            if (off >= most) break;
+            const int4 t = make_int4(__shfl_up(x.x, off, 64), __shfl_up(x.y, off, 64), __shfl_up(x.z, off, 64), __shfl_up(x.w, off, 64));
+            if (lane >= off) x.x += t.x, x.y += t.y, x.z += t.z, x.w += t.w;
+        }
+        return x;
+    };
+    const auto minus = [](int4 a, int4 b) { return make_int4(a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w); };
+    const int4 incl = inclusive(v, 64);
+    if (n_waves == 1) {
+        *total = make_int4(__shfl(incl.x, 63, 64), __shfl(incl.y, 63, 64), __shfl(incl.z, 63, 64), __shfl(incl.w, 63, 64));
+        return minus(incl, v);
     }
-    __syncthreads();  // (whoever still reads sm from an earlier use is done)
     if (lane == 63) sm[wave] = incl;
     __syncthreads();
     if (wave == 0) {
-        int w = lane < NWAVES ? sm[lane] : 0;
-#pragma unroll
-        for (int off = 1; off < NWAVES; off <<= 1) {
-            const int t = __shfl_up(w, off, 64);
-            if (lane >= off) w += t;
-        }
-        if (lane < NWAVES) sm[lane] = w;          // inclusive sums of the waves
+        const int4 w = inclusive(lane < n_waves ? sm[lane] : make_int4(0, 0, 0, 0), PK_THREADS / 64);
+        if (lane < n_waves) sm[lane] = w;          // inclusive sums of the waves
     }
     __syncthreads();
-    const int before = wave > 0 ? sm[wave - 1] : 0;
-    *total = sm[NWAVES - 1];
-    __syncthreads();  // (the caller may write sm next)
-    return before + incl - v;
+    *total = sm[n_waves - 1];
+    const int4 e = minus(incl, v);
+    if (wave == 0) return e;
+    const int4 before = sm[wave - 1];
+    return make_int4(before.x + e.x, before.y + e.y, before.z + e.z, before.w + e.w);
 }
 
 __global__ void __launch_bounds__(PK_THREADS) pack_batch_kernel(
@@ -52,28 +58,35 @@ __global__ void __launch_bounds__(PK_THREADS) pack_batch_kernel(
     int32_t *block_tables, int max_blocks, int32_t *num_blocks, int32_t *free_list, int32_t *free_count,
     int block_size, int32_t *cu_seqlens, int32_t *token_pos, int32_t *slot_mapping, int32_t *kv_lens,
     int32_t *status, int32_t *items, int items_cap) {
-    __shared__ int sm[PK_THREADS];
+    __shared__ int4 sm[PK_THREADS / 64];
+    __shared__ int2 s_key[PK_THREADS], s_partials[PK_THREADS / 64];
     __shared__ int s_cu[PK_THREADS + 1];
+    __shared__ int4 s_seq[PK_THREADS];  // position, slot, blocks it had, blocks taken by the sequences before it
     const int tid = threadIdx.x;
     const bool act = tid < batch;
-    int slot = 0, pos = 0, ql = 0, have = 0, need = 0;
+    int slot = 0, pos = 0, ql = 0, have = 0, need = 0, block = 0;
+    const int F = *free_count;
     if (act) {
         slot = seq_slots[tid];
         pos = positions[tid];
         ql = q_lens ? q_lens[tid] : 1;
         have = num_blocks[slot];
+        block = block_tables[(size_t)slot * max_blocks + min(max(pos / block_size, 0), max_blocks - 1)];  // where the first new token goes, if it is there
         int end = pos + ql;
         int want = end > 0 ? (end - 1) / block_size + 1 : 0;
         need = want > have ? want - have : 0;
     }
-    int total_need, total_q;
-    const int rank = block_exclusive_scan(need, sm, &total_need);
-    const int cu = block_exclusive_scan(ql, sm, &total_q);
-    const int F = *free_count;
+    const int len = act ? pos + ql : 0;
+    const int full[2] = {len / ATTN_TPW, len / (ATTN_TPW / 2)}, rest[2] = {len % ATTN_TPW, len % (ATTN_TPW / 2)};
+    int4 totals;
+    const int4 ahead = block_exclusive_scan4(make_int4(need, ql, full[0], full[1]), sm, &totals);
+    const int rank = ahead.x, cu = ahead.y, off[2] = {ahead.z, ahead.w};
+    const int total_need = totals.x, total_q = totals.y, total_full[2] = {totals.z, totals.w};
     bool fail = total_need > F || total_q != total_tokens;
     if (act && have + need > max_blocks) fail = true;
     // any thread's failure fails the step
     const bool any_fail = __syncthreads_or(fail ? 1 : 0) != 0;
+    const bool ones = !q_lens || __syncthreads_and(!act || ql == 1) != 0;  // one new token each
     if (any_fail) {
         if (tid == 0) {
             *status = 1;
@@ -89,30 +102,32 @@ __global__ void __launch_bounds__(PK_THREADS) pack_batch_kernel(
         // that for the kernels that take half as many tokens per workgroup (grouped queries). Equal (full) items
         // first, in batch order; then the partial last items from the longest down, so that the kernel's last
         // workgroups are its smallest. The second list sits behind the first one's capacity.
-        const int len = act ? pos + ql : 0;
+        // A partial item's key in each list: its tokens, then the earlier sequence (0: none). The items ahead of it are those of larger keys.
+        int key[2], before[2] = {0, 0}, partials[2] = {0, 0};
+#pragma unroll
+        for (int which = 0; which < 2; which++) key[which] = rest[which] > 0 ? rest[which] * PK_THREADS + PK_THREADS - 1 - tid : 0;
+        s_key[tid] = make_int2(key[0], key[1]);
+        const int2 in_wave = make_int2(__popcll(__ballot(key[0] > 0)), __popcll(__ballot(key[1] > 0)));
+        if ((tid & 63) == 0) s_partials[tid >> 6] = in_wave;
+        __syncthreads();
+        for (int w = 0; w < (int)blockDim.x >> 6; w++) partials[0] += s_partials[w].x, partials[1] += s_partials[w].y;
+        if (act) {
+#pragma unroll 8
+            for (int j = 0; j < batch; j++) {
+                const int2 other = s_key[j];
+                before[0] += other.x > key[0];
+                before[1] += other.y > key[1];
+            }
+        }
+#pragma unroll
         for (int which = 0; which < 2; which++) {
-            const int tpw = which == 0 ? ATTN_TPW : ATTN_TPW / 2;
             const int cap = which == 0 ? items_cap : 2 * items_cap;
             int32_t *list = which == 0 ? items : items + (items_cap + 1) * 4;
-            const int full = len / tpw, rest = len % tpw;
-            int total_full;
-            const int off = block_exclusive_scan(full, sm, &total_full);
-            sm[tid] = rest;
-            __syncthreads();
-            int before = 0, partials = 0;  // partial items ahead of this one; partial items in all
-            if (act || tid == 0) {  // (the threads without a sequence write nothing below)
-                for (int j = 0; j < batch; j++) {
-                    const int rj = sm[j];
-                    partials += rj > 0;
-                    before += (rj > rest) || (rj == rest && rj > 0 && j < tid);
-                }
-            }
-            __syncthreads();
-            const int n_items = total_full + partials;
+            const int n_items = total_full[which] + partials[which];
             if (act && n_items <= cap) {
                 int4 *rec = (int4 *)(list + 4);  // one 16-byte record per item: everything a workgroup needs to start
-                for (int s2 = 0; s2 < full; s2++) rec[off + s2] = make_int4(tid, s2, len, slot);
-                if (rest > 0) rec[total_full + before] = make_int4(tid, full, len, slot);
+                for (int s2 = 0; s2 < full[which]; s2++) rec[off[which] + s2] = make_int4(tid, s2, len, slot);
+                if (rest[which] > 0) rec[total_full[which] + before[which]] = make_int4(tid, full[which], len, slot);
             }
             if (tid == 0) list[0] = n_items <= cap ? n_items : -1;  // -1: the list did not fit, not to be used
         }
@@ -123,6 +138,7 @@ __global__ void __launch_bounds__(PK_THREADS) pack_batch_kernel(
         num_blocks[slot] = have + need;
         kv_lens[tid] = pos + ql;
         s_cu[tid] = cu;
+        s_seq[tid] = make_int4(pos, slot, have, rank);
         cu_seqlens[tid] = cu;
     }
     if (tid == 0) {
@@ -131,8 +147,17 @@ __global__ void __launch_bounds__(PK_THREADS) pack_batch_kernel(
         s_cu[batch] = total_q;
         cu_seqlens[batch] = total_q;
     }
+    if (ones) {  // (a new block's number from where the sequence takes it: not a trip behind the store of it)
+        if (act) {
+            const int j = pos / block_size - have;
+            if (j >= 0 && pos >= 0) block = free_list[F - 1 - (rank + j)];
+            token_pos[tid] = pos;
+            slot_mapping[tid] = block * block_size + pos % block_size;
+        }
+        return;
+    }
     __syncthreads();
-    for (int t = tid; t < total_q; t += PK_THREADS) {
+    for (int t = tid; t < total_q; t += blockDim.x) {
         // binary search: largest i with s_cu[i] <= t
         int lo = 0, hi = batch - 1;
         while (lo < hi) {
@@ -142,10 +167,11 @@ __global__ void __launch_bounds__(PK_THREADS) pack_batch_kernel(
             else
                 hi = mid - 1;
         }
-        const int p = positions[lo] + (t - s_cu[lo]);
+        const int4 seq = s_seq[lo];
+        const int p = seq.x + (t - s_cu[lo]), j = p / block_size - seq.z;
+        const int blk = j >= 0 && p >= 0 ? free_list[F - 1 - (seq.w + j)] : block_tables[(size_t)seq.y * max_blocks + p / block_size];
         token_pos[t] = p;
-        const int sl = seq_slots[lo];
-        slot_mapping[t] = block_tables[(size_t)sl * max_blocks + p / block_size] * block_size + p % block_size;
+        slot_mapping[t] = blk * block_size + p % block_size;
     }
 }
 
@@ -172,7 +198,11 @@ extern "C" int vx_pack_batch(vx_backend *be, const int32_t *seq_slots, const int
     if (batch <= 32767 && per_seq <= 65535 &&
         ensure_ws(be, (void **)&be->items.buf, &be->items.bytes, (3 * cap + 2) * 4 * sizeof(int32_t), "attention work list") == VX_OK)
         items = be->items.buf;
-    pack_batch_kernel<<<1, PK_THREADS, 0, be->stream>>>(seq_slots, positions, q_lens, batch, total_tokens,
+    // A wave for every 64 sequences or new tokens. Bound by what follows one another: trips to memory, shuffles, barriers. With 16 waves always,
+    // four scans one behind the other, the ranks in two passes of eight instructions a sequence and each new token's block read back behind
+    // the store of it 32 sequences of one token each took 12.0 us, now 5.7; one sequence 8.2, now 6.4.
+    const int threads = std::min(PK_THREADS, ceil_div(std::max(batch, total_tokens), 64) * 64);
+    pack_batch_kernel<<<1, threads, 0, be->stream>>>(seq_slots, positions, q_lens, batch, total_tokens,
                                                         block_tables, max_blocks, num_blocks, free_list, free_count,
                                                         block_size, cu_seqlens, token_pos, slot_mapping, kv_lens,
                                                         status, items, (int)cap);
