@@ -510,6 +510,15 @@ def test_attention_geometries(be, act, geom):
     run_attention(be, act, Batch(be, *SINGLE, seed=2), *geom)
 
 
+# Every sequence in one piece: the workgroup writes the results itself, from its waves' parts; groups of more heads than waves, value
+# sizes that fill the last 64 or do not, one to four waves with keys
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("geom", [(8, 1, 128, 128), (20, 1, 64, 32), (4, 2, 256, 256), (3, 1, 96, 40), (4, 4, 40, 96), (6, 1, 192, 160)])
+def test_attention_of_one_piece(be, geom, gated):
+    for lens in ([1, 1, 1, 1, 1, 1], [1, 3, 1, 1, 2, 1]):
+        run_attention(be, BF16, Batch(be, [0, 20, 31, 32, 70, 120], lens, seed=7), *geom, seed=3, gated=gated)
+
+
 @pytest.mark.parametrize("act", ACTS)
 def test_attention_options(be, act):
     """No gate, no bias, no temperature, a temperature per position, bias tables of one entry and too long for LDS."""

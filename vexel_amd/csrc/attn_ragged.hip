@@ -232,6 +232,12 @@ __global__ void __launch_bounds__(256, (prefill_waves<KD, VD, QT, MAPS>())) pref
     }
 }
 
+// Each of the four waves keeps an output of its own in LDS where they fit: they are then added up where a result is written, without turns.
+template <int VD, int MAPS> constexpr int decode_areas() { return MAPS * 16 * (VD * 16 + 4) * 4 * 4 <= 48 * 1024 ? 4 : 1; }
+
+// Bound by trips to memory one behind the other (a short sequence's keys are few bytes), so what does not depend on another load is asked for with
+// it: the sequence's numbers; its blocks, queries, gate; its keys, values and the bias tables. 32 sequences of 44 tokens, 16 / 4 heads x 128,
+// with a gate: 10.9 -> 9.2 us.
 template <int KD, int VD, int MAPS>
 __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode_kernel(Args a) {
     constexpr int QT = MAPS;
@@ -242,46 +248,67 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
     const int g = blockIdx.x % a.p.kv_heads, h0 = blockIdx.x / a.p.kv_heads * 16;  // 16 of the group's query heads
     int seq, piece;
     if (a.items) {
-        if ((int)blockIdx.y >= a.items[0]) return;
-        seq = a.items[4 + 4 * blockIdx.y], piece = a.items[5 + 4 * blockIdx.y];
+        // (one trip for the three: the list has room for every workgroup of the grid)
+        int n = __builtin_amdgcn_readfirstlane(a.items[0]), s = __builtin_amdgcn_readfirstlane(a.items[4 + 4 * blockIdx.y]),
+            c = __builtin_amdgcn_readfirstlane(a.items[5 + 4 * blockIdx.y]);
+        asm volatile("" : "+s"(n), "+s"(s), "+s"(c));
+        if ((int)blockIdx.y >= n) return;
+        seq = __builtin_amdgcn_readfirstlane(s), piece = __builtin_amdgcn_readfirstlane(c);
     } else {
         piece = blockIdx.y, seq = blockIdx.z;
     }
-    const int row = a.one_token ? seq : a.cu[seq];
-    if (!a.one_token && a.cu[seq + 1] - row != 1) return;
-    const int len = a.kv_lens[seq], pos = len - 1, first = first_key(a.p, pos);
+    const int32_t *cu = a.one_token ? a.kv_lens : a.cu;
+    int c0 = __builtin_amdgcn_readfirstlane(cu[seq]), c1 = __builtin_amdgcn_readfirstlane(cu[seq + (a.one_token ? 0 : 1)]),
+        len = __builtin_amdgcn_readfirstlane(a.kv_lens[seq]), table = __builtin_amdgcn_readfirstlane(a.rows[seq]);
+    asm volatile("" : "+s"(c0), "+s"(c1), "+s"(len), "+s"(table));  // (one trip for the four)
+    if (!a.one_token && c1 - c0 != 1) return;
+    const int row = a.one_token ? seq : c0, pos = len - 1, first = first_key(a.p, pos);
     const int start = first / 32 * 32, p_lo = (a.from_start ? 0 : start) + piece * a.piece, k_lo = max(p_lo, start), k_hi = min(len, p_lo + a.piece);
     if (k_lo >= k_hi) return;
-    load_lut(a, g, s_lut);
     const int last_blk = pos / BS;
-    const int32_t *bt = a.tables + (size_t)a.rows[seq] * a.max_blocks;
-
+    const int32_t *bt = a.tables + (size_t)table * a.max_blocks;
+    const int g_hi = (k_hi + 31) / 32, g_lo = k_lo / 32 + wave;
+    int gi = g_lo;
+    int b0 = bt[min(2 * gi, last_blk)], b1 = bt[min(2 * gi + 1, last_blk)];
+    int n0 = bt[min(2 * gi + 8, last_blk)], n1 = bt[min(2 * gi + 9, last_blk)];
     Queries<KD, VD, QT> qs;
+    const int hq = min(h0 + (lane & 15), a.group - 1);  // this lane's query head of the group
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+        const bf16 *q = (const bf16 *)a.p.q + (size_t)row * a.p.ldq + ((g * a.group + hq) * MAPS + t) * a.p.k_dim;
+#pragma unroll
+        for (int kk = 0; kk < KD; kk++) qs.q[t][kk] = load_q(q, kk * 32 + (lane >> 4) * 8, a.p.k_dim, a.vec_q);
+    }
+    const bool finishes = MAPS == 1 && a.pieces == 1;  // this workgroup's results are whole
+    const int vd = a.p.v_dim;
+    bf16 gate[(VD + 3) / 4] = {};  // of the wave's first head, in the order in which it is written
+    if (finishes && a.p.gate && wave < min(16, a.group - h0)) {
+#pragma unroll
+        for (int i = 0; i < (VD + 3) / 4; i++)
+            gate[i] = ((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + (g * a.group + h0 + wave) * vd + min(lane + 64 * i, vd - 1)];
+    }
+    Keys<KD, VD, MAPS, true> ks;
+    ks.init(a, g, lane);
+    if (gi < g_hi) {
+        ks.load_k(b0, b1);
+        ks.load_v(b0, b1, lane);
+    }
     qs.clear();
     const float factor = score_factor(a.p, pos);
 #pragma unroll
     for (int t = 0; t < QT; t++) {
-        const int hh = min(h0 + (lane & 15), a.group - 1), h = g * a.group + hh;
+        const int h = g * a.group + hq;
         qs.pos[t] = pos;
         qs.lo[t] = first;
-        qs.lut[t] = (a.lut_lds ? hh : h) * a.p.bias_len;
+        qs.lut[t] = (a.lut_lds ? hq : h) * a.p.bias_len;
         qs.qs[t] = factor;
         qs.far[t] = score_offset(a.p, h);
-        const bf16 *q = (const bf16 *)a.p.q + (size_t)row * a.p.ldq + (h * MAPS + t) * a.p.k_dim;
-#pragma unroll
-        for (int kk = 0; kk < KD; kk++) qs.q[t][kk] = load_q(q, kk * 32 + (lane >> 4) * 8, a.p.k_dim, a.vec_q);
     }
-    Keys<KD, VD, MAPS, true> ks;
-    ks.init(a, g, lane);
-    const int g_hi = (k_hi + 31) / 32;
-    int gi = k_lo / 32 + wave;
+    load_lut(a, g, s_lut);
     if (gi < g_hi) {
-        int b0 = bt[min(2 * gi, last_blk)], b1 = bt[min(2 * gi + 1, last_blk)];
-        int n0 = bt[min(2 * gi + 8, last_blk)], n1 = bt[min(2 * gi + 9, last_blk)];
-        ks.load_k(b0, b1);
         for (; gi < g_hi; gi += 4) {
             const int f0 = bt[min(2 * gi + 16, last_blk)], f1 = bt[min(2 * gi + 17, last_blk)];
-            ks.load_v(b0, b1, lane);
+            if (gi > g_lo) ks.load_v(b0, b1, lane);
             const bool more = gi + 4 < g_hi;
             const int k0 = gi * 32;
             b0 = n0, b1 = n1, n0 = f0, n1 = f1;
@@ -297,44 +324,66 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
         if (lane < 16) s_m[wave][t * 16 + lane] = qs.m[t], s_l[wave][t * 16 + lane] = l;
     }
     __syncthreads();  // (the bias tables in s_dyn are done with as well)
-    float *s_o = s_dyn;  // [QT * 16][VD * 16 + 4]
-    constexpr int LDO = VD * 16 + 4;
-    for (int w = 0; w < 4; w++) {
-        if (wave == w) {
+    constexpr int LDO = VD * 16 + 4, AREAS = decode_areas<VD, MAPS>(), AREA = MAPS * 16 * LDO;
+    float *s_o = s_dyn;  // [AREAS][QT * 16][VD * 16 + 4]
+    if constexpr (AREAS == 4) {
 #pragma unroll
-            for (int t = 0; t < QT; t++) {
-                const int c = t * 16 + (lane & 15);
-                const float mg = fmaxf(fmaxf(s_m[0][c], s_m[1][c]), fmaxf(s_m[2][c], s_m[3][c]));
-                const float f = qs.m[t] > -INFINITY ? __builtin_amdgcn_exp2f(qs.m[t] - mg) : 0.f;
+        for (int t = 0; t < QT; t++)
 #pragma unroll
-                for (int v = 0; v < VD; v++) {
-                    f32x4 *dst = (f32x4 *)(s_o + c * LDO + v * 16 + (lane >> 4) * 4);
-                    const f32x4 x = qs.o[t][v] * f;
-                    *dst = w == 0 ? x : *dst + x;
+            for (int v = 0; v < VD; v++) *(f32x4 *)(s_o + wave * AREA + (t * 16 + (lane & 15)) * LDO + v * 16 + (lane >> 4) * 4) = qs.o[t][v];
+        __syncthreads();
+    } else {
+        for (int w = 0; w < 4; w++) {
+            if (wave == w) {
+#pragma unroll
+                for (int t = 0; t < QT; t++) {
+                    const int c = t * 16 + (lane & 15);
+                    const float mg = fmaxf(fmaxf(s_m[0][c], s_m[1][c]), fmaxf(s_m[2][c], s_m[3][c]));
+                    const float f = qs.m[t] > -INFINITY ? __builtin_amdgcn_exp2f(qs.m[t] - mg) : 0.f;
+#pragma unroll
+                    for (int v = 0; v < VD; v++) {
+                        f32x4 *dst = (f32x4 *)(s_o + c * LDO + v * 16 + (lane >> 4) * 4);
+                        const f32x4 x = qs.o[t][v] * f;
+                        *dst = w == 0 ? x : *dst + x;
+                    }
                 }
             }
+            __syncthreads();
         }
-        __syncthreads();
     }
-    const int vd = a.p.v_dim;
     for (int i = wave; i < MAPS * min(16, a.group - h0); i += 4) {
         const int hh = i / MAPS, c = i % MAPS * 16 + hh;
         float *dst = a.partial + ((((size_t)seq * a.p.heads + g * a.group + h0 + hh) * MAPS + i % MAPS) * a.pieces + piece) * (vd + 2);
-        float mg = -INFINITY, l = 0.f;
+        float mg = -INFINITY, l = 0.f, f[4];
+#pragma unroll
         for (int w = 0; w < 4; w++) mg = fmaxf(mg, s_m[w][c]);
-        for (int w = 0; w < 4; w++) l += s_m[w][c] > -INFINITY ? s_l[w][c] * __builtin_amdgcn_exp2f(s_m[w][c] - mg) : 0.f;
-        if (MAPS == 1 && a.pieces == 1) {  // what merge_kernel makes of one piece
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            f[w] = s_m[w][c] > -INFINITY ? __builtin_amdgcn_exp2f(s_m[w][c] - mg) : 0.f;
+            l += s_m[w][c] > -INFINITY ? s_l[w][c] * f[w] : 0.f;
+        }
+        const auto output = [&](int d) __attribute__((always_inline)) {
+            if constexpr (AREAS == 1) return s_o[c * LDO + d];
+            float o = s_o[c * LDO + d] * f[0];
+#pragma unroll
+            for (int w = 1; w < AREAS; w++) o += s_o[w * AREA + c * LDO + d] * f[w];
+            return o;
+        };
+        if (finishes) {  // what merge_kernel makes of one piece
             const int h = g * a.group + h0 + hh;
             const float inv = a.p.out_scale / (l + sink_term(a.p, h, mg));
-            for (int d = lane; d < vd; d += 64) {
-                float o = s_o[c * LDO + d] * inv;
-                if (a.p.gate) o *= sigmoid_f((float)((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + h * vd + d]);
+#pragma unroll
+            for (int x = 0; x < (VD + 3) / 4; x++) {
+                const int d = lane + 64 * x;
+                if (d >= vd) break;
+                float o = output(d) * inv;
+                if (a.p.gate) o *= sigmoid_f((float)(i == wave ? gate[x] : ((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + h * vd + d]));
                 ((bf16 *)a.p.out)[(size_t)row * a.p.ldo + h * vd + d] = (bf16)o;
             }
             continue;
         }
         if (lane == 0) dst[0] = mg, dst[1] = l;
-        for (int d = lane; d < vd; d += 64) dst[2 + d] = s_o[c * LDO + d];
+        for (int d = lane; d < vd; d += 64) dst[2 + d] = output(d);
     }
 }
 
@@ -428,7 +477,7 @@ void launch_prefill(vx_backend *be, Args a, const vx_ragged *b) {
 
 template <int KD, int VD, int MAPS>
 void launch_decode(vx_backend *be, const Args &a, dim3 grid) {
-    const size_t lut = a.lut_lds ? (size_t)a.group * a.p.bias_len * 4 : 0, o = (size_t)MAPS * 16 * (VD * 16 + 4) * 4;
+    const size_t lut = a.lut_lds ? (size_t)a.group * a.p.bias_len * 4 : 0, o = (size_t)decode_areas<VD, MAPS>() * MAPS * 16 * (VD * 16 + 4) * 4;
     decode_kernel<KD, VD, MAPS><<<grid, 256, lut > o ? lut : o, be->stream>>>(a);
 }
 
