@@ -506,3 +506,57 @@ def test_fused_qkv_with_packed_v_in_q6_k(be, rows, hq, hk, d, hidden, fqk):
     for p in list(dev.values()) + [dx, dnw, dpos, dslots, dpool, dq]:
         be.free(p)
     be.reset_pool()
+
+
+# Q|K|V rows over 2048 wide where the streaming launch and the one that finishes its rows take the place of the kernel that finishes its
+# own (12288 x 4096, Q4_K also 13824 x 4608), and where they do not: small matrices, Q4_0 rows over 4096 wide
+@pytest.mark.parametrize("fmt,heads,hidden,streamed", [(nx.FMT_Q4_0, 32, 4096, True), (nx.FMT_Q8_0, 32, 4096, True), (nx.FMT_Q4_K, 36, 4608, True),
+                                                       (nx.FMT_Q8_0, 20, 2560, False), (nx.FMT_Q4_0, 18, 2304, False), (nx.FMT_Q4_0, 34, 4352, False)])
+@pytest.mark.parametrize("rows", [2, 17, 32])
+def test_qkv_streamed_or_finished_in_one_launch(rows, fmt, heads, hidden, streamed):
+    from vexel_amd.backend import HipBackend
+    be = HipBackend(0)          # (scratch that no other test has grown)
+    rng = np.random.default_rng(rows + hidden)
+    d, bs, nblocks, theta, eps = 128, 16, 4, 10000.0, 1e-5
+    n = heads * d
+    raw = [qz.random_quant(fmt, rng, n, hidden) for _ in range(3)]
+    qws = [_packed(be, w, n, hidden, fmt)[1] for w in raw]
+    x, nw = rng.standard_normal((rows, hidden)).astype(np.float32), (1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32)
+    positions, slots = rng.integers(0, 100, rows).astype(np.int32), rng.permutation(nblocks * bs)[:rows].astype(np.int32)
+    h = nx.rmsnorm(x, nw, rows, hidden, eps)
+    q, k, v = (nx.matmul_quant(fmt, h, w, rows, n, hidden) for w in raw)
+    want_q, want_k = nx.rope_positions(q, k, d, heads, heads, positions, d, theta, False)
+    dx, dnw, dpos, dslots = (be.upload(a, permanent=True) for a in (x, nw, positions, slots))
+    per_block = 2 * bs * n
+    dpool, dq = be.alloc_permanent(nblocks * per_block * 2), be.alloc_permanent(rows * n * 4)
+
+    def step():
+        be.decode_attn_qkv(dx, dnw, eps, True, *qws, rows, dpos, dslots, dpool, True, heads, heads, d, bs, theta, dq)
+
+    def check():
+        _close(be.download(dq, (rows, n), np.float32), want_q, 2e-4, 2e-5 * np.abs(want_q).max(), "Q")
+        pool = nx.f16_to_f32_array(be.download(dpool, (nblocks * per_block,), np.uint16)).reshape(nblocks, 2, bs, n)
+        for part, want in enumerate((want_k, v)):
+            got = pool[slots // bs, part, slots % bs]
+            _close(got, nx.f16_to_f32_array(nx.f32_to_f16_array(want)), 2e-3, 2e-3 * np.abs(want).max(), "K" if part == 0 else "V")
+        be.to_device(dq, np.full((rows, n), np.nan, dtype=np.float32))
+
+    be.rmsnorm_prepare(dx, dnw, None, rows, hidden, eps)
+    be.rope_table_prepare(dpos, rows, d, theta)
+    if streamed:
+        be.sync()
+        be.graph_begin_capture()    # no scratch for slices' sums yet: the launch that needs none
+        be.rope_table_prepare(dpos, rows, d, theta)
+        step()
+        graph = be.graph_end_capture()
+        for _ in range(3):
+            be.graph_launch(graph)
+            be.sync()
+            check()
+        be.graph_destroy(graph)
+        be.rmsnorm_prepare(dx, dnw, None, rows, hidden, eps)
+        be.rope_table_prepare(dpos, rows, d, theta)
+    step()
+    assert not streamed or be.last_matmul_kernel() == "qstream_kernel"
+    check()
+    be.close()

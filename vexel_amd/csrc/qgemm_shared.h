@@ -54,6 +54,8 @@ struct QkvEpi {
 // copy (vx_qweight_pack), 2 <= M <= 64 and the shape fits. stream_gemm leaves the K slices' raw sums in
 // be->part_ws as [slice][M][N] (*ks_out slices) or, given an epilogue, finishes the Q|K|V rows itself.
 bool stream_gemm_ok(vx_backend *be, int fmt, const uint8_t *const *w, const int *n_end, int nseg, int N, int K, int M, bool epi);
+// Bytes of the K slices' sums that stream_gemm leaves without an epilogue; 0: it does not take the call.
+size_t stream_gemm_sums(vx_backend *be, int fmt, const uint8_t *const *w, const int *n_end, int nseg, int N, int K, int M);
 int stream_gemm(vx_backend *be, int fmt, const uint8_t *const *w, const int *n_end, int nseg, int N, int K, int M, int mpad,
                 const PrepView &pv, const QkvEpi *epi, int *ks_out);
 
