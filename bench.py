@@ -336,7 +336,7 @@ def time_step_gemms(be, mr, c, rows):
                      "frac": round(nbytes / us / 1e3 / HBM_PEAK_GBS, 4), "kernel": kernel}
         if name == "Q|K|V":
             fused = time_fused_qkv(be, lw, c, rows, acts[k])
-            if fused is not None:   # what the step launches for Q|K|V: the projection with RoPE and the KV store in its epilogue
+            if fused is not None:   # what the step launches for Q|K|V: the projection with RoPE and the KV store, in its epilogue or in a launch behind it
                 res[name]["us_projection_alone"] = res[name]["us"]
                 res[name]["kernel_projection_alone"] = res[name]["kernel"]
                 res[name]["kernel"] = be.last_matmul_kernel()
@@ -356,7 +356,7 @@ def time_step_gemms(be, mr, c, rows):
             "us_per_layer": total_us, "launches": res,
             "note": "HIP events around back-to-back launches over all layers' weights; us: the projection launch alone, "
                     "as the fused decode blocks issue it (K slices' sums consumed by the next prepare kernel; Q|K|V: "
-                    "with its RoPE + KV-store epilogue, timed as vx_decode_attn_qkv minus the prepare kernel alone); "
+                    "with RoPE + KV store, timed as vx_decode_attn_qkv minus the prepare kernel alone); "
                     "us_with_reduction: with the separate reduction kernel of the unfused call"}
 
 
