@@ -2525,11 +2525,12 @@ int vx_prefill_attn_qkv(vx_backend *be, const float *x, const float *norm_weight
         // 2386, 16 rows 2526 -> 2483, 2 rows the same. Eight layers of 15360 x 5120: Q4_K 2 rows 857 -> 833, 12 rows 949 -> 928, 32 rows 1222 ->
         // 1207. The other way round: Q4_0 6912 x 2304 541 -> 566, 7680 x 2560 564 -> 588 (Q8_0 535 -> 542), 5120 x 3072 569 -> 579, and Q4_0 with rows
         // over 4096 (15360 x 5120, 32 rows 1143 -> 1163). (A captured step whose scratch would have to grow for it keeps the one launch.)
-        const size_t sums = stream_gemm_sums(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows);
+        const bool whole = pl.r > 0 && pl.ks == 1;
+        const size_t sums = whole ? stream_gemm_sums(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows) : 0;
         const size_t bytes = (size_t)ntot * (k / 32) * (wq->fmt == VX_Q8_0 ? 34 : 18);
         const bool streams = sums > 0 && (wq->fmt == VX_Q8_0 || wq->fmt == VX_Q4_K || (wq->fmt == VX_Q4_0 && k <= 4096)) &&
                              bytes >= (size_t)41 << 19 && (!be->capturing || sums <= be->part_ws_bytes);
-        const bool one_launch = (pl.r > 0 && pl.ks == 1 && !streams) || stream_gemm_ok(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows, true);
+        const bool one_launch = (whole && !streams) || stream_gemm_ok(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows, true);
         if (!no_epi && !gen && table && one_launch && mpad_for(rows) <= 32 && (head_dim & (head_dim - 1)) == 0 &&
             head_dim >= 4 && ((uintptr_t)kv_pool % 16) == 0 && ((uintptr_t)q_out % 16) == 0) {
             QkvEpi epi;
