@@ -265,3 +265,71 @@ def test_pages_of_expected_transfers(tmp_path, helpers):
     subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "vexel_amd", "csrc"), str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe), str(helpers)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stdout)
+
+
+# Which pages the caller of a transfer makes itself while another destination, its own, or a part of its own is announced.
+BESIDE = SENDER[:SENDER.index("int main(")].replace("#define memcpy copy_slowly", r"""#include <sys/mman.h>
+static char *made_from = nullptr;
+static size_t made_bytes = 0;
+static int noted_madvise(void *a, size_t n, int what) {  // (of the caller's, one after the other)
+    if (std::this_thread::get_id() == caller) {
+        if (!made_from) made_from = (char *)a;
+        made_bytes += n;
+    }
+    return madvise(a, n, what);
+}
+#define madvise noted_madvise
+#define memcpy copy_slowly""") + r"""
+static const size_t SLOT = vx::Mover::SENT_SLOT, N = 10 * SLOT;
+static char *fresh() { return (char *)mmap(nullptr, N, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0); }
+static void add(std::vector<vx::Mover::Piece> &to, char *dst, const char *src) {
+    for (size_t at = 0; at < N; at += SLOT) to.push_back({dst + at, src ? src + at : nullptr, SLOT});
+}
+static bool missing(const char *p) {
+    unsigned char in_core[N / 4096];
+    if (mincore((void *)p, N, in_core) != 0) return true;
+    for (unsigned char c : in_core)
+        if (!(c & 1)) return true;
+    return false;
+}
+int main(int argc, char **argv) {
+    caller = std::this_thread::get_id();
+    vx::Mover m;
+    m.marks = (uint64_t *)calloc(vx::Mover::SENT_SLOTS * vx::Mover::MARK_STEP, 8);
+    m.sender = late = new Late;
+    late->hold = true;  // (the first piece comes when all pages that the caller makes have been made)
+    if (!m.start(atoi(argv[1]))) return 2;
+    std::string from(N, 0);
+    for (size_t k = 0; k < N; k++) from[k] = (char)(k * 2654435761u >> 13);
+    for (const char *what : {"other", "own", "part"}) {
+        char *x = fresh(), *y = fresh();
+        std::vector<vx::Mover::Piece> announced, pieces;
+        add(announced, what[1] == 'w' ? x : y, nullptr);
+        const int token = m.expect(announced);
+        if (token == 0) return 3;
+        for (const auto end = std::chrono::steady_clock::now() + std::chrono::seconds(20); missing(announced[0].dst); std::this_thread::yield())
+            if (std::chrono::steady_clock::now() > end) return 4;
+        if (what[0] == 'p') add(pieces, y, from.data());
+        add(pieces, x, from.data());
+        made_from = nullptr, made_bytes = 0;
+        vx::Mover::Job job(pieces);
+        if (m.move(0, job) != 0 || memcmp(x, from.data(), N) != 0) return 5;
+        if (what[0] == 'p' && memcmp(y, from.data(), N) != 0) return 6;
+        if (what[1] == 'w' ? made_bytes != 0 : made_from != x || made_bytes != N) return 7;
+        m.forget(token);
+        munmap(x, N);
+        munmap(y, N);
+        printf("%s ok\n", what);
+    }
+    return 0;
+}
+"""
+
+
+@pytest.mark.parametrize("helpers", [1, 6])
+def test_pages_beside_an_announcement(tmp_path, helpers):
+    src, exe = tmp_path / "beside.cpp", tmp_path / "beside"
+    src.write_text(BESIDE)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "vexel_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe), str(helpers)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "other ok\nown ok\npart ok\n", (r.returncode, r.stdout)

@@ -9,6 +9,7 @@
 #include <condition_variable>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 namespace vx {
@@ -64,6 +65,7 @@ struct Mover {
     bool stop = false;
     // Destinations of a transfer that is still to come (expect).
     std::vector<Piece> ahead;
+    std::vector<std::pair<const char *, const char *>> ahead_ranges;  // what they cover, [from, to)
     std::atomic<int> ahead_next{0};
     bool making = false;              // a helper is at it
     std::atomic<int> ahead_token{0};  // which expect() it is, 0: none
@@ -168,6 +170,11 @@ struct Mover {
     int expect(std::vector<Piece> pieces) {
         std::lock_guard<std::mutex> g(mu);
         if (ahead_token.load() != 0 || workers.empty() || pieces.empty()) return 0;
+        ahead_ranges.clear();
+        for (const Piece &p : pieces) {
+            if (!ahead_ranges.empty() && ahead_ranges.back().second == p.dst) ahead_ranges.back().second += p.bytes;
+            else ahead_ranges.push_back({p.dst, p.dst + p.bytes});
+        }
         ahead = std::move(pieces);
         ahead_next.store(0);
         tokens = tokens == 0x7FFFFFFF ? 1 : tokens + 1;
@@ -184,6 +191,16 @@ struct Mover {
         ahead.clear();
         ahead_token.store(0);
     }
+    // Whether a helper makes this piece's pages, or has made them: what is announced is not what every transfer writes, and the
+    // helpers may have been busy ever since.
+    bool made_ahead(const Piece &p) {
+        if (ahead_token.load() == 0) return false;
+        std::lock_guard<std::mutex> g(mu);
+        if (ahead_token.load() == 0 || (!making && ahead_next.load() == 0)) return false;
+        for (const auto &r : ahead_ranges)
+            if (r.first <= p.dst && p.dst + p.bytes <= r.second) return true;
+        return false;
+    }
     bool pages_wanted() const { return !making && ahead_next.load() < (int)ahead.size(); }
     void make_ahead() {
         for (;;) {
@@ -199,7 +216,7 @@ struct Mover {
         left.wait(l, [&] { return inside == 0; });
     }
     // move() with a sender: the caller enqueues up to SENT_MOST pieces whenever their slots are free, and copies what has arrived
-    // in between; while nothing has, it makes the destination's pages. It never waits for a piece without asking now and then whether the stream still works.
+    // in between; while nothing has, it makes the destination's pages (those that no helper makes). It never waits for a piece without asking now and then whether the stream still works.
     hipError_t move_sent(hipStream_t stream, Job &j) {
         const int n = (int)j.pieces.size();
         hipError_t err = hipSuccess;
@@ -222,8 +239,8 @@ struct Mover {
                 wake_workers(j);
             }
             if (awake && take_arrived(j)) continue;  // (not before: piece 256 may take the slot that says that they can be woken)
-            made = ahead_token.load() != 0 ? n : std::max(made, j.next.load());
-            if (made < n) made = make_pages(j.pieces[made]) ? made + 1 : n;
+            made = std::max(made, j.next.load());
+            if (made < n) made = made_ahead(j.pieces[made]) || make_pages(j.pieces[made]) ? made + 1 : n;
             else std::this_thread::yield();
             if (polls % 8192 == 0) {  // a stream that has ended without the pieces will not bring them
                 bool over = false;
