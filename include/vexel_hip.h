@@ -260,7 +260,8 @@ typedef struct vx_qweight {
  * vx_qweight_unpack, vx_free of the matrix, a library write into its bytes or vx_backend_destroy. While it exists,
  * every quantized matmul entry point and fused decode block that is given the matrix (by the same data pointer, alone
  * or as part of a Q|K|V or gate|up group) with 2 .. 64 activation rows streams the packed copy, and with more than 64 rows reads
- * it tile by tile; a single row reads the GGUF rows, which stay where they are. vx_dequantize_packed: gguf.Dequantize of the packed copy
+ * it tile by tile; a single row reads the GGUF rows, which stay where they are. The call also grows the library's scratch to what a
+ * decode step's Q|K|V of such matrices needs, so that a captured step takes the launches of an eager one. vx_dequantize_packed: gguf.Dequantize of the packed copy
  * (pkg/gguf/dequant.go:16-145, 272-470), bit for bit what vx_dequantize gives for the rows. */
 int vx_qweight_pack(vx_backend *be, const vx_qweight *w);
 int vx_qweight_unpack(vx_backend *be, const vx_qweight *w);

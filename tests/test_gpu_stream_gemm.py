@@ -509,7 +509,8 @@ def test_fused_qkv_with_packed_v_in_q6_k(be, rows, hq, hk, d, hidden, fqk):
 
 
 # Q|K|V rows over 2048 wide where the streaming launch and the one that finishes its rows take the place of the kernel that finishes its
-# own (12288 x 4096, Q4_K also 13824 x 4608), and where they do not: small matrices, Q4_0 rows over 4096 wide
+# own (12288 x 4096, Q4_K also 13824 x 4608), and where they do not: small matrices, Q4_0 rows over 4096 wide. A captured step takes the
+# same launches as one that is not, whatever ran before it.
 @pytest.mark.parametrize("fmt,heads,hidden,streamed", [(nx.FMT_Q4_0, 32, 4096, True), (nx.FMT_Q8_0, 32, 4096, True), (nx.FMT_Q4_K, 36, 4608, True),
                                                        (nx.FMT_Q8_0, 20, 2560, False), (nx.FMT_Q4_0, 18, 2304, False), (nx.FMT_Q4_0, 34, 4352, False)])
 @pytest.mark.parametrize("rows", [2, 17, 32])
@@ -534,29 +535,62 @@ def test_qkv_streamed_or_finished_in_one_launch(rows, fmt, heads, hidden, stream
         be.decode_attn_qkv(dx, dnw, eps, True, *qws, rows, dpos, dslots, dpool, True, heads, heads, d, bs, theta, dq)
 
     def check():
-        _close(be.download(dq, (rows, n), np.float32), want_q, 2e-4, 2e-5 * np.abs(want_q).max(), "Q")
-        pool = nx.f16_to_f32_array(be.download(dpool, (nblocks * per_block,), np.uint16)).reshape(nblocks, 2, bs, n)
+        got_q = be.download(dq, (rows, n), np.float32)
+        _close(got_q, want_q, 2e-4, 2e-5 * np.abs(want_q).max(), "Q")
+        bits = be.download(dpool, (nblocks * per_block,), np.uint16).reshape(nblocks, 2, bs, n)
+        pool = nx.f16_to_f32_array(bits.ravel()).reshape(bits.shape)
         for part, want in enumerate((want_k, v)):
             got = pool[slots // bs, part, slots % bs]
             _close(got, nx.f16_to_f32_array(nx.f32_to_f16_array(want)), 2e-3, 2e-3 * np.abs(want).max(), "K" if part == 0 else "V")
         be.to_device(dq, np.full((rows, n), np.nan, dtype=np.float32))
+        stored = bits[slots // bs, :, slots % bs]
+        bits[slots // bs, :, slots % bs] = 0x7E00
+        be.to_device(dpool, bits)
+        return got_q, stored
 
+    kernel = "qstream_kernel" if streamed else "qgemm_wave_kernel"
     be.rmsnorm_prepare(dx, dnw, None, rows, hidden, eps)
+    be.sync()
+    be.graph_begin_capture()    # (before any call has asked for scratch for slices' sums)
     be.rope_table_prepare(dpos, rows, d, theta)
-    if streamed:
-        be.sync()
-        be.graph_begin_capture()    # no scratch for slices' sums yet: the launch that needs none
-        be.rope_table_prepare(dpos, rows, d, theta)
-        step()
-        graph = be.graph_end_capture()
-        for _ in range(3):
-            be.graph_launch(graph)
-            be.sync()
-            check()
-        be.graph_destroy(graph)
-        be.rmsnorm_prepare(dx, dnw, None, rows, hidden, eps)
-        be.rope_table_prepare(dpos, rows, d, theta)
     step()
-    assert not streamed or be.last_matmul_kernel() == "qstream_kernel"
-    check()
+    recorded = be.last_matmul_kernel()
+    graph = be.graph_end_capture()
+    assert recorded == kernel
+    be.rope_table_prepare(dpos, rows, d, theta)
+    step()
+    assert be.last_matmul_kernel() == kernel
+    eager = check()
+    for _ in range(3):
+        be.graph_launch(graph)
+        be.sync()
+        got = check()
+        assert all(np.array_equal(a, b) for a, b in zip(got, eager))
+    be.graph_destroy(graph)
     be.close()
+
+
+@pytest.mark.parametrize("fmt", [nx.FMT_Q4_0, nx.FMT_Q8_0, nx.FMT_Q4_K])
+def test_streamed_qkv_rows_do_not_depend_on_the_batch(be, fmt):
+    rng = np.random.default_rng(11)
+    heads, kv_heads, d, hidden, bs, nblocks, theta, eps = 36, 30, 128, 4096, 16, 4, 10000.0, 1e-5
+    qd, kvd = heads * d, kv_heads * d
+    dev, qws = zip(*[_packed(be, qz.random_quant(fmt, rng, n, hidden), n, hidden, fmt) for n in (qd, kvd, kvd)])
+    x, nw = rng.standard_normal((32, hidden)).astype(np.float32), (1.0 + 0.1 * rng.standard_normal(hidden)).astype(np.float32)
+    positions, slots = rng.integers(0, 100, 32).astype(np.int32), rng.permutation(nblocks * bs)[:32].astype(np.int32)
+    dx, dnw, dpos, dslots = (be.upload(a, permanent=True) for a in (x, nw, positions, slots))
+    per_block = 2 * bs * kvd
+    dpool, dq = be.alloc_permanent(nblocks * per_block * 2), be.alloc_permanent(32 * qd * 4)
+    want = None
+    for rows in (32, 17, 16, 2):
+        be.rope_table_prepare(dpos, rows, d, theta)
+        be.decode_attn_qkv(dx, dnw, eps, False, *qws, rows, dpos, dslots, dpool, True, heads, kv_heads, d, bs, theta, dq)
+        assert be.last_matmul_kernel() == "qstream_kernel"
+        pool = be.download(dpool, (nblocks * per_block,), np.uint16).reshape(nblocks, 2, bs, kvd)
+        got = be.download(dq, (rows, qd), np.float32), pool[slots // bs, :, slots % bs][:rows]
+        want = want or got
+        assert all(np.array_equal(a, b[:rows]) for a, b in zip(got, want)), rows
+        be.fill_zero(dpool, nblocks * per_block * 2)
+    for p in list(dev) + [dx, dnw, dpos, dslots, dpool, dq]:
+        be.free(p)
+    be.reset_pool()

@@ -1832,7 +1832,7 @@ WavePlan wave_plan(vx_backend *be, int fmt, const Segs &segs, int N, int K, int 
         }
     }
     // more than 6 tiles a workgroup would spill registers: taller matrices (output heads) stay on qgemm_kernel
-    const int max_r = rows64 ? 3 : (fmt == VX_Q8_0 ? 4 : (fmt == VX_BF16 ? 2 : 6));  // (wider staging leaves room for fewer tiles)
+    const int max_r = rows64 ? 3 : (fmt == VX_Q8_0 ? 4 : (fmt == VX_BF16 ? 2 : WAVE_TILES_MOST));  // (wider staging leaves room for fewer tiles)
     const bool rounds = fmt == VX_BF16 || rows64;
     if (tiles > max_r * cus && !rounds) return none;
     static const int rs[] = {1, 2, 3, 4, 6};
@@ -2519,17 +2519,9 @@ int vx_prefill_attn_qkv(vx_backend *be, const float *x, const float *norm_weight
         const bool table = be->rope_tab_pos == positions && be->rope_tab_rows >= rows && be->rope_tab_dim == head_dim &&
                            be->rope_tab_theta == theta && be->rope_tab_epoch == be->write_epoch;
         static const bool no_epi = getenv("VEXEL_HIP_NO_QKV_EPILOGUE") != nullptr;
-        // Matrices that could be streamed but not with the epilogue (rows over 2048 wide): from 20.5 MiB on the streaming launch and the one
-        // that finishes its rows are the shorter pair, and K in slices leaves less error (1.00e-7 against 1.15e-7 at 4096 wide). Whole steps of 32
-        // layers of 12288 x 4096 at context 100: Q8_0 2 rows 2662 -> 2523 us, 8 rows 2838 -> 2712, 24 rows 3421 -> 3247; Q4_0 8 rows 2444 ->
-        // 2386, 16 rows 2526 -> 2483, 2 rows the same. Eight layers of 15360 x 5120: Q4_K 2 rows 857 -> 833, 12 rows 949 -> 928, 32 rows 1222 ->
-        // 1207. The other way round: Q4_0 6912 x 2304 541 -> 566, 7680 x 2560 564 -> 588 (Q8_0 535 -> 542), 5120 x 3072 569 -> 579, and Q4_0 with rows
-        // over 4096 (15360 x 5120, 32 rows 1143 -> 1163). (A captured step whose scratch would have to grow for it keeps the one launch.)
+        // (matrices with rows over 2048 wide could be streamed, but not with the epilogue: see qkv_streams)
         const bool whole = pl.r > 0 && pl.ks == 1;
-        const size_t sums = whole ? stream_gemm_sums(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows) : 0;
-        const size_t bytes = (size_t)ntot * (k / 32) * (wq->fmt == VX_Q8_0 ? 34 : 18);
-        const bool streams = sums > 0 && (wq->fmt == VX_Q8_0 || wq->fmt == VX_Q4_K || (wq->fmt == VX_Q4_0 && k <= 4096)) &&
-                             bytes >= (size_t)41 << 19 && (!be->capturing || sums <= be->part_ws_bytes);
+        const bool streams = whole && qkv_streams(be, wq->fmt, ntot, k) && stream_gemm_ok(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows, false);
         const bool one_launch = (whole && !streams) || stream_gemm_ok(be, wq->fmt, segs.w, segs.n_end, 3, ntot, k, rows, true);
         if (!no_epi && !gen && table && one_launch && mpad_for(rows) <= 32 && (head_dim & (head_dim - 1)) == 0 &&
             head_dim >= 4 && ((uintptr_t)kv_pool % 16) == 0 && ((uintptr_t)q_out % 16) == 0) {

@@ -54,8 +54,11 @@ struct QkvEpi {
 // copy (vx_qweight_pack), 2 <= M <= 64 and the shape fits. stream_gemm leaves the K slices' raw sums in
 // be->part_ws as [slice][M][N] (*ks_out slices) or, given an epilogue, finishes the Q|K|V rows itself.
 bool stream_gemm_ok(vx_backend *be, int fmt, const uint8_t *const *w, const int *n_end, int nseg, int N, int K, int M, bool epi);
-// Bytes of the K slices' sums that stream_gemm leaves without an epilogue; 0: it does not take the call.
-size_t stream_gemm_sums(vx_backend *be, int fmt, const uint8_t *const *w, const int *n_end, int nseg, int N, int K, int M);
+constexpr int WAVE_TILES_MOST = 6;  // weight tiles of a workgroup of qgemm_wave_kernel
+// A Q|K|V matrix [N, K] that qgemm_wave_kernel would take whole and the streaming kernel only without the epilogue (rows over 2048
+// wide, K-quants): whether the streaming launch and the one that finishes its rows serve it. By format and shape only, and never for
+// want of scratch (vx_qweight_pack makes the room), so that a captured step records what an eager one launches: same bits.
+bool qkv_streams(const vx_backend *be, int fmt, int N, int K);
 int stream_gemm(vx_backend *be, int fmt, const uint8_t *const *w, const int *n_end, int nseg, int N, int K, int M, int mpad,
                 const PrepView &pv, const QkvEpi *epi, int *ks_out);
 
