@@ -235,66 +235,62 @@ __global__ void __launch_bounds__(256, (prefill_waves<KD, VD, QT, MAPS>())) pref
 // Each of the four waves keeps an output of its own in LDS where they fit: they are then added up where a result is written, without turns.
 template <int VD, int MAPS> constexpr int decode_areas() { return MAPS * 16 * (VD * 16 + 4) * 4 * 4 <= 48 * 1024 ? 4 : 1; }
 
-// Bound by trips to memory one behind the other (a short sequence's keys are few bytes), so what does not depend on another load is asked for with
-// it: the sequence's numbers; its blocks, queries, gate; its keys, values and the bias tables. 32 sequences of 44 tokens, 16 / 4 heads x 128,
-// with a gate: 10.9 -> 9.2 us.
+// Bound by trips to memory one behind the other (a short sequence's keys are few bytes). Where the four outputs fit, a sequence's numbers are
+// asked for together and the gate with the queries. Back to back, with the merge where there is one, us: 32 sequences of 16 / 4 heads x 128 with a
+// gate, 44 tokens 6.8 -> 5.9, 600 18.8 -> 17.8, 2000 32.0 -> 31.2, one of 4000 17.6 -> 16.7; with a bias table of 512 7.7 -> 6.9, 21.0 -> 20.5, 35.7 -> 34.2,
+// 18.6 -> 17.9. Block numbers ahead of the queries (600 tokens: 19.0), values ahead of the loop as well (19.4) and bias tables behind the keys (with
+// them 23.1) were slower. Wider forms are the slower for all this (192 / 160 columns, 44 tokens 8.0 -> 8.3, 600 30.1 -> 30.6; 256 with a
+// bias table, 600 38.8 -> 39.1; two maps of 128, 2000 66.0 -> 66.8): they read one number after the other, and the gate where they write.
 template <int KD, int VD, int MAPS>
 __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode_kernel(Args a) {
     constexpr int QT = MAPS;
+    constexpr bool NARROW = decode_areas<VD, MAPS>() == 4;
     extern __shared__ float s_dyn[];
     __shared__ float s_m[4][QT * 16], s_l[4][QT * 16];
     float *s_lut = s_dyn;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = blockIdx.x % a.p.kv_heads, h0 = blockIdx.x / a.p.kv_heads * 16;  // 16 of the group's query heads
-    int seq, piece;
-    if (a.items) {
-        // (one trip for the three: the list has room for every workgroup of the grid)
-        int n = __builtin_amdgcn_readfirstlane(a.items[0]), s = __builtin_amdgcn_readfirstlane(a.items[4 + 4 * blockIdx.y]),
-            c = __builtin_amdgcn_readfirstlane(a.items[5 + 4 * blockIdx.y]);
-        asm volatile("" : "+s"(n), "+s"(s), "+s"(c));
-        if ((int)blockIdx.y >= n) return;
-        seq = __builtin_amdgcn_readfirstlane(s), piece = __builtin_amdgcn_readfirstlane(c);
-    } else {
-        piece = blockIdx.y, seq = blockIdx.z;
-    }
-    const int32_t *cu = a.one_token ? a.kv_lens : a.cu;
-    int c0 = __builtin_amdgcn_readfirstlane(cu[seq]), c1 = __builtin_amdgcn_readfirstlane(cu[seq + (a.one_token ? 0 : 1)]),
+    int seq, piece, row, len, table;
+    if constexpr (NARROW) {
+        if (a.items) {
+            // (one trip for the three: the list has room for every workgroup of the grid)
+            int n = __builtin_amdgcn_readfirstlane(a.items[0]), s = __builtin_amdgcn_readfirstlane(a.items[4 + 4 * blockIdx.y]),
+                c = __builtin_amdgcn_readfirstlane(a.items[5 + 4 * blockIdx.y]);
+            asm volatile("" : "+s"(n), "+s"(s), "+s"(c));
+            if ((int)blockIdx.y >= n) return;
+            seq = __builtin_amdgcn_readfirstlane(s), piece = __builtin_amdgcn_readfirstlane(c);
+        } else {
+            piece = blockIdx.y, seq = blockIdx.z;
+        }
+        const int32_t *cu = a.one_token ? a.kv_lens : a.cu;
+        int c0 = __builtin_amdgcn_readfirstlane(cu[seq]), c1 = __builtin_amdgcn_readfirstlane(cu[seq + (a.one_token ? 0 : 1)]);
         len = __builtin_amdgcn_readfirstlane(a.kv_lens[seq]), table = __builtin_amdgcn_readfirstlane(a.rows[seq]);
-    asm volatile("" : "+s"(c0), "+s"(c1), "+s"(len), "+s"(table));  // (one trip for the four)
-    if (!a.one_token && c1 - c0 != 1) return;
-    const int row = a.one_token ? seq : c0, pos = len - 1, first = first_key(a.p, pos);
+        asm volatile("" : "+s"(c0), "+s"(c1), "+s"(len), "+s"(table));  // (one trip for the four)
+        if (!a.one_token && c1 - c0 != 1) return;
+        row = a.one_token ? seq : c0;
+    } else {
+        if (a.items) {
+            if ((int)blockIdx.y >= a.items[0]) return;
+            seq = a.items[4 + 4 * blockIdx.y], piece = a.items[5 + 4 * blockIdx.y];
+        } else {
+            piece = blockIdx.y, seq = blockIdx.z;
+        }
+        row = a.one_token ? seq : a.cu[seq];
+        if (!a.one_token && a.cu[seq + 1] - row != 1) return;
+        len = a.kv_lens[seq], table = a.rows[seq];
+    }
+    const int pos = len - 1, first = first_key(a.p, pos);
     const int start = first / 32 * 32, p_lo = (a.from_start ? 0 : start) + piece * a.piece, k_lo = max(p_lo, start), k_hi = min(len, p_lo + a.piece);
     if (k_lo >= k_hi) return;
+    load_lut(a, g, s_lut);
     const int last_blk = pos / BS;
     const int32_t *bt = a.tables + (size_t)table * a.max_blocks;
-    const int g_hi = (k_hi + 31) / 32, g_lo = k_lo / 32 + wave;
-    int gi = g_lo;
-    int b0 = bt[min(2 * gi, last_blk)], b1 = bt[min(2 * gi + 1, last_blk)];
-    int n0 = bt[min(2 * gi + 8, last_blk)], n1 = bt[min(2 * gi + 9, last_blk)];
+    const int g_hi = (k_hi + 31) / 32;
+    int gi = k_lo / 32 + wave;
     Queries<KD, VD, QT> qs;
-    const int hq = min(h0 + (lane & 15), a.group - 1);  // this lane's query head of the group
-#pragma unroll
-    for (int t = 0; t < QT; t++) {
-        const bf16 *q = (const bf16 *)a.p.q + (size_t)row * a.p.ldq + ((g * a.group + hq) * MAPS + t) * a.p.k_dim;
-#pragma unroll
-        for (int kk = 0; kk < KD; kk++) qs.q[t][kk] = load_q(q, kk * 32 + (lane >> 4) * 8, a.p.k_dim, a.vec_q);
-    }
-    const bool finishes = MAPS == 1 && a.pieces == 1;  // this workgroup's results are whole
-    const int vd = a.p.v_dim;
-    bf16 gate[(VD + 3) / 4] = {};  // of the wave's first head, in the order in which it is written
-    if (finishes && a.p.gate && wave < min(16, a.group - h0)) {
-#pragma unroll
-        for (int i = 0; i < (VD + 3) / 4; i++)
-            gate[i] = ((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + (g * a.group + h0 + wave) * vd + min(lane + 64 * i, vd - 1)];
-    }
-    Keys<KD, VD, MAPS, true> ks;
-    ks.init(a, g, lane);
-    if (gi < g_hi) {
-        ks.load_k(b0, b1);
-        ks.load_v(b0, b1, lane);
-    }
     qs.clear();
     const float factor = score_factor(a.p, pos);
+    const int hq = min(h0 + (lane & 15), a.group - 1);  // this lane's query head of the group
 #pragma unroll
     for (int t = 0; t < QT; t++) {
         const int h = g * a.group + hq;
@@ -303,12 +299,27 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
         qs.lut[t] = (a.lut_lds ? hq : h) * a.p.bias_len;
         qs.qs[t] = factor;
         qs.far[t] = score_offset(a.p, h);
+        const bf16 *q = (const bf16 *)a.p.q + (size_t)row * a.p.ldq + ((g * a.group + hq) * MAPS + t) * a.p.k_dim;
+#pragma unroll
+        for (int kk = 0; kk < KD; kk++) qs.q[t][kk] = load_q(q, kk * 32 + (lane >> 4) * 8, a.p.k_dim, a.vec_q);
     }
-    load_lut(a, g, s_lut);
+    const bool finishes = MAPS == 1 && a.pieces == 1;  // this workgroup's results are whole
+    const int vd = a.p.v_dim;
+    bf16 gate[(VD + 3) / 4] = {};  // of the wave's first head, in the order in which it is written
+    if (NARROW && finishes && a.p.gate && wave < min(16, a.group - h0)) {
+#pragma unroll
+        for (int i = 0; i < (VD + 3) / 4; i++)
+            gate[i] = ((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + (g * a.group + h0 + wave) * vd + min(lane + 64 * i, vd - 1)];
+    }
+    Keys<KD, VD, MAPS, true> ks;
+    ks.init(a, g, lane);
     if (gi < g_hi) {
+        int b0 = bt[min(2 * gi, last_blk)], b1 = bt[min(2 * gi + 1, last_blk)];
+        int n0 = bt[min(2 * gi + 8, last_blk)], n1 = bt[min(2 * gi + 9, last_blk)];
+        ks.load_k(b0, b1);
         for (; gi < g_hi; gi += 4) {
             const int f0 = bt[min(2 * gi + 16, last_blk)], f1 = bt[min(2 * gi + 17, last_blk)];
-            if (gi > g_lo) ks.load_v(b0, b1, lane);
+            ks.load_v(b0, b1, lane);
             const bool more = gi + 4 < g_hi;
             const int k0 = gi * 32;
             b0 = n0, b1 = n1, n0 = f0, n1 = f1;
@@ -377,7 +388,7 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
                 const int d = lane + 64 * x;
                 if (d >= vd) break;
                 float o = output(d) * inv;
-                if (a.p.gate) o *= sigmoid_f((float)(i == wave ? gate[x] : ((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + h * vd + d]));
+                if (a.p.gate) o *= sigmoid_f((float)(NARROW && i == wave ? gate[x] : ((const bf16 *)a.p.gate)[(size_t)row * a.p.ldg + h * vd + d]));
                 ((bf16 *)a.p.out)[(size_t)row * a.p.ldo + h * vd + d] = (bf16)o;
             }
             continue;
