@@ -1059,6 +1059,29 @@ def test_paged_decode_single_batched_ragged(be, f16, shape):
     be.reset_pool()
 
 
+def test_scratch_that_cannot_grow():
+    """Partial sums of terabytes: an error before any launch, the old scratch is gone and kept graphs are told so, and the next calls work."""
+    from vexel_amd.backend import HipBackend, VexelError
+    be = HipBackend(0)
+    rng = np.random.default_rng(5)
+    B, hq, d, bs, nblocks = 3, 8, 128, 16, 8
+    pool = _make_pool(rng, True, nblocks, bs, hq, d)
+    table = rng.permutation(nblocks)[:6].reshape(3, 2).astype(np.int32)
+    lens = [17, 32, 20]
+    q = rng.standard_normal((B, hq, d)).astype(np.float32)
+    sc = np.float32(1 / math.sqrt(d))
+    want = np.stack([nx.sdpa_paged_decode(q[i], pool, table[i], 2, bs, hq, hq, d, sc, lens[i] - bs) for i in range(B)])
+    dq, dpool, dt, dl, do = be.upload(q), be.upload(pool), be.upload(table), be.upload(np.array(lens, dtype=np.int32)), be.alloc(q.nbytes)
+    for _ in range(2):
+        be.sdpa_paged_decode_ragged(dq, dpool, True, dt, dl, do, B, 2, bs, hq, hq, d, sc, 32)
+        _close(be.download(do, q.shape, np.float32), want, 1e-5, 3e-6, "paged ragged")
+        gen = be.scratch_generation()
+        with pytest.raises(VexelError, match="scratch"):
+            be.sdpa_paged_decode_ragged(dq, dpool, True, dt, dl, do, 1024, 1 << 26, bs, hq, hq, d, sc, 1 << 30)
+        assert be.scratch_generation() > gen
+    be.close()
+
+
 @pytest.mark.parametrize("hq,hk,d", [(8, 2, 128), (16, 2, 64), (6, 2, 128)])
 def test_paged_decode_grouped_queries_value_ranges(be, hq, hk, d):
     """The grouped-query kernel scales every query row by a power of two before it splits it into two f16 halves and

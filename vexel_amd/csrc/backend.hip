@@ -35,14 +35,16 @@ int ensure_ws(vx_backend *be, void **ptr, size_t *cap, size_t bytes, const char 
     if (*ptr) VX_CHECK_HIP(hipFree(*ptr));
     *ptr = nullptr;
     *cap = 0;
+    be->scratch_gen++;  // (also when no larger one is to be had: a recorded graph holds the old address)
     size_t want = bytes + bytes / 4;
     hipError_t e = hipMalloc(ptr, want);
     if (e != hipSuccess) {
+        *ptr = nullptr;
+        (void)hipGetLastError();  // (not the next launch's error)
         set_error("hipMalloc(%zu) for %s scratch failed: %s", want, what, hipGetErrorString(e));
         return VX_ERR_OOM;
     }
     *cap = want;
-    be->scratch_gen++;
     return VX_OK;
 }
 
