@@ -282,7 +282,7 @@ int vx_decode_attn_qkv_supported(const vx_qweight *wq, const vx_qweight *wk, con
  * stands, a vx_decode_attn_qkv call with the same positions pointer, at most 32 rows, an unbiased interleaved whole-head
  * RoPE and weights laid out for a single K slice rotates and stores its rows inside the projection launch (one launch
  * per layer less), with the same arithmetic; a call of that RoPE whose projection leaves K slices' sums (more rows, the
- * formats with a min term, V in another format, vx_prefill_attn_qkv) reads its cos / sin from the table in the RoPE +
+ * formats with a min term, large packed matrices, V in another format, vx_prefill_attn_qkv) reads its cos / sin from the table in the RoPE +
  * store launch that follows. The table falls whenever the library writes to a caller's buffer, whichever it is (vx_pack_batch,
  * vx_decode_advance, vx_to_device, vx_to_device_staged, vx_to_device_staged_many, vx_copy_buffer, vx_fill_zero) or frees
  * one (vx_free), with vx_reset_pool and with graphs (vx_graph_begin_capture, vx_graph_end_capture, vx_graph_launch); a
