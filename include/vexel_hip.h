@@ -886,6 +886,21 @@ typedef struct vx_scan_args {
 int vx_scan_state_pad(int states);  /* 16, 32, .. 256; -1 beyond 256 */
 int vx_selective_scan(vx_backend *be, int act, const vx_ragged *b, const vx_scan_args *p);
 
+/* The whole branch of a step with one row per sequence (q_lens NULL), in two launches: vx_conv_silu(conv), the map x_w [x_n, x_k] of its
+ * result (VX_LIN_SPLIT: dt_k columns in the activation type, then B | C), the map dt_w [dt_n, dt_k] of the former with bias dt_bias
+ * (VX_LIN_SOFTPLUS), vx_selective_scan(scan; its dt and bc unused, x = conv.out): the same results. For sizes that vx_scan_step_takes
+ * says 1 to; others, and other steps, take the calls one by one. attn (or NULL): vx_attn_ragged(attn) as well, which neither reads nor
+ * writes what the branch does; in the branch's second launch where its geometry allows. */
+typedef struct vx_scan_step_args {
+    vx_conv_args conv;
+    vx_scan_args scan;
+    const void *x_w, *dt_w;
+    int x_n, x_k, dt_n, dt_k;
+    const float *dt_bias;
+} vx_scan_step_args;
+int vx_scan_step_takes(vx_backend *be, int act, const vx_ragged *b, const vx_scan_step_args *p);
+int vx_scan_step(vx_backend *be, int act, const vx_ragged *b, const vx_scan_step_args *p, const vx_attn_args *attn);
+
 /* Wall-clock helpers on the backend stream (HIP events), for benchmarks. */
 int vx_timer_start(vx_backend *be);
 int vx_timer_stop_ms(vx_backend *be, float *ms);

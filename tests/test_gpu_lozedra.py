@@ -420,6 +420,106 @@ def test_selective_scan(be, act, states, channels):
     be.free(state)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("channels,states,rank,attn", [(2048, 16, 64, None), (2024, 11, 100, (10, 2, 112)), (3976, 3, 300, (4, 4, 64)), (4096, 16, 128, (16, 4, 128))])
+def test_scan_step_is_the_separate_calls(be, rows, channels, states, rank, attn):
+    """The scan branch of a step of single rows in two launches: outputs, convolved inputs and both states after two steps are bit for
+    bit those of the four calls (row tiles of 16 with one over, channels that end inside a workgroup's 32 and inside a step of the
+    map's inputs, one to two steps of the rank for a wave), for sequences at position 0, within the first taps and later, with leavings of an earlier owner in every slot. So is attention beside it (in the same launch for heads of 112 and 128, of
+    one piece and, where a sequence is long, of several; in its own for 64)."""
+    from vexel_amd.backend import VxAttnArgs, VxScanStepArgs
+    rng = np.random.default_rng(rows + channels)
+    k, dt_k, pad, taps, n16 = -(-channels // 64) * 64, -(-rank // 64) * 64, 16, 4, -(-channels // 16) * 16
+    w_x, w_dt = np.zeros((dt_k + 2 * pad, channels)), rng.standard_normal((channels, rank)) / np.sqrt(rank)
+    for first, n in ((0, rank), (dt_k, states), (dt_k + pad, states)):
+        w_x[first:first + n] = rng.standard_normal((n, channels)) / np.sqrt(channels)
+    x_w, x_n, x_k = packed(be, w_x)
+    dt_w, dt_n, _ = packed(be, w_dt, k_pad=dt_k)
+    assert (x_k, dt_n) == (k, n16)
+    ld, cat = 2 * n16 + 8, channels + 24
+    xs = [grid(rng.standard_normal((rows, ld)), BF16) for _ in range(2)]
+    a2 = np.zeros((channels, pad), dtype=np.float32)
+    a2[:, :states] = -np.exp(rng.uniform(np.log(0.002), np.log(8.0), (channels, states))) / np.log(2.0)
+    conv_w, conv_b, D, bias = (rng.standard_normal(s).astype(np.float32) for s in ((taps, channels), channels, channels, channels))
+    start = [int(s) for s in np.resize([0, 1, 2, 3, 40, 300 if channels == 2024 else 50], rows)]
+    slots = rng.permutation(rows + 2)[:rows].tolist()
+    left, left_c = np.full((rows + 2, channels, pad), 1e3, dtype=np.float32), np.full((rows + 2, taps - 1, channels), 1e3)
+    for i, s in zip(slots, start):
+        if s:
+            left[i] = rng.standard_normal((channels, pad))
+            left_c[i, max(0, taps - 1 - s):] = rng.standard_normal((taps - 1, channels))[max(0, taps - 1 - s):]
+    dev = [be.upload(v) for v in (conv_w, conv_b, a2, D, bias)]
+    res = []
+    if attn:
+        heads, kv_heads, dim = attn
+        tables = Batch(be, [s + 1 for s in start], [1] * rows, slots=slots)
+        pool = up(be, rng.standard_normal((tables.pool_blocks, 2 * kv_heads * dim * BS)), BF16)
+        q = up(be, rng.standard_normal((rows, 2 * heads * dim)), BF16)
+        table = be.upload(rng.standard_normal((heads, 20)).astype(np.float32))
+    for fused in (True, False):
+        state, hist = be.upload(left), up(be, left_c, BF16)
+        outs = []
+        for step in range(2):
+            bt = Batch(be, [s + step for s in start], [1] * rows, slots=slots)
+            x, xc, out = up(be, xs[step], BF16), blank(be, (rows, k), BF16), blank(be, (rows, cat + 1), BF16)
+            p = VxScanStepArgs()
+            c, s = p.conv, p.scan
+            c.channels, c.taps, c.x, c.ldx, c.w, c.b, c.state, c.out, c.ldo = channels, taps, x, ld, dev[0], dev[1], hist, xc, k
+            s.channels, s.states, s.a2, s.d, s.x, s.z, s.ldx, s.ldz = channels, states, dev[2], dev[3], xc, x + n16 * 2, k, ld
+            s.state, s.out_scale, s.out, s.ldo, s.out_cols = state, 0.6, out, cat + 1, cat
+            p.x_w, p.dt_w, p.x_n, p.x_k, p.dt_n, p.dt_k, p.dt_bias = x_w, dt_w, x_n, x_k, dt_n, dt_k, dev[4]
+            at = None
+            if attn:
+                seen = blank(be, (rows, heads * dim), BF16)
+                at = VxAttnArgs()
+                at.heads, at.kv_heads, at.k_dim, at.v_dim, at.scale, at.bias, at.bias_len = heads, kv_heads, dim, dim, dim ** -0.5, table, 20
+                at.q, at.ldq, at.gate, at.ldg, at.pool, at.out_scale = q, 2 * heads * dim, q + heads * dim * 2, 2 * heads * dim, pool, 0.7
+                at.out, at.ldo = seen, heads * dim
+            if fused:
+                assert be.scan_step(BF16, bt.c, p, at)
+            else:
+                if attn:
+                    be.attn_ragged(BF16, bt.c, at)
+                dtr, bc, dt = blank(be, (rows, dt_k), BF16), blank(be, (rows, 2 * pad), F32), blank(be, (rows, dt_n), F32)
+                be.conv_silu(BF16, bt.c, c)
+                be.linear(BF16, xc, k, x_w, x_n, x_k, rows, lin_out(kind=3, out=dtr, ldo=dt_k, cols=dt_k, split=dt_k, out2=bc, ldo2=2 * pad))
+                be.linear(BF16, dtr, dt_k, dt_w, dt_n, dt_k, rows, lin_out(kind=4, out=dt, ldo=dt_n, cols=channels, bias=dev[4]))
+                s.dt, s.bc, s.lddt = dt, bc, dt_n
+                be.selective_scan(BF16, bt.c, s)
+            outs += [down(be, xc, (rows, k), BF16), down(be, out, (rows, cat + 1), BF16)]
+            if attn:
+                outs.append(down(be, seen, (rows, heads * dim), BF16))
+                assert np.isfinite(outs[-1]).all()
+        res.append(outs + [be.download(state, left.shape, np.float32), down(be, hist, left_c.shape, BF16)])
+    for x, y in zip(*res):
+        assert np.array_equal(x, y, equal_nan=True)
+    assert np.isfinite(res[0][1][:, :cat]).all() and np.any(res[0][1][:, :channels] != 0)
+    be.reset_pool()
+
+
+def test_scan_step_leaves_other_sizes_alone(be):
+    """What the two launches do not take is said before anything is done: steps with several rows of a sequence, float32, other tap
+    counts, more than 16 states, narrow or unaligned channels."""
+    from vexel_amd.backend import VxScanStepArgs
+    one, many = Batch(be, [3, 4], [1, 1]), Batch(be, [3, 4], [1, 2])
+
+    def takes(act=BF16, batch=one, **change):
+        v = dict(channels=2048, taps=4, states=16, ldx=4096, x=1 << 20)
+        v.update(change)
+        p = VxScanStepArgs()
+        c, s, at = p.conv, p.scan, 1 << 20
+        c.channels, c.taps, c.x, c.ldx, c.w, c.b, c.state, c.out, c.ldo = v["channels"], v["taps"], v["x"], v["ldx"], at, at, at, at, 2048
+        s.channels, s.states, s.a2, s.d, s.x, s.z, s.ldx, s.ldz = v["channels"], v["states"], at, at, at, at, 2048, 4096
+        s.state, s.out, s.ldo, s.out_cols = at, at, 2048, 2048
+        p.x_w, p.dt_w, p.x_n, p.x_k, p.dt_n, p.dt_k, p.dt_bias = at, at, 96, 2048 if v["channels"] > 1024 else 1024, 2048, 64, at
+        return be.lib_call("vx_scan_step_takes", be._h, act, C.byref(batch.c), C.byref(p))
+
+    assert takes() == 1
+    assert takes(channels=2040) == 1
+    assert 0 == takes(act=F32) == takes(batch=many) == takes(taps=3) == takes(states=17) == takes(channels=1000) == takes(channels=2044) == takes(ldx=4092)
+    assert 0 == takes(x=(1 << 20) + 8)
+
+
 # ---------------------------------------------------------------- attention
 class Cache:
     """Random keys and values of every sequence, in the pool's layout on the device."""

@@ -107,6 +107,10 @@ class VxScanArgs(C.Structure):
                        "ptr out; int ldo out_cols")
 
 
+class VxScanStepArgs(C.Structure):
+    _fields_ = [("conv", VxConvArgs), ("scan", VxScanArgs)] + _fields("ptr x_w dt_w; int x_n x_k dt_n dt_k; ptr dt_bias")
+
+
 class VexelError(RuntimeError):
     def __init__(self, code, msg):
         super().__init__("vexel_hip error %d: %s" % (code, msg))
@@ -547,6 +551,13 @@ class HipBackend:
 
     def selective_scan(self, act, batch, args):
         self.call("vx_selective_scan", act, C.byref(batch), C.byref(args))
+
+    def scan_step(self, act, batch, args, attn=None):
+        """-> whether the branch's two launches take these sizes (nothing was done otherwise)"""
+        if not self._lib.vx_scan_step_takes(self._h, act, C.byref(batch), C.byref(args)):
+            return False
+        self.call("vx_scan_step", act, C.byref(batch), C.byref(args), C.byref(attn) if attn is not None else None)
+        return True
 
     # ---- graph capture / timing
     def graph_begin_capture(self):

@@ -13,7 +13,7 @@ SYNTH_LIB = os.path.join(HERE, "libvexel_synth.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
 SOURCES = ["backend.hip", "transfer.hip", "elementwise.hip", "attention.hip", "qgemm.hip", "qstream.hip", "qmatvec.hip", "pack.hip", "sampler.hip", "medusa.hip",
-           "linear.hip", "mixers.hip", "attn_ragged.hip", "attn_latent.hip", "heads.hip",
+           "linear.hip", "mixers.hip", "scan_step.hip", "attn_ragged.hip", "attn_latent.hip", "heads.hip",
            "decay.hip", "experts.hip", "forget.hip", "attn_talk.hip"]
 HOST_SOURCES = ["runtime.cpp", "gguf.cpp", "scheduler.cpp", "layers.cpp", "checkpoint.cpp"]
 

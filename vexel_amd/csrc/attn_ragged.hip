@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "attn_tiles.h"
+#include "scan_step.h"
 
 using namespace vx;
 
@@ -242,25 +243,24 @@ template <int VD, int MAPS> constexpr int decode_areas() { return MAPS * 16 * (V
 // them 23.1) were slower. Wider forms are the slower for all this (192 / 160 columns, 44 tokens 8.0 -> 8.3, 600 30.1 -> 30.6; 256 with a
 // bias table, 600 38.8 -> 39.1; two maps of 128, 2000 66.0 -> 66.8): they read one number after the other, and the gate where they write.
 template <int KD, int VD, int MAPS>
-__global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode_kernel(Args a) {
+__device__ __forceinline__ void one_row(const Args &a, float *s_dyn, int bx, int by, int bz) {
     constexpr int QT = MAPS;
     constexpr bool NARROW = decode_areas<VD, MAPS>() == 4;
-    extern __shared__ float s_dyn[];
     __shared__ float s_m[4][QT * 16], s_l[4][QT * 16];
     float *s_lut = s_dyn;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = blockIdx.x % a.p.kv_heads, h0 = blockIdx.x / a.p.kv_heads * 16;  // 16 of the group's query heads
+    const int g = bx % a.p.kv_heads, h0 = bx / a.p.kv_heads * 16;  // 16 of the group's query heads
     int seq, piece, row, len, table;
     if constexpr (NARROW) {
         if (a.items) {
             // (one trip for the three: the list has room for every workgroup of the grid)
-            int n = __builtin_amdgcn_readfirstlane(a.items[0]), s = __builtin_amdgcn_readfirstlane(a.items[4 + 4 * blockIdx.y]),
-                c = __builtin_amdgcn_readfirstlane(a.items[5 + 4 * blockIdx.y]);
+            int n = __builtin_amdgcn_readfirstlane(a.items[0]), s = __builtin_amdgcn_readfirstlane(a.items[4 + 4 * by]),
+                c = __builtin_amdgcn_readfirstlane(a.items[5 + 4 * by]);
             asm volatile("" : "+s"(n), "+s"(s), "+s"(c));
-            if ((int)blockIdx.y >= n) return;
+            if (by >= n) return;
             seq = __builtin_amdgcn_readfirstlane(s), piece = __builtin_amdgcn_readfirstlane(c);
         } else {
-            piece = blockIdx.y, seq = blockIdx.z;
+            piece = by, seq = bz;
         }
         const int32_t *cu = a.one_token ? a.kv_lens : a.cu;
         int c0 = __builtin_amdgcn_readfirstlane(cu[seq]), c1 = __builtin_amdgcn_readfirstlane(cu[seq + (a.one_token ? 0 : 1)]);
@@ -270,10 +270,10 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
         row = a.one_token ? seq : c0;
     } else {
         if (a.items) {
-            if ((int)blockIdx.y >= a.items[0]) return;
-            seq = a.items[4 + 4 * blockIdx.y], piece = a.items[5 + 4 * blockIdx.y];
+            if (by >= a.items[0]) return;
+            seq = a.items[4 + 4 * by], piece = a.items[5 + 4 * by];
         } else {
-            piece = blockIdx.y, seq = blockIdx.z;
+            piece = by, seq = bz;
         }
         row = a.one_token ? seq : a.cu[seq];
         if (!a.one_token && a.cu[seq + 1] - row != 1) return;
@@ -398,6 +398,25 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
     }
 }
 
+template <int KD, int VD, int MAPS>
+__global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode_kernel(Args a) {
+    extern __shared__ float s_dyn[];
+    one_row<KD, VD, MAPS>(a, s_dyn, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// The same launch with the scan branch's second half (scan_step.h) behind it: the two read the same projection and write side by side, and
+// either is a chain of trips to memory that leaves most of the chip idle. Attention, the longer of the two, has the first workgroups. 32 sequences of
+// 16 / 4 heads x 128 beside 4096 channels x 16 states: 9.7 us and 9.2 us one behind the other, 12.7 together.
+template <int KD, int VD>
+__global__ void __launch_bounds__(256, 2) attn_scan_kernel(Args a, StepArgs s, int gx, int gy, int n_attn, int scan_x) {
+    extern __shared__ float s_dyn[];
+    const int id = blockIdx.x;
+    if (id < n_attn)
+        one_row<KD, VD, 1>(a, s_dyn, id % gx, id / gx % gy, id / gx / gy);
+    else
+        scan_step::scan_project(s, (id - n_attn) % scan_x, (id - n_attn) / scan_x);
+}
+
 template <int MAPS>
 __global__ void __launch_bounds__(64) merge_kernel(Args a) {
     const int h = blockIdx.x, seq = blockIdx.y, vd = a.p.v_dim;
@@ -486,14 +505,28 @@ void launch_prefill(vx_backend *be, Args a, const vx_ragged *b) {
     if (a.tiles > 0) prefill_kernel<KD, VD, QT, KS, MAPS><<<a.tiles * a.p.kv_heads, 256, lut > o ? lut : o, be->stream>>>(a);
 }
 
+struct Beside {  // the scan's workgroups that may join a launch of decode_kernel
+    const StepArgs *scan;
+    bool taken;
+};
+
 template <int KD, int VD, int MAPS>
-void launch_decode(vx_backend *be, const Args &a, dim3 grid) {
+void launch_decode(vx_backend *be, const Args &a, dim3 grid, Beside *side) {
     const size_t lut = a.lut_lds ? (size_t)a.group * a.p.bias_len * 4 : 0, o = (size_t)decode_areas<VD, MAPS>() * MAPS * 16 * (VD * 16 + 4) * 4;
+    if constexpr (MAPS == 1 && KD == 4 && VD == 8) {
+        if (side) {
+            using namespace scan_step;
+            const int n = (int)(grid.x * grid.y * grid.z), sx = ceil_div(side->scan->p.scan.channels, CH), sy = ceil_div(side->scan->rows, ROWS);
+            attn_scan_kernel<KD, VD><<<n + sx * sy, 256, lut > o ? lut : o, be->stream>>>(a, *side->scan, grid.x, grid.y, n, sx);
+            side->taken = true;
+            return;
+        }
+    }
     decode_kernel<KD, VD, MAPS><<<grid, 256, lut > o ? lut : o, be->stream>>>(a);
 }
 
 template <int KD, int VD, int MAPS = 1>
-int run_fast(vx_backend *be, Args a, const vx_ragged *b) {
+int run_fast(vx_backend *be, Args a, const vx_ragged *b, Beside *side) {
     bool any_many = false, any_one = !b->q_lens && a.p.min_rows <= 1;
     int64_t many = 0;
     a.min_rows = a.p.min_rows > 2 ? a.p.min_rows : 2;
@@ -554,7 +587,7 @@ int run_fast(vx_backend *be, Args a, const vx_ragged *b) {
             grid = dim3(a.p.kv_heads, b->n_seqs * a.pieces, 1);
         }
         grid.x *= ceil_div(a.group, 16);
-        launch_decode<KD, VD, MAPS>(be, a, grid);
+        launch_decode<KD, VD, MAPS>(be, a, grid, side);
         VX_CHECK_LAUNCH();
         if (MAPS > 1 || a.pieces > 1) {  // (one piece of at most 128 or 256 keys is the result: a launch of 4.4 us less per layer)
             merge_kernel<MAPS><<<dim3(a.p.heads, b->n_seqs), 64, 0, be->stream>>>(a);
@@ -564,24 +597,7 @@ int run_fast(vx_backend *be, Args a, const vx_ragged *b) {
     return VX_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-size_t vx_kv_block_elems2(int block_size, int k_heads, int k_dim, int v_heads, int v_dim) {
-    if (block_size < 1 || k_heads < 1 || k_dim < 1 || v_heads < 1 || v_dim < 1) return 0;
-    return (size_t)block_size * ((size_t)k_heads * ((k_dim + 7) & ~7) + (size_t)v_heads * v_dim);
-}
-
-size_t vx_kv_block_elems(int block_size, int kv_heads, int k_dim, int v_dim) { return vx_kv_block_elems2(block_size, kv_heads, k_dim, kv_heads, v_dim); }
-
-int vx_attn_ragged_fast(int act, int block_size, int heads, int kv_heads, int k_dim, int v_dim) {
-    if (heads < 1 || kv_heads < 1 || heads % kv_heads) return 0;
-    const int wide = k_dim > v_dim ? k_dim : v_dim, group = heads / kv_heads;
-    return act == VX_ACT_BF16 && block_size == BS && k_dim >= 1 && v_dim >= 1 && wide <= 256 && group <= (wide <= 128 ? 64 : 16);
-}
-
-int vx_attn_ragged(vx_backend *be, int act, const vx_ragged *b, const vx_attn_args *p) {
+int attn_ragged(vx_backend *be, int act, const vx_ragged *b, const vx_attn_args *p, Beside *side) {
     int rc = enter(be);
     if (rc) return rc;
     rc = check_ragged(b, "vx_attn_ragged");
@@ -620,17 +636,17 @@ int vx_attn_ragged(vx_backend *be, int act, const vx_ragged *b, const vx_attn_ar
     if (fast) {
         const int wide = p->k_dim > p->v_dim ? p->k_dim : p->v_dim;
         if (maps == 2) {
-            if (wide <= 64) return run_fast<2, 4, 2>(be, a, b);
-            if (p->k_dim <= 64 && p->v_dim <= 128) return run_fast<2, 8, 2>(be, a, b);
-            if (wide <= 128) return run_fast<4, 8, 2>(be, a, b);
-            return run_fast<4, 16, 2>(be, a, b);
+            if (wide <= 64) return run_fast<2, 4, 2>(be, a, b, side);
+            if (p->k_dim <= 64 && p->v_dim <= 128) return run_fast<2, 8, 2>(be, a, b, side);
+            if (wide <= 128) return run_fast<4, 8, 2>(be, a, b, side);
+            return run_fast<4, 16, 2>(be, a, b, side);
         }
-        if (wide <= 64) return run_fast<2, 4>(be, a, b);
-        if (wide <= 96) return run_fast<3, 6>(be, a, b);
-        if (wide <= 128) return run_fast<4, 8>(be, a, b);
-        if (p->k_dim <= 192 && p->v_dim <= 128) return run_fast<6, 8>(be, a, b);
-        if (wide <= 192) return run_fast<6, 12>(be, a, b);
-        return run_fast<8, 16>(be, a, b);
+        if (wide <= 64) return run_fast<2, 4>(be, a, b, side);
+        if (wide <= 96) return run_fast<3, 6>(be, a, b, side);
+        if (wide <= 128) return run_fast<4, 8>(be, a, b, side);
+        if (p->k_dim <= 192 && p->v_dim <= 128) return run_fast<6, 8>(be, a, b, side);
+        if (wide <= 192) return run_fast<6, 12>(be, a, b, side);
+        return run_fast<8, 16>(be, a, b, side);
     }
     PlainAttn t;
     memset(&t, 0, sizeof t);
@@ -664,5 +680,33 @@ int vx_attn_ragged(vx_backend *be, int act, const vx_ragged *b, const vx_attn_ar
     VX_CHECK_LAUNCH();
     return VX_OK;
 }
+
+}  // namespace
+
+namespace vx {
+int attn_beside(vx_backend *be, int act, const vx_ragged *b, const vx_attn_args *p, const StepArgs &scan, bool *beside) {
+    Beside side{&scan, false};
+    const int rc = attn_ragged(be, act, b, p, &side);
+    *beside = side.taken;
+    return rc;
+}
+}  // namespace vx
+
+extern "C" {
+
+size_t vx_kv_block_elems2(int block_size, int k_heads, int k_dim, int v_heads, int v_dim) {
+    if (block_size < 1 || k_heads < 1 || k_dim < 1 || v_heads < 1 || v_dim < 1) return 0;
+    return (size_t)block_size * ((size_t)k_heads * ((k_dim + 7) & ~7) + (size_t)v_heads * v_dim);
+}
+
+size_t vx_kv_block_elems(int block_size, int kv_heads, int k_dim, int v_dim) { return vx_kv_block_elems2(block_size, kv_heads, k_dim, kv_heads, v_dim); }
+
+int vx_attn_ragged_fast(int act, int block_size, int heads, int kv_heads, int k_dim, int v_dim) {
+    if (heads < 1 || kv_heads < 1 || heads % kv_heads) return 0;
+    const int wide = k_dim > v_dim ? k_dim : v_dim, group = heads / kv_heads;
+    return act == VX_ACT_BF16 && block_size == BS && k_dim >= 1 && v_dim >= 1 && wide <= 256 && group <= (wide <= 128 ? 64 : 16);
+}
+
+int vx_attn_ragged(vx_backend *be, int act, const vx_ragged *b, const vx_attn_args *p) { return attn_ragged(be, act, b, p, nullptr); }
 
 }  // extern "C"

@@ -374,25 +374,28 @@ int run_mixers(vh_model *m, const LayerRun &r, const vx_ragged &b, const MixActs
     VXC(vx_linear(m->be, x.act, a.h, width_pad, l.in.w, l.in.n, l.in.k, rows, &o));
     const int attn_cols = l.has_attn ? l.attn.heads * l.attn.v_dim : 0;
     if (!l.has_scan && attn_cols < ldc) VXC(vx_fill_zero(m->be, a.cat, (size_t)rows * ldc * es));
+    bool attended = !l.has_attn;
+    vx_attn_args at_;
+    memset(&at_, 0, sizeof at_);
+    if (l.has_attn) {
+        const AttnMixer &t = l.attn;
+        at_.heads = t.heads, at_.kv_heads = t.kv_heads, at_.k_dim = t.k_dim, at_.v_dim = t.v_dim;
+        at_.scale = t.scale, at_.temp_coef = t.temp_coef, at_.temp_every = t.temp_every;
+        at_.bias = t.bias, at_.bias_len = t.bias_len;
+        at_.q = at(a.proj, t.q_col, es), at_.ldq = ldp;
+        at_.gate = t.gate ? at(a.proj, t.g_col, es) : nullptr, at_.ldg = ldp;
+        at_.pool = r.kv, at_.out_scale = t.out_scale, at_.out = a.cat, at_.ldo = ldc;
+    }
     if (l.has_scan) {
         const ScanMixer &s = l.scan;
-        vx_conv_args cv;
-        memset(&cv, 0, sizeof cv);
+        vx_scan_step_args st;
+        memset(&st, 0, sizeof st);
+        vx_conv_args &cv = st.conv;
         cv.channels = s.channels, cv.taps = s.taps;
         cv.x = at(a.proj, s.x_col, es), cv.ldx = ldp;
         cv.w = s.conv_w, cv.b = s.conv_b, cv.state = r.conv;
         cv.out = a.xc, cv.ldo = s.x.k;
-        VXC(vx_conv_silu(m->be, x.act, &b, &cv));
-        o = plain(a.dtr, 0, s.dt_pad, s.dt_pad, 1);
-        o.kind = VX_LIN_SPLIT;
-        o.split = s.dt_pad, o.out2 = a.bc, o.ldo2 = 2 * s.pad;
-        VXC(vx_linear(m->be, x.act, a.xc, s.x.k, s.x.w, s.x.n, s.x.k, rows, &o));
-        o = plain(a.dt, 1, s.dt.n, s.channels, 1);
-        o.kind = VX_LIN_SOFTPLUS;
-        o.bias = s.dt_bias;
-        VXC(vx_linear(m->be, x.act, a.dtr, s.dt_pad, s.dt.w, s.dt.n, s.dt.k, rows, &o));
-        vx_scan_args sc;
-        memset(&sc, 0, sizeof sc);
+        vx_scan_args &sc = st.scan;
         sc.channels = s.channels, sc.states = s.states;
         sc.a2 = s.a2, sc.d = s.d;
         sc.x = a.xc, sc.ldx = s.x.k;
@@ -400,20 +403,24 @@ int run_mixers(vh_model *m, const LayerRun &r, const vx_ragged &b, const MixActs
         sc.dt = a.dt, sc.lddt = s.dt.n, sc.bc = a.bc;
         sc.state = r.state, sc.out_scale = s.out_scale;
         sc.out = at(a.cat, attn_cols, es), sc.ldo = ldc, sc.out_cols = ldc - attn_cols;
-        VXC(vx_selective_scan(m->be, x.act, &b, &sc));
+        st.x_w = s.x.w, st.x_n = s.x.n, st.x_k = s.x.k, st.dt_w = s.dt.w, st.dt_n = s.dt.n, st.dt_k = s.dt.k, st.dt_bias = s.dt_bias;
+        if (vx_scan_step_takes(m->be, x.act, &b, &st)) {
+            VXC(vx_scan_step(m->be, x.act, &b, &st, l.has_attn ? &at_ : nullptr));
+            attended = true;
+        } else {
+            VXC(vx_conv_silu(m->be, x.act, &b, &cv));
+            o = plain(a.dtr, 0, s.dt_pad, s.dt_pad, 1);
+            o.kind = VX_LIN_SPLIT;
+            o.split = s.dt_pad, o.out2 = a.bc, o.ldo2 = 2 * s.pad;
+            VXC(vx_linear(m->be, x.act, a.xc, s.x.k, s.x.w, s.x.n, s.x.k, rows, &o));
+            o = plain(a.dt, 1, s.dt.n, s.channels, 1);
+            o.kind = VX_LIN_SOFTPLUS;
+            o.bias = s.dt_bias;
+            VXC(vx_linear(m->be, x.act, a.dtr, s.dt_pad, s.dt.w, s.dt.n, s.dt.k, rows, &o));
+            VXC(vx_selective_scan(m->be, x.act, &b, &sc));
+        }
     }
-    if (l.has_attn) {
-        const AttnMixer &t = l.attn;
-        vx_attn_args at_;
-        memset(&at_, 0, sizeof at_);
-        at_.heads = t.heads, at_.kv_heads = t.kv_heads, at_.k_dim = t.k_dim, at_.v_dim = t.v_dim;
-        at_.scale = t.scale, at_.temp_coef = t.temp_coef, at_.temp_every = t.temp_every;
-        at_.bias = t.bias, at_.bias_len = t.bias_len;
-        at_.q = at(a.proj, t.q_col, es), at_.ldq = ldp;
-        at_.gate = t.gate ? at(a.proj, t.g_col, es) : nullptr, at_.ldg = ldp;
-        at_.pool = r.kv, at_.out_scale = t.out_scale, at_.out = a.cat, at_.ldo = ldc;
-        VXC(vx_attn_ragged(m->be, x.act, &b, &at_));
-    }
+    if (!attended) VXC(vx_attn_ragged(m->be, x.act, &b, &at_));
     return run_out(m, l, rows, a, slices);
 }
 

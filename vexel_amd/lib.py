@@ -153,6 +153,8 @@ SIGNATURES = {
     "vx_conv_silu": (_i, [_vp, _i, _vp, _vp]),
     "vx_scan_state_pad": (_i, [_i]),
     "vx_selective_scan": (_i, [_vp, _i, _vp, _vp]),
+    "vx_scan_step_takes": (_i, [_vp, _i, _vp, _vp]),
+    "vx_scan_step": (_i, [_vp, _i, _vp, _vp, _vp]),
     "vx_timer_start": (_i, [_vp]),
     "vx_timer_stop_ms": (_i, [_vp, C.POINTER(_f)]),
 }
