@@ -703,6 +703,38 @@ def test_single_row_qkv_finishes_its_rows(be, fqk, fv):
     be.reset_pool()
 
 
+@pytest.mark.parametrize("fqk", [nx.FMT_Q4_K, nx.FMT_Q5_K])
+@pytest.mark.parametrize("hq,hk,d", [(4, 1, 64), (26, 2, 128), (32, 32, 128), (40, 40, 128)])
+def test_single_row_qkv_of_two_formats_in_one_launch(be, fqk, hq, hk, d):
+    """Q and K of one format, V in Q6_K, one row: the launch that takes both (a last pass of few rows, one trip, two trips of Q|K and
+    one of V, two of either) gives what the separate operations give."""
+    rng = np.random.default_rng(fqk + hq)
+    hidden, bs, nblocks, eps, theta = hq * d, 16, 8, 1e-5, 10000.0
+    kvd = hk * d
+    dims, fm = dict(wq=(hidden, hidden), wk=(kvd, hidden), wv=(kvd, hidden)), dict(wq=fqk, wk=fqk, wv=nx.FMT_Q6_K)
+    dW = {n: be.upload(np.resize(qz.random_quant(fm[n], rng, 64, hidden).reshape(64, -1), (dims[n][0], qz.random_quant(fm[n], rng, 1, hidden).size)))
+          for n in dims}
+    qw = {n: be.qweight(fm[n], dW[n], *dims[n]) for n in dims}
+    x, n1 = (rng.standard_normal((1, hidden)) * 2).astype(np.float32), rng.standard_normal(hidden).astype(np.float32)
+    pool = _make_pool(rng, True, nblocks, bs, hk, d)
+    dx, dn1, dpool, dpool2 = be.upload(x), be.upload(n1), be.upload(pool), be.upload(pool)
+    dpos, dslots = be.upload(np.array([1234], dtype=np.int32)), be.upload(np.array([77], dtype=np.int32))
+    dnorm, dq, dk, dv, dq2 = (be.alloc(n * 4) for n in (hidden, hidden, kvd, kvd, hidden))
+    be.rmsnorm(dx, dn1, dnorm, 1, hidden, eps)
+    for name, out in (("wq", dq), ("wk", dk), ("wv", dv)):
+        be.matmul_quant(fm[name], dnorm, dW[name], out, None, 1, dims[name][0], hidden)
+    be.rope_store_paged(dq, dk, dv, dpos, dslots, dpool, True, 1, hq, hk, d, bs, theta)
+    be.rope_table_prepare(dpos, 1, d, theta)
+    be.decode_attn_qkv(dx, dn1, eps, False, qw["wq"], qw["wk"], qw["wv"], 1, dpos, dslots, dpool2, True, hq, hk, d, bs, theta, dq2)
+    q_ref, q = be.download(dq, (hidden,), np.float32), be.download(dq2, (hidden,), np.float32)
+    assert np.all(np.abs(q - q_ref) <= 2e-5 * np.abs(q_ref).max() + 1e-6)   # (the norm is applied to the sums here, to the row there)
+    ref, got = (nx.f16_to_f32_array(be.download(p, pool.shape, pool.dtype)) for p in (dpool, dpool2))
+    assert np.all(np.abs(got - ref) <= np.abs(ref) * 2.0 ** -10 + 1e-4 * max(1.0, np.abs(ref).max() / 8))
+    was = nx.f16_to_f32_array(pool)
+    assert np.count_nonzero(got != was) > 1.9 * kvd and np.count_nonzero(got != was) <= 2 * kvd   # (every row of K and V, nothing else)
+    be.reset_pool()
+
+
 # (query heads, kv heads, head size): a workgroup's columns are one 256-column chunk, a quarter or half of one,
 # four of them, one and a half (two KV heads make three chunks: merged in the kernel), three and a half and five
 # sixteenths (7 chunks per two KV heads, 5 per sixteen heads of 80: more than a workgroup merges at once, the

@@ -209,6 +209,9 @@ bool matvec_ok(int fmt, const void *const *ws, const int *ns, int nw, int k);
 // two matrices of equal height n, out[i] = silu(W0[i] . a) * (W1[i] . a), i < n.
 int run_matvec_fused(vx_backend *be, int fmt, const void *const *ws, const int *ns, int nw, int k, const MatvecSource &src,
                      float *out, const float *residual, int pair);
+// Matrices of one format and a last one of another in one launch that finishes its rows (src.rope); VX_ERR_UNSUPPORTED, and nothing
+// done, where no kernel takes the two formats together.
+int run_matvec_two(vx_backend *be, int fmt, const void *const *ws, const int *ns, int nw, int fmt2, const void *w2, int n2, int k, const MatvecSource &src);
 
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -2419,8 +2419,10 @@ int vx_prefill_attn_qkv(vx_backend *be, const float *x, const float *norm_weight
             src.x = x;
             src.norm_w = norm_weight;
             src.eps = eps;
-            if (finish_rows()) {  // both launches finish their own rows
+            if (finish_rows()) {  // the launch, or both launches, finish their own rows
                 src.rope = rope_of();
+                rc = run_matvec_two(be, wq->fmt, mw, mn, 2, wv->fmt, wv->data, wv->n, k, src);
+                if (rc != VX_ERR_UNSUPPORTED) return rc;
                 rc = run_matvec_fused(be, wq->fmt, mw, mn, 2, k, src, (float *)be->part_ws, nullptr, 0);
                 if (rc == VX_OK) {
                     src.rope.first = wq->n + wk->n;

@@ -920,16 +920,17 @@ struct K3_Q6_K {  // share (n, a, h): low and high nibbles of ql[64 n + 32 a + 1
     }
 };
 
+// Workgroup `block` of `blocks`; smem: planes [shares + 1][MV2_XSTRIDE] (the last share zeros).
 template <class F>
-__global__ void __launch_bounds__(MV_THREADS) qmatvec3_kernel(const MvArgs p, const int n_passes) {
-    constexpr int DEPTH = 2;  // (three: 3 - 20 % slower, a wave less per SIMD)
-    extern __shared__ __attribute__((aligned(16))) uint32_t smem[];  // planes [shares + 1][MV2_XSTRIDE] (the last share zeros)
+__device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, const int block, const int blocks) {
+    extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
     __shared__ float s_ss[MV_WAVES];
+    constexpr int DEPTH = 2;  // (three: 3 - 20 % slower, a wave less per SIMD)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int K = p.K, n_shares = K / 32, pair = p.pair;
     const int steps = (n_shares + 63) / 64;
-    const int n_waves = gridDim.x * MV_WAVES;
+    const int n_waves = blocks * MV_WAVES;
     const int share = lane % F::SHARES;
     struct Load2 {
         typename F::Load r[2];
@@ -964,7 +965,7 @@ __global__ void __launch_bounds__(MV_THREADS) qmatvec3_kernel(const MvArgs p, co
     // The activation's first loads go ahead of the weights': behind them they would wait for all of those.
     if (tid < n_shares) load_x(tid);
     __builtin_amdgcn_sched_barrier(0);
-    int q = blockIdx.x * MV_WAVES + wave, t = 0;  // what is worked on
+    int q = block * MV_WAVES + wave, t = 0;  // what is worked on
     int iq = q, it = 0;                           // what is asked for next
     auto next = [&]() __attribute__((always_inline)) {
         const Load2 l = issue(iq, it);
@@ -1076,31 +1077,80 @@ __global__ void __launch_bounds__(MV_THREADS) qmatvec3_kernel(const MvArgs p, co
     }
 }
 
-// Launches the third form when it serves the call: an activation row from memory, planes that fit LDS.
 template <class F>
-bool launch_third_form(vx_backend *be, MvArgs &a) {
+__global__ void __launch_bounds__(MV_THREADS) qmatvec3_kernel(const MvArgs p, const int n_passes) {
+    matvec3<F>(p, n_passes, blockIdx.x, gridDim.x);
+}
+
+// Q|K of one format and V of another in one launch: the first workgroups take Q|K. A launch of its own for V is mostly what every launch
+// costs before its first weights and behind its last (Q|K 8192 x 4096 of Q4_K 9.6 us and V 4096 x 4096 of Q6_K 5.9, together 11.6).
+template <class F, class G>
+__global__ void __launch_bounds__(MV_THREADS) qmatvec3_two_kernel(const MvArgs p, const int passes, const int blocks, const MvArgs p2, const int passes2) {
+    if ((int)blockIdx.x < blocks)
+        matvec3<F>(p, passes, blockIdx.x, blocks);
+    else
+        matvec3<G>(p2, passes2, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
+}
+
+// Whether the third form serves the call: an activation row from memory, planes that fit LDS.
+template <class F>
+bool third_form_ok(MvArgs &a) {
     static const bool off = getenv("VEXEL_HIP_MATVEC_FIRST_FORM") != nullptr;
-    const size_t lds = (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4;
-    if (off || a.mode == MV_MERGED_ATTENTION || lds > 120 * 1024) return false;
+    if (off || a.mode == MV_MERGED_ATTENTION || (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4 > 120 * 1024) return false;
     if (a.rope.q_out && (a.pair > 0 || a.residual || a.rope.qd % 2 != 0 || a.rope.kvd % 2 != 0 || a.rope.first % 2 != 0 || a.N % 2 != 0 ||
                          (a.rope.head_dim & (a.rope.head_dim - 1)) != 0 || ((uintptr_t)a.rope.q_out & 7) != 0))
         return false;
     a.row_bytes = (size_t)(a.K / (32 * F::SHARES)) * F::BYTES;
-    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_kernel<F>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-    (void)attr;
-    // workgroups a compute unit holds, asked for once per length of the row (backends may call from several threads)
-    constexpr int LONGEST = 120 * 1024 / (MV2_XSTRIDE * 4);
-    static std::atomic<int> resident[LONGEST + 1];
-    std::atomic<int> &known = resident[a.K / 32];
+    return true;
+}
+
+// Workgroups of a kernel of the third form that a compute unit holds, asked for once per length of the row (backends may call from several threads).
+template <class Kernel>
+int third_form_resident(Kernel *kernel, std::atomic<int> *resident, int k, size_t lds) {
+    std::atomic<int> &known = resident[k / 32];
     int per_cu = known.load(std::memory_order_relaxed);
     if (per_cu == 0) {
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, qmatvec3_kernel<F>, MV_THREADS, lds) != hipSuccess || per_cu < 1) per_cu = 1;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, MV_THREADS, lds) != hipSuccess || per_cu < 1) per_cu = 1;
         known.store(per_cu, std::memory_order_relaxed);
     }
+    return per_cu;
+}
+constexpr int MV3_LONGEST = 120 * 1024 / (MV2_XSTRIDE * 4);
+
+// Launches the third form when it serves the call.
+template <class F>
+bool launch_third_form(vx_backend *be, MvArgs &a) {
+    if (!third_form_ok<F>(a)) return false;
+    const size_t lds = (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4;
+    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_kernel<F>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    (void)attr;
+    static std::atomic<int> resident[MV3_LONGEST + 1];
+    const int per_cu = third_form_resident(qmatvec3_kernel<F>, resident, a.K, lds);
     const int n_passes = a.pair > 0 ? a.pair : ceil_div(a.N, 2);
     // as many workgroups as fit at once, or fewer when that makes every wave's number of passes equal
     const int wgs = ceil_div(n_passes, MV_WAVES), trips = ceil_div(wgs, per_cu * device_cus(be));
     qmatvec3_kernel<F><<<ceil_div(wgs, trips), MV_THREADS, lds, be->stream>>>(a, n_passes);
+    return true;
+}
+
+// Two of them in one launch, K and the activation row the same.
+template <class F, class G>
+bool launch_third_form_two(vx_backend *be, MvArgs &a, MvArgs &b) {
+    if (!third_form_ok<F>(a) || !third_form_ok<G>(b)) return false;
+    const size_t lds = (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4;
+    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_two_kernel<F, G>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    (void)attr;
+    static std::atomic<int> resident[MV3_LONGEST + 1];
+    const int room = std::max(2, third_form_resident(qmatvec3_two_kernel<F, G>, resident, a.K, lds) * device_cus(be));
+    const int pa = ceil_div(a.N, 2), pb = ceil_div(b.N, 2), wa = ceil_div(pa, MV_WAVES), wb = ceil_div(pb, MV_WAVES);
+    // all resident at once, with the fewest trips of either; of the two, one more goes to the one that has the most workgroups
+    int ta = 1, tb = 1;
+    while (ceil_div(wa, ta) + ceil_div(wb, tb) > room) {
+        if (ceil_div(wa, ta) >= ceil_div(wb, tb)) ta++;
+        else tb++;
+    }
+    const int ga = ceil_div(wa, ta), gb = ceil_div(wb, tb);
+    qmatvec3_two_kernel<F, G><<<ga + gb, MV_THREADS, lds, be->stream>>>(a, pa, ga, b, pb);
     return true;
 }
 
@@ -1311,13 +1361,11 @@ int run_matvec(vx_backend *be, int fmt, const float *a, const void *b, float *ou
     return run_matvec_fused(be, fmt, ws, ns, 1, k, src, out, residual, 0);
 }
 
-// The general form: nw <= 3 matrices of one format and K, rows concatenated; the activation row from `src`;
-// pair != 0: two matrices of equal height, out[i] = silu(row i of the first) * (row i of the second).
-int run_matvec_fused(vx_backend *be, int fmt, const void *const *ws, const int *ns, int nw, int k, const MatvecSource &src,
-                     float *out, const float *residual, int pair) {
+static int matvec_args(int fmt, const void *const *ws, const int *ns, int nw, int k, const MatvecSource &src, float *out, const float *residual, int pair,
+                       MvArgs &a) {
     const size_t rb = mv_row_bytes(fmt, k);
     if (rb == 0 || nw < 1 || nw > 3) return VX_ERR_UNSUPPORTED;
-    MvArgs a = {};
+    a = MvArgs{};
     const uint8_t *w[3] = {nullptr, nullptr, nullptr};
     int end[3] = {0, 0, 0}, tot = 0;
     for (int i = 0; i < 3; i++) {
@@ -1348,7 +1396,30 @@ int run_matvec_fused(vx_backend *be, int fmt, const void *const *ws, const int *
         a.mode = src.norm_w ? MV_RMSNORM : MV_PLAIN;
         a.x = src.x; a.norm_w = src.norm_w; a.eps = src.eps;
     }
-    return launch_fmt(be, fmt, a);
+    return VX_OK;
+}
+
+// The general form: nw <= 3 matrices of one format and K, rows concatenated; the activation row from `src`;
+// pair != 0: two matrices of equal height, out[i] = silu(row i of the first) * (row i of the second).
+int run_matvec_fused(vx_backend *be, int fmt, const void *const *ws, const int *ns, int nw, int k, const MatvecSource &src,
+                     float *out, const float *residual, int pair) {
+    MvArgs a;
+    const int rc = matvec_args(fmt, ws, ns, nw, k, src, out, residual, pair, a);
+    return rc ? rc : launch_fmt(be, fmt, a);
+}
+
+int run_matvec_two(vx_backend *be, int fmt, const void *const *ws, const int *ns, int nw, int fmt2, const void *w2, int n2, int k, const MatvecSource &src) {
+    MvArgs a, b;
+    if (!src.rope.q_out) return VX_ERR_UNSUPPORTED;
+    MatvecSource rest = src;
+    for (int i = 0; i < nw; i++) rest.rope.first += ns[i];
+    int rc = matvec_args(fmt, ws, ns, nw, k, src, nullptr, nullptr, 0, a);
+    if (!rc) rc = matvec_args(fmt2, &w2, &n2, 1, k, rest, nullptr, nullptr, 0, b);
+    if (rc) return rc;
+    if (!(fmt2 == VX_Q6_K && ((fmt == VX_Q4_K && launch_third_form_two<K3_Q4_K, K3_Q6_K>(be, a, b)) || (fmt == VX_Q5_K && launch_third_form_two<K3_Q5_K, K3_Q6_K>(be, a, b)))))
+        return VX_ERR_UNSUPPORTED;
+    VX_CHECK_LAUNCH();
+    return VX_OK;
 }
 
 }  // namespace vx
