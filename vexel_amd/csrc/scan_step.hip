@@ -33,30 +33,21 @@ __device__ __forceinline__ bf16x8 convolved(const bf16x8 (&v)[TAPS], const f32x8
     return o;
 }
 
-template <int MT>
 __global__ void __launch_bounds__(64 * PW, 2) conv_project_kernel(StepArgs a) {
-    __shared__ f32x4 red[PW][MT][64];
+    __shared__ f32x4 red[PW][64];
     const vx_conv_args &p = a.p.conv;
     const int lane = threadIdx.x & 63, wave = wave_id();
     const int steps = a.p.x_k >> 5, slices = gridDim.y, slice = blockIdx.y, tile = blockIdx.x;
     const int s0 = (int)((int64_t)steps * slice / slices), s1 = (int)((int64_t)steps * (slice + 1) / slices);
     const bf16 *w = (const bf16 *)a.p.x_w + (size_t)tile * steps * 512 + lane * 8;
-    int pos[MT];
-    const bf16 *x[MT], *st[MT];
-    f32x4 acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; m++) {
-        const int row = min(m * 16 + (lane & 15), a.rows - 1);
-        pos[m] = a.pos[row];
-        x[m] = (const bf16 *)p.x + (size_t)row * p.ldx;
-        st[m] = (const bf16 *)p.state + (size_t)a.slots[row] * (TAPS - 1) * p.channels;
-        acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    // (everything that the steps of a turn read is asked for ahead of the first sum: a wave has two to four steps, and a trip to memory for each
-    // was half of the launch)
-    constexpr int U = MT == 4 ? 1 : 2;
+    const int own = blockIdx.z * 16 + (lane & 15), row = min(own, a.rows - 1), pos = a.pos[row];
+    const bf16 *x = (const bf16 *)p.x + (size_t)row * p.ldx, *st = (const bf16 *)p.state + (size_t)a.slots[row] * (TAPS - 1) * p.channels;
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    // (everything that two steps read is asked for ahead of the first sum: a wave has up to four steps, and a trip to memory for each was half
+    // of the launch)
+    constexpr int U = 2;
     for (int sb = s0 + wave; sb < s1; sb += U * PW) {
-        bf16x8 wf[U], v[U][MT][TAPS];
+        bf16x8 wf[U], v[U][TAPS];
         f32x8 cw[U][TAPS], cb[U];
         int c[U];
 #pragma unroll
@@ -68,37 +59,29 @@ __global__ void __launch_bounds__(64 * PW, 2) conv_project_kernel(StepArgs a) {
             cb[u] = *(const f32x8 *)(p.b + cc);
 #pragma unroll
             for (int t = 0; t < TAPS; t++) cw[u][t] = *(const f32x8 *)(p.w + (size_t)t * p.channels + cc);
+            v[u][TAPS - 1] = *(const bf16x8 *)(x + cc);
 #pragma unroll
-            for (int m = 0; m < MT; m++) {
-                v[u][m][TAPS - 1] = *(const bf16x8 *)(x[m] + cc);
-#pragma unroll
-                for (int t = 0; t + 1 < TAPS; t++) v[u][m][t] = *(const bf16x8 *)(st[m] + (size_t)t * p.channels + cc);
-            }
+            for (int t = 0; t + 1 < TAPS; t++) v[u][t] = *(const bf16x8 *)(st + (size_t)t * p.channels + cc);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (sb + u * PW >= s1) break;
+            bf16x8 o = convolved(v[u], cw[u], cb[u], pos);
+            if (c[u] >= p.channels)  // (columns that pad the inputs)
 #pragma unroll
-            for (int m = 0; m < MT; m++) {
-                bf16x8 o = convolved(v[u][m], cw[u], cb[u], pos[m]);
-                if (c[u] >= p.channels)  // (columns that pad the inputs)
-#pragma unroll
-                    for (int e = 0; e < 8; e++) o[e] = (bf16)0.f;
-                if (const int row = m * 16 + (lane & 15); tile == 0 && row < a.rows) *(bf16x8 *)((bf16 *)p.out + (size_t)row * p.ldo + c[u]) = o;
-                acc[m] = mma(wf[u], o, acc[m]);
-            }
+                for (int e = 0; e < 8; e++) o[e] = (bf16)0.f;
+            if (tile == 0 && own < a.rows) *(bf16x8 *)((bf16 *)p.out + (size_t)own * p.ldo + c[u]) = o;
+            acc = mma(wf[u], o, acc);
         }
     }
-#pragma unroll
-    for (int m = 0; m < MT; m++) red[wave][m][lane] = acc[m];
+    red[wave][lane] = acc;
     __syncthreads();
-    for (int i = threadIdx.x; i < MT * 64; i += 64 * PW) {
-        const int l = i & 63, m = i >> 6, row = m * 16 + (l & 15);
-        f32x4 v = red[0][m][l];
+    if (wave == 0 && own < a.rows) {
+        f32x4 v = red[0][lane];
 #pragma unroll
-        for (int k = 1; k < PW; k++) v += red[k][m][l];
-        if (row < a.rows) *(f32x4 *)(a.part + ((size_t)slice * a.rows + row) * a.p.x_n + tile * 16 + (l >> 4) * 4) = v;
+        for (int k = 1; k < PW; k++) v += red[k][lane];
+        *(f32x4 *)(a.part + ((size_t)slice * a.rows + own) * a.p.x_n + tile * 16 + (lane >> 4) * 4) = v;
     }
 }
 
@@ -139,13 +122,7 @@ int vx_scan_step(vx_backend *be, int act, const vx_ragged *b, const vx_scan_step
     rc = ensure_ws(be, &be->part_ws, &be->part_ws_bytes, (size_t)a.slices * b->rows * p->x_n * 4, "partial sums");
     if (rc) return rc;
     a.part = (float *)be->part_ws;
-    const dim3 grid(p->x_n >> 4, a.slices);
-    if (b->rows <= 16)
-        conv_project_kernel<1><<<grid, 64 * PW, 0, be->stream>>>(a);
-    else if (b->rows <= 32)
-        conv_project_kernel<2><<<grid, 64 * PW, 0, be->stream>>>(a);
-    else
-        conv_project_kernel<4><<<grid, 64 * PW, 0, be->stream>>>(a);
+    conv_project_kernel<<<dim3(p->x_n >> 4, a.slices, ceil_div(b->rows, ROWS)), 64 * PW, 0, be->stream>>>(a);
     VX_CHECK_LAUNCH();
     bool beside = false;
     if (attn) {
