@@ -4,12 +4,12 @@
 // Each of the five is a launch's fixed time and a trip or two to memory (3.8 - 8 us), and a few megabytes at most. What lets them join is that
 // a decode step's rows are few enough to be computed again by every workgroup that reads them:
 //  * conv_project_kernel: a row tile of the split map and a slice of its inputs, as linear_few_kernel; a lane's operand, eight channels of a
-//    row, is convolved in its registers instead of loaded. (Ten row tiles convolve the same channels, 16 K outputs a workgroup: 2 of its 9 us.)
+//    row, is convolved in its registers instead of loaded. (Ten row tiles convolve the same channels, 8 K outputs a workgroup: about 1 us.)
 //  * scan_project (scan_step.h): 32 channels of 16 rows. The waves add up the slices of the rows' low-rank part as a matrix operand and
 //    multiply, add up B and C and move the convolution's history; then two lanes a channel and row step the states, which were asked for
 //    at the start.
-// 32 rows, 4096 channels x 16 states, rank 128, in a traced step, us: the five launches 5.0 + 4.6 + 3.7 + 4.2 + 7.7, these two 9.3 + 9.2; the second one with
-// single-token attention (9.5 - 10 alone) beside it 12.7. The step of a bfloat16 model of four such layers 585 -> 525.
+// 32 rows, 4096 channels x 16 states, rank 128, in a traced step, us: the five launches 5.0 + 4.6 + 3.7 + 4.2 + 7.7, these two 6.6 + 9.2; the second one with
+// single-token attention (9.5 - 10 alone) beside it 12.7. (A workgroup of two row tiles convolved twice as much: 9.1.) The step of a bfloat16 model of four such layers with its logits 585 -> 520 - 531.
 #include <string.h>
 
 #include "scan_step.h"
