@@ -667,6 +667,27 @@ def test_matvec_by_shares(be, fmt, n, k):
     be.reset_pool()
 
 
+@pytest.mark.parametrize("fmt,k", [(f, k) for f in FMTS_SHARES for k in (2048, 2304, 4096, 8448)] +
+                         [(f, k) for f in (nx.FMT_Q4_0, nx.FMT_Q8_0) for k in (32, 2016, 2080, 4128)])
+def test_matvec_planes_by_four_threads(be, fmt, k):
+    """The activation's planes are made by four threads a share up to 64 shares and by one beyond, in one turn up to 256 and in several
+    from there on: every share's elements take part once, also where one is far larger than the rest of its share."""
+    n = 16
+    rng = np.random.default_rng(k + fmt)
+    w = qz.random_quant(fmt, rng, n, k).reshape(n, -1)
+    a = rng.standard_normal((1, k)).astype(np.float32)
+    a[0, ::37] *= 100.0                                               # (another place in every share)
+    deq = nx.dequantize(fmt, w, n * k).reshape(-1, k).astype(np.float64)
+    # (an element is off by 2^-21 of its share's largest, which is up to some 500 times its own size; float32 roundings per share beside it)
+    share = np.abs(a.reshape(-1, 32)).max(1).repeat(32)[None].astype(np.float64)
+    lim = 2.0 ** -21 * (share @ np.abs(deq).T)[0] + 1e-6 * (np.abs(a.astype(np.float64)) @ np.abs(deq).T)[0]
+    dout = be.alloc(n * 4)
+    be.matmul_quant(fmt, be.upload(a), be.upload(w), dout, None, 1, n, k)
+    err = np.abs(be.download(dout, (n,), np.float32) - (a.astype(np.float64) @ deq.T)[0])
+    assert np.all(err <= lim), np.max(err / lim)
+    be.reset_pool()
+
+
 @pytest.mark.parametrize("fqk,fv", [(nx.FMT_Q4_K, nx.FMT_Q6_K), (nx.FMT_Q5_K, nx.FMT_Q6_K), (nx.FMT_Q6_K, nx.FMT_Q6_K),
                                     (nx.FMT_Q4_0, nx.FMT_Q4_0), (nx.FMT_Q8_0, nx.FMT_Q8_0), (nx.FMT_Q4_0, nx.FMT_Q8_0)])
 def test_single_row_qkv_finishes_its_rows(be, fqk, fv):

@@ -85,37 +85,47 @@ struct XInt {
     uint32_t p[3][8];  // plane, dword j = elements 4j .. 4j+3
     int s0, s1;        // sum of xi over elements 0-15 / 16-31
     float inv;         // activation = xi * inv
+    // scale = 2^(BITS - 2 - exponent(m)) and its inverse; zero, denormal-range and non-finite maxima take 1 (such rows give
+    // zeros or garbage either way: the float path would too)
+    static __device__ __forceinline__ float scale_of(float m, float &inv) {
+        const int ex = (int)((__float_as_uint(m) >> 23) & 0xFF);
+        const bool usable = ex > BITS && ex < 255;
+        inv = usable ? __uint_as_float((uint32_t)(ex - (BITS - 2)) << 23) : 1.f;
+        return usable ? __uint_as_float((uint32_t)(127 + BITS - 2 + 127 - ex) << 23) : 1.f;
+    }
+    // four elements' dwords of the planes; -> the sum of their xi
+    static __device__ __forceinline__ int four(const float *v, float scale, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
+        uint32_t xi[4];
+        int sum = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            // adding 1.5 * 2^23 rounds v * scale (|.| < 2^22) to an integer, to nearest even, in the low
+            // mantissa bits: the float's bits are 0x4B400000 + xi
+            const uint32_t bits = __float_as_uint(fmaf(v[k], scale, 12582912.f));
+            xi[k] = bits - 0x4B400000u;
+            sum += (int)xi[k];
+        }
+        // v_perm_b32(hi, lo, sel): selector bytes 0-3 pick from lo, 4-7 from hi
+        const uint32_t a01 = __builtin_amdgcn_perm(xi[1], xi[0], 0x05010400u);  // x0.b0 x1.b0 x0.b1 x1.b1
+        const uint32_t a23 = __builtin_amdgcn_perm(xi[3], xi[2], 0x05010400u);
+        const uint32_t c01 = __builtin_amdgcn_perm(xi[1], xi[0], 0x0c0c0602u);  // x0.b2 x1.b2 0 0
+        const uint32_t c23 = __builtin_amdgcn_perm(xi[3], xi[2], 0x0c0c0602u);
+        p0 = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
+        p1 = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
+        p2 = __builtin_amdgcn_perm(c23, c01, 0x05040100u);
+        return sum;
+    }
     __device__ __forceinline__ void prep(const float *v) {
         float m = 0.f;
 #pragma unroll
         for (int i = 0; i < 32; i++) m = fmaxf(m, fabsf(v[i]));
-        // scale = 2^(BITS - 2 - exponent(m)); zero, denormal-range and non-finite maxima take 1 (such rows give
-        // zeros or garbage either way: the float path would too)
-        const int ex = (int)((__float_as_uint(m) >> 23) & 0xFF);
-        const bool usable = ex > BITS && ex < 255;
-        const float scale = usable ? __uint_as_float((uint32_t)(127 + BITS - 2 + 127 - ex) << 23) : 1.f;
-        inv = usable ? __uint_as_float((uint32_t)(ex - (BITS - 2)) << 23) : 1.f;
+        const float scale = scale_of(m, inv);
         s0 = s1 = 0;
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            uint32_t xi[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                // adding 1.5 * 2^23 rounds v * scale (|.| < 2^22) to an integer, to nearest even, in the low
-                // mantissa bits: the float's bits are 0x4B400000 + xi
-                const uint32_t bits = __float_as_uint(fmaf(v[4 * j + k], scale, 12582912.f));
-                xi[k] = bits - 0x4B400000u;
-                if (j < 4) s0 += (int)xi[k];
-                else s1 += (int)xi[k];
-            }
-            // v_perm_b32(hi, lo, sel): selector bytes 0-3 pick from lo, 4-7 from hi
-            const uint32_t a01 = __builtin_amdgcn_perm(xi[1], xi[0], 0x05010400u);  // x0.b0 x1.b0 x0.b1 x1.b1
-            const uint32_t a23 = __builtin_amdgcn_perm(xi[3], xi[2], 0x05010400u);
-            const uint32_t c01 = __builtin_amdgcn_perm(xi[1], xi[0], 0x0c0c0602u);  // x0.b2 x1.b2 0 0
-            const uint32_t c23 = __builtin_amdgcn_perm(xi[3], xi[2], 0x0c0c0602u);
-            p[0][j] = __builtin_amdgcn_perm(a23, a01, 0x05040100u);
-            p[1][j] = __builtin_amdgcn_perm(a23, a01, 0x07060302u);
-            p[2][j] = __builtin_amdgcn_perm(c23, c01, 0x05040100u);
+            const int sum = four(v + 4 * j, scale, p[0][j], p[1][j], p[2][j]);
+            if (j < 4) s0 += sum;
+            else s1 += sum;
         }
     }
     // acc[p] += sum over the 4 unsigned code bytes of c times byte p of elements 4j .. 4j+3 (codes below 128)
@@ -920,8 +930,12 @@ struct K3_Q6_K {  // share (n, a, h): low and high nibbles of ql[64 n + 32 a + 1
     }
 };
 
-// Workgroup `block` of `blocks`; smem: planes [shares + 1][MV2_XSTRIDE] (the last share zeros).
-template <class F>
+// Workgroup `block` of `blocks`; smem: planes [shares + 1][MV2_XSTRIDE] (the last share zeros). QUARTERS: a share's planes are made by four
+// neighbouring threads, half a run each, which rows of up to MV3_QUARTERS elements take in one turn; by a thread a share three of the
+// four waves of a row of 2048 stand by. (Longer rows: by two threads a share 1 % of a 7B step slower, its products wait for weights.)
+// Q4_0 in a step, us: 2560 x 2048 5.3 -> 4.65, 11264 x 2048 8.2 -> 7.3, 2048 x 2048 4.1 the same.
+constexpr int MV3_QUARTERS = MV_THREADS / 4 * 32;
+template <class F, bool QUARTERS>
 __device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, const int block, const int blocks) {
     extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
     __shared__ float s_ss[MV_WAVES];
@@ -951,19 +965,22 @@ __device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, cons
         return l;
     };
 
-    // share j of the activation row: two runs of 16 elements
+    // share j of the activation row, two runs of 16 elements, or quarter i of it all
     float4 xv[8], nv[8];
-    auto load_x = [&](int j) __attribute__((always_inline)) {
-        const size_t at = (size_t)(j / F::SHARES) * (32 * F::SHARES) + F::first(j % F::SHARES);
+    auto load_x = [&](int i) __attribute__((always_inline)) {
+        constexpr int V = QUARTERS ? 2 : 8;
+        const int j = QUARTERS ? i >> 2 : i;
+        const size_t at = (size_t)(j / F::SHARES) * (32 * F::SHARES) + F::first(j % F::SHARES) + (QUARTERS ? (i >> 1 & 1) * F::APART + (i & 1) * 8 : 0);
 #pragma unroll
-        for (int i = 0; i < 8; i++) xv[i] = *(const float4 *)(p.x + at + (i < 4 ? 0 : F::APART - 16) + 4 * i);
+        for (int e = 0; e < V; e++) xv[e] = *(const float4 *)(p.x + at + (e < 4 ? 0 : F::APART - 16) + 4 * e);
         if (p.mode == MV_RMSNORM) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) nv[i] = *(const float4 *)(p.norm_w + at + (i < 4 ? 0 : F::APART - 16) + 4 * i);
+            for (int e = 0; e < V; e++) nv[e] = *(const float4 *)(p.norm_w + at + (e < 4 ? 0 : F::APART - 16) + 4 * e);
         }
     };
+    const int n_parts = QUARTERS ? n_shares * 4 : n_shares;
     // The activation's first loads go ahead of the weights': behind them they would wait for all of those.
-    if (tid < n_shares) load_x(tid);
+    if (tid < n_parts) load_x(tid);
     __builtin_amdgcn_sched_barrier(0);
     int q = block * MV_WAVES + wave, t = 0;  // what is worked on
     int iq = q, it = 0;                           // what is asked for next
@@ -978,16 +995,17 @@ __device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, cons
     for (int i = 0; i < DEPTH - 1; i++) l[i] = next();
     __builtin_amdgcn_sched_barrier(0);
     float ss = 0.f;
-    for (int j = tid; j < n_shares; j += MV_THREADS) {
+    for (int j = tid; j < n_parts; j += MV_THREADS) {
+        constexpr int E = QUARTERS ? 8 : 32;
         if (j != tid) load_x(j);
-        float v[32];
+        float v[E];
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
+        for (int i = 0; i < E / 4; i++) {
             v[4 * i] = xv[i].x; v[4 * i + 1] = xv[i].y; v[4 * i + 2] = xv[i].z; v[4 * i + 3] = xv[i].w;
         }
         if (p.mode == MV_RMSNORM) {
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
+            for (int i = 0; i < E / 4; i++) {
                 const float wv[4] = {nv[i].x, nv[i].y, nv[i].z, nv[i].w};
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
@@ -996,17 +1014,49 @@ __device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, cons
                 }
             }
         }
-        XInt<F::BITS> x;
-        x.prep(v);
-        uint32_t *dst = smem + (size_t)j * MV2_XSTRIDE;
-#pragma unroll
-        for (int pl = 0; pl < 3; pl++) {
-            *(mv_u32x4 *)(dst + pl * 8) = mv_u32x4{x.p[pl][0], x.p[pl][1], x.p[pl][2], x.p[pl][3]};
-            *(mv_u32x4 *)(dst + pl * 8 + 4) = mv_u32x4{x.p[pl][4], x.p[pl][5], x.p[pl][6], x.p[pl][7]};
-        }
-        // what the format's value() needs of the planes as a whole
+        uint32_t *dst = smem + (size_t)(QUARTERS ? j >> 2 : j) * MV2_XSTRIDE;
         const bool bytes = std::is_same<F, K3_Q8_0>::value;
-        *(mv_u32x4 *)(dst + 24) = mv_u32x4{(uint32_t)(bytes ? x.plane_sum(0) : x.s0), (uint32_t)(bytes ? x.plane_sum(1) : x.s1), __float_as_uint(x.inv), 0u};
+        if constexpr (QUARTERS) {
+            // (the four threads' lanes are neighbours, and all on or all off)
+            const auto beside = [](auto x, auto two) __attribute__((always_inline)) {
+                return __builtin_bit_cast(decltype(x), __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), two() ? 0x4e : 0xb1, 0xf, 0xf, false));
+            };
+            const std::false_type one;
+            const std::true_type two;
+            float m = 0.f, inv;
+#pragma unroll
+            for (int e = 0; e < E; e++) m = fmaxf(m, fabsf(v[e]));
+            m = fmaxf(m, beside(m, one));
+            m = fmaxf(m, beside(m, two));
+            const float scale = XInt<F::BITS>::scale_of(m, inv);
+            uint32_t pl[3][2];
+            const int sum = XInt<F::BITS>::four(v, scale, pl[0][0], pl[1][0], pl[2][0]) + XInt<F::BITS>::four(v + 4, scale, pl[0][1], pl[1][1], pl[2][1]);
+#pragma unroll
+            for (int x = 0; x < 3; x++) *(mv_u32x2 *)(dst + x * 8 + (j & 3) * 2) = mv_u32x2{pl[x][0], pl[x][1]};
+            // what the format's value() needs of the planes as a whole: the byte sums of planes 0 and 1, or the runs' sums
+            int s[2];
+            if (bytes) {
+#pragma unroll
+                for (int x = 0; x < 2; x++) {
+                    s[x] = (int)__builtin_amdgcn_udot4(0x01010101u, pl[x][1], __builtin_amdgcn_udot4(0x01010101u, pl[x][0], 0u, false), false);
+                    s[x] += beside(s[x], one);
+                    s[x] += beside(s[x], two);
+                }
+            } else {
+                s[0] = sum + beside(sum, one);
+                s[1] = beside(s[0], two);
+            }
+            if ((j & 3) == 0) *(mv_u32x4 *)(dst + 24) = mv_u32x4{(uint32_t)s[0], (uint32_t)s[1], __float_as_uint(inv), 0u};
+        } else {
+            XInt<F::BITS> x;
+            x.prep(v);
+#pragma unroll
+            for (int pl = 0; pl < 3; pl++) {
+                *(mv_u32x4 *)(dst + pl * 8) = mv_u32x4{x.p[pl][0], x.p[pl][1], x.p[pl][2], x.p[pl][3]};
+                *(mv_u32x4 *)(dst + pl * 8 + 4) = mv_u32x4{x.p[pl][4], x.p[pl][5], x.p[pl][6], x.p[pl][7]};
+            }
+            *(mv_u32x4 *)(dst + 24) = mv_u32x4{(uint32_t)(bytes ? x.plane_sum(0) : x.s0), (uint32_t)(bytes ? x.plane_sum(1) : x.s1), __float_as_uint(x.inv), 0u};
+        }
     }
     if (tid < MV2_XSTRIDE) smem[(size_t)n_shares * MV2_XSTRIDE + tid] = 0u;
     if (p.mode == MV_RMSNORM) {
@@ -1077,19 +1127,19 @@ __device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, cons
     }
 }
 
-template <class F>
+template <class F, bool QUARTERS>
 __global__ void __launch_bounds__(MV_THREADS) qmatvec3_kernel(const MvArgs p, const int n_passes) {
-    matvec3<F>(p, n_passes, blockIdx.x, gridDim.x);
+    matvec3<F, QUARTERS>(p, n_passes, blockIdx.x, gridDim.x);
 }
 
 // Q|K of one format and V of another in one launch: the first workgroups take Q|K. A launch of its own for V is mostly what every launch
 // costs before its first weights and behind its last (Q|K 8192 x 4096 of Q4_K 9.6 us and V 4096 x 4096 of Q6_K 5.9, together 11.6).
-template <class F, class G>
+template <class F, class G, bool QUARTERS>
 __global__ void __launch_bounds__(MV_THREADS) qmatvec3_two_kernel(const MvArgs p, const int passes, const int blocks, const MvArgs p2, const int passes2) {
     if ((int)blockIdx.x < blocks)
-        matvec3<F>(p, passes, blockIdx.x, blocks);
+        matvec3<F, QUARTERS>(p, passes, blockIdx.x, blocks);
     else
-        matvec3<G>(p2, passes2, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
+        matvec3<G, QUARTERS>(p2, passes2, (int)blockIdx.x - blocks, (int)gridDim.x - blocks);
 }
 
 // Whether the third form serves the call: an activation row from memory, planes that fit LDS.
@@ -1117,31 +1167,35 @@ int third_form_resident(Kernel *kernel, std::atomic<int> *resident, int k, size_
 }
 constexpr int MV3_LONGEST = 120 * 1024 / (MV2_XSTRIDE * 4);
 
+template <class F, bool QUARTERS>
+void launch_third_form_as(vx_backend *be, const MvArgs &a) {
+    const size_t lds = (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4;
+    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_kernel<F, QUARTERS>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    (void)attr;
+    static std::atomic<int> resident[MV3_LONGEST + 1];
+    const int per_cu = third_form_resident(qmatvec3_kernel<F, QUARTERS>, resident, a.K, lds);
+    const int n_passes = a.pair > 0 ? a.pair : ceil_div(a.N, 2);
+    // as many workgroups as fit at once, or fewer when that makes every wave's number of passes equal
+    const int wgs = ceil_div(n_passes, MV_WAVES), trips = ceil_div(wgs, per_cu * device_cus(be));
+    qmatvec3_kernel<F, QUARTERS><<<ceil_div(wgs, trips), MV_THREADS, lds, be->stream>>>(a, n_passes);
+}
+
 // Launches the third form when it serves the call.
 template <class F>
 bool launch_third_form(vx_backend *be, MvArgs &a) {
     if (!third_form_ok<F>(a)) return false;
-    const size_t lds = (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4;
-    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_kernel<F>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
-    (void)attr;
-    static std::atomic<int> resident[MV3_LONGEST + 1];
-    const int per_cu = third_form_resident(qmatvec3_kernel<F>, resident, a.K, lds);
-    const int n_passes = a.pair > 0 ? a.pair : ceil_div(a.N, 2);
-    // as many workgroups as fit at once, or fewer when that makes every wave's number of passes equal
-    const int wgs = ceil_div(n_passes, MV_WAVES), trips = ceil_div(wgs, per_cu * device_cus(be));
-    qmatvec3_kernel<F><<<ceil_div(wgs, trips), MV_THREADS, lds, be->stream>>>(a, n_passes);
+    if (a.K <= MV3_QUARTERS) launch_third_form_as<F, true>(be, a);
+    else launch_third_form_as<F, false>(be, a);
     return true;
 }
 
-// Two of them in one launch, K and the activation row the same.
-template <class F, class G>
-bool launch_third_form_two(vx_backend *be, MvArgs &a, MvArgs &b) {
-    if (!third_form_ok<F>(a) || !third_form_ok<G>(b)) return false;
+template <class F, class G, bool QUARTERS>
+void launch_third_form_two_as(vx_backend *be, const MvArgs &a, const MvArgs &b) {
     const size_t lds = (size_t)(a.K / 32 + 1) * MV2_XSTRIDE * 4;
-    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_two_kernel<F, G>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
+    static const hipError_t attr = hipFuncSetAttribute((const void *)qmatvec3_two_kernel<F, G, QUARTERS>, hipFuncAttributeMaxDynamicSharedMemorySize, 128 * 1024);
     (void)attr;
     static std::atomic<int> resident[MV3_LONGEST + 1];
-    const int room = std::max(2, third_form_resident(qmatvec3_two_kernel<F, G>, resident, a.K, lds) * device_cus(be));
+    const int room = std::max(2, third_form_resident(qmatvec3_two_kernel<F, G, QUARTERS>, resident, a.K, lds) * device_cus(be));
     const int pa = ceil_div(a.N, 2), pb = ceil_div(b.N, 2), wa = ceil_div(pa, MV_WAVES), wb = ceil_div(pb, MV_WAVES);
     // all resident at once, with the fewest trips of either; of the two, one more goes to the one that has the most workgroups
     int ta = 1, tb = 1;
@@ -1150,7 +1204,15 @@ bool launch_third_form_two(vx_backend *be, MvArgs &a, MvArgs &b) {
         else tb++;
     }
     const int ga = ceil_div(wa, ta), gb = ceil_div(wb, tb);
-    qmatvec3_two_kernel<F, G><<<ga + gb, MV_THREADS, lds, be->stream>>>(a, pa, ga, b, pb);
+    qmatvec3_two_kernel<F, G, QUARTERS><<<ga + gb, MV_THREADS, lds, be->stream>>>(a, pa, ga, b, pb);
+}
+
+// Two of them in one launch, K and the activation row the same.
+template <class F, class G>
+bool launch_third_form_two(vx_backend *be, MvArgs &a, MvArgs &b) {
+    if (!third_form_ok<F>(a) || !third_form_ok<G>(b)) return false;
+    if (a.K <= MV3_QUARTERS) launch_third_form_two_as<F, G, true>(be, a, b);
+    else launch_third_form_two_as<F, G, false>(be, a, b);
     return true;
 }
 
