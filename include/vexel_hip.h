@@ -65,7 +65,8 @@ void vx_reset_pool(vx_backend *be);
 /* Backend.ToDevice / ToHost: the host buffer may be reused as soon as the call returns. */
 int vx_to_device(vx_backend *be, void *dst, const void *src_host, size_t bytes);
 int vx_to_host(vx_backend *be, void *dst_host, const void *src, size_t bytes);
-/* vx_to_host of n ranges with one wait; a null src or zero bytes is left out. */
+/* vx_to_host of n ranges with one wait; a null src or zero bytes is left out. Everything enqueued before is done when either returns (unless
+ * there was nothing to bring). */
 int vx_to_host_many(vx_backend *be, int n, void *const *dst_host, const void *const *src, const size_t *bytes);
 /* A hint, ahead of the work whose results a later vx_to_host_many will bring: threads of the backend make the destinations' pages
  * (large ordinary memory only) while the caller enqueues it. The memory stays valid until vx_to_host_forget has returned, which

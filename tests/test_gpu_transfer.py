@@ -65,6 +65,29 @@ def test_download_after_device_work_and_between_smaller_ones(be):
         be.free(p)
 
 
+# one byte; both sides of a slot; all eight slots; more ranges than slots and a range that begins inside an allocation (both ways);
+# a total beyond the pinned part
+@pytest.mark.parametrize("sizes", [[1], [64 * KB], [64 * KB + 1], [512 * KB], [4, 128000], [4, 0, 448 * KB], [100] * 8, [100] * 9, [300 * KB, 200 * KB], [4, 512 * KB]])
+def test_small_download_by_marks(be, sizes):
+    """What the caller waits for by marks: the bytes of the work enqueued last, call after call into the same slots, at odd addresses."""
+    rng = np.random.default_rng(sum(sizes))
+    n = sum(sizes) + 64
+    a, b = (rng.integers(0, 256, n, dtype=np.uint8) for _ in range(2))
+    da, db, dc = be.upload(a, permanent=True), be.upload(b, permanent=True), be.alloc_permanent(n)
+    at = np.concatenate([[3], 3 + np.cumsum(sizes)[:-1]]).astype(int)
+    for i in range(12):
+        for k in range(11 + i % 2):                   # (the last copy is of b, of a, of b, ...)
+            be.copy_buffer(db if k % 2 == 0 else da, 0, dc, 0, n)
+        want = b if (10 + i % 2) % 2 == 0 else a
+        out = [np.zeros(s + 2, dtype=np.uint8) for s in sizes]
+        be.call("vx_to_host_many", len(sizes), (C.c_void_p * len(sizes))(*[o.ctypes.data + 1 for o in out]),
+                (C.c_void_p * len(sizes))(*[int(dc + x) for x in at]), (C.c_size_t * len(sizes))(*sizes))
+        for o, x, s in zip(out, at, sizes):
+            assert np.array_equal(o[1:-1], want[x:x + s]) and o[0] == 0 and o[-1] == 0, (i, x)
+    for p in (da, db, dc):
+        be.free(p)
+
+
 def test_staged_uploads(be):
     """Each upload's bytes are taken when the call returns, also once the staging memory has been used up several times."""
     rows, size = 1500, 1000

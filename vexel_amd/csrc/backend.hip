@@ -89,6 +89,7 @@ int vx_backend_create(int device_id, vx_backend **out) {
     be->host_stage_bytes = 1 << 20;
     // (coherent: kernels read staged uploads there, whose bytes the host writes anew between launches)
     VX_CHECK_HIP(hipHostMalloc(&be->host_stage, be->host_stage_bytes, hipHostMallocCoherent));
+    memset(be->host_stage, 0, be->host_stage_bytes);  // (no download's mark is there yet)
     be->misc_ws_bytes = 1 << 20;
     VX_CHECK_HIP(hipMalloc(&be->misc_ws, be->misc_ws_bytes));
     VX_CHECK_HIP(hipMalloc(&be->rope_tab, (size_t)VX_ROPE_TAB_ROWS * VX_ROPE_TAB_PAIRS * 2 * sizeof(float)));

@@ -139,6 +139,7 @@ struct vx_backend {
     size_t host_stage_bytes = 0;
     size_t stage_used = 0;       // of its part for staged uploads: what the stream may still read
     std::mutex stage_mu;         // (its parts are shared by the threads that call)
+    uint64_t note_mark = 0;      // the last mark of a small download (no mark is ever used again)
     vx::Mover *mover = nullptr;  // large downloads (transfer.hip), from the first one on
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;

@@ -826,8 +826,7 @@ int mix_step(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_t *q_l
     void *dst[2] = {argmax_out, logits_out};
     const void *src[2] = {d_am, logits_out ? logits : nullptr};
     const size_t bytes[2] = {(size_t)n_want * 4, (size_t)n_want * c.vocab * 4};
-    VXC(vx_to_host_many(be, 2, dst, src, bytes));
-    VXC(vx_sync(be));
+    VHC(bring(be, 2, dst, src, bytes));
     std::lock_guard<std::mutex> g(m->pool.mu);
     for (int i = 0; i < n_seqs; i++)
         if (SeqState *s = find_seq(m, seq_ids[i])) s->seq_len = pos[i] + q_lens[i];

@@ -287,6 +287,15 @@ struct Expected {
     Expected &operator=(const Expected &) = delete;
 };
 
+// The end of a step: what it leaves for the caller, and everything it enqueued is done. (A download waits for all that; the runtime's wait
+// behind one by marks was another 30 us of a step.)
+inline int bring(vx_backend *be, int n, void *const *dst, const void *const *src, const size_t *bytes) {
+    bool any = false;
+    for (int i = 0; i < n; i++) any = any || (src[i] && bytes[i] > 0);
+    const int rc = any ? vx_to_host_many(be, n, dst, src, bytes) : vx_sync(be);
+    return rc == VX_OK ? (int)VH_OK : fail("%s", vx_last_error());
+}
+
 // A model whose mixer program is complete in m->mix (weights included): caches, states, activations.
 int mix_finish(vh_model *m);
 // Embedding of b.rows tokens -> layer runs -> final norm and head of n_want rows (want: device row numbers, NULL = the

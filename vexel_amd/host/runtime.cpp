@@ -947,8 +947,7 @@ int vh_decode_batched(vh_model *m, const int32_t *tokens, const int64_t *seq_ids
     void *dst[2] = {argmax_out, logits_out};
     const void *src[2] = {argmax_out ? m->d_next : nullptr, logits_out ? m->logits : nullptr};
     const size_t bytes[2] = {(size_t)batch * 4, (size_t)batch * c.vocab * 4};
-    VXC(vx_to_host_many(m->be, 2, dst, src, bytes));
-    VXC(vx_sync(m->be));                                                             // decode.go:651
+    VHC(bring(m->be, 2, dst, src, bytes));                                           // decode.go:651
     return VH_OK;
 }
 
@@ -975,7 +974,6 @@ int vh_sample_last_logits(vh_model *m, int rows, const float *temperature, const
                 VXC(vx_logit_softcap(be, m->logits + (size_t)r * m->cfg.vocab, m->cfg.vocab, m->arch.final_softcap));
     VXC(vx_sample_rows(be, m->logits, rows, m->cfg.vocab, d_t, d_k, d_p, d_u, d_out));
     VXC(vx_to_host(be, tokens_out, d_out, (size_t)rows * 4));
-    VXC(vx_sync(be));
     return VH_OK;
 }
 
@@ -1152,9 +1150,10 @@ int vh_prefill(vh_model *m, const int32_t *tokens, int n, int64_t seq_id, int st
         VHC(norm_for(m, last, m->final_norm, norm, out_rows, hw, 1, &prep));
         VHC(mm(m, prep, norm, m->lm_head, logits, nullptr, out_rows));
     }
-    if (logits_out) VXC(vx_to_host(be, logits_out, logits, (size_t)out_rows * c.vocab * 4));
-    VXC(vx_sync(be));
-    return VH_OK;
+    void *dst = logits_out;
+    const void *src = logits_out ? logits : nullptr;
+    const size_t bytes = (size_t)out_rows * c.vocab * 4;
+    return bring(be, 1, &dst, &src, &bytes);
 }
 
 // ------------------------------------------------------------------ a step of portions and single tokens
@@ -1445,8 +1444,7 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
             out_row += sr[i].rows;
         }
     }
-    VXC(vx_to_host_many(be, (int)dst.size(), dst.data(), from.data(), bytes.data()));
-    VXC(vx_sync(be));
+    VHC(bring(be, (int)dst.size(), dst.data(), from.data(), bytes.data()));
 
     // greedy acceptance per sequence, then the moves that make each accepted path contiguous
     std::vector<int32_t> chain_off(1, 0), move_src, move_dst;
