@@ -455,6 +455,26 @@ int vx_pack_batch(vx_backend *be, const int32_t *seq_slots, const int32_t *posit
                   int batch, int total_tokens, int32_t *block_tables, int max_blocks, int32_t *num_blocks,
                   int32_t *free_list, int32_t *free_count, int block_size, int32_t *cu_seqlens,
                   int32_t *token_pos, int32_t *slot_mapping, int32_t *kv_lens, int32_t *status);
+/* The start of a step of one new token a sequence in one launch (more than 64 sequences, and uploads beyond 64 KiB: as the
+ * calls it stands for): what vx_to_device_staged of `bytes` bytes to dst, vx_pack_batch with one new token each,
+ * vx_embedding of the batch's ids (a null table: none) and vx_rope_table_prepare of token_pos (rope_dim 0: none) leave when
+ * called in that order. seq_slots, positions and ids point into what is uploaded: dst .. dst + bytes. Not during capture.
+ * No counterpart in the reference. */
+typedef struct {
+    void *dst;
+    const void *src_host;
+    size_t bytes;
+    const int32_t *seq_slots, *positions;
+    int batch, max_blocks, block_size;
+    int32_t *block_tables, *num_blocks, *free_list, *free_count;
+    int32_t *cu_seqlens, *token_pos, *slot_mapping, *kv_lens, *status;
+    const int32_t *ids;
+    const float *table;
+    float *out;
+    int vocab, dim, rope_dim;
+    float rope_theta;
+} vx_step_begin_args;
+int vx_step_begin(vx_backend *be, const vx_step_begin_args *args);
 
 /* End of a device-driven decode step (host restatement: scheduler/scheduler.go:432-446 greedy arm +
  * scheduler/sequence.go:136-141): out_log[step*batch + i] = next_tokens[i] where step = *step_counter,

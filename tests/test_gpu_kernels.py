@@ -1788,6 +1788,65 @@ def test_pack_batch_by_waves(be, batch, q_lens):
     be.reset_pool()
 
 
+# a lane, a wave and one sequence more (separate launches); a row of one part with an end, of several, of no whole vectors; ids out of range;
+# without embeddings and angles; another upload's ids
+@pytest.mark.parametrize("batch,dim,rope,case", [(1, 512, 64, ""), (3, 2052, 128, "ids"), (31, 1030, 0, ""), (64, 516, 256, "ids"), (65, 512, 64, ""),
+                                                 (7, 0, 0, ""), (7, 4096, 80, "elsewhere"), (64, 30, 514, "")])
+def test_step_begin_is_the_separate_calls(be, batch, dim, rope, case):
+    """One launch of a step's upload, packing, embeddings and angles leaves what the four calls leave, bit for bit."""
+    from vexel_amd.backend import VxStepBeginArgs
+    rng = np.random.default_rng(batch + dim)
+    bs, mb, vocab, theta = 16, 80, 50, 10000.0
+    pos = rng.integers(0, 1200, batch).astype(np.int32)
+    pos[::3] = pos[::3] // bs * bs
+    had = (pos + bs - 1) // bs
+    slots = rng.permutation(batch).astype(np.int32)
+    perm = rng.permutation(int(had.sum()) + batch + 5).astype(np.int32)
+    tables, nblk = rng.integers(0, 99, (batch, mb)).astype(np.int32), np.zeros(batch, np.int32)
+    nblk[slots] = had
+    ids = rng.integers(0, vocab, batch).astype(np.int32)
+    if case == "ids":
+        ids[0], ids[-1] = -1, vocab
+    up = np.concatenate([ids, np.full(3, -7, np.int32), slots, pos, np.arange(1500, dtype=np.int32)])
+    dtab = be.upload(rng.standard_normal((vocab, max(dim, 1))).astype(np.float32))
+    d, hq, hk, hidden = rope, 2, 1, 2 * rope
+    if rope in (64, 128):
+        qw = {n: be.qweight(nx.FMT_Q8_0, be.upload(qz.random_quant(nx.FMT_Q8_0, rng, r, 512)), r, 512) for n, r in (("wq", hq * d), ("wk", d), ("wv", d))}
+        dx, dn = be.upload(rng.standard_normal((batch, 512)).astype(np.float32)), be.upload(np.ones(512, dtype=np.float32))
+        dslot = be.upload(rng.permutation(batch * bs)[:batch].astype(np.int32))
+    results = []
+    for one in (False, True):
+        old = dict(tables=tables, nblk=nblk, free=perm, count=np.array([perm.size], np.int32), up=np.full(up.size, 9, np.int32), cu=np.full(batch + 1, 9, np.int32),
+                   out=np.full((batch, max(dim, 1)), 3, np.float32), **{n: np.full(batch, 9, np.int32) for n in ("tp", "sm", "kl")}, st=np.array([9], np.int32))
+        b = {n: be.upload(v) for n, v in old.items()}
+        at = lambda n: b["up"] + 4 * n
+        d_ids = be.upload(ids) if case == "elsewhere" else at(0)
+        d_slots, d_pos = at(batch + 3), at(2 * batch + 3)
+        dpool, dq = be.upload(np.zeros(batch * bs * 2 * max(d, 1), np.float16)), be.alloc(batch * hq * d * 4 + 4)
+        if one:
+            be.step_begin(VxStepBeginArgs(b["up"], up.ctypes.data, up.nbytes, d_slots, d_pos, batch, mb, bs, b["tables"], b["nblk"], b["free"], b["count"],
+                                          b["cu"], b["tp"], b["sm"], b["kl"], b["st"], d_ids, dtab if dim else None, b["out"], vocab, dim, rope, theta))
+        else:
+            be.call("vx_to_device_staged", b["up"], up.ctypes.data, up.nbytes)
+            be.pack_batch(d_slots, d_pos, 0, batch, batch, b["tables"], mb, b["nblk"], b["free"], b["count"], bs, b["cu"], b["tp"], b["sm"], b["kl"], b["st"])
+            if dim:
+                be.call("vx_embedding", d_ids, batch, dtab, b["out"], vocab, dim)
+            if rope:
+                be.rope_table_prepare(b["tp"], batch, rope, theta)
+        res = [be.download(b[n], v.shape, np.uint32) for n, v in old.items()]
+        if rope in (64, 128):  # (the positions change behind the library's back: the table's are what counts)
+            _overwrite(be, b["tp"], pos[::-1] + 1)
+            results.append(res)
+            be.decode_attn_qkv(dx, dn, 1e-5, False, qw["wq"], qw["wk"], qw["wv"], batch, b["tp"], dslot, dpool, True, hq, hk, d, bs, theta, dq)
+            res += [be.download(dq, (batch, hq * d), np.uint32), be.download(dpool, (batch * bs * 2 * d,), np.uint16)]
+        else:
+            results.append(res)
+    assert results[0][list(old).index("st")][0] == 0
+    for want, got in zip(*results):
+        assert np.array_equal(want, got)
+    be.reset_pool()
+
+
 def test_pack_batch_bit_exact(be):
     rng = np.random.default_rng(40)
     bs, max_blocks, nslots, pool_blocks = 16, 20, 12, 150

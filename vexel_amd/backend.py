@@ -111,6 +111,12 @@ class VxScanStepArgs(C.Structure):
     _fields_ = [("conv", VxConvArgs), ("scan", VxScanArgs)] + _fields("ptr x_w dt_w; int x_n x_k dt_n dt_k; ptr dt_bias")
 
 
+class VxStepBeginArgs(C.Structure):
+    _fields_ = _fields("ptr dst src_host; i64 bytes; ptr seq_slots positions; int batch max_blocks block_size; "
+                       "ptr block_tables num_blocks free_list free_count cu_seqlens token_pos slot_mapping kv_lens status ids table out; "
+                       "int vocab dim rope_dim; float rope_theta")
+
+
 class VexelError(RuntimeError):
     def __init__(self, code, msg):
         super().__init__("vexel_hip error %d: %s" % (code, msg))
@@ -481,6 +487,10 @@ class HipBackend:
         self.call("vx_pack_batch", seq_slots, positions, q_lens, batch, total_tokens, block_tables, max_blocks,
                   num_blocks, free_list, free_count, block_size, cu_seqlens, token_pos, slot_mapping, kv_lens,
                   status)
+
+    def step_begin(self, args):
+        """args: VxStepBeginArgs; upload, pack_batch, embedding and rope_table_prepare of a step of one new token a sequence"""
+        self.call("vx_step_begin", C.byref(args))
 
     # ---- ragged mixed batches (structures: VxRagged and the Vx*Args above)
     def fill_zero(self, dst, nbytes):

@@ -169,6 +169,18 @@ inline void items_written(vx_backend *be, const void *dst, size_t bytes) {
     if (a < k + (size_t)be->items.batch * 4 && k < a + bytes) be->items.valid = false;
 }
 
+// The backend's table holds the angles of these positions from the launch just made on (vx_rope_table_prepare).
+inline void rope_table_stands(vx_backend *be, const int32_t *positions, int rows, int head_dim, float theta) {
+    be->rope_tab_pos = positions, be->rope_tab_rows = rows, be->rope_tab_dim = head_dim, be->rope_tab_theta = theta;
+    be->rope_tab_epoch = be->write_epoch;
+}
+
+// transfer.hip: a small upload's bytes in pinned memory that kernels read, until the next call that asks for it: the caller holds
+// be->stage_mu from before it to behind the launch that reads them. At most 64 KiB.
+int stage_upload(vx_backend *be, const void *src_host, size_t bytes, const char **at);
+// transfer.hip: whether a kernel can read and write these bytes by itself: memory of this device, within one allocation.
+bool device_memory(const vx_backend *be, const void *at, size_t bytes);
+
 // transfer.hip: ends the threads of large downloads and gives their memory back.
 void mover_destroy(Mover *m);
 

@@ -40,6 +40,7 @@
 
 #include "prep_tiles.h"
 #include "qgemm_shared.h"
+#include "rope_angle.h"
 
 using namespace vx;
 
@@ -1648,10 +1649,7 @@ __global__ void rope_store_partials_kernel(const float *__restrict__ P, int KS, 
 // position per row), once per step instead of once per layer. grid = rows, block = head_dim / 2.
 __global__ void rope_table_kernel(const int32_t *__restrict__ positions, float2 *__restrict__ tab, int head_dim, float theta) {
     const int row = blockIdx.x, j = threadIdx.x, half = head_dim / 2;
-    const double ex = (double)(2 * j) / (double)head_dim;
-    const float freq = (float)(1.0 / pow((double)theta, ex));
-    const float angle = __fmul_rn((float)positions[row], freq);
-    tab[(size_t)row * half + j] = make_float2((float)cos((double)angle), (float)sin((double)angle));
+    tab[(size_t)row * half + j] = rope_angle(positions[row], j, head_dim, theta);
 }
 
 size_t fmt_row_bytes(int fmt, int k) {
@@ -2326,11 +2324,7 @@ int vx_rope_table_prepare(vx_backend *be, const int32_t *positions, int rows, in
     if (rows > VX_ROPE_TAB_ROWS || head_dim / 2 > VX_ROPE_TAB_PAIRS) return VX_OK;  // no table: the calls keep their own arithmetic
     rope_table_kernel<<<rows, head_dim / 2, 0, be->stream>>>(positions, (float2 *)be->rope_tab, head_dim, theta);
     VX_CHECK_LAUNCH();
-    be->rope_tab_pos = positions;
-    be->rope_tab_rows = rows;
-    be->rope_tab_dim = head_dim;
-    be->rope_tab_theta = theta;
-    be->rope_tab_epoch = be->write_epoch;
+    rope_table_stands(be, positions, rows, head_dim, theta);
     return VX_OK;
 }
 

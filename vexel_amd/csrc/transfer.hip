@@ -95,8 +95,10 @@ struct KernelSender : Mover::Sender {
     hipError_t lost() override { return hipErrorUnknown; }
 };
 
-// Whether the kernel can read these bytes: memory of the device within one allocation (the runtime's copy says what is wrong with others).
-bool readable(const vx_backend *be, const void *src, size_t bytes) {
+}  // namespace
+
+// (The runtime's copy says what is wrong with other memory.)
+bool device_memory(const vx_backend *be, const void *src, size_t bytes) {
     hipPointerAttribute_t a;
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
@@ -107,6 +109,7 @@ bool readable(const vx_backend *be, const void *src, size_t bytes) {
     return ok;
 }
 
+namespace {
 // Coherent pinned memory for the ring and its marks: what a kernel has written there is seen by the host while the kernel runs.
 // Without it the runtime's copies fill the ring.
 void use_sender(Mover *m) {
@@ -152,7 +155,7 @@ static int download_noted(vx_backend *be, int n, void *const *dst, const void *c
     char *to[SLOTS];
     for (int i = 0; i < n; i++) {
         if (!src[i] || bytes[i] == 0) continue;
-        if (a.count + (int)((bytes[i] + Mover::SENT_SLOT - 1) / Mover::SENT_SLOT) > SLOTS || !readable(be, src[i], bytes[i])) return VX_ERR_UNSUPPORTED;
+        if (a.count + (int)((bytes[i] + Mover::SENT_SLOT - 1) / Mover::SENT_SLOT) > SLOTS || !device_memory(be, src[i], bytes[i])) return VX_ERR_UNSUPPORTED;
         for (size_t at = 0; at < bytes[i]; at += Mover::SENT_SLOT, a.count++) {
             a.src[a.count] = (const char *)src[i] + at, a.bytes[a.count] = (uint32_t)std::min(Mover::SENT_SLOT, bytes[i] - at);
             to[a.count] = (char *)dst[i] + at;
@@ -218,7 +221,7 @@ static int download(vx_backend *be, int n, void *const *dst, const void *const *
     }
     // pieces of a slot; of the runtime's larger slots an eighth, so that the threads have something to share, of 256 KiB up
     bool by_sender = mover->sender != nullptr;
-    for (int i = 0; i < n && by_sender; i++) by_sender = !src[i] || bytes[i] == 0 || readable(be, src[i], bytes[i]);
+    for (int i = 0; i < n && by_sender; i++) by_sender = !src[i] || bytes[i] == 0 || device_memory(be, src[i], bytes[i]);
     const size_t most = by_sender ? Mover::SENT_SLOT : std::min(Mover::SLOT, std::max((size_t)256 << 10, total / 8 / 4096 * 4096));
     std::vector<Mover::Piece> pieces;
     for (int i = 0; i < n; i++) {
@@ -230,6 +233,20 @@ static int download(vx_backend *be, int n, void *const *dst, const void *const *
     Mover::Job job(std::move(pieces));
     job.by_sender = by_sender;
     VX_CHECK_HIP(mover->move(be->stream, job));
+    return VX_OK;
+}
+
+int stage_upload(vx_backend *be, const void *src_host, size_t bytes, const char **at) {
+    const size_t room = (bytes + 63) / 64 * 64;
+    VX_REQUIRE(bytes <= UP_MOST, "staged upload of %zu bytes", bytes);
+    if (be->stage_used + room > UP_BYTES) {
+        VX_CHECK_HIP(hipStreamSynchronize(be->stream));
+        be->stage_used = 0;
+    }
+    char *to = (char *)be->host_stage + UP_AT + be->stage_used;
+    be->stage_used += room;
+    memcpy(to, src_host, bytes);
+    *at = to;
     return VX_OK;
 }
 
@@ -300,15 +317,9 @@ int vx_to_device_staged(vx_backend *be, void *dst, const void *src_host, size_t 
     VX_REQUIRE(src_host != nullptr, "vx_to_device_staged: null source");
     VX_REQUIRE(!be->capturing, "vx_to_device_staged during graph capture");
     items_written(be, dst, bytes);
-    const size_t room = (bytes + 63) / 64 * 64;
     std::lock_guard<std::mutex> g(be->stage_mu);
-    if (be->stage_used + room > UP_BYTES) {
-        VX_CHECK_HIP(hipStreamSynchronize(be->stream));
-        be->stage_used = 0;
-    }
-    char *at = (char *)be->host_stage + UP_AT + be->stage_used;
-    be->stage_used += room;
-    memcpy(at, src_host, bytes);
+    const char *at;
+    if (rc = stage_upload(be, src_host, bytes, &at); rc) return rc;
     VX_CHECK_HIP(hipMemcpyAsync(dst, at, bytes, hipMemcpyHostToDevice, be->stream));
     return VX_OK;
 }
@@ -345,7 +356,7 @@ int vx_to_device_staged_many(vx_backend *be, int n, void *const *dst, const void
     };
     for (int i = 0; i < n; i++) {
         if (!dst[i] || bytes[i] == 0) continue;
-        if (bytes[i] > UP_MOST || !readable(be, dst[i], bytes[i])) {
+        if (bytes[i] > UP_MOST || !device_memory(be, dst[i], bytes[i])) {
             if (rc = launch(); rc) return rc;
             g.unlock();
             if (rc = vx_to_device_staged(be, dst[i], src_host[i], bytes[i]); rc) return rc;

@@ -248,6 +248,12 @@ int embed(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, float *out) 
     return VH_OK;
 }
 
+// Where embed() leaves the rows of a program that begins with plain embeddings; null: of another.
+float *embedded_rows(const MixModel &x, const MixActs &a) {
+    if (x.pairs || x.branch_norm) return nullptr;
+    return x.post_norm ? a.hist : a.emb ? a.emb : a.x;
+}
+
 // the experts of every row, from the router's logits z (float32, in slices)
 int run_router(vh_model *m, const MixLayer &l, int rows, const MixActs &a, const float *z, int slices, int ldz) {
     const ExpertMlp &e = l.moe;
@@ -537,12 +543,12 @@ int head_logits(vh_model *m, const MixActs &a, int n, float *logits) {
 }
 
 // Layers whose norms precede the sublayers: the seams add what the last one left, normed, and norm what the next one reads.
-int forward_pre_norm(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, const MixActs &a, const int32_t *want, int n_want) {
+int forward_pre_norm(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, const MixActs &a, const int32_t *want, int n_want, bool embedded) {
     const MixModel &x = *m->mix;
     const vh_config &c = m->cfg;
     const int rows = b.rows, width_pad = pad_to(c.hidden, 64);
     float *emb = a.emb ? a.emb : a.x;
-    VHC(embed(m, b, d_tokens, emb));
+    if (!embedded) VHC(embed(m, b, d_tokens, emb));
     VHC(rot_tables(m, b, a));
     vx_residual_norm_args s;
     memset(&s, 0, sizeof s);
@@ -599,11 +605,11 @@ int forward_pre_norm(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, c
 // Layers whose norms follow the residual sums; the sublayers read the stream itself, and every layer's result is kept for the
 // averages of those behind it.
 int forward_post_norm(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, const MixActs &a, const MixExpand *ex, const int32_t *want,
-                      int n_want) {
+                      int n_want, bool embedded) {
     const MixModel &x = *m->mix;
     const vh_config &c = m->cfg;
     const int rows = b.rows, n_runs = (int)x.runs.size();
-    VHC(embed(m, b, d_tokens, a.hist));
+    if (!embedded) VHC(embed(m, b, d_tokens, a.hist));
     VHC(rot_tables(m, b, a));
     vx_post_norm_args s;
     memset(&s, 0, sizeof s);
@@ -680,10 +686,11 @@ int forward_branch_norm(vh_model *m, const vx_ragged &b, const int32_t *d_tokens
 }  // namespace
 
 int mix_forward(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, const MixActs &a, const MixExpand *ex, const int32_t *want,
-                int n_want, float *logits) {
+                int n_want, float *logits, bool embedded) {
     if (b.rows > a.rows) return fail("internal: %d rows, activations for %d", b.rows, a.rows);
     VHC(m->mix->branch_norm ? forward_branch_norm(m, b, d_tokens, a, want, n_want)
-        : m->mix->post_norm ? forward_post_norm(m, b, d_tokens, a, ex, want, n_want) : forward_pre_norm(m, b, d_tokens, a, want, n_want));
+        : m->mix->post_norm ? forward_post_norm(m, b, d_tokens, a, ex, want, n_want, embedded)
+                           : forward_pre_norm(m, b, d_tokens, a, want, n_want, embedded));
     return n_want > 0 ? head_logits(m, a, n_want, logits) : (int)VH_OK;
 }
 
@@ -799,7 +806,6 @@ int mix_step(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_t *q_l
     memcpy(h, pos.data(), (size_t)n_seqs * 4), h += n_seqs;
     memcpy(h, q_lens, (size_t)n_seqs * 4), h += n_seqs;
     if (n_want) memcpy(h, want_rows, (size_t)n_want * 4);
-    VXC(vx_to_device_staged(be, d, host.data(), up * 4));
     int32_t *d_tok = d, *d_slots = d + T, *d_pos = d_slots + n_seqs, *d_q = d_pos + n_seqs, *d_want = d_q + n_seqs;
     int32_t *d_cu = d + up, *d_tp = d_cu + n_seqs + 1, *d_sm = d_tp + T, *d_kvl = d_sm + T;
     MixActs acts = m->mix->perm;
@@ -810,13 +816,26 @@ int mix_step(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_t *q_l
         if (!logits) return fail("logits of %d rows: %s", n_want, vx_last_error());
     }
     MixExpand ex;
-    if (!one_each) VHC(plan_expand(m, n_seqs, q_lens, lens, seq_tables, &ex));
-    VXC(vx_pack_batch(be, d_slots, d_pos, one_each ? nullptr : d_q, n_seqs, T, m->d_tables, c.max_blocks_per_seq, m->d_num_blocks,
-                      m->d_free, m->d_free_count, c.block_size, d_cu, d_tp, d_sm, d_kvl, m->d_status));
+    float *const embedded = one_each ? embedded_rows(*m->mix, acts) : nullptr;
+    if (one_each) {
+        vx_step_begin_args a;
+        memset(&a, 0, sizeof a);
+        a.dst = d, a.src_host = host.data(), a.bytes = up * 4, a.seq_slots = d_slots, a.positions = d_pos, a.batch = n_seqs;
+        a.max_blocks = c.max_blocks_per_seq, a.block_size = c.block_size, a.block_tables = m->d_tables, a.num_blocks = m->d_num_blocks;
+        a.free_list = m->d_free, a.free_count = m->d_free_count, a.cu_seqlens = d_cu, a.token_pos = d_tp, a.slot_mapping = d_sm, a.kv_lens = d_kvl;
+        a.status = m->d_status;
+        if (embedded) a.ids = d_tok, a.table = m->embedding, a.out = embedded, a.vocab = c.vocab, a.dim = c.hidden;
+        VXC(vx_step_begin(be, &a));
+    } else {
+        VXC(vx_to_device_staged(be, d, host.data(), up * 4));
+        VHC(plan_expand(m, n_seqs, q_lens, lens, seq_tables, &ex));
+        VXC(vx_pack_batch(be, d_slots, d_pos, d_q, n_seqs, T, m->d_tables, c.max_blocks_per_seq, m->d_num_blocks, m->d_free, m->d_free_count,
+                          c.block_size, d_cu, d_tp, d_sm, d_kvl, m->d_status));
+    }
     const Expected expected(be, logits_out, (size_t)n_want * c.vocab * 4);
     const vx_ragged b{T, n_seqs, one_each ? nullptr : q_lens, max_kv, d_cu, d_tp, d_sm, d_slots, d_kvl, m->d_tables, c.max_blocks_per_seq,
                       c.block_size};
-    VHC(mix_forward(m, b, d_tok, acts, ex.rows > 0 ? &ex : nullptr, n_want ? d_want : nullptr, n_want, logits));
+    VHC(mix_forward(m, b, d_tok, acts, ex.rows > 0 ? &ex : nullptr, n_want ? d_want : nullptr, n_want, logits, embedded != nullptr));
     int32_t *d_am = nullptr;
     if (n_want > 0 && argmax_out) {
         d_am = n_want <= c.max_batch ? m->d_next : (int32_t *)vx_alloc(be, (size_t)n_want * 4);

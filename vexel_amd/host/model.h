@@ -299,9 +299,9 @@ inline int bring(vx_backend *be, int n, void *const *dst, const void *const *src
 // A model whose mixer program is complete in m->mix (weights included): caches, states, activations.
 int mix_finish(vh_model *m);
 // Embedding of b.rows tokens -> layer runs -> final norm and head of n_want rows (want: device row numbers, NULL = the
-// first n_want) -> logits [n_want, vocab].
+// first n_want) -> logits [n_want, vocab]. embedded: the rows' embeddings are there.
 int mix_forward(vh_model *m, const vx_ragged &b, const int32_t *d_tokens, const MixActs &a, const MixExpand *ex, const int32_t *want,
-                int n_want, float *logits);
+                int n_want, float *logits, bool embedded = false);
 // One mixed step (vh_step) of such a model.
 int mix_step(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_t *q_lens, const int32_t *tokens, int n_want,
              const int32_t *want_rows, float *logits_out, int32_t *argmax_out);

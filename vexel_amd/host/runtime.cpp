@@ -342,8 +342,9 @@ int execute_layer_decode(vh_model *m, int layer, int rows, int max_kv_len, const
     return layer_tail(m, w, m->x, m->norm, m->attn, m->gate, m->up, rows);
 }
 
-// embedding -> layers -> final norm -> lm_head -> argmax for a decode batch (decode.go:404-452)
-int forward_decode(vh_model *m, int rows, int max_kv_len) {
+// embedding -> layers -> final norm -> lm_head -> argmax for a decode batch (decode.go:404-452); begun: the embeddings and the rows' angles
+// are there (vx_step_begin)
+int forward_decode(vh_model *m, int rows, int max_kv_len, bool begun = false) {
     const vh_config &c = m->cfg;
     if (m->mix) {
         const vx_ragged b{rows, rows, nullptr, max_kv_len, m->d_cu, m->d_token_pos, m->d_slot_map, m->d_slots, m->d_kv_lens, m->d_tables,
@@ -352,12 +353,12 @@ int forward_decode(vh_model *m, int rows, int max_kv_len) {
         VXC(vx_argmax_rows(m->be, m->logits, rows, c.vocab, m->d_next));
         return VH_OK;
     }
-    VXC(vx_embedding(m->be, m->d_tokens, rows, m->embedding, m->x, c.vocab, c.hidden));
+    if (!begun) VXC(vx_embedding(m->be, m->d_tokens, rows, m->embedding, m->x, c.vocab, c.hidden));
     VHC(g_scale_embedding(m, m->x, rows));
     const bool head_prepared = rows > 1 && m->fused && (!m->general || m->fused_ok) && fast(m->lm_head) && c.hidden % 256 == 0;
     bool chained = false;
     // the step's RoPE angles once for all layers: the fused Q|K|V launches then rotate and store their own rows
-    if (m->fused && !m->general) VXC(vx_rope_table_prepare(m->be, m->d_token_pos, rows, c.head_dim, c.rope_theta));
+    if (!begun && m->fused && !m->general) VXC(vx_rope_table_prepare(m->be, m->d_token_pos, rows, c.head_dim, c.rope_theta));
     for (int l = 0; l < c.num_layers; l++) {
         const float *next_norm = l + 1 < c.num_layers ? (rows > 1 && attn_fusable(m, l + 1) ? m->layers[l + 1].attn_norm : nullptr)
                                                       : (head_prepared ? m->final_norm : nullptr);
@@ -928,22 +929,28 @@ int vh_decode_batched(vh_model *m, const int32_t *tokens, const int64_t *seq_ids
     std::copy(tokens, tokens + batch, in.begin());                                    // decode.go:389-395
     std::copy(slots.begin(), slots.end(), in.begin() + mb);
     std::copy(positions, positions + batch, in.begin() + 2 * mb);
-    VXC(vx_to_device_staged(m->be, m->d_tokens, in.data(), in.size() * 4));
     bool at_end = true;  // every sequence decodes at its end: kv length = position + 1
     for (int i = 0; i < batch; i++) at_end = at_end && kv_lens[i] == positions[i] + 1;
     if (at_end) {
-        // The blocks are there already (host pool, mirrored above), so the packing kernel allocates nothing and
+        // The blocks are there already (host pool, mirrored above), so the packing allocates nothing and
         // only derives slots and lengths on the device, and leaves the attention's work list with them.
-        VXC(vx_pack_batch(m->be, m->d_slots, m->d_pos_in, nullptr, batch, batch, m->d_tables, c.max_blocks_per_seq,
-                          m->d_num_blocks, m->d_free, m->d_free_count, c.block_size, m->d_cu, m->d_token_pos,
-                          m->d_slot_map, m->d_kv_lens, m->d_status));
+        vx_step_begin_args a;
+        memset(&a, 0, sizeof a);
+        a.dst = m->d_tokens, a.src_host = in.data(), a.bytes = in.size() * 4;
+        a.seq_slots = m->d_slots, a.positions = m->d_pos_in, a.batch = batch, a.max_blocks = c.max_blocks_per_seq, a.block_size = c.block_size;
+        a.block_tables = m->d_tables, a.num_blocks = m->d_num_blocks, a.free_list = m->d_free, a.free_count = m->d_free_count;
+        a.cu_seqlens = m->d_cu, a.token_pos = m->d_token_pos, a.slot_mapping = m->d_slot_map, a.kv_lens = m->d_kv_lens, a.status = m->d_status;
+        a.ids = m->d_tokens, a.table = m->embedding, a.out = m->x, a.vocab = c.vocab, a.dim = c.hidden;
+        if (m->fused && !m->general) a.rope_dim = c.head_dim, a.rope_theta = c.rope_theta;
+        VXC(vx_step_begin(m->be, &a));
     } else {
+        VXC(vx_to_device_staged(m->be, m->d_tokens, in.data(), in.size() * 4));
         VXC(vx_to_device_staged(m->be, m->d_token_pos, positions, (size_t)batch * 4));
         VXC(vx_to_device_staged(m->be, m->d_slot_map, slot_map.data(), (size_t)batch * 4));
         VXC(vx_to_device_staged(m->be, m->d_kv_lens, kv_lens.data(), (size_t)batch * 4));
     }
     const Expected expected(m->be, logits_out, (size_t)batch * c.vocab * 4);
-    VHC(forward_decode(m, batch, max_kv));
+    VHC(forward_decode(m, batch, max_kv, at_end));
     void *dst[2] = {argmax_out, logits_out};
     const void *src[2] = {argmax_out ? m->d_next : nullptr, logits_out ? m->logits : nullptr};
     const size_t bytes[2] = {(size_t)batch * 4, (size_t)batch * c.vocab * 4};

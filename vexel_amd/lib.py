@@ -113,6 +113,7 @@ SIGNATURES = {
     "vx_paged_kv_copy_shifted": (_i, [_vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f]),
     "vx_paged_kv_move": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i]),
     "vx_pack_batch": (_i, [_vp, _vp, _vp, _vp, _i, _i, _vp, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp]),
+    "vx_step_begin": (_i, [_vp, _vp]),
     "vx_decode_advance": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "vx_graph_begin_capture": (_i, [_vp]),
     "vx_graph_end_capture": (_i, [_vp, C.POINTER(_vp)]),
