@@ -420,6 +420,32 @@ def test_selective_scan(be, act, states, channels):
     be.free(state)
 
 
+# 16 chunks, which the carry asks for in one trip, one row more, a third trip with one chunk
+@pytest.mark.parametrize("rows", [1024, 1025, 2049])
+@pytest.mark.parametrize("states", [16, 30])
+def test_selective_scan_of_many_chunks(be, rows, states):
+    from vexel_amd.backend import VxScanArgs
+    rng = np.random.default_rng(rows + states)
+    channels, pad = 11, -(-states // 16) * 16
+    A = -np.exp(rng.uniform(np.log(1e-4), np.log(1.0), (channels, states)))   # (states that last over the whole prompt)
+    D = rng.standard_normal(channels).astype(np.float32)
+    x, z = (grid(rng.standard_normal((rows, channels)), BF16) for _ in range(2))
+    dt = np.exp(rng.uniform(-6, 0, (rows, channels))).astype(np.float32)
+    bc = np.zeros((rows, 2, pad), dtype=np.float32)
+    bc[:, :, :states] = rng.standard_normal((rows, 2, states))
+    y, _ = lz.selective_scan(x.astype(np.float64), dt.astype(np.float64), A, bc[:, 0, :states], bc[:, 1, :states], D)
+    a2 = np.zeros((channels, pad), dtype=np.float32)
+    a2[:, :states] = A / np.log(2.0)
+    bt = Batch(be, [0], [rows], slots=[1])
+    p = VxScanArgs()
+    p.channels, p.states, p.a2, p.d, p.state = channels, states, be.upload(a2), be.upload(D), be.upload(np.full((2, channels, pad), 1e3, dtype=np.float32))
+    p.x, p.z, p.ldx, p.ldz, p.dt, p.bc, p.lddt = up(be, x, BF16), up(be, z, BF16), channels, channels, be.upload(dt), be.upload(bc), channels
+    p.out_scale, p.out, p.ldo, p.out_cols = 1.0, blank(be, (rows, channels), BF16), channels, channels
+    be.selective_scan(BF16, bt.c, p)
+    close(down(be, p.out, (rows, channels), BF16), y * lz.silu(z.astype(np.float64)), BF16, rows)
+    be.reset_pool()
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 33, 64])
 @pytest.mark.parametrize("channels,states,rank,attn", [(2048, 16, 64, None), (2024, 11, 100, (10, 2, 112)), (3976, 3, 300, (4, 4, 64)), (4096, 16, 128, (16, 4, 128))])
 def test_scan_step_is_the_separate_calls(be, rows, channels, states, rank, attn):

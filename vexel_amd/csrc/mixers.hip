@@ -602,21 +602,30 @@ __global__ void __launch_bounds__(256) scan_kernel(ScanArgs a) {
         for (int i = threadIdx.x; i < tn * 2 * pad / 4; i += 256) ((f32x4 *)s_bc)[i] = src[i];
         __syncthreads();
         constexpr int U = 4;
-        float ndt[U], nx[U], nz[U];
+        // Every lane of a channel has the rows' sums; of U rows each writes OWN, u % LP == sub, so that gates are not worked out by lanes that
+        // write nothing (2048 rows of 4096 channels, two lanes each: 44.1 us with the first lane writing all, now 42.2; the rest is
+        // the states' exponentials and multiply-adds, which one lane a channel with two waves a SIMD takes 43.3 for).
+        constexpr int TURN = LP < U ? LP : U, OWN = U / TURN;
+        float ndt[U], nx[U], nz[OWN];
         auto fetch = [&](int t) {
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 const int tt = t0 + min(t + u, tn - 1);
                 ndt[u] = dt[(size_t)tt * p.lddt];
                 nx[u] = (float)x[(size_t)tt * p.ldx];
-                if (FINAL) nz[u] = (float)z[(size_t)tt * p.ldz];
+            }
+            if (FINAL) {
+#pragma unroll
+                for (int i = 0; i < OWN; i++) nz[i] = (float)z[(size_t)(t0 + min(t + i * TURN + sub, tn - 1)) * p.ldz];
             }
         };
         fetch(0);
         for (int t = 0; t < tn; t += U) {
-            float cdt[U], cx[U], cz[U];
+            float cdt[U], cx[U], cz[OWN], y[U];
 #pragma unroll
-            for (int u = 0; u < U; u++) cdt[u] = ndt[u], cx[u] = nx[u], cz[u] = FINAL ? nz[u] : 0.f;
+            for (int u = 0; u < U; u++) cdt[u] = ndt[u], cx[u] = nx[u], y[u] = 0.f;
+#pragma unroll
+            for (int i = 0; i < OWN; i++) cz[i] = FINAL ? nz[i] : 0.f;
             if (t + U < tn) fetch(t + U);
 #pragma unroll
             for (int u = 0; u < U; u++) {
@@ -628,15 +637,23 @@ __global__ void __launch_bounds__(256) scan_kernel(ScanArgs a) {
                 for (int n = 0; n < NS; n++) S[n] = fmaf(__builtin_amdgcn_exp2f(cdt[u] * A[n]), S[n], dx * B[n]);
                 if (FINAL) {
                     const f32x8 C = load8(b + pad);
-                    float y = 0.f;
 #pragma unroll
-                    for (int n = 0; n < NS; n++) y = fmaf(S[n], C[n], y);
+                    for (int n = 0; n < NS; n++) y[u] = fmaf(S[n], C[n], y[u]);
 #pragma unroll
-                    for (int off = LP / 2; off > 0; off >>= 1) y += __shfl_xor(y, off, 64);
-                    if (sub == 0 && live)
-                        out[(size_t)(t0 + t + u) * p.ldo] = (T)(p.out_scale * (fmaf(D, cx[u], y) * silu_f(cz[u])));
+                    for (int off = LP / 2; off > 0; off >>= 1) y[u] += __shfl_xor(y[u], off, 64);  // (the same sum in every lane)
                 } else {
                     sum += cdt[u];
+                }
+            }
+            if (FINAL) {
+#pragma unroll
+                for (int i = 0; i < OWN; i++) {
+                    float own = y[i * TURN], ox = cx[i * TURN];
+#pragma unroll
+                    for (int k = 1; k < TURN; k++)
+                        if (sub == k) own = y[i * TURN + k], ox = cx[i * TURN + k];
+                    const int row = t + i * TURN + sub;
+                    if (sub < TURN && row < tn && live) out[(size_t)(t0 + row) * p.ldo] = (T)(p.out_scale * (fmaf(D, ox, own) * silu_f(cz[i])));
                 }
             }
         }
@@ -667,7 +684,7 @@ __global__ void __launch_bounds__(256) scan_carry_kernel(ScanArgs a) {
     const int c = (int)(e / a.pad);
     const float A = p.a2[e];
     float S = a.pos[a.cu[seq]] > 0 ? p.state[(size_t)a.slots[seq] * per + e] : 0.f;
-    constexpr int U = 4;
+    constexpr int U = 16;  // (chunks asked for in one trip; 32 of them with four a trip 8.6 us, now 6.5)
     for (int k = 0; k < chunks; k += U) {
         float own[U], sd[U];
 #pragma unroll
