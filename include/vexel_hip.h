@@ -405,6 +405,14 @@ int vx_sdpa_paged_tree_batched(vx_backend *be, const float *q, const void *kv_po
                                int entries, const int32_t *row_info, const uint8_t *tree_masks,
                                const int32_t *mask_offsets, float *out, int rows, int max_tree_rows,
                                int num_q_heads, int num_kv_heads, int head_dim, float scale, int max_kv_len);
+/* The same for two rows and more, its result left inside the backend as the prepared activation that a vx_decode_ffn with
+ * attn = NULL, called next, takes (heads * head_dim and ffn_k, the columns of the widest activation of that call,
+ * multiples of 256): a launch and a trip of the rows through memory less. */
+int vx_sdpa_paged_tree_batched_ffn(vx_backend *be, const float *q, const void *kv_pool, const int32_t *block_tables,
+                                   int max_blocks, const int32_t *entry_table_rows, const int32_t *entry_kv_lens,
+                                   int entries, const int32_t *row_info, const uint8_t *tree_masks,
+                                   const int32_t *mask_offsets, int rows, int max_tree_rows, int num_q_heads,
+                                   int num_kv_heads, int head_dim, float scale, int max_kv_len, int ffn_k);
 
 /* Copies num_tokens token rows (K and V of every KV head) from src_slots[i] to dst_slots[i] of one layer's paged
  * pool (device int32 arrays, slot = physical block * block_size + offset; the two sets must not overlap) and

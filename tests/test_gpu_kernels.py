@@ -1552,6 +1552,51 @@ def test_tree_keys_and_splits_of_every_count(be, hq, hk, d, n, start):
     be.reset_pool()
 
 
+# a tile of rows; rows that pad the activation (48 and 36 of 64); one chunk of columns and several, of two heads and of four
+@pytest.mark.parametrize("hq,hk,d", [(4, 4, 128), (6, 2, 128), (8, 2, 64), (4, 4, 64)])
+@pytest.mark.parametrize("n,start", [(3, 0), (33, 530)])
+def test_tree_rows_as_the_next_call_takes_them(be, hq, hk, d, n, start):
+    """Attention of candidate trees into the second half of the layer: what it gives through rows in memory, up to the rounding of operands with a
+    factor per 256 columns instead of per row; refused for one row, and where the rows have been overwritten meanwhile."""
+    from vexel_amd.backend import VexelError
+    rng = np.random.default_rng(n + hq + d)
+    fmt, hidden, ffn, bs, nblocks, eps = nx.FMT_Q8_0, 512, 768, 16, 60, 1e-5
+    dims = dict(wo=(hidden, hq * d), w1=(ffn, hidden), w3=(ffn, hidden), w2=(hidden, ffn))
+    qw = {k: be.qweight(fmt, be.upload(qz.random_quant(fmt, rng, *v)), *v) for k, v in dims.items()}
+    rg = be._lib.vx_sdpa_paged_tree_rows_per_entry(1, bs, hq, hk, d)
+    pad = -(-n // rg) * rg
+    mb = (start + n + bs - 1) // bs
+    table = rng.integers(0, nblocks - 5, (1, mb)).astype(np.int32)
+    table[0, start // bs:] = nblocks - 5 + np.arange(mb - start // bs)
+    mask = np.array(hl.build_tree_attention_mask(n, [int(rng.integers(-1, i)) if i else -1 for i in range(n)]), dtype=np.uint8)
+    info = np.array([[0, start, min(r, n - 1), n] for r in range(pad)], dtype=np.int32)
+    x, q = (rng.standard_normal((pad, c)).astype(np.float32) for c in (hidden, hq * d))
+    q[:, :d] *= 8                                                     # (heads of different size: factors that differ between chunks)
+    up = [be.upload(q), be.upload(_make_pool(rng, True, nblocks, bs, hk, d)), be.upload(table), mb, be.upload(np.zeros(pad // rg, dtype=np.int32)),
+          be.upload(np.full(pad // rg, start, dtype=np.int32)), pad // rg, be.upload(info), be.upload(mask), be.upload(np.zeros(pad, dtype=np.int32))]
+    tail = [n, hq, hk, d, np.float32(1 / math.sqrt(d)), start]
+    dnw, attn = be.upload(np.ones(hidden, dtype=np.float32)), be.alloc(q.nbytes)
+    outs = []
+    for into in (False, True):
+        dx = be.upload(x)
+        if into:
+            be.call("vx_sdpa_paged_tree_batched_ffn", *up, pad, *tail, ffn)
+        else:
+            be.call("vx_sdpa_paged_tree_batched", *up, attn, pad, *tail)
+        be.decode_ffn(None if into else attn, dx, qw["wo"], dnw, eps, qw["w1"], qw["w3"], qw["w2"], pad, None)
+        outs.append(be.download(dx, (pad, hidden), np.float32))
+    assert np.all(np.abs(outs[1] - outs[0]) <= 2e-5 * np.abs(outs[0]).max())
+    be.call("vx_sdpa_paged_tree_batched_ffn", *up, pad, *tail, ffn)
+    be.rmsnorm_prepare(be.upload(x), dnw, None, pad, hidden, eps)
+    with pytest.raises(VexelError):
+        be.decode_ffn(None, dx, qw["wo"], dnw, eps, qw["w1"], qw["w3"], qw["w2"], pad, None)
+    with pytest.raises(VexelError):
+        be.call("vx_sdpa_paged_tree_batched_ffn", *up, 1, *tail, ffn)
+    with pytest.raises(VexelError):
+        be.call("vx_sdpa_paged_tree_batched", *up, None, pad, *tail)
+    be.reset_pool()
+
+
 @pytest.mark.parametrize("hq,hk,d,half", [(8, 8, 128, False), (8, 8, 128, True), (8, 2, 64, False), (8, 2, 64, True),
                                           (16, 2, 128, False), (16, 2, 128, True), (6, 2, 128, False), (10, 2, 64, False),
                                           (14, 2, 128, True)])

@@ -802,6 +802,12 @@ __device__ __forceinline__ half8 read_columns(const _Float16 *a, const _Float16 
     return r;
 }
 
+// Where an attention kernel leaves its rows as the prepared activation of the output projection.
+struct AttnPrep {
+    PrepView pv;
+    int mpad = 0;
+};
+
 // Many query rows of one sequence over its paged F16 context, each row with its own number of visible keys (the
 // later chunks of a prompt, linear verification): paged_decode_gqa_kernel's two matrix-core products and operand
 // layouts, with QT tiles of 16 consecutive query rows of one head per wave instead of 16 (row, head) queries of one
@@ -1158,20 +1164,33 @@ __global__ void __launch_bounds__(D) paged_merge_kernel(const float *__restrict_
 // is the same in all lanes, so the others are passed over instead of being added with a weight of 0, and 64 registers let all of those
 // rows' waves run at once (15.6 -> 13.9 us; 128 rows 10.7 -> 9.4, 64 rows 7.7 -> 6.9; four heads a workgroup: 16.7). Heads of 128 would
 // take 66 registers and spill four of them for that, 12 bytes a lane.
-template <int D>
-__global__ void __launch_bounds__(64, 8) tree_merge_kernel(const float *__restrict__ partial, const float *__restrict__ q,
+// PREP: the rows as the prepared activation of the output projection instead: a workgroup has the heads of a 256-column chunk, a wave
+// each, and one of them puts their columns there; grid.y goes on over the rows that pad the activation. (256 rows of 32
+// heads of 128: 14.7 us for 13.7 and a launch of 6.8 that read the rows again; 16 trees on a 7B Q6_K model 14.49 -> 14.21 ms.)
+template <int D, bool PREP>
+__global__ void __launch_bounds__(PREP ? 64 * 256 / D : 64, 8) tree_merge_kernel(const float *__restrict__ partial, const float *__restrict__ q,
                                                        const _Float16 *__restrict__ pool, const int32_t *__restrict__ bt_matrix,
                                                        int max_blocks, const int4 *__restrict__ info,
                                                        const uint8_t *__restrict__ masks, const int32_t *__restrict__ mask_off,
                                                        float *__restrict__ out, int num_q_heads, int num_kv_heads, float scale,
-                                                       int max_splits) {
+                                                       int max_splits, int rows, AttnPrep prep) {
+    constexpr int HEADS = PREP ? 256 / D : 1;  // of a workgroup
+    __shared__ __attribute__((aligned(16))) float s_y[PREP ? 256 : 1];
+    if (PREP && (int)blockIdx.y >= rows) {
+        if (threadIdx.x < 64) {
+            const float zero[4] = {0.f, 0.f, 0.f, 0.f};
+            write_chunk(prep.pv, blockIdx.y, blockIdx.x, zero, prep.mpad);
+            if (blockIdx.x == 0 && threadIdx.x == 0) prep.pv.inv_scale[blockIdx.y] = 0.f;
+        }
+        return;
+    }
     constexpr int MAXN = 64;  // rows of one tree (checked on the host)
     constexpr int KPP = 8;      // keys per pass: eight lanes share a key,
     constexpr int EL = D / 8;   // this many elements each
     constexpr int C = D / 64;   // columns of the output per lane
     typedef _Float16 halfc __attribute__((ext_vector_type(C)));
     typedef float floatc __attribute__((ext_vector_type(C)));
-    const int qh = blockIdx.x, row = blockIdx.y, lane = threadIdx.x;
+    const int sub = HEADS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, qh = blockIdx.x * HEADS + sub, row = blockIdx.y, lane = threadIdx.x & 63;
     const int4 inf = info[row];
     const int start = inf.y, r = inf.z, n = inf.w;
     const int kvh = qh / (num_q_heads / num_kv_heads);
@@ -1207,7 +1226,8 @@ __global__ void __launch_bounds__(64, 8) tree_merge_kernel(const float *__restri
             if (j0 + j < n && (vis >> (j0 + j) & 1)) vv[j] = *(const halfc *)(row_at(j0 + j) + part + lane * C);
         }
     };
-    __shared__ float s_s[MAXN];
+    __shared__ float s_scores[HEADS][MAXN];
+    float *const s_s = s_scores[sub];
     const float *qp = q + ((size_t)row * num_q_heads + qh) * D + (lane % 8) * EL;
     float qf[EL];
 #pragma unroll
@@ -1266,7 +1286,19 @@ __global__ void __launch_bounds__(64, 8) tree_merge_kernel(const float *__restri
             for (int e = 0; e < C; e++) A[e] = fmaf(f, (float)vv[j][e], A[e]);
         }
     }
-    *(floatc *)(out + ((size_t)row * num_q_heads + qh) * D + lane * C) = (L > 0.f) ? A / L : (floatc)0.f;
+    const floatc y = (L > 0.f) ? A / L : (floatc)0.f;
+    if (!PREP) {
+        *(floatc *)(out + ((size_t)row * num_q_heads + qh) * D + lane * C) = y;
+        return;
+    }
+    *(floatc *)(s_y + sub * D + lane * C) = y;
+    __syncthreads();
+    if (sub == 0) {
+        const float4 t = *(const float4 *)(s_y + lane * 4);
+        const float four[4] = {t.x, t.y, t.z, t.w};
+        write_chunk(prep.pv, row, blockIdx.x, four, prep.mpad);
+        if (blockIdx.x == 0 && lane == 0) prep.pv.inv_scale[row] = 1.f;
+    }
 }
 
 // --------------------------------------------------------------------------------------------
@@ -2091,14 +2123,15 @@ int vx_sdpa_paged_tree_rows_per_entry(int pool_is_f16, int block_size, int num_q
     return G <= 8 ? 16 / G : 0;  // 16 queries (row, head) per K/V row fill the matrix-core tile: 16, 8, 5, 4, 3, 2, 2, 2 rows
 }
 
-int vx_sdpa_paged_tree_batched(vx_backend *be, const float *q, const void *kv_pool, const int32_t *block_tables,
-                               int max_blocks, const int32_t *entry_table_rows, const int32_t *entry_kv_lens, int entries,
-                               const int32_t *row_info, const uint8_t *tree_masks, const int32_t *mask_offsets, float *out,
-                               int rows, int max_tree_rows, int num_q_heads, int num_kv_heads, int head_dim, float scale,
-                               int max_kv_len) {
+// ffn_k > 0: the rows as the prepared activation of a vx_decode_ffn whose widest activation has ffn_k columns, instead of out
+static int tree_batched(vx_backend *be, const float *q, const void *kv_pool, const int32_t *block_tables,
+                        int max_blocks, const int32_t *entry_table_rows, const int32_t *entry_kv_lens, int entries,
+                        const int32_t *row_info, const uint8_t *tree_masks, const int32_t *mask_offsets, float *out,
+                        int rows, int max_tree_rows, int num_q_heads, int num_kv_heads, int head_dim, float scale,
+                        int max_kv_len, int ffn_k) {
     int rc = enter(be);
     if (rc) return rc;
-    VX_REQUIRE(q && kv_pool && block_tables && entry_table_rows && entry_kv_lens && row_info && tree_masks && mask_offsets && out,
+    VX_REQUIRE(q && kv_pool && block_tables && entry_table_rows && entry_kv_lens && row_info && tree_masks && mask_offsets && (out || ffn_k > 0),
                "vx_sdpa_paged_tree_batched: null pointer");
     const int rg_max = vx_sdpa_paged_tree_rows_per_entry(1, HOT_BS, num_q_heads, num_kv_heads, head_dim);
     if (rg_max == 0) {
@@ -2115,6 +2148,9 @@ int vx_sdpa_paged_tree_batched(vx_backend *be, const float *q, const void *kv_po
     VX_REQUIRE(((uintptr_t)kv_pool % 16) == 0 && max_kv_len >= 0, "vx_sdpa_paged_tree_batched: bad pool alignment / length");
     if (rows == 0) return VX_OK;
     const int max_splits = max_kv_len > 0 ? ceil_div(max_kv_len, TPW) : 1;
+    AttnPrep prep;
+    if (ffn_k > 0)
+        if (rc = prep_for_ffn(be, rows, num_q_heads * head_dim, ffn_k, &prep.pv, &prep.mpad); rc) return rc;
     const size_t need = (size_t)rows * num_q_heads * max_splits * (head_dim + 2) * sizeof(float);
     rc = ensure_ws(be, &be->attn_ws, &be->attn_ws_bytes, need, "attention");
     if (rc) return rc;
@@ -2138,17 +2174,40 @@ int vx_sdpa_paged_tree_batched(vx_backend *be, const float *q, const void *kv_po
 #undef VX_TREE
         VX_CHECK_LAUNCH();
     }
-    const dim3 mgrid(num_q_heads, rows);
-    if (head_dim == 128)
-        tree_merge_kernel<128><<<mgrid, 64, 0, be->stream>>>(ws, q, pool, block_tables, max_blocks, (const int4 *)row_info,
-                                                             tree_masks, mask_offsets, out, num_q_heads, num_kv_heads, scale,
-                                                             max_splits);
-    else
-        tree_merge_kernel<64><<<mgrid, 64, 0, be->stream>>>(ws, q, pool, block_tables, max_blocks, (const int4 *)row_info,
-                                                           tree_masks, mask_offsets, out, num_q_heads, num_kv_heads, scale,
-                                                           max_splits);
+#define VX_TREE_MERGE(DD, PREP)                                                                                                  \
+    tree_merge_kernel<DD, PREP><<<dim3(PREP ? num_q_heads * DD / 256 : num_q_heads, PREP ? prep.mpad : rows), PREP ? 64 * 256 / DD : 64, 0, \
+                                  be->stream>>>(ws, q, pool, block_tables, max_blocks, (const int4 *)row_info, tree_masks,       \
+                                                mask_offsets, out, num_q_heads, num_kv_heads, scale, max_splits, rows, prep)
+    if (ffn_k > 0) {
+        if (head_dim == 128) VX_TREE_MERGE(128, true);
+        else VX_TREE_MERGE(64, true);
+    } else {
+        if (head_dim == 128) VX_TREE_MERGE(128, false);
+        else VX_TREE_MERGE(64, false);
+    }
+#undef VX_TREE_MERGE
     VX_CHECK_LAUNCH();
+    if (ffn_k > 0) prepared_for_ffn(be, rows, num_q_heads, head_dim);
     return VX_OK;
+}
+
+int vx_sdpa_paged_tree_batched(vx_backend *be, const float *q, const void *kv_pool, const int32_t *block_tables,
+                               int max_blocks, const int32_t *entry_table_rows, const int32_t *entry_kv_lens, int entries,
+                               const int32_t *row_info, const uint8_t *tree_masks, const int32_t *mask_offsets, float *out,
+                               int rows, int max_tree_rows, int num_q_heads, int num_kv_heads, int head_dim, float scale,
+                               int max_kv_len) {
+    return tree_batched(be, q, kv_pool, block_tables, max_blocks, entry_table_rows, entry_kv_lens, entries, row_info, tree_masks, mask_offsets,
+                        out, rows, max_tree_rows, num_q_heads, num_kv_heads, head_dim, scale, max_kv_len, 0);
+}
+
+int vx_sdpa_paged_tree_batched_ffn(vx_backend *be, const float *q, const void *kv_pool, const int32_t *block_tables,
+                                   int max_blocks, const int32_t *entry_table_rows, const int32_t *entry_kv_lens, int entries,
+                                   const int32_t *row_info, const uint8_t *tree_masks, const int32_t *mask_offsets, int rows,
+                                   int max_tree_rows, int num_q_heads, int num_kv_heads, int head_dim, float scale,
+                                   int max_kv_len, int ffn_k) {
+    VX_REQUIRE(ffn_k > 0 && rows > 1, "vx_sdpa_paged_tree_batched_ffn: %d rows before activations of %d columns", rows, ffn_k);
+    return tree_batched(be, q, kv_pool, block_tables, max_blocks, entry_table_rows, entry_kv_lens, entries, row_info, tree_masks, mask_offsets,
+                        nullptr, rows, max_tree_rows, num_q_heads, num_kv_heads, head_dim, scale, max_kv_len, ffn_k);
 }
 
 }  // extern "C"

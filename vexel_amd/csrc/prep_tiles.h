@@ -126,5 +126,9 @@ __device__ __forceinline__ void split_merge4(const float *__restrict__ part, int
 // Makes the prepared-activation workspace hold an [m,k] activation whose rows carry the factor 1 and returns its
 // view, when the chunk-wise kernels serve the shape (qgemm.hip); VX_ERR_UNSUPPORTED when they do not.
 int prep_begin_chunked(vx_backend *be, int m, int k, PrepView *pv, int *mpad);
+// The same for several rows of any number, in a workspace that the vx_decode_ffn that follows has no reason to move (its widest activation has ffn_k
+// columns); then, behind the launch that has written them, that they are what its attn = NULL takes.
+int prep_for_ffn(vx_backend *be, int m, int k, int ffn_k, PrepView *pv, int *mpad);
+void prepared_for_ffn(vx_backend *be, int m, int num_q_heads, int head_dim);
 
 }  // namespace vx

@@ -2314,6 +2314,16 @@ int prep_begin_chunked(vx_backend *be, int m, int k, PrepView *pv, int *mpad) {
     *mpad = mpad_for(m);
     return prep_begin(be, m, k, pv);
 }
+int prep_for_ffn(vx_backend *be, int m, int k, int ffn_k, PrepView *pv, int *mpad) {
+    VX_REQUIRE(m > 1 && k % 256 == 0 && ffn_k % 256 == 0 && k * (int64_t)4 <= 64 * 1024, "attention into vx_decode_ffn: %d rows of %d columns, activations of %d", m, k, ffn_k);
+    if (int rc = prep_reserve(be, m, std::max(k, ffn_k)); rc) return rc;
+    *mpad = mpad_for(m);
+    return prep_begin(be, m, k, pv);
+}
+void prepared_for_ffn(vx_backend *be, int m, int num_q_heads, int head_dim) {
+    be->split.batch = m, be->split.num_q_heads = num_q_heads, be->split.head_dim = head_dim;
+    be->split.max_splits = be->split.tokens_per_split = 0, be->split.kv_lens = nullptr, be->split.plain = nullptr, be->split.merged = 1;
+}
 }  // namespace vx
 }
 int vx_rope_table_prepare(vx_backend *be, const int32_t *positions, int rows, int head_dim, float theta) {
@@ -2662,6 +2672,7 @@ int vx_decode_ffn(vx_backend *be, const float *attn, float *x, const vx_qweight 
     const bool merged = !attn && be->split.merged && be->gemm_ws == ws_before && be->gemm_ws_bytes == ws_bytes_before &&
                         be->prep_m == rows && be->prep_k == wo->k;
     be->split.merged = 0;
+    VX_REQUIRE(attn || merged || be->split.kv_lens, "vx_decode_ffn: attn = NULL, and the prepared rows that attention left are gone");
     // attention output -> Wo -> partials
     if (attn) {
         rc = vx_prepare_act(be, attn, rows, wo->k);

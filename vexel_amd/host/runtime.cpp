@@ -1397,7 +1397,15 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
             VXC(vx_rope_store_paged(be, q, k, v, d_pos, d_slot, m->kv[l], c.kv_fp16, n, c.num_heads, c.num_kv_heads,
                                     c.head_dim, c.block_size, c.rope_theta));
         }
-        if (rg) {  // every tree in two launches, each sequence's context read once per entry of rg rows
+        const bool ffn_fused = !tail_general && m->fused && n > 1 && w.wo.data && w.w1.data && w.w2.data && w.w3.data &&
+                               vx_decode_ffn_supported(&w.wo, &w.w1, &w.w3, &w.w2);
+        // (attention then leaves its rows as that half's prepared activation)
+        const bool into_ffn = rg && ffn_fused && c.num_heads * c.head_dim % 256 == 0 && (size_t)w.wo.k * 4 <= 64 * 1024;
+        if (into_ffn) {
+            VXC(vx_sdpa_paged_tree_batched_ffn(be, q, m->kv[l], m->d_tables, c.max_blocks_per_seq, d_ent_rows, d_ent_lens, entries, d_info, d_mask,
+                                               d_moff, n, max_rows, c.num_heads, c.num_kv_heads, c.head_dim, scale, max_start,
+                                               std::max(w.w1.n, w.wo.n)));
+        } else if (rg) {  // every tree in two launches, each sequence's context read once per entry of rg rows
             VXC(vx_sdpa_paged_tree_batched(be, q, m->kv[l], m->d_tables, c.max_blocks_per_seq, d_ent_rows, d_ent_lens, entries,
                                            d_info, d_mask, d_moff, attn, n, max_rows, c.num_heads, c.num_kv_heads, c.head_dim,
                                            scale, max_start));
@@ -1415,12 +1423,10 @@ int vh_verify_tree(vh_model *m, int n_seqs, const int64_t *seq_ids, const int32_
             VHC(g_tail(m, l, x, norm, attn, gate, up, n));
             continue;
         }
-        const bool ffn_fused = m->fused && n > 1 && w.wo.data && w.w1.data && w.w2.data && w.w3.data &&
-                               vx_decode_ffn_supported(&w.wo, &w.w1, &w.w3, &w.w2);
         if (ffn_fused) {
             const float *next_norm = l + 1 < c.num_layers ? (attn_fusable(m, l + 1) ? m->layers[l + 1].attn_norm : nullptr)
                                                           : (head_prepared ? m->final_norm : nullptr);
-            VXC(vx_decode_ffn(be, attn, x, &w.wo, w.ffn_norm, c.eps, &w.w1, &w.w3, &w.w2, n, next_norm));
+            VXC(vx_decode_ffn(be, into_ffn ? nullptr : attn, x, &w.wo, w.ffn_norm, c.eps, &w.w1, &w.w3, &w.w2, n, next_norm));
             chained = next_norm != nullptr;
         } else {
             VHC(layer_tail(m, w, x, norm, attn, gate, up, n));
