@@ -194,6 +194,13 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
                                     const int32_t *block_table, float *out, const int32_t *kv_lens,
                                     int num_blocks, int block_size, int num_q_heads, int num_kv_heads,
                                     int head_dim, float scale, int query_len);
+/* The same, its result left inside the backend as the prepared activation that a vx_decode_ffn with attn = NULL, called
+ * next, takes (ffn_k: the columns of that call's widest activation, a multiple of 256); where _supported says so. */
+int vx_sdpa_paged_multiquery_ffn_supported(int pool_is_f16, int block_size, int num_q_heads, int num_kv_heads, int head_dim,
+                                           int query_len);
+int vx_sdpa_paged_multiquery_ffn(vx_backend *be, const float *q, const void *kv_pool, int pool_is_f16, const int32_t *block_table,
+                                 const int32_t *kv_lens, int num_blocks, int block_size, int num_q_heads, int num_kv_heads,
+                                 int head_dim, float scale, int query_len, int ffn_k);
 
 /* ---- batched-decode entry points the reference lacks ------------------------- */
 /* (its batch is a host loop, runtime/decode.go:623-650; these run the whole batch in one

@@ -1552,6 +1552,43 @@ def test_tree_keys_and_splits_of_every_count(be, hq, hk, d, n, start):
     be.reset_pool()
 
 
+# one share of the steps, two and four; rows that end inside a tile, inside the activation's last 32 and on their edge; heads of a chunk: two and four
+@pytest.mark.parametrize("hq,hk,d,n,start", [(8, 2, 128, 16, 5), (8, 4, 128, 77, 300), (12, 2, 128, 40, 0), (32, 8, 128, 300, 40), (32, 8, 128, 1025, 10), (8, 2, 64, 33, 100),
+                                             (32, 8, 64, 520, 70), (32, 8, 64, 1100, 0)])
+def test_multiquery_rows_as_the_next_call_takes_them(be, hq, hk, d, n, start):
+    """Many rows' attention into the second half of the layer: what it gives through rows in memory (the same bits where those get a factor per 256
+    columns, too: from 257 rows on); geometries without that form are refused."""
+    from vexel_amd.backend import VexelError
+    rng = np.random.default_rng(n + hq + d)
+    fmt, hidden, ffn, bs, nblocks, eps = nx.FMT_Q8_0, 512, 768, 16, 100, 1e-5
+    dims = dict(wo=(hidden, hq * d), w1=(ffn, hidden), w3=(ffn, hidden), w2=(hidden, ffn))
+    qw = {k: be.qweight(fmt, be.upload(qz.random_quant(fmt, rng, *v)), *v) for k, v in dims.items()}
+    mb = (start + n + bs - 1) // bs
+    lens = (start + 1 + np.arange(n)).astype(np.int32)
+    x, q = (rng.standard_normal((n, c)).astype(np.float32) for c in (hidden, hq * d))
+    q[:, :d] *= 8
+    dq, dpool, dt, dl = be.upload(q), be.upload(_make_pool(rng, True, nblocks, bs, hk, d)), be.upload(rng.integers(0, nblocks, mb).astype(np.int32)), be.upload(lens)
+    dnw, attn, sc = be.upload(np.ones(hidden, dtype=np.float32)), be.alloc(q.nbytes), np.float32(1 / math.sqrt(d))
+    outs = []
+    assert be.lib_call("vx_sdpa_paged_multiquery_ffn_supported", 1, bs, hq, hk, d, n) == 1
+    for into in (False, True):
+        dx = be.upload(x)
+        if into:
+            be.call("vx_sdpa_paged_multiquery_ffn", dq, dpool, 1, dt, dl, mb, bs, hq, hk, d, sc, n, ffn)
+        else:
+            be.call("vx_sdpa_paged_decode_multiquery", dq, dpool, 1, dt, attn, dl, mb, bs, hq, hk, d, sc, n)
+        be.decode_ffn(None if into else attn, dx, qw["wo"], dnw, eps, qw["w1"], qw["w3"], qw["w2"], n, None)
+        outs.append(be.download(dx, (n, hidden), np.float32))
+    if n > 256:
+        assert np.array_equal(*outs)
+    assert np.all(np.abs(outs[1] - outs[0]) <= 2e-5 * np.abs(outs[0]).max())
+    for bad in ((0, bs, hq, hk, d, n), (1, 32, hq, hk, d, n), (1, bs, hk, hk, d, n), (1, bs, hq, hk, 80, n), (1, bs, hq, hk, d, 15)):
+        assert be.lib_call("vx_sdpa_paged_multiquery_ffn_supported", *bad) == 0
+        with pytest.raises(VexelError):
+            be.call("vx_sdpa_paged_multiquery_ffn", dq, dpool, bad[0], dt, dl, mb, *bad[1:5], sc, bad[5], ffn)
+    be.reset_pool()
+
+
 # a tile of rows; rows that pad the activation (48 and 36 of 64); one chunk of columns and several, of two heads and of four
 @pytest.mark.parametrize("hq,hk,d", [(4, 4, 128), (6, 2, 128), (8, 2, 64), (4, 4, 64)])
 @pytest.mark.parametrize("n,start", [(3, 0), (33, 530)])

@@ -829,17 +829,20 @@ struct AttnPrep {
 // A row's reference lies 10 below its largest score (the weights are 2^10 p) and follows it once that is more than 15 above: a weight
 // fits f16 as long as its exponent, a difference of two floats that are near each other and so exact, stays below 16.
 constexpr float MQ_MOST = 15.f;
-template <int D, int QT, int KS, int NSUB = 4>
+// PREP: the rows as the prepared activation of the output projection instead (as tree_merge_kernel does): a workgroup has the neighbouring heads
+// of its 256-column chunks, G being a multiple of their number, and its row tiles go on over the rows that pad the activation. (512 rows
+// over 4096 keys, 32 / 8 heads of 128: 93.0 us for 91.4 and a launch of 6.3 that read the rows again.)
+template <int D, int QT, int KS, int NSUB = 4, bool PREP = false>
 __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *__restrict__ q, const _Float16 *__restrict__ pool,
                                                          const int32_t *__restrict__ table, const int32_t *__restrict__ kv_lens,
                                                          float *__restrict__ out, int query_len, int max_keys, int num_q_heads,
-                                                         int num_kv_heads, float scale) {
+                                                         int num_kv_heads, float scale, AttnPrep prep = AttnPrep()) {
     constexpr int NS = D / 32, NT = D / 16;
     const int kvh = blockIdx.x % num_kv_heads, nth = blockIdx.x / num_kv_heads, G = num_q_heads / num_kv_heads;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sub = wave % NSUB, ksub = wave / NSUB;  // which of the workgroup's NSUB (head, row group) pairs, which share of the blocks
-    const int row_groups = (query_len + 16 * QT - 1) / (16 * QT);
+    const int row_groups = ((PREP ? prep.mpad : query_len) + 16 * QT - 1) / (16 * QT);
     const bool idle = nth * NSUB + sub >= G * row_groups;  // (a wave without work walks no block; it still meets the others)
     const int combo = min(nth * NSUB + sub, G * row_groups - 1);
     const int head = kvh * G + combo % G, r0 = (combo / G) * 16 * QT;
@@ -1083,11 +1086,12 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
             }
         }
         __syncthreads();
-        if (ksub > 0) return;
+        if (!PREP && ksub > 0) return;
     }
-    if (idle) return;
+    if (!PREP && idle) return;
 #pragma unroll
     for (int t = 0; t < QT; t++) {
+        if (PREP && ksub > 0) break;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int row = 4 * g4 + i, qi = r0 + 16 * t + row;
@@ -1108,8 +1112,8 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
                 w[0] = 1.f;
             }
             const float inv = L > 0.f ? 1.f / L : 0.f;
-            if (qi >= query_len) continue;
-            float *op = out + (size_t)qi * qs + (size_t)head * D + c16;
+            if (!PREP && qi >= query_len) continue;
+            float *op = PREP ? nullptr : out + (size_t)qi * qs + (size_t)head * D + c16;
 #pragma unroll
             for (int e = 0; e < NT; e++) {
                 float acc = o[t][e][i] * w[0];
@@ -1117,8 +1121,33 @@ __global__ void __launch_bounds__(64 * NSUB * KS) paged_mq_kernel(const float *_
 #pragma unroll
                     for (int k2 = 1; k2 < KS; k2++) acc += s_o[k2 - 1][sub][t][e * 4 + i][lane] * w[k2];
                 }
-                op[16 * e] = acc * inv;
+                if (PREP) o[t][e][i] = acc * inv;
+                else op[16 * e] = acc * inv;
             }
+        }
+    }
+    if constexpr (PREP) {
+        constexpr int HEADS = 256 / D, ROWS = 16 * QT, PITCH = D + 4;  // heads of a chunk; floats of a head's row
+        static_assert(NSUB % HEADS == 0 && NSUB * ROWS * PITCH * 4 <= SMEM, "whole chunks that fit where the steps were");
+        float(*const s_y)[ROWS][PITCH] = (float(*)[ROWS][PITCH])smem;
+        __syncthreads();  // (the other shares' results have been read)
+        if (ksub == 0) {
+#pragma unroll
+            for (int t = 0; t < QT; t++)
+#pragma unroll
+                for (int e = 0; e < NT; e++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) s_y[sub][16 * t + 4 * g4 + i][16 * e + c16] = o[t][e][i];
+        }
+        __syncthreads();
+        for (int u = wave; u < NSUB / HEADS * ROWS; u += NSUB * KS) {
+            const int first = u / ROWS * HEADS, r = u % ROWS, c0 = nth * NSUB + first, row = c0 / G * ROWS + r, chunk = (kvh * G + c0 % G) / HEADS;
+            if (c0 >= G * row_groups || row >= prep.mpad) continue;
+            const bool real = row < query_len;
+            const float4 v = *(const float4 *)&s_y[first + lane / (D / 4)][r][lane % (D / 4) * 4];
+            const float y[4] = {real ? v.x : 0.f, real ? v.y : 0.f, real ? v.z : 0.f, real ? v.w : 0.f};
+            write_chunk(prep.pv, row, chunk, y, prep.mpad);
+            if (chunk == 0 && lane == 0) prep.pv.inv_scale[row] = real ? 1.f : 0.f;
         }
     }
 }
@@ -2030,21 +2059,31 @@ int vx_sdpa_paged_decode_split_supported(int pool_is_f16, int block_size, int nu
            ((head_dim == 80 || head_dim == 96) && G == 1);
 }
 
-int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *kv_pool, int pool_is_f16,
-                                    const int32_t *block_table, float *out, const int32_t *kv_lens, int num_blocks,
-                                    int block_size, int num_q_heads, int num_kv_heads, int head_dim, float scale,
-                                    int query_len) {
+// (the LDS-tiled kernel instead, to compare)
+static bool mq_lds_tiles() {
+    static const bool on = getenv("VEXEL_HIP_MQ_LDS_TILES") != nullptr;
+    return on;
+}
+
+int vx_sdpa_paged_multiquery_ffn_supported(int pool_is_f16, int block_size, int num_q_heads, int num_kv_heads, int head_dim, int query_len) {
+    return pool_is_f16 && block_size == HOT_BS && query_len >= 16 && (head_dim == 64 || head_dim == 128) && num_kv_heads > 0 &&
+           num_q_heads % num_kv_heads == 0 && num_q_heads / num_kv_heads % (256 / head_dim) == 0 && num_q_heads * head_dim <= 16 * 1024 && !mq_lds_tiles();
+}
+
+// ffn_k > 0: the rows as the prepared activation of a vx_decode_ffn whose widest activation has ffn_k columns, instead of out
+static int multiquery(vx_backend *be, const float *q, const void *kv_pool, int pool_is_f16, const int32_t *block_table, float *out,
+                      const int32_t *kv_lens, int num_blocks, int block_size, int num_q_heads, int num_kv_heads, int head_dim, float scale,
+                      int query_len, int ffn_k) {
     int rc = enter(be);
     if (rc) return rc;
-    VX_REQUIRE(q && kv_pool && block_table && out && kv_lens, "vx_sdpa_paged_decode_multiquery: null pointer");
+    VX_REQUIRE(q && kv_pool && block_table && (out || ffn_k > 0) && kv_lens, "vx_sdpa_paged_decode_multiquery: null pointer");
     VX_REQUIRE(num_blocks >= 1 && block_size >= 1 && query_len >= 0, "vx_sdpa_paged_decode_multiquery: bad counts");
     VX_REQUIRE(head_dim > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0, "vx_sdpa_paged_decode_multiquery: bad head counts");
     // Chunks of a prompt and verification rows over an F16 pool: the matrix-core kernels (16-token blocks: a tile of
     // 16 query rows per wave straight from the pool; other block sizes: K/V tiles of 32 keys staged in LDS for 64
     // queries). A handful of rows, other head sizes and float32 pools keep the one-workgroup-per-query kernel.
-    static const bool lds_tiles = getenv("VEXEL_HIP_MQ_LDS_TILES") != nullptr;  // (the LDS-tiled kernel instead, to compare)
     if (pool_is_f16 && query_len >= 16 && (head_dim == 64 || head_dim == 128) && ((uintptr_t)kv_pool % 16) == 0 &&
-        block_size == HOT_BS && ((uintptr_t)q % 16) == 0 && ((uintptr_t)out % 16) == 0 && !lds_tiles) {
+        block_size == HOT_BS && ((uintptr_t)q % 16) == 0 && ((uintptr_t)out % 16) == 0 && !mq_lds_tiles()) {
         constexpr int QT = 1;
         const int G = num_q_heads / num_kv_heads, combos = G * ceil_div(query_len, 16 * QT);
         // the blocks of a row tile shared out over 1, 2 or 4 waves: two waves per SIMD and more cover each other's
@@ -2053,6 +2092,20 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
         const int share = waves >= 2048 ? 1 : (waves >= 1024 ? 2 : 4);
         const _Float16 *pool = (const _Float16 *)kv_pool;
         const int max_keys = num_blocks * block_size;
+        if (ffn_k > 0) {
+            AttnPrep prep;
+            if (rc = prep_for_ffn(be, query_len, num_q_heads * head_dim, ffn_k, &prep.pv, &prep.mpad); rc) return rc;
+            const int padded = G * ceil_div(prep.mpad, 16 * QT);
+#define VX_MQ(DD, KK, NS)                                                                                                 \
+    if (head_dim == DD && share == KK)                                                                                    \
+        paged_mq_kernel<DD, QT, KK, NS, true><<<num_kv_heads * ceil_div(padded, NS), 64 * NS * KK, 0, be->stream>>>(         \
+            q, pool, block_table, kv_lens, nullptr, query_len, max_keys, num_q_heads, num_kv_heads, scale, prep);
+            VX_MQ(128, 1, 4) VX_MQ(128, 2, 4) VX_MQ(128, 4, 2) VX_MQ(64, 1, 4) VX_MQ(64, 2, 4) VX_MQ(64, 4, 4)
+#undef VX_MQ
+            VX_CHECK_LAUNCH();
+            prepared_for_ffn(be, query_len, num_q_heads, head_dim);
+            return VX_OK;
+        }
 #define VX_MQ(DD, KK, NS)                                                                                                 \
     if (head_dim == DD && share == KK)                                                                                    \
         paged_mq_kernel<DD, QT, KK, NS><<<num_kv_heads * ceil_div(combos, NS), 64 * NS * KK, 0, be->stream>>>(               \
@@ -2063,6 +2116,7 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
         VX_CHECK_LAUNCH();
         return VX_OK;
     }
+    VX_REQUIRE(out, "vx_sdpa_paged_multiquery_ffn: unaligned pointer");
     if (pool_is_f16 && query_len >= 16 && (head_dim == 64 || head_dim == 128) && ((uintptr_t)kv_pool % 8) == 0) {
         PagedSrc src = {(const _Float16 *)kv_pool, block_table, kv_lens, block_size};
         dim3 grid(ceil_div(query_len, FA_BQ), num_q_heads);
@@ -2089,6 +2143,23 @@ int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *
     p.block_size = block_size;
     p.kv_lens = kv_lens;
     return run_generic(be, p, query_len);
+}
+
+int vx_sdpa_paged_decode_multiquery(vx_backend *be, const float *q, const void *kv_pool, int pool_is_f16,
+                                    const int32_t *block_table, float *out, const int32_t *kv_lens, int num_blocks,
+                                    int block_size, int num_q_heads, int num_kv_heads, int head_dim, float scale,
+                                    int query_len) {
+    return multiquery(be, q, kv_pool, pool_is_f16, block_table, out, kv_lens, num_blocks, block_size, num_q_heads, num_kv_heads, head_dim, scale,
+                      query_len, 0);
+}
+
+int vx_sdpa_paged_multiquery_ffn(vx_backend *be, const float *q, const void *kv_pool, int pool_is_f16, const int32_t *block_table,
+                                 const int32_t *kv_lens, int num_blocks, int block_size, int num_q_heads, int num_kv_heads, int head_dim,
+                                 float scale, int query_len, int ffn_k) {
+    VX_REQUIRE(ffn_k > 0 && vx_sdpa_paged_multiquery_ffn_supported(pool_is_f16, block_size, num_q_heads, num_kv_heads, head_dim, query_len),
+               "vx_sdpa_paged_multiquery_ffn: %d rows of %d / %d heads x %d", query_len, num_q_heads, num_kv_heads, head_dim);
+    return multiquery(be, q, kv_pool, pool_is_f16, block_table, nullptr, kv_lens, num_blocks, block_size, num_q_heads, num_kv_heads, head_dim, scale,
+                      query_len, ffn_k);
 }
 
 int vx_sdpa_paged_tree(vx_backend *be, const float *q, const void *kv_pool, int pool_is_f16,

@@ -1064,14 +1064,22 @@ int vh_prefill(vh_model *m, const int32_t *tokens, int n, int64_t seq_id, int st
     for (int l = 0; l < c.num_layers; l++) {
         const vh_layer_weights &w = m->layers[l];
         const bool attn_fused = later && attn_fusable(m, l);
+        const bool ffn_fused = tails_fusable && w.wo.data && w.w1.data && w.w2.data && w.w3.data &&
+                               vx_decode_ffn_supported(&w.wo, &w.w1, &w.w3, &w.w2);
+        const bool into_ffn = attn_fused && ffn_fused && (size_t)w.wo.k * 4 <= 64 * 1024 &&
+                              vx_sdpa_paged_multiquery_ffn_supported(c.kv_fp16, c.block_size, c.num_heads, c.num_kv_heads, c.head_dim, n);
         if (attn_fused) {
             const vh_layer_extras &e = m->extras[l];
             VXC(vx_decode_attn_qkv_ex(be, x, w.attn_norm, c.eps, chained ? 1 : 0, &w.wq, &w.wk, &w.wv, e.wq_bias, e.wk_bias,
                                       e.wv_bias, n, d_pos, d_slot, m->kv[l], c.kv_fp16, c.num_heads, c.num_kv_heads, c.head_dim,
                                       c.block_size, c.rope_theta, m->arch.rope_dim, m->arch.rope_neox, q));
             chained = false;
-            VXC(vx_sdpa_paged_decode_multiquery(be, q, m->kv[l], c.kv_fp16, d_bt, attn, d_kvl, (int)table.size(),
-                                                c.block_size, c.num_heads, c.num_kv_heads, c.head_dim, scale, n));
+            if (into_ffn)  // (the rows as that half's prepared activation)
+                VXC(vx_sdpa_paged_multiquery_ffn(be, q, m->kv[l], c.kv_fp16, d_bt, d_kvl, (int)table.size(), c.block_size, c.num_heads,
+                                                 c.num_kv_heads, c.head_dim, scale, n, std::max(w.w1.n, w.wo.n)));
+            else
+                VXC(vx_sdpa_paged_decode_multiquery(be, q, m->kv[l], c.kv_fp16, d_bt, attn, d_kvl, (int)table.size(),
+                                                    c.block_size, c.num_heads, c.num_kv_heads, c.head_dim, scale, n));
         } else if (first && attn_fusable(m, l)) {
             const vh_layer_extras &e = m->extras[l];
             VXC(vx_prefill_attn_qkv(be, x, w.attn_norm, c.eps, chained ? 1 : 0, &w.wq, &w.wk, &w.wv, e.wq_bias, e.wk_bias,
@@ -1136,10 +1144,9 @@ int vh_prefill(vh_model *m, const int32_t *tokens, int n, int64_t seq_id, int st
                 VXC(vx_sdpa_prefill(be, q, k, v, attn, n, c.num_heads, c.num_kv_heads, c.head_dim, scale));
             }
         }
-        if (tails_fusable && w.wo.data && w.w1.data && w.w2.data && w.w3.data &&
-            vx_decode_ffn_supported(&w.wo, &w.w1, &w.w3, &w.w2)) {                      // block.go:981-1077
+        if (ffn_fused) {                                                                   // block.go:981-1077
             const float *next_norm = l + 1 < c.num_layers && (later || first) && attn_fusable(m, l + 1) ? m->layers[l + 1].attn_norm : nullptr;
-            VXC(vx_decode_ffn(be, attn, x, &w.wo, w.ffn_norm, c.eps, &w.w1, &w.w3, &w.w2, n, next_norm));
+            VXC(vx_decode_ffn(be, into_ffn ? nullptr : attn, x, &w.wo, w.ffn_norm, c.eps, &w.w1, &w.w3, &w.w2, n, next_norm));
             chained = next_norm != nullptr;
         } else if (m->general) {
             VHC(g_tail(m, l, x, norm, attn, gate, up, n));

@@ -109,6 +109,8 @@ SIGNATURES = {
     "vx_sdpa_paged_tree_rows_per_entry": (_i, [_i, _i, _i, _i, _i]),
     "vx_sdpa_paged_tree_batched": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i]),
     "vx_sdpa_paged_tree_batched_ffn": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _i]),
+    "vx_sdpa_paged_multiquery_ffn_supported": (_i, [_i, _i, _i, _i, _i, _i]),
+    "vx_sdpa_paged_multiquery_ffn": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f, _i, _i]),
     "vx_rope_shift": (_i, [_vp, _vp, _i, _i, _i, _i, _f]),
     "vx_sample_rows": (_i, [_vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _vp]),
     "vx_paged_kv_copy_shifted": (_i, [_vp, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _f]),
