@@ -1589,6 +1589,25 @@ def test_multiquery_rows_as_the_next_call_takes_them(be, hq, hk, d, n, start):
     be.reset_pool()
 
 
+# the last rows prepared row by row, the first by chunks, padded and whole tiles, one wave a workgroup and four (32 and 16 chunks of 96 and 256 rows)
+@pytest.mark.parametrize("rows,k", [(64, 512), (65, 512), (96, 256), (97, 8192), (256, 4096), (257, 768)])
+def test_activations_prepared_by_rows_and_by_chunks(be, rows, k):
+    """The product against float64. An operand is off by at most 2^-22 of its chunk's (or row's) largest, which the factors from 2^-6 to 2^6 between
+    chunks leave below 2^-16 of the sums of magnitudes, and so is a float32 sum of k terms in slices of 1024 and fewer."""
+    rng = np.random.default_rng(rows + k)
+    n, fmt = 96, nx.FMT_Q8_0
+    a = (rng.uniform(0.5, 1.0, (rows, k)) * rng.choice([-1, 1], (rows, k))).astype(np.float32)
+    a *= np.repeat(2.0 ** rng.integers(-6, 7, (rows, k // 256)), 256, axis=1).astype(np.float32)
+    w = qz.random_quant(fmt, rng, n, k)
+    dw, do = be.upload(w), be.alloc(rows * n * 4)
+    be.prepare_act(be.upload(a), rows, k)
+    be.matmul_quant_prepared(fmt, dw, do, None, rows, n, k)
+    exact = nx.dequantize(fmt, w, n * k).reshape(n, k).astype(np.float64)
+    err = np.abs(be.download(do, (rows, n), np.float32) - a.astype(np.float64) @ exact.T)
+    assert np.all(err <= 2.0 ** -16 * (np.abs(a).astype(np.float64) @ np.abs(exact).T))
+    be.reset_pool()
+
+
 # a tile of rows; rows that pad the activation (48 and 36 of 64); one chunk of columns and several, of two heads and of four
 @pytest.mark.parametrize("hq,hk,d", [(4, 4, 128), (6, 2, 128), (8, 2, 64), (4, 4, 64)])
 @pytest.mark.parametrize("n,start", [(3, 0), (33, 530)])

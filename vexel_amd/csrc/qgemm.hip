@@ -1450,7 +1450,7 @@ __global__ void __launch_bounds__(64) chunk_merge_kernel(const float *__restrict
     if (c == 0 && lane == 0) pv.inv_scale[r] = r < M ? 1.f : 0.f;
 }
 
-//   a plain activation row by row and chunk by chunk, row factor 1 (big prompt chunks: see vx_prepare_act)
+//   a plain activation row by row and chunk by chunk, row factor 1 (more than 64 rows: see vx_prepare_act)
 __global__ void __launch_bounds__(256) chunk_plain_kernel(const float *__restrict__ a, int M, int K, PrepView pv, int Mpad) {
     const int c = blockIdx.x, r = wave_row(), lane = threadIdx.x & 63;
     float y[4] = {0.f, 0.f, 0.f, 0.f};
@@ -2117,10 +2117,12 @@ int vx_prepare_act(vx_backend *be, const float *a, int m, int k) {
     rc = prep_begin(be, m, k, &pv);
     if (rc) return rc;
     const int mpad = mpad_for(m);
-    // beyond 256 rows a wave per row and 256-column chunk (each chunk with its own power-of-two factor): many small
-    // workgroups instead of one of 1024 threads per row; up to there the row kernel, whose bits the decode paths share
-    if (m > 256)
-        chunk_plain_kernel<<<dim3(k / 256, mpad / 4), 256, 0, be->stream>>>(a, m, k, pv, mpad);
+    // beyond 64 rows a wave per row and 256-column chunk (each chunk with its own power-of-two factor): many small workgroups instead of one of 1024
+    // threads per row, which starts late and reduces twice (back to back, 77 and 256 rows of 4096 columns 5.0 and 6.7 -> 3.7 and 4.1 us, of 11008 7.7
+    // and 13.0 -> 4.3 and 7.7; a prompt of 77 rows on a 7B Q4_0 model 4860 -> 4813); up to there the row kernel, whose bits the decode paths share
+    const int waves = waves_per_group(k / 256, mpad);
+    if (m > 64)
+        chunk_plain_kernel<<<dim3(k / 256, mpad / waves), 64 * waves, 0, be->stream>>>(a, m, k, pv, mpad);
     else
         prepare_kernel<PREP_PLAIN, false><<<mpad, PREP_THREADS, 0, be->stream>>>(a, nullptr, nullptr, m, k, 0.f, pv, mpad);
     VX_CHECK_LAUNCH();
