@@ -3,6 +3,10 @@ copy dequantises to the reference's values bit for bit, the products match the C
 (backend/cpu/cpu.go:842-911) to float32 summation order on every cut of the matrix the planner makes, a row's bits
 do not depend on the batch it sits in (2 .. 32 rows; 33 .. 64 rows), and the fused decode blocks give the oracle's
 layer with packed weights."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -10,6 +14,7 @@ from oracle import numerics as nx
 from oracle import quantize as qz
 
 pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.fixture(scope="module")
@@ -349,7 +354,6 @@ def test_default_configuration_takes_the_kernels_the_benchmark_reports(be):
     """With no environment switch set, a packed matrix runs the streaming kernel at 2 .. 64 rows and the many-rows
     kernel beyond, one row the matrix-vector kernel, and an unpacked matrix the kernels over the GGUF rows: the paths
     bench.py times are the paths a default process takes."""
-    import os
     if [k for k in os.environ if k.startswith("VEXEL_HIP_")]:
         pytest.skip("a VEXEL_HIP_* switch is set: this is not the default configuration")
     rng = np.random.default_rng(21)
@@ -594,3 +598,40 @@ def test_streamed_qkv_rows_do_not_depend_on_the_batch(be, fmt):
     for p in list(dev) + [dx, dnw, dpos, dslots, dpool, dq]:
         be.free(p)
     be.reset_pool()
+
+
+def qkv_with_and_without_angles(rows_min):
+    """(In a process of its own, whose VEXEL_HIP_ROWS_MIN is rows_min.)"""
+    from vexel_amd.backend import HipBackend
+    be = HipBackend(0)
+    rng = np.random.default_rng(rows_min)
+    hq, hk, d, hidden, bs, nblocks, theta, eps, fmt = 4, 2, 64, 512, 16, 8, 10000.0, 1e-5, nx.FMT_Q8_0
+    dims = dict(wq=(hq * d, hidden), wk=(hk * d, hidden), wv=(hk * d, hidden))
+    qw = {n: be.qweight(fmt, be.upload(qz.random_quant(fmt, rng, *v)), *v) for n, v in dims.items()}
+    dnw, pool0 = be.upload(np.ones(hidden, dtype=np.float32)), np.zeros(nblocks * 2 * bs * hk * d, dtype=np.float16)
+    for rows in (rows_min - 1, rows_min, 32):
+        dx = be.upload(rng.standard_normal((rows, hidden)).astype(np.float32))
+        dpos, dslots = be.upload(np.arange(rows, dtype=np.int32) * 5), be.upload(rng.permutation(nblocks * bs)[:rows].astype(np.int32))
+        got = []
+        for table in (True, False):
+            dpool, dq = be.upload(pool0), be.alloc(rows * hq * d * 4)
+            if table:
+                be.rope_table_prepare(dpos, rows, d, theta)
+            else:
+                be.to_device(dpos, np.arange(rows, dtype=np.int32) * 5)   # (the table falls)
+            be.decode_attn_qkv(dx, dnw, eps, False, qw["wq"], qw["wk"], qw["wv"], rows, dpos, dslots, dpool, True, hq, hk, d, bs, theta, dq)
+            assert be.last_matmul_kernel() == ("qgemm_wave_kernel" if table or rows < rows_min else "qgemm_rows_kernel"), (rows, table)
+            got.append((be.download(dq, (rows, hq * d), np.float32), be.download(dpool, pool0.shape, np.float16).astype(np.float32)))
+        for a, b, rel in zip(*got, (2e-5, 2.0 ** -10)):               # (float32 sums in another order; rounded to f16)
+            assert np.abs(b).max() > 0 and np.all(np.abs(a - b) <= rel * np.abs(b).max())
+    be.close()
+
+
+@pytest.mark.parametrize("rows_min", [3, 17])
+def test_switch_for_many_rows_leaves_the_rows_that_are_finished_alone(rows_min):
+    """VEXEL_HIP_ROWS_MIN moves batches to a kernel that leaves sums, also where a step's table of angles lets the Q|K|V launch finish its rows: those
+    stay with the kernel that does."""
+    r = subprocess.run([sys.executable, "-c", "import test_gpu_stream_gemm as t; t.qkv_with_and_without_angles(%d)" % rows_min],
+                       cwd=os.path.dirname(os.path.abspath(__file__)), env=dict(os.environ, VEXEL_HIP_ROWS_MIN=str(rows_min), PYTHONPATH=ROOT),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]

@@ -2003,15 +2003,21 @@ int launch_gemm_fmt(vx_backend *be, int fmt, const Segs &segs, int N, float *out
             return VX_OK;
         }
     }
-    if (tiles_gemm_ok(be, fmt, segs.w, segs.n_end, 3, N, K, M)) {  // packed copies and a batch beyond the streaming kernel's
+    // An epilogue has no output beside it: what the streaming kernel does not take is for the wave-private one with the whole K, whatever the
+    // switches make of the kernels for many rows.
+    if (fin) {
+        const WavePlan whole = wave_plan(be, fmt, segs, N, K, M);
+        VX_REQUIRE(whole.r > 0 && whole.ks == 1, "Q|K|V of %d rows, %d x %d: no kernel finishes the rows", M, N, K);
+    }
+    if (!fin && tiles_gemm_ok(be, fmt, segs.w, segs.n_end, 3, N, K, M)) {  // packed copies and a batch beyond the streaming kernel's
         int ks = 1;
         const int mpad = mpad_for(M);
         const PrepView spv = prep_view(be, mpad, K);
         // (a pending 1/rms: this launch folds it into the plain row factors beside its own work, for whoever
         // consumes its K slices' sums)
         const bool fold = to_partials && be->prep_norm_k > 0;
-        const RowNorm fin = cur_row_norm(be);
-        int rc = tiles_gemm(be, fmt, segs.w, segs.n_end, 3, N, K, M, mpad, spv, out, residual, to_partials, &ks, fold ? &fin : nullptr);
+        const RowNorm pending = cur_row_norm(be);
+        int rc = tiles_gemm(be, fmt, segs.w, segs.n_end, 3, N, K, M, mpad, spv, out, residual, to_partials, &ks, fold ? &pending : nullptr);
         if (rc != VX_ERR_UNSUPPORTED) {
             if (rc) return rc;
             if (fold) be->prep_norm_k = 0;
@@ -2026,12 +2032,12 @@ int launch_gemm_fmt(vx_backend *be, int fmt, const Segs &segs, int N, float *out
             return VX_OK;
         }
     }
-    const WavePlan rp = rows_plan(be, fmt, segs, N, K, M);
+    const WavePlan rp = fin ? WavePlan{0, 1} : rows_plan(be, fmt, segs, N, K, M);
     if (rp.r > 0) {
         be->last_matmul = "qgemm_rows_kernel";
         return launch_gemm_rows_r<WQ8_0>(be, rp, segs, N, out, residual, to_partials, M, K, ks_out);
     }
-    const QkvEpi epi = epi_in ? *epi_in : QkvEpi{};  // (with an epilogue the caller has checked that the wave plan applies)
+    const QkvEpi epi = epi_in ? *epi_in : QkvEpi{};
     const WavePlan pl = wave_plan(be, fmt, segs, N, K, M);
     if (pl.r > 0) {
         be->last_matmul = "qgemm_wave_kernel";
