@@ -3,6 +3,9 @@ inputs. Integer/byte results (dequantised weights, scatter layout, argmax, packi
 compared bit-exactly; floating point within the stated tolerances."""
 import ctypes
 import math
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -12,6 +15,7 @@ from oracle import quantize as qz
 from oracle import host_logic as hl
 
 pytestmark = pytest.mark.gpu
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 FMTS = [nx.FMT_Q4_0, nx.FMT_Q8_0, nx.FMT_Q4_K, nx.FMT_Q6_K]
 FMTS_MFMA = FMTS + [nx.FMT_Q5_0, nx.FMT_Q5_K]      # the formats with matrix-vector and MFMA kernels
@@ -1606,6 +1610,34 @@ def test_activations_prepared_by_rows_and_by_chunks(be, rows, k):
     err = np.abs(be.download(do, (rows, n), np.float32) - a.astype(np.float64) @ exact.T)
     assert np.all(err <= 2.0 ** -16 * (np.abs(a).astype(np.float64) @ np.abs(exact).T))
     be.reset_pool()
+
+
+def small_chunk_beside_a_large_one(rows):
+    """-> what a product makes of a chunk of columns whose elements are 2^-60 of those in the chunk before, which meets weights of zero"""
+    from vexel_amd.backend import HipBackend
+    be = HipBackend(0)
+    rng = np.random.default_rng(rows)
+    n, k, fmt = 64, 512, nx.FMT_Q8_0
+    a = rng.uniform(0.5, 1.0, (rows, k)).astype(np.float32)
+    a[:, 256:] *= np.float32(2.0 ** -60)
+    w = qz.random_quant(fmt, rng, n, k).reshape(n, 2, -1)
+    w[:, 0] = 0
+    do = be.alloc(rows * n * 4)
+    be.prepare_act(be.upload(a), rows, k)
+    be.matmul_quant_prepared(fmt, be.upload(w), do, None, rows, n, k)
+    got = be.download(do, (rows, n), np.float32).astype(np.float64) * 2.0 ** 60
+    be.close()
+    return got
+
+
+@pytest.mark.parametrize("switch,rows,by_rows", [(False, 64, True), (False, 65, False), (True, 65, True), (True, 256, True), (True, 257, False)])
+def test_switch_for_preparing_by_rows(switch, rows, by_rows):
+    """VEXEL_HIP_PREP_ROW_KERNELS: up to 256 rows a factor per row, beside which so small a chunk is nothing; else one per chunk."""
+    code = "import sys, numpy as np, test_gpu_kernels as t; sys.exit(7 if np.any(t.small_chunk_beside_a_large_one(%d)) else 8)" % rows
+    env = {k: v for k, v in os.environ.items() if not k.startswith("VEXEL_HIP_")}
+    env.update(PYTHONPATH=ROOT, **({"VEXEL_HIP_PREP_ROW_KERNELS": "1"} if switch else {}))
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.abspath(__file__)), env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == (8 if by_rows else 7), r.stderr[-2000:]
 
 
 # a tile of rows; rows that pad the activation (48 and 36 of 64); one chunk of columns and several, of two heads and of four

@@ -453,6 +453,17 @@ def test_scan_step_is_the_separate_calls(be, rows, channels, states, rank, attn)
     bit those of the four calls (row tiles of 16 with one over, channels that end inside a workgroup's 32 and inside a step of the
     map's inputs, one to two steps of the rank for a wave), for sequences at position 0, within the first taps and later, with leavings of an earlier owner in every slot. So is attention beside it (in the same launch for heads of 112 and 128, of
     one piece and, where a sequence is long, of several; in its own for 64)."""
+    scan_step_both_ways(be, rows, channels, states, rank, attn, 20)
+
+
+# tables up to which the joint launch stays within 64 KiB of LDS, and one entry more; the largest that attention keeps there, and one more
+@pytest.mark.parametrize("bias_len", [2912, 2913, 3072, 3073])
+def test_scan_step_beside_attention_with_a_large_table(be, bias_len):
+    """Attention's table of four heads a group in LDS beside what the scan's workgroups keep there."""
+    scan_step_both_ways(be, 17, 2048, 16, 64, (16, 4, 128), bias_len)
+
+
+def scan_step_both_ways(be, rows, channels, states, rank, attn, bias_len):
     from vexel_amd.backend import VxAttnArgs, VxScanStepArgs
     rng = np.random.default_rng(rows + channels)
     k, dt_k, pad, taps, n16 = -(-channels // 64) * 64, -(-rank // 64) * 64, 16, 4, -(-channels // 16) * 16
@@ -481,7 +492,7 @@ def test_scan_step_is_the_separate_calls(be, rows, channels, states, rank, attn)
         tables = Batch(be, [s + 1 for s in start], [1] * rows, slots=slots)
         pool = up(be, rng.standard_normal((tables.pool_blocks, 2 * kv_heads * dim * BS)), BF16)
         q = up(be, rng.standard_normal((rows, 2 * heads * dim)), BF16)
-        table = be.upload(rng.standard_normal((heads, 20)).astype(np.float32))
+        table = be.upload(rng.standard_normal((heads, bias_len)).astype(np.float32))
     for fused in (True, False):
         state, hist = be.upload(left), up(be, left_c, BF16)
         outs = []
@@ -498,7 +509,7 @@ def test_scan_step_is_the_separate_calls(be, rows, channels, states, rank, attn)
             if attn:
                 seen = blank(be, (rows, heads * dim), BF16)
                 at = VxAttnArgs()
-                at.heads, at.kv_heads, at.k_dim, at.v_dim, at.scale, at.bias, at.bias_len = heads, kv_heads, dim, dim, dim ** -0.5, table, 20
+                at.heads, at.kv_heads, at.k_dim, at.v_dim, at.scale, at.bias, at.bias_len = heads, kv_heads, dim, dim, dim ** -0.5, table, bias_len
                 at.q, at.ldq, at.gate, at.ldg, at.pool, at.out_scale = q, 2 * heads * dim, q + heads * dim * 2, 2 * heads * dim, pool, 0.7
                 at.out, at.ldo = seen, heads * dim
             if fused:

@@ -2100,6 +2100,12 @@ int finalize_row_norm(vx_backend *be) {
     return VX_OK;
 }
 
+// VEXEL_HIP_PREP_ROW_KERNELS=1 (measurements): prepares by rows where they once were.
+bool prep_row_kernels() {
+    static const bool on = getenv("VEXEL_HIP_PREP_ROW_KERNELS") != nullptr;
+    return on;
+}
+
 int run_prepared(vx_backend *be, int fmt, const void *b, float *out, const float *residual, int m, int n, int k) {
     Segs segs;
     segs.w[0] = segs.w[1] = segs.w[2] = (const uint8_t *)b;
@@ -2127,7 +2133,7 @@ int vx_prepare_act(vx_backend *be, const float *a, int m, int k) {
     // threads per row, which starts late and reduces twice (back to back, 77 and 256 rows of 4096 columns 5.0 and 6.7 -> 3.7 and 4.1 us, of 11008 7.7
     // and 13.0 -> 4.3 and 7.7; a prompt of 77 rows on a 7B Q4_0 model 4860 -> 4813); up to there the row kernel, whose bits the decode paths share
     const int waves = waves_per_group(k / 256, mpad);
-    if (m > 64)
+    if (m > (prep_row_kernels() ? 256 : 64))
         chunk_plain_kernel<<<dim3(k / 256, mpad / waves), 64 * waves, 0, be->stream>>>(a, m, k, pv, mpad);
     else
         prepare_kernel<PREP_PLAIN, false><<<mpad, PREP_THREADS, 0, be->stream>>>(a, nullptr, nullptr, m, k, 0.f, pv, mpad);
@@ -2307,11 +2313,10 @@ static Segs make_segs(const vx_qweight *const *ws, int nw, int *ntot) {
 }
 
 // The chunk-parallel prepares (a wave per row and 256-column chunk) cover decode batches, prompt chunks and trees of
-// up to 512 rows; larger ones keep the one-workgroup-per-row kernels. VEXEL_HIP_PREP_ROW_KERNELS=1 (measurements):
-// those from 65 rows on, as before the many-rows GEMM folded the pending 1/rms in.
+// up to 512 rows; larger ones keep the one-workgroup-per-row kernels. With the switch those from 65 rows on, as before the
+// many-rows GEMM folded the pending 1/rms in.
 bool chunk_prepare_ok(int rows, int k) {
-    static const bool row_kernels = getenv("VEXEL_HIP_PREP_ROW_KERNELS") != nullptr;
-    return mpad_for(rows) <= (row_kernels ? 64 : VX_PREP_SYNC_ROWS) && k / 256 <= VX_PREP_SYNC_CHUNKS;
+    return mpad_for(rows) <= (prep_row_kernels() ? 64 : VX_PREP_SYNC_ROWS) && k / 256 <= VX_PREP_SYNC_CHUNKS;
 }
 
 extern "C++" {
