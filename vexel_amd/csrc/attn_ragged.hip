@@ -406,7 +406,8 @@ __global__ void __launch_bounds__(256, VD <= 8 && MAPS * KD <= 6 ? 2 : 1) decode
 
 // The same launch with the scan branch's second half (scan_step.h) behind it: the two read the same projection and write side by side, and
 // either is a chain of trips to memory that leaves most of the chip idle. Attention, the longer of the two, has the first workgroups. 32 sequences of
-// 16 / 4 heads x 128 beside 4096 channels x 16 states: 9.7 us and 9.2 us one behind the other, 12.7 together.
+// 16 / 4 heads x 128 beside 4096 channels x 16 states: 9.7 us and 9.2 us one behind the other, 12.7 together. (A large bias table and what the scan keeps
+// in LDS are 66.5 KiB together; a workgroup may have 160, and two still fit a compute unit, which is what their registers allow.)
 template <int KD, int VD>
 __global__ void __launch_bounds__(256, 2) attn_scan_kernel(Args a, StepArgs s, int gx, int gy, int n_attn, int scan_x) {
     extern __shared__ float s_dyn[];
