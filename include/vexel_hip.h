@@ -66,7 +66,8 @@ void vx_reset_pool(vx_backend *be);
 int vx_to_device(vx_backend *be, void *dst, const void *src_host, size_t bytes);
 int vx_to_host(vx_backend *be, void *dst_host, const void *src, size_t bytes);
 /* vx_to_host of n ranges with one wait; a null src or zero bytes is left out. Everything enqueued before is done when either returns (unless
- * there was nothing to bring). */
+ * there was nothing to bring). The calling thread does not sleep meanwhile: these two and vx_sync keep a core busy for as long as the
+ * device takes. */
 int vx_to_host_many(vx_backend *be, int n, void *const *dst_host, const void *const *src, const size_t *bytes);
 /* A hint, ahead of the work whose results a later vx_to_host_many will bring: threads of the backend make the destinations' pages
  * (large ordinary memory only) while the caller enqueues it. The memory stays valid until vx_to_host_forget has returned, which

@@ -144,8 +144,9 @@ static Mover *mover_of(vx_backend *be) {
     return be->mover;
 }
 
-// A small download. The runtime's takes a copy of its own for every range, and its wait for the stream falls asleep behind work of some 40 us,
-// where waking up takes another 15 - 20. One launch of send_kernel instead, into the pinned megabyte's slots, and the caller looks at its marks: 4
+// A small download. The runtime's takes a copy of its own for every range, and its wait for the stream comes back 15 - 20 us late behind more than six
+// launches. One launch of send_kernel instead, into the pinned megabyte's slots, and the caller looks at its marks, which keeps its core busy as the
+// runtime's wait does (either takes as much processor time as it lasts, behind 5 us of work and behind 13 ms): 4
 // bytes behind 0, 1, 6, 8 and 20 short kernels 12.7, 15.8, 30, 62 and 106 us -> 8.9, 12, 27, 33 and 68, 128 KB behind 1, 8 and 20 of them 27, 65 and
 // 105 -> 17, 38 and 74 (behind none, where the runtime copies at once, 13.7 -> 14.4), all eight slots of 64 KiB 40, 102 -> 38, 96 behind 1 and 20.
 // VX_ERR_UNSUPPORTED, with nothing done, where a range is nothing that a kernel can read or the ranges need more slots.
