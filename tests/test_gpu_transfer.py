@@ -3,6 +3,7 @@ of pieces, straight to pinned memory) and staged uploads, byte for byte."""
 import ctypes as C
 import mmap
 import os
+import time
 
 import numpy as np
 import pytest
@@ -86,6 +87,38 @@ def test_small_download_by_marks(be, sizes):
             assert np.array_equal(o[1:-1], want[x:x + s]) and o[0] == 0 and o[-1] == 0, (i, x)
     for p in (da, db, dc):
         be.free(p)
+
+
+# both sides of where the runtime's copy takes over, from addresses of every alignment, with and without work ahead
+@pytest.mark.parametrize("ahead", [0, 9])
+@pytest.mark.parametrize("off", [0, 4, 1, 2, 3])
+@pytest.mark.parametrize("size", [1, 3, 7, 4 * KB, 4 * KB + 1, 16 * KB, 16 * KB + 3, 64 * KB + 2, 512 * KB - 64])
+def test_small_download_with_and_without_work_ahead(be, size, off, ahead):
+    rng = np.random.default_rng(size + off)
+    a, b = (rng.integers(0, 256, size + 16, dtype=np.uint8) for _ in range(2))
+    da, db, dc = be.upload(a, permanent=True), be.upload(b, permanent=True), be.upload(a, permanent=True)
+    out = np.zeros(size + 2, dtype=np.uint8)
+    for turn in range(3):
+        be.sync()
+        for k in range(ahead):                        # (the last copy is of b)
+            be.copy_buffer(da if k % 2 else db, 0, dc, 0, size + 16)
+        be.call("vx_to_host", out.ctypes.data + 1, int(dc) + off, size)
+        assert np.array_equal(out[1:-1], (b if ahead else a)[off:off + size]) and out[0] == 0 and out[-1] == 0
+    for p in (da, db, dc):
+        be.free(p)
+
+
+def test_small_download_of_a_stream_at_rest_from_any_address(be):
+    """64 KiB with nothing ahead take as long from an odd address as from an aligned one (byte by byte in a kernel it was 2.6 times as long)."""
+    d = be.alloc_permanent(1 * MB)
+    out, took = np.zeros(64 * KB, dtype=np.uint8), {0: [], 1: []}
+    for off in [0, 1] * 40:
+        be.sync()
+        t = time.perf_counter()
+        be.call("vx_to_host", out.ctypes.data, int(d) + off, out.size)
+        took[off].append(time.perf_counter() - t)
+    assert np.median(took[1]) < 1.5 * np.median(took[0]), {k: np.median(v) * 1e6 for k, v in took.items()}
+    be.free(d)
 
 
 def test_staged_uploads(be):

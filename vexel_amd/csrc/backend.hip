@@ -15,13 +15,18 @@ void set_error(const char *fmt, ...) {
     va_end(ap);
 }
 
-int enter(vx_backend *be) {
+int enter_to_wait(vx_backend *be) {
     if (!be) {
         set_error("null backend");
         return VX_ERR_INVALID;
     }
     VX_CHECK_HIP(hipSetDevice(be->device));
     return VX_OK;
+}
+
+int enter(vx_backend *be) {
+    if (be) be->at_rest.store(false, std::memory_order_relaxed);
+    return enter_to_wait(be);
 }
 
 int ensure_ws(vx_backend *be, void **ptr, size_t *cap, size_t bytes, const char *what) {
@@ -221,10 +226,11 @@ int vx_to_device(vx_backend *be, void *dst, const void *src_host, size_t bytes) 
 }
 
 int vx_sync(vx_backend *be) {
-    int rc = enter(be);
+    int rc = enter_to_wait(be);
     if (rc) return rc;
     VX_REQUIRE(!be->capturing, "vx_sync during graph capture");
     VX_CHECK_HIP(hipStreamSynchronize(be->stream));
+    be->at_rest.store(true, std::memory_order_relaxed);
     return VX_OK;
 }
 

@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <stdio.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <unordered_map>
@@ -140,6 +141,7 @@ struct vx_backend {
     size_t stage_used = 0;       // of its part for staged uploads: what the stream may still read
     std::mutex stage_mu;         // (its parts are shared by the threads that call)
     uint64_t note_mark = 0;      // the last mark of a small download (no mark is ever used again)
+    std::atomic<bool> at_rest{false};  // no call that may enqueue since one saw the stream done (a hint: where it is wrong a download is slower)
     vx::Mover *mover = nullptr;  // large downloads (transfer.hip), from the first one on
 
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -186,6 +188,8 @@ void mover_destroy(Mover *m);
 
 // Makes be->device current on the calling thread (Go moves goroutines across OS threads).
 int enter(vx_backend *be);
+// The same of a call that enqueues nothing which outlasts it.
+int enter_to_wait(vx_backend *be);
 // Ensures a library scratch buffer holds at least `bytes`; fails during capture if it must grow.
 int ensure_ws(vx_backend *be, void **ptr, size_t *cap, size_t bytes, const char *what);
 // Looks up, once per backend and with its device current, where that device keeps the fixed partial-sum area of

@@ -30,6 +30,10 @@ __device__ __forceinline__ void copy_bytes(char *dst, const char *src, uint32_t 
     } else if ((at & 3) == 0) {
         for (uint32_t k = tid; k < n / 4; k += threads) ((uint32_t *)dst)[k] = ((const uint32_t *)src)[k];
         done = n / 4 * 4;
+    } else if (((uintptr_t)dst & 3) == 0) {  // (the two words that hold a word's bytes; of memory that begins and ends on words)
+        const uint32_t *words = (const uint32_t *)((uintptr_t)src & ~(uintptr_t)3), off = (uintptr_t)src & 3;
+        for (uint32_t k = tid; k < n / 4; k += threads) ((uint32_t *)dst)[k] = __builtin_amdgcn_alignbyte(words[k + 1], words[k], off);
+        done = n / 4 * 4;
     }
     for (uint32_t k = done + tid; k < n; k += threads) dst[k] = src[k];
 }
@@ -148,15 +152,28 @@ static Mover *mover_of(vx_backend *be) {
 // launches. One launch of send_kernel instead, into the pinned megabyte's slots, and the caller looks at its marks, which keeps its core busy as the
 // runtime's wait does (either takes as much processor time as it lasts, behind 5 us of work and behind 13 ms): 4
 // bytes behind 0, 1, 6, 8 and 20 short kernels 12.7, 15.8, 30, 62 and 106 us -> 8.9, 12, 27, 33 and 68, 128 KB behind 1, 8 and 20 of them 27, 65 and
-// 105 -> 17, 38 and 74 (behind none, where the runtime copies at once, 13.7 -> 14.4), all eight slots of 64 KiB 40, 102 -> 38, 96 behind 1 and 20.
-// VX_ERR_UNSUPPORTED, with nothing done, where a range is nothing that a kernel can read or the ranges need more slots.
+// 105 -> 17, 38 and 74, all eight slots of 64 KiB 40, 102 -> 38, 96 behind 1 and 20.
+// The runtime's is the sooner one where nothing is ahead and one range comes that is long for a workgroup a slot (64, 128 and 512 KiB 12.3, 15.0 and 30.1 us
+// against 16.8, 18.6 and 33.7; 16 KiB 14.3 and 14.1; from an address that is no multiple of 16, by words, 16 KiB 14.2 and 15.3, 64 KiB 12.4 and 22.8). Whether
+// something is ahead is not asked of the stream: the question costs it 12 us.
+// VX_ERR_UNSUPPORTED, with nothing done, for such a one, where a range is nothing that a kernel can read, and where the ranges need more slots.
 static int download_noted(vx_backend *be, int n, void *const *dst, const void *const *src, const size_t *bytes) {
     constexpr int SLOTS = (int)(DOWN_BYTES / Mover::SENT_SLOT);
+    constexpr size_t LONG = 16 << 10, LONG_APART = 4 << 10;
+    int ranges = 0;
+    size_t slots = 0;
+    bool is_long = false;
+    for (int i = 0; i < n; i++) {
+        if (!src[i] || bytes[i] == 0) continue;
+        ranges++, slots += (bytes[i] + Mover::SENT_SLOT - 1) / Mover::SENT_SLOT;
+        is_long = is_long || bytes[i] > ((uintptr_t)src[i] % 16 == 0 ? LONG : LONG_APART);
+    }
+    if (slots > SLOTS || (ranges == 1 && is_long && be->at_rest.load(std::memory_order_relaxed))) return VX_ERR_UNSUPPORTED;
     SendArgs a = {};
     char *to[SLOTS];
     for (int i = 0; i < n; i++) {
         if (!src[i] || bytes[i] == 0) continue;
-        if (a.count + (int)((bytes[i] + Mover::SENT_SLOT - 1) / Mover::SENT_SLOT) > SLOTS || !device_memory(be, src[i], bytes[i])) return VX_ERR_UNSUPPORTED;
+        if (!device_memory(be, src[i], bytes[i])) return VX_ERR_UNSUPPORTED;
         for (size_t at = 0; at < bytes[i]; at += Mover::SENT_SLOT, a.count++) {
             a.src[a.count] = (const char *)src[i] + at, a.bytes[a.count] = (uint32_t)std::min(Mover::SENT_SLOT, bytes[i] - at);
             to[a.count] = (char *)dst[i] + at;
@@ -258,17 +275,20 @@ using namespace vx;
 extern "C" {
 
 int vx_to_host_many(vx_backend *be, int n, void *const *dst_host, const void *const *src, const size_t *bytes) {
-    int rc = enter(be);
+    int rc = enter_to_wait(be);
     if (rc) return rc;
     if (n == 0) return VX_OK;
     VX_REQUIRE(n > 0 && dst_host && src && bytes, "vx_to_host: bad arguments");
     VX_REQUIRE(!be->capturing, "vx_to_host during graph capture");
+    bool any = false;
+    for (int i = 0; i < n; i++) any = any || (src[i] && bytes[i] > 0);
     try {
         rc = download(be, n, dst_host, src, bytes);
     } catch (...) {
         set_error("vx_to_host: out of host memory");
         return VX_ERR_OOM;
     }
+    if (rc == VX_OK && any) be->at_rest.store(true, std::memory_order_relaxed);
     return rc;
 }
 
@@ -304,7 +324,7 @@ void vx_to_host_forget(vx_backend *be, int token) {
 }
 
 int vx_to_host(vx_backend *be, void *dst_host, const void *src, size_t bytes) {
-    int rc = enter(be);
+    int rc = enter_to_wait(be);
     if (rc) return rc;
     if (!src || bytes == 0) return VX_OK;
     return vx_to_host_many(be, 1, &dst_host, &src, &bytes);
