@@ -934,6 +934,8 @@ struct K3_Q6_K {  // share (n, a, h): low and high nibbles of ql[64 n + 32 a + 1
 // neighbouring threads, half a run each, which rows of up to MV3_QUARTERS elements take in one turn; by a thread a share three of the
 // four waves of a row of 2048 stand by. (Longer rows: by two threads a share 1 % of a 7B step slower, its products wait for weights.)
 // Q4_0 in a step, us: 2560 x 2048 5.3 -> 4.65, 11264 x 2048 8.2 -> 7.3, 2048 x 2048 4.1 the same.
+// Back to back, 1024 to 2048 elements: Q4_0 and Q8_0 1 - 9 % shorter up to 16384 rows (but 11264 x 1536 of Q8_0, 6.4 -> 6.75); K-quants 3 - 5 % at 2560 rows,
+// beyond from 4 % longer (14336 and 32000 rows of Q4_K, 32000 of Q5_K) to 7 % shorter.
 constexpr int MV3_QUARTERS = MV_THREADS / 4 * 32;
 template <class F, bool QUARTERS>
 __device__ __forceinline__ void matvec3(const MvArgs p, const int n_passes, const int block, const int blocks) {
